@@ -36,6 +36,27 @@ using fvp::set_error;
 
 struct fvp_schur;
 
+// Pattern tables of a factorisation (see bj_factor), the rows as level-ordered
+// slots: per slot its record, per L entry the position of its pivot u_kk, and
+// the byte offsets of the u_kj that update each entry of the row.
+struct FactorTab {
+    DevBuf<uint4> slot, out;
+    DevBuf<unsigned> piv;
+    DevBuf<uint2> off;
+    int nc = 1;  // longest row in entries, in units of 16
+    void release() { slot.release(); out.release(); piv.release(); off.release(); }
+};
+
+// One triangle of the one-workgroup ILU(0) solve (see ilu0_solve)
+struct IluTri {
+    DevBuf<int> pptr;                  // pieces: first slot of each, then the slot count
+    DevBuf<unsigned> row;              // per slot: row | entries << 16
+    DevBuf<unsigned short> col;        // per slot: o_win columns
+    DevBuf<double> val;                // the current factor: per slot its o_win entries, then (U) the slots' inverted pivots
+    int npieces = 0, nslots = 0;
+    void release() { pptr.release(); row.release(); col.release(); val.release(); }
+};
+
 struct fvp_csr {
     int device = 0;
     hipStream_t stream = nullptr, own_stream = nullptr;
@@ -60,26 +81,28 @@ struct fvp_csr {
     int factor_mode = -1;                   // staging form of the last block factorisation (bj_factor)
     DevBuf<int> b_roff, b_rowid, b_own;     // per block: first local row; global row of each local row; owned range
     DevBuf<double> b_zn2;                   // per block: its share of ||z||^2 of the last scaled solve
-    DevBuf<int> b_ia, b_src, b_diag;        // row pointers into the block arrays, source entry, diagonal position
-    DevBuf<unsigned short> b_ja;            // local column
+    DevBuf<int> b_ia, b_src;                // row pointers into the block arrays, source entry
     DevBuf<double> b_lu;
     DevBuf<float> b_lu32;                   // FP32 factor (FVP_PRECON_BJILU0_F32)
-    DevBuf<int> b_lev_l, b_lev_u;           // per block: level pointer range [b_lev[b], b_lev[b+1]) into *_lptr
-    DevBuf<int> b_lptr_l, b_lptr_u;         // level -> rows range in *_rows
-    DevBuf<unsigned short> b_rows_l, b_rows_u;  // local rows grouped by level
-    DevBuf<unsigned> fac_rec, fac_pair;     // factorisation: per entry its pair record (2 words), the pairs
-    DevBuf<long> fac_pbase;                 // per block: its first pair
+    FactorTab fac;                          // block factorisation (bj_factor), its slots the s_lptr_l order
+    // global ILU(0) in one workgroup: its factor tables, and per triangle the
+    // solve's pieces and padded row windows (see ilu0_solve)
+    bool one = false;
+    FactorTab ofac;
+    DevBuf<int> o_fptr;                     // {0, n}, {0, pieces}, then the factorisation's pieces of slots
+    IluTri otri[2];
+    int o_threads = 64, o_win = 0;
+    size_t o_lds = 0;
     // the solve's levels: the factor's levels cut into pieces of at most 32 rows
     DevBuf<int> s_lev_l, s_lev_u, s_lptr_l, s_lptr_u;
     int s_levmax_l = 0, s_levmax_u = 0;
     int s_maxslots = 0;                     // most slots of one block's triangle
     // packed solve layout per triangle (see bj_solve): per slot its meta word
-    // pair, per block its entry base, per entry its source in b_lu (-1:
-    // padding) and local column, the values of the current factor; per U slot
-    // the source of its diagonal and the inverted diagonal
+    // pair, per block its entry base, per entry its local column (0-valued
+    // entries pad odd rows) and the current factor's value, which bj_factor
+    // writes; per U slot the inverted diagonal
     DevBuf<unsigned> meta_l, meta_u;
     DevBuf<long> ebase_l, ebase_u;
-    DevBuf<int> esrc_l, esrc_u, dsrc;
     DevBuf<unsigned short> col_l, col_u;
     DevBuf<double> val_l, val_u, dinv;
     DevBuf<float> val32_l, val32_u, dinv32;
@@ -614,89 +637,281 @@ constexpr int kBjFactorThreads = 512;
 // wavefront's accesses in issue order; no wait for outstanding memory loads)
 __device__ __forceinline__ void wave_lds_order() { asm volatile("" ::: "memory"); }
 
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+// workgroup barrier for LDS data: waits for LDS accesses only, so global loads
+// issued ahead stay in flight across it
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
 }
 
-// The update pairs of the factorisation are precomputed from the pattern: for
-// the L entry e = (i, k) of a block, rec[e] = {first pair, count | pos(u_kk) << 16}
-// and each pair packs the block positions of u_kj (low half) and a_ij (high
-// half) for the columns j > k that rows i and k share.  A group of kBjGroup
-// lanes factors one row (IKJ order: for each L entry in column order,
-// l_ik = a_ik u_kk^-1, then a_ij -= l_ik u_kj over the entry's pairs, one pair
-// per lane); kBjFactorThreads / kBjGroup rows of a level are in flight per
-// workgroup.  The records of a row are held in the group's registers and the
-// pairs of the next L entry are loaded while the current one is applied.
-// STAGED: the block's values are staged in LDS; otherwise the factorisation
-// works in place on the block's values in memory.
+// Factorisation (IKJ order).  Rows of one level only need rows of earlier
+// levels, so when a level begins every u_kj that its rows use is final: a group
+// of kBjGroup lanes holds one row in registers (entry j in lane j mod 16), loads
+// all the u_kj and pivots of its L entries in one round, and runs the row's
+// chain (l_ik = a_ik u_kk^-1, then a_ij -= l_ik u_kj for the columns both rows
+// have) in registers with broadcasts inside the group.  What bounds it is the
+// level chain (one round of loads, the row's chain, one barrier per level) and,
+// inside it, instruction issue (about 250 per wavefront and level), so everything
+// that does not depend on values is loaded ahead (slot records two levels, pivot
+// positions, offsets and the row's own values one), and L entries that no row of
+// a wavefront has are skipped four at a time.  The pattern gives per L entry
+// (i, k) the position of u_kk, and per entry j of row i one byte: the distance
+// from u_kk to u_kj in row k, or 0.  Eight bytes (eight L entries) are one load
+// per lane.  141k-node box, FP32, 1024-row blocks, one overlap layer: 110 us,
+// packing of the solve's copies included; pairs read, modified and written in
+// memory one L entry after another, and a packing pass, took 500 + 25 us.
+// STAGED: the block's values are held in LDS; otherwise in place in memory.
 constexpr int kBjGroup = 16;
+constexpr int kAhead = 2;  // offset words of eight L entries loaded a level ahead
 
-__device__ __forceinline__ uint2 group_shfl(uint2 v, int src) {
-    return make_uint2((unsigned)__shfl((int)v.x, src, kBjGroup), (unsigned)__shfl((int)v.y, src, kBjGroup));
+// x of lane K of each 16-lane row, in every lane of that row
+template <int K>
+__device__ __forceinline__ int row_bcast(int x) {
+    return __builtin_amdgcn_update_dpp(0, x, 0x150 + K, 0xf, 0xf, true);
+}
+template <int K>
+__device__ __forceinline__ unsigned row_bcast(unsigned x) { return (unsigned)row_bcast<K>((int)x); }
+template <int K>
+__device__ __forceinline__ float row_bcast(float x) { return __int_as_float(row_bcast<K>(__float_as_int(x))); }
+template <int K>
+__device__ __forceinline__ double row_bcast(double x) {
+    const long long b = __double_as_longlong(x);
+    const unsigned lo = (unsigned)row_bcast<K>((int)(unsigned)b), hi = (unsigned)row_bcast<K>((int)(b >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-template <typename T, bool STAGED>
+// What a row needs besides the other rows' values, loaded a level ahead.
+template <typename T, int NC>
+struct FacRow {
+    int s0, len, d;           // first entry, entries, L entries
+    unsigned tab, l0;         // its first offset word, its first L entry
+    uint4 out;                // where the solve's packed copies of its L part, its U part and its pivot go
+    T a[NC];                  // this lane's entries
+    unsigned piv;             // pivot position of L entry `lane`
+    unsigned off[2 * kAhead][NC];  // distances, four L entries a word, 0: none
+};
+
+template <typename T, int NC>
+__device__ __forceinline__ void fac_row_load(FacRow<T, NC> &w, uint4 m, uint4 out, int gl,
+                                             const unsigned *__restrict__ piv, const uint2 *__restrict__ off,
+                                             const T *val) {
+    w.s0 = (int)m.x;
+    w.len = (int)(m.y & 0xffu);
+    w.d = (int)((m.y >> 8) & 0xffu);
+    w.tab = m.z;
+    w.l0 = m.w;
+    w.out = out;
+    const int nch = (w.len + kBjGroup - 1) / kBjGroup;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) w.a[c] = gl + kBjGroup * c < w.len ? val[w.s0 + gl + kBjGroup * c] : T(0);
+    w.piv = gl < w.d ? piv[w.l0 + gl] : 0u;
+#pragma unroll
+    for (int b = 0; b < kAhead; ++b)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const uint2 o = 8 * b < w.d && c < nch ? off[(size_t)(w.tab + b * nch + c) * kBjGroup + gl]
+                                                   : make_uint2(0u, 0u);
+            w.off[2 * b][c] = o.x;
+            w.off[2 * b + 1][c] = o.y;
+        }
+}
+
+// L entries 4 B .. 4 B + 3 of a row: their u_kj (an entry without one loads the pivot, unused)
+template <int B, typename T, int NC>
+__device__ __forceinline__ void fac_load_u(const FacRow<T, NC> &w, bool wide, const T *val, T (&u)[4][NC]) {
+    constexpr int K0 = 4 * B;
+    const unsigned p[4] = {row_bcast<K0>(w.piv), row_bcast<K0 + 1>(w.piv), row_bcast<K0 + 2>(w.piv),
+                           row_bcast<K0 + 3>(w.piv)};
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+            if (c == 0 || wide) u[k][c] = val[p[k] + ((w.off[B][c] >> (8 * k)) & 0xffu)];
+}
+
+// L entry K: l_ik = a_ik u_kk^-1 (lane K's product, final since only earlier L
+// entries update entry K), then the row's entries that row k has too
+template <int K, typename T, int NC>
+__device__ __forceinline__ void fac_step(FacRow<T, NC> &w, bool wide, T pv, const T (&u)[4][NC]) {
+    const T lik = row_bcast<K>(w.a[0] * pv);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        if (c > 0 && !wide) break;
+        const T t = w.a[c] - lik * u[K & 3][c];
+        w.a[c] = (w.off[K / 4][c] & (0xffu << (8 * (K & 3)))) ? t : w.a[c];
+    }
+}
+
+template <int B, typename T, int NC>
+__device__ __forceinline__ void fac_chain(FacRow<T, NC> &w, bool wide, T pv, const T (&u)[4][NC]) {
+    fac_step<4 * B>(w, wide, pv, u);
+    fac_step<4 * B + 1>(w, wide, pv, u);
+    fac_step<4 * B + 2>(w, wide, pv, u);
+    fac_step<4 * B + 3>(w, wide, pv, u);
+}
+
+// One row, once every row that it uses is final: the u_kj of its first sixteen L
+// entries in one round of loads, then their chain; more L entries one at a time.
+template <typename T, int NC>
+__device__ __forceinline__ void fac_row(FacRow<T, NC> &w, int gl, const unsigned *__restrict__ piv,
+                                        const uint2 *__restrict__ off, const T *val) {
+    // uniform: batches, and entries past the sixteenth, that no row of the wavefront has
+    const bool b1 = __any(w.d > 4), b2 = __any(w.d > 8), b3 = __any(w.d > 12);
+    const bool wide = NC > 1 && __any(w.len > kBjGroup);
+    const T pv = val[w.piv];
+    T u0[4][NC], u1[4][NC], u2[4][NC], u3[4][NC];
+    fac_load_u<0>(w, wide, val, u0);
+    if (b1) fac_load_u<1>(w, wide, val, u1);
+    if (b2) fac_load_u<2>(w, wide, val, u2);
+    if (b3) fac_load_u<3>(w, wide, val, u3);
+    fac_chain<0>(w, wide, pv, u0);
+    if (b1) fac_chain<1>(w, wide, pv, u1);
+    if (b2) fac_chain<2>(w, wide, pv, u2);
+    if (b3) fac_chain<3>(w, wide, pv, u3);
+    if (gl < w.d) w.a[0] *= pv;
+    if (NC > 1 && __any(w.d > 8 * kAhead)) {
+        const int nch = (w.len + kBjGroup - 1) / kBjGroup;
+        for (int k = 8 * kAhead; __any(k < w.d); ++k) {
+            const bool in = k < w.d;
+            T ak = T(0);
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                const T q = __shfl(w.a[c], k & (kBjGroup - 1), kBjGroup);
+                if (c == k / kBjGroup) ak = q;
+            }
+            const unsigned pk = in ? piv[w.l0 + k] : 0u;
+            const T lik = in ? ak * val[pk] : T(0);
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                const uint2 o2 = in && c < nch ? off[(size_t)(w.tab + (k >> 3) * nch + c) * kBjGroup + gl]
+                                               : make_uint2(0u, 0u);
+                const unsigned o = ((k & 4 ? o2.y : o2.x) >> (8 * (k & 3))) & 0xffu;
+                if (o) w.a[c] -= lik * val[pk + o];
+                if (in && gl + kBjGroup * c == k) w.a[c] = lik;
+            }
+        }
+    }
+}
+
+// The factored row to val and to the solve's packed copies, its pivot inverted
+// (a zero pivot sets the flag).
+template <typename T, int NC>
+__device__ __forceinline__ void fac_row_store(const FacRow<T, NC> &w, int gl, T *val, T *__restrict__ vl,
+                                              T *__restrict__ vu, T *__restrict__ vd, int *__restrict__ flag) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        const int e = gl + kBjGroup * c;
+        T v = w.a[c];
+        if (e == w.d) {
+            if (v == T(0)) { atomicOr(flag, 1); v = T(0); }
+            else v = T(1) / v;
+        }
+        if (e < w.len) {
+            val[w.s0 + e] = v;
+            T *const p = e < w.d ? vl + w.out.x + e : e > w.d ? vu + w.out.y + (e - w.d - 1) : vd + w.out.z;
+            *p = v;
+        }
+    }
+}
+
+// One workgroup per block b: values ia[roff[b]] ... ia[roff[b + 1]] of lu, the
+// slots of its level pieces (at most kBjFactorThreads / kBjGroup each)
+// lptr[blev[b]] ... lptr[blev[b + 1]].  src null: lu already holds the values to
+// factor.  vl, vu, vd: the solve's packed L, U and inverted diagonal.  STAGED: values and piece pointers (npmax + 1 ints) in LDS, so that a
+// barrier waits for LDS accesses only and rows are loaded kRing levels ahead.
+template <typename T, int NC, bool STAGED>
 __global__ void __launch_bounds__(kBjFactorThreads) bj_factor(
-    const int *__restrict__ roff, const int *__restrict__ ia, const int *__restrict__ diag,
-    const int *__restrict__ src, const double *__restrict__ a, const uint2 *__restrict__ rec,
-    const long *__restrict__ pbase, const unsigned *__restrict__ pairs, const int *__restrict__ blev,
-    const int *__restrict__ lptr, const unsigned short *__restrict__ rows, T *__restrict__ lu,
-    int *__restrict__ flag) {
+    const int *__restrict__ roff, const int *__restrict__ ia, const int *__restrict__ src,
+    const double *__restrict__ a, const uint4 *__restrict__ slot, const uint4 *__restrict__ sout,
+    const unsigned *__restrict__ piv, const uint2 *__restrict__ off, const int *__restrict__ blev,
+    const int *__restrict__ lptr, T *lu, T *__restrict__ vl, T *__restrict__ vu, T *__restrict__ vd,
+    int *__restrict__ flag, int npmax) {
     extern __shared__ double smem[];
     const int b = blockIdx.x;
-    const int base = roff[b];
-    const int cnt = roff[b + 1] - base;
-    const int z0 = ia[base], nzb = ia[base + cnt] - z0;
-    T *val = STAGED ? (T *)smem : lu + z0;
-    for (int k = threadIdx.x; k < nzb; k += blockDim.x) val[k] = (T)a[src[z0 + k]];
-    if (!STAGED) __threadfence_block();
-    __syncthreads();
-    const int gl = threadIdx.x & (kBjGroup - 1), g = threadIdx.x / kBjGroup, ng = blockDim.x / kBjGroup;
-    const unsigned *pr = pairs + pbase[b];
-    const uint2 *rb = rec + z0;
-    for (int l = blev[b]; l < blev[b + 1]; ++l) {
-        for (int t = lptr[l] + g; t < lptr[l + 1]; t += ng) {
-            const int r = rows[t];
-            const int s0 = ia[base + r] - z0, d = diag[base + r] - z0 - s0;
-            uint2 rc = gl < d ? rb[s0 + gl] : make_uint2(0u, 0u);  // records kk = gl (mod kBjGroup)
-            uint2 cur = group_shfl(rc, 0);
-            unsigned q = gl < (cur.y & 0xffffu) ? pr[cur.x + gl] : 0u;
-            for (int kk = 0; kk < d; ++kk) {
-                const int k1 = kk + 1;
-                if (k1 < d && (k1 & (kBjGroup - 1)) == 0) rc = k1 + gl < d ? rb[s0 + k1 + gl] : make_uint2(0u, 0u);
-                uint2 nxt = make_uint2(0u, 0u);
-                unsigned qn = 0u;
-                if (k1 < d) {
-                    nxt = group_shfl(rc, k1 & (kBjGroup - 1));
-                    qn = gl < (nxt.y & 0xffffu) ? pr[nxt.x + gl] : 0u;
-                }
-                const int np = (int)(cur.y & 0xffffu);
-                const T lik = val[s0 + kk] * val[cur.y >> 16];  // u_kk is stored inverted
-                if (gl < np) val[q >> 16] -= lik * val[q & 0xffffu];
-                for (int j = gl + kBjGroup; j < np; j += kBjGroup) {
-                    const unsigned q2 = pr[cur.x + j];
-                    val[q2 >> 16] -= lik * val[q2 & 0xffffu];
-                }
-                wave_lds_sync();
-                if (gl == 0) val[s0 + kk] = lik;
-                wave_lds_sync();
-                cur = nxt;
-                q = qn;
-            }
-            if (gl == 0) {
-                const T piv = val[s0 + d];
-                if (piv == T(0)) { atomicOr(flag, 1); val[s0 + d] = T(0); }
-                else val[s0 + d] = T(1) / piv;
-            }
-            wave_lds_sync();
-        }
-        if (!STAGED) __threadfence_block();
-        __syncthreads();
-    }
+    const int z0 = ia[roff[b]], nzb = ia[roff[b + 1]] - z0;
+    const int l0 = blev[b], nl = blev[b + 1] - l0;
+    int *pp = reinterpret_cast<int *>(smem);
+    T *val = STAGED ? reinterpret_cast<T *>(smem + (npmax + 2) / 2) : lu + z0;
+    if (src)
+        for (int k = threadIdx.x; k < nzb; k += kBjFactorThreads) val[k] = (T)a[src[z0 + k]];
+    else if (STAGED)
+        for (int k = threadIdx.x; k < nzb; k += kBjFactorThreads) val[k] = lu[z0 + k];
     if (STAGED)
-        for (int k = threadIdx.x; k < nzb; k += blockDim.x) lu[z0 + k] = val[k];
+        for (int k = threadIdx.x; k <= nl; k += kBjFactorThreads) pp[k] = lptr[l0 + k];
+    else
+        __threadfence_block();
+    __syncthreads();
+    if (nl == 0) return;
+    const int gl = threadIdx.x & (kBjGroup - 1), g = threadIdx.x / kBjGroup;
+    // piece l's slot of this group: a group without a row takes the piece's last
+    // slot (loads stay in range) and stores nothing
+    auto slot_of = [&](int l, bool &have) {
+        const int lc = min(l, nl - 1);
+        const int p0 = STAGED ? pp[lc] : lptr[l0 + lc], p1 = STAGED ? pp[lc + 1] : lptr[l0 + lc + 1];
+        have = l < nl && p0 + g < p1;
+        return min(p0 + g, p1 - 1);
+    };
+    // a wavefront none of whose groups has a row in a piece skips the work on it
+    if (STAGED) {
+        constexpr int kRing = 4;
+        FacRow<T, NC> w[kRing];
+        bool have[kRing], have1[kRing];
+        uint4 m[kRing], o[kRing];
+#pragma unroll
+        for (int q = 0; q < kRing; ++q) {
+            const int sl = slot_of(q, have[q]);
+            m[q] = slot[sl];
+            o[q] = sout[sl];
+        }
+#pragma unroll
+        for (int q = 0; q < kRing; ++q) fac_row_load(w[q], m[q], o[q], gl, piv, off, val);
+#pragma unroll
+        for (int q = 0; q < kRing; ++q) {
+            const int sl = slot_of(q + kRing, have1[q]);
+            m[q] = slot[sl];
+            o[q] = sout[sl];
+        }
+        for (int lb = 0; lb < nl; lb += kRing) {
+#pragma unroll
+            for (int q = 0; q < kRing; ++q) {
+                if (__any(have[q])) {
+                    fac_row(w[q], gl, piv, off, val);
+                    if (have[q]) fac_row_store(w[q], gl, val, vl, vu, vd, flag);
+                }
+                fac_row_load(w[q], m[q], o[q], gl, piv, off, val);
+                have[q] = have1[q];
+                const int sl = slot_of(lb + q + 2 * kRing, have1[q]);
+                m[q] = slot[sl];
+                o[q] = sout[sl];
+                lds_barrier();
+            }
+        }
+        for (int k = threadIdx.x; k < nzb; k += kBjFactorThreads) lu[z0 + k] = val[k];
+    } else {
+        bool have, have1, have2;
+        FacRow<T, NC> w;
+        const int sl0 = slot_of(0, have), sl1 = slot_of(1, have1);
+        fac_row_load(w, slot[sl0], sout[sl0], gl, piv, off, val);
+        uint4 m1 = slot[sl1], o1 = sout[sl1];
+        for (int l = 0; l < nl; ++l) {
+            FacRow<T, NC> nx;
+            fac_row_load(nx, m1, o1, gl, piv, off, val);
+            const int sl = slot_of(l + 2, have2);
+            const uint4 m2 = slot[sl], o2 = sout[sl];
+            if (__any(have)) {
+                fac_row(w, gl, piv, off, val);
+                if (have) fac_row_store(w, gl, val, vl, vu, vd, flag);
+            }
+            __threadfence_block();
+            __syncthreads();
+            w = nx;
+            have = have1;
+            m1 = m2;
+            o1 = o2;
+            have1 = have2;
+        }
+    }
 }
 
 // Solve: one wavefront per block.  Only the block's solution, its overflow
@@ -721,16 +936,6 @@ constexpr int kBjRow = 12;
 #ifndef BJ_AHEAD_F64
 #define BJ_AHEAD_F64 4
 #endif
-
-// After a factorisation: the packed values (src < 0: padding, zero) and, for
-// U, every slot's inverted diagonal.
-template <typename T>
-__global__ void bj_pack_vals(long n, const int *__restrict__ src, const T *__restrict__ lu, T *__restrict__ val) {
-    long k = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    const int q = src[k];
-    val[k] = q >= 0 ? lu[q] : T(0);
-}
 
 constexpr int kBjHalf = kBjRow / 2;  // window entries per lane of a pair
 
@@ -1064,6 +1269,129 @@ __global__ void __launch_bounds__(64) bj_solve(const int *__restrict__ roff, con
     if (yn2) {  // this block's share of ||y||^2 (owned rows partition the rows)
         q = wave_reduce(q);
         if (threadIdx.x == 0) yn2[b] = q;
+    }
+}
+
+// Global ILU(0) solve of a matrix whose solution fits the LDS, in one
+// workgroup: y = U^-1 L^-1 (x / xdiv).  Rows lie in level order, one lane per
+// row; a level wider than the workgroup is cut into pieces.  Per slot a padded
+// window of KW entries, so a piece's loads have fixed addresses and go out kA
+// pieces ahead; the chain per piece is one batch of LDS reads, the row's sum and
+// one LDS store.  One wavefront needs no barrier (the LDS runs its accesses in
+// order); wider workgroups meet at one per piece.  A 4 141-node slice (141 levels
+// per triangle) takes 52 us, and its factorisation 282 us; one launch per level
+// and triangle (the form that matrices outside these limits keep) took 707 to
+// 1075 us, and 1500 us.  The chain bounds it: 0.18 us per level.
+// kOneWidth: rows per level, on average over both triangles, up to which one
+// workgroup is used: a launch per level costs 2.5 us in the solve and 10 us in
+// the factorisation, one workgroup 0.2 us per piece of up to 1024 rows and 2 us
+// per 32 rows of a level.
+constexpr long kOneWidth = 256;
+
+template <int KW>
+struct IluWin {
+    double a[KW];
+    unsigned c[KW / 2];
+    unsigned rm;
+    double d;
+    bool have;
+};
+
+template <int KW, int TH, bool UPPER>
+__device__ __forceinline__ void ilu0_sweep(double *v, double *spare, int np, const int *pp,
+                                           const unsigned *__restrict__ row, const unsigned short *__restrict__ col,
+                                           const double *__restrict__ val, const double *__restrict__ dinv) {
+    constexpr int kA = KW <= 4 ? (TH > 256 ? 4 : 8) : KW == 8 ? (TH > 256 ? 2 : 4) : KW == 16 ? 2 : 1;
+    const int t = threadIdx.x;
+    auto load = [&](IluWin<KW> &w, int p) {
+        const int pc = min(p, np - 1), p0 = pp[pc], p1 = pp[pc + 1];
+        const int sl = min(p0 + t, p1 - 1);  // a lane without a row reads the piece's last
+        w.have = p < np && p0 + t < p1;
+        w.rm = row[sl];
+        const double2 *pa = reinterpret_cast<const double2 *>(val + (size_t)sl * KW);
+        const unsigned *pc2 = reinterpret_cast<const unsigned *>(col + (size_t)sl * KW);
+#pragma unroll
+        for (int k = 0; k < KW / 2; ++k) {
+            const double2 q = pa[k];
+            w.a[2 * k] = q.x;
+            w.a[2 * k + 1] = q.y;
+            w.c[k] = pc2[k];
+        }
+        w.d = UPPER ? dinv[sl] : 0.;
+    };
+    IluWin<KW> w[kA];
+#pragma unroll
+    for (int q = 0; q < kA; ++q) load(w[q], q);
+    for (int pb = 0; pb < np; pb += kA) {
+#pragma unroll
+        for (int q = 0; q < kA; ++q) {
+            const int r = (int)(w[q].rm & 0xffffu), kn = (int)(w[q].rm >> 16);
+            double xv[KW];
+#pragma unroll
+            for (int k = 0; k < KW; ++k) xv[k] = v[(k & 1) ? w[q].c[k / 2] >> 16 : w[q].c[k / 2] & 0xffffu];
+            const double vr = v[r];
+            double s = 0.;
+#pragma unroll
+            for (int k = 0; k < KW; ++k) s += k < kn ? w[q].a[k] * xv[k] : 0.;
+            s = vr - s;
+            if (UPPER) s *= w[q].d;
+            *(w[q].have ? v + r : spare) = s;
+            load(w[q], pb + q + kA);
+            if (TH > 64) lds_barrier();
+            else wave_lds_order();
+        }
+    }
+}
+
+template <int KW, int TH>
+__global__ void __launch_bounds__(TH) ilu0_solve(int n, int npl, const int *__restrict__ ppl,
+                                                 const unsigned *__restrict__ row_l,
+                                                 const unsigned short *__restrict__ col_l,
+                                                 const double *__restrict__ val_l, int npu,
+                                                 const int *__restrict__ ppu, const unsigned *__restrict__ row_u,
+                                                 const unsigned short *__restrict__ col_u,
+                                                 const double *__restrict__ val_u, const double *__restrict__ x,
+                                                 const double *__restrict__ xdiv, double *__restrict__ y,
+                                                 double *__restrict__ yn2) {
+    extern __shared__ double smem[];
+    double *v = smem, *spare = v + n + threadIdx.x;
+    int *pl = reinterpret_cast<int *>(v + n + TH), *pu = pl + npl + 1;
+    for (int k = threadIdx.x; k <= npl; k += TH) pl[k] = ppl[k];
+    for (int k = threadIdx.x; k <= npu; k += TH) pu[k] = ppu[k];
+    constexpr int kStage = 8;  // loads in flight per lane
+    for (int i0 = threadIdx.x; i0 < n; i0 += TH * kStage) {
+        double q[kStage], d[kStage];
+#pragma unroll
+        for (int u = 0; u < kStage; ++u) {
+            const int i = min(i0 + TH * u, n - 1);
+            q[u] = x[i];
+            d[u] = xdiv ? xdiv[i] : 1.;
+        }
+#pragma unroll
+        for (int u = 0; u < kStage; ++u)
+            if (i0 + TH * u < n) v[i0 + TH * u] = xdiv ? q[u] / d[u] : q[u];
+    }
+    __syncthreads();
+    ilu0_sweep<KW, TH, false>(v, spare, npl, pl, row_l, col_l, val_l, nullptr);
+    __syncthreads();
+    ilu0_sweep<KW, TH, true>(v, spare, npu, pu, row_u, col_u, val_u, val_u + (size_t)n * KW);
+    __syncthreads();
+    double q = 0.;
+    for (int i = threadIdx.x; i < n; i += TH) {
+        const double s = v[i];
+        y[i] = s;
+        q += s * s;
+    }
+    if (yn2) {
+        q = wave_reduce(q);
+        __syncthreads();
+        if ((threadIdx.x & 63) == 0) v[threadIdx.x >> 6] = q;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double tot = 0.;
+            for (int k = 0; k < TH / 64; ++k) tot += v[k];
+            yn2[0] = tot;
+        }
     }
 }
 
@@ -1693,6 +2021,9 @@ static int csr_gemv_impl(fvp_csr *A, double alpha, const double *x, double beta,
     return 0;
 }
 
+static int build_one(fvp_csr *A, const std::vector<int> &diag, const std::vector<int> &lrows,
+                     const std::vector<int> &urows);
+
 // level sets of the L (forward) and U (backward) dependency DAGs
 static int build_levels(fvp_csr *A, const std::vector<int> &diag) {
     const int n = A->n;
@@ -1721,8 +2052,150 @@ static int build_levels(fvp_csr *A, const std::vector<int> &diag) {
     std::vector<int> lrows, urows;
     group(lev, nl, A->lptr_h, lrows);
     group(ulev, nu, A->uptr_h, urows);
-    if (A->lrows.upload(lrows.data(), n) || A->urows.upload(urows.data(), n)) return -1;
+    if (build_one(A, diag, lrows, urows)) return -1;
+    if (!A->one && (A->lrows.upload(lrows.data(), n) || A->urows.upload(urows.data(), n))) return -1;
     A->levels = true;
+    return 0;
+}
+
+// The tables of bj_factor: roff, bia, bja, bdiag describe the blocks (local
+// columns, entry positions over all blocks), rows the local rows as slots in
+// level order (block b's slots are [roff[b], roff[b + 1])), out per slot the
+// places of its packed L part, U part and pivot; no row is longer than 64
+// entries.
+template <typename Col, typename Row>
+static int factor_tables(FactorTab &F, int nb, const std::vector<int> &roff, const std::vector<int> &bia,
+                         const std::vector<Col> &bja, const std::vector<int> &bdiag, const std::vector<Row> &rows,
+                         const std::vector<uint4> &out, int maxrow) {
+    const int total = roff[nb];
+    std::vector<uint4> slot(total);
+    std::vector<unsigned> piv;
+    size_t units = 0;  // offset batches of one 16-lane group
+    for (int i = 0; i < total; ++i) {
+        const int len = bia[i + 1] - bia[i], d = bdiag[i] - bia[i];
+        units += (size_t)((d + 7) / 8) * ((len + kBjGroup - 1) / kBjGroup);
+    }
+    if (units > 0xffffffffu) { set_error("too many entries for the factorisation's tables"); return -1; }
+    std::vector<unsigned char> off(units * kBjGroup * 8, (unsigned char)0);
+    piv.reserve(bdiag.empty() ? 0 : (size_t)bia[total] / 2);
+    int widest = 0;
+    for (int b = 0; b < nb; ++b) widest = std::max(widest, roff[b + 1] - roff[b]);
+    std::vector<int> pos(widest, -1);
+    size_t tab = 0;
+    for (int b = 0; b < nb; ++b) {
+        const int base = roff[b], z0 = bia[base];
+        for (int sl = base; sl < roff[b + 1]; ++sl) {
+            const int i = base + (int)rows[sl];
+            const int e0 = bia[i], len = bia[i + 1] - e0, d = bdiag[i] - e0;
+            const int nch = (len + kBjGroup - 1) / kBjGroup;
+            slot[sl] = make_uint4((unsigned)(e0 - z0), (unsigned)len | ((unsigned)d << 8), (unsigned)tab,
+                                  (unsigned)piv.size());
+            for (int j = 0; j < len; ++j) pos[bja[e0 + j]] = j;
+            for (int k = 0; k < d; ++k) {
+                const int row = base + (int)bja[e0 + k], kd = bdiag[row];
+                piv.push_back((unsigned)(kd - z0));
+                for (int m = kd + 1; m < bia[row + 1]; ++m) {
+                    const int j = pos[bja[m]];
+                    if (j < 0) continue;
+                    const size_t unit = tab + (size_t)(k / 8) * nch + j / kBjGroup;
+                    off[(unit * kBjGroup + j % kBjGroup) * 8 + k % 8] = (unsigned char)(m - kd);
+                }
+            }
+            for (int j = 0; j < len; ++j) pos[bja[e0 + j]] = -1;
+            tab += (size_t)((d + 7) / 8) * nch;
+        }
+    }
+    if (piv.empty()) piv.push_back(0u);
+    if (off.empty()) off.resize(8 * kBjGroup, (unsigned char)0);
+    F.nc = maxrow <= kBjGroup ? 1 : maxrow <= 2 * kBjGroup ? 2 : 4;
+    return F.slot.upload(slot.data(), slot.size()) || F.out.upload(out.data(), out.size()) || F.piv.upload(piv.data(), piv.size()) ||
+           F.off.upload(reinterpret_cast<const uint2 *>(off.data()), off.size() / 8);
+}
+
+// pieces of at most `width` slots of each level
+static void level_pieces(const std::vector<int> &lptr, int width, std::vector<int> &pieces) {
+    pieces.assign(1, lptr[0]);
+    for (size_t l = 0; l + 1 < lptr.size(); ++l)
+        for (int p = lptr[l]; p < lptr[l + 1]; p += width) pieces.push_back(std::min(p + width, lptr[l + 1]));
+}
+
+// Global ILU(0) in one workgroup (see ilu0_solve): the tables of its
+// factorisation and of its solve, where the pattern allows them.
+static int build_one(fvp_csr *A, const std::vector<int> &diag, const std::vector<int> &lrows,
+                     const std::vector<int> &urows) {
+    const int n = A->n;
+    A->one = false;
+    if (hipDeviceGetAttribute(&A->lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, A->device) != hipSuccess)
+        A->lds_max = 64 * 1024;
+    int maxrow = 0, maxtri = 1;
+    for (int i = 0; i < n; ++i) {
+        maxrow = std::max(maxrow, A->ia_h[i + 1] - A->ia_h[i]);
+        maxtri = std::max({maxtri, diag[i] - A->ia_h[i], A->ia_h[i + 1] - diag[i] - 1});
+    }
+    const int win = maxtri <= 4 ? 4 : maxtri <= 8 ? 8 : maxtri <= 16 ? 16 : 32;
+    if (maxrow > 64 || maxtri > win || n > 65536) return 0;
+    // wide levels are worth a launch each (the whole device on one level); one
+    // workgroup takes kBjFactorThreads / kBjGroup rows of a level at a time
+    const long levels = (long)(A->lptr_h.size() - 1 + A->uptr_h.size() - 1);
+    if (2L * n > kOneWidth * levels) return 0;
+    // threads: the count that makes the sweep's pieces cheapest (a piece's cost
+    // grows with the wavefronts that meet at its barrier)
+    std::vector<int> pieces[2];
+    double best = 1e300;
+    for (int th : {64, 256, 1024}) {
+        std::vector<int> pl, pu;
+        level_pieces(A->lptr_h, th, pl);
+        level_pieces(A->uptr_h, th, pu);
+        const size_t lds = 8 * (size_t)(n + th) + 4 * (pl.size() + pu.size());
+        const double cost = (double)(pl.size() + pu.size()) * (th == 64 ? 1.0 : th == 256 ? 1.3 : 1.8);
+        if (lds > (size_t)A->lds_max || cost >= best) continue;
+        best = cost;
+        A->o_threads = th;
+        A->o_lds = lds;
+        pieces[0].swap(pl);
+        pieces[1].swap(pu);
+    }
+    if (pieces[0].empty()) return 0;
+    A->o_win = win;
+    std::vector<uint4> out(n);  // by row at first, then by slot of L's level order
+    for (int t = 0; t < 2; ++t) {
+        const std::vector<int> &order = t ? urows : lrows;
+        std::vector<unsigned> row(n);
+        std::vector<unsigned short> col((size_t)n * win, 0);
+        for (int sl = 0; sl < n; ++sl) {
+            const int i = order[sl], k0 = t ? diag[i] + 1 : A->ia_h[i], k1 = t ? A->ia_h[i + 1] : diag[i];
+            row[sl] = (unsigned)i | ((unsigned)(k1 - k0) << 16);
+            for (int k = 0; k < win; ++k) {
+                const size_t q = (size_t)sl * win + k;
+                col[q] = (unsigned short)(k0 + k < k1 ? A->ja_h[k0 + k] : i);
+            }
+            (t ? out[i].y : out[i].x) = (unsigned)(sl * win);
+            if (t) out[i].z = (unsigned)sl;
+        }
+        IluTri &T = A->otri[t];
+        T.npieces = (int)pieces[t].size() - 1;
+        T.nslots = n;
+        if (T.pptr.upload(pieces[t].data(), pieces[t].size()) || T.row.upload(row.data(), n) ||
+            T.col.upload(col.data(), col.size()) || T.val.alloc((size_t)n * win + (t ? n : 0)))
+            return -1;
+        FVP_HIP(hipMemsetAsync(T.val.p, 0, sizeof(double) * T.val.n, A->stream));  // the windows' padding stays zero
+    }
+    std::vector<uint4> by(n);
+    for (int sl = 0; sl < n; ++sl) by[sl] = out[lrows[sl]];
+    std::vector<int> fp;
+    level_pieces(A->lptr_h, kBjFactorThreads / kBjGroup, fp);
+    const int head[4] = {0, n, 0, (int)fp.size() - 1};
+    fp.insert(fp.begin(), head, head + 4);
+    if (A->o_fptr.upload(fp.data(), fp.size()) ||
+        factor_tables(A->ofac, 1, {0, n}, A->ia_h, A->ja_h, diag, lrows, by, maxrow))
+        return -1;
+    for (const void *f :
+         {(const void *)ilu0_solve<4, 64>, (const void *)ilu0_solve<8, 64>, (const void *)ilu0_solve<16, 64>,
+          (const void *)ilu0_solve<32, 64>, (const void *)ilu0_solve<4, 256>, (const void *)ilu0_solve<8, 256>,
+          (const void *)ilu0_solve<16, 256>, (const void *)ilu0_solve<32, 256>, (const void *)ilu0_solve<4, 1024>,
+          (const void *)ilu0_solve<8, 1024>, (const void *)ilu0_solve<16, 1024>, (const void *)ilu0_solve<32, 1024>})
+        (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, A->lds_max);
+    A->one = true;
     return 0;
 }
 
@@ -1819,58 +2292,24 @@ static int build_bj(fvp_csr *A) {
     }
     if (maxrow > 64) { set_error("block-Jacobi ILU(0) supports rows of at most 64 block entries"); return -1; }
     if (maxnz > 65535) { set_error("block-Jacobi ILU(0): more than 65535 entries in one block"); return -1; }
-    // the factorisation's update pairs (see bj_factor)
-    std::vector<unsigned> frec(2 * bsrc.size(), 0u), fpair;
-    std::vector<long> fpbase(nb + 1, 0);
-    {
-        std::vector<int> pos(maxrows, -1);
-        for (int b = 0; b < nb; ++b) {
-            const int base = roff[b], cnt = roff[b + 1] - base, z0 = bia[base];
-            fpbase[b] = (long)fpair.size();
-            for (int r = 0; r < cnt; ++r) {
-                const int s0 = bia[base + r], s1 = bia[base + r + 1], dd = bdiag[base + r];
-                for (int q = s0; q < s1; ++q) pos[bja[q]] = q - z0;
-                for (int e = s0; e < dd; ++e) {
-                    const int k = bja[e], kd = bdiag[base + k], ke = bia[base + k + 1];
-                    const long start = (long)fpair.size() - fpbase[b];
-                    unsigned count = 0;
-                    for (int m = kd + 1; m < ke; ++m) {
-                        const int p = pos[bja[m]];
-                        if (p >= 0) { fpair.push_back((unsigned)(m - z0) | ((unsigned)p << 16)); ++count; }
-                    }
-                    frec[2 * (size_t)e] = (unsigned)start;
-                    frec[2 * (size_t)e + 1] = count | ((unsigned)(kd - z0) << 16);
-                }
-                for (int q = s0; q < s1; ++q) pos[bja[q]] = -1;
-            }
-        }
-        fpbase[nb] = (long)fpair.size();
-        if (fpair.empty()) fpair.push_back(0u);  // a block-diagonal matrix has no pairs
-    }
-    if (A->fac_rec.upload(frec.data(), frec.size()) || A->fac_pair.upload(fpair.data(), fpair.size()) ||
-        A->fac_pbase.upload(fpbase.data(), nb + 1))
-        return -1;
     const bool ident = A->overlap == 0;  // rows of block b are [b bs, ...): no row list needed
     if (A->b_ia.upload(bia.data(), total + 1) || A->b_src.upload(bsrc.data(), bsrc.size()) ||
-        A->b_diag.upload(bdiag.data(), total) || A->b_ja.upload(bja.data(), bja.size()) ||
-        A->b_lu.alloc(bsrc.size()) || A->b_roff.upload(roff.data(), nb + 1) ||
-        A->b_own.upload(own.data(), own.size()) || (!ident && A->b_rowid.upload(rowid.data(), total)) ||
-        A->b_lev_l.upload(blev_l.data(), nb + 1) || A->b_lev_u.upload(blev_u.data(), nb + 1) ||
-        A->b_lptr_l.upload(lptr_l.data(), lptr_l.size()) || A->b_lptr_u.upload(lptr_u.data(), lptr_u.size()) ||
-        A->b_rows_l.upload(rows_l.data(), rows_l.size()) || A->b_rows_u.upload(rows_u.data(), rows_u.size()))
+        A->b_roff.upload(roff.data(), nb + 1) ||
+        A->b_own.upload(own.data(), own.size()) || (!ident && A->b_rowid.upload(rowid.data(), total)))
         return -1;
     if (ident) A->b_rowid.release();
+    A->b_lu.release();
     A->b_lu32.release();
     {
         // packed solve layout (see bj_solve)
         std::vector<int> ovp(nb + 1, 0);
         std::vector<long> ovpos;
         std::vector<uint8_t> ovtri;
-        std::vector<int> dsr;
+        std::vector<uint4> out(total);  // by row at first, then by slot of L's level order
+        long ndiag = 0;
         struct Tri {
             std::vector<unsigned> meta;
             std::vector<long> ebase;
-            std::vector<int> esrc;
             std::vector<unsigned short> col;
         } tr[2];
         for (int t = 0; t < 2; ++t) tr[t].ebase.assign(nb + 1, 0);
@@ -1880,7 +2319,7 @@ static int build_bj(fvp_csr *A) {
             int nov = 0;
             for (int tri = 0; tri < 2; ++tri) {
                 Tri &T = tr[tri];
-                const long eb = (long)T.esrc.size();
+                const long eb = (long)T.col.size();
                 T.ebase[b] = eb;
                 const std::vector<int> &lptr = tri ? lptr_u : lptr_l;
                 const std::vector<int> &blev = tri ? blev_u : blev_l;
@@ -1890,32 +2329,38 @@ static int build_bj(fvp_csr *A) {
                     const int i = base + r;
                     const int k0 = tri ? bdiag[i] + 1 : bia[i], k1 = tri ? bia[i + 1] : bdiag[i];
                     const int kn = k1 - k0;
-                    const long kl = (long)T.esrc.size() - eb;
+                    const long kl = (long)T.col.size() - eb;
                     if (kl > 65535 || nov > 65535) {
                         set_error("block-Jacobi ILU(0): more than 65535 entries in one block triangle");
                         return -1;
                     }
                     T.meta.push_back((unsigned)kl | ((unsigned)nov << 16));
                     T.meta.push_back((unsigned)r | ((unsigned)kn << 16));
+                    (tri ? out[i].y : out[i].x) = (unsigned)T.col.size();
+                    if (tri) out[i].z = (unsigned)ndiag++;
                     for (int k = k0; k < k1; ++k) {
                         if (k - k0 >= kBjRow) {
-                            ovpos.push_back((long)T.esrc.size());
+                            ovpos.push_back((long)T.col.size());
                             ovtri.push_back((uint8_t)tri);
                             ++nov;
                         }
-                        T.esrc.push_back(k);
                         T.col.push_back(bja[k]);
                     }
-                    if (kn & 1) { T.esrc.push_back(-1); T.col.push_back((unsigned short)r); }
-                    if (tri) dsr.push_back(bdiag[i]);
+                    if (kn & 1) T.col.push_back((unsigned short)r);
                 }
             }
             ovp[b + 1] = ovp[b] + nov;
             ovmax = std::max(ovmax, nov);
         }
         for (int t = 0; t < 2; ++t) {  // the last windows read up to kBjRow entries past the end
-            tr[t].ebase[nb] = (long)tr[t].esrc.size();
-            for (int k = 0; k < kBjRow; ++k) { tr[t].esrc.push_back(-1); tr[t].col.push_back(0); }
+            tr[t].ebase[nb] = (long)tr[t].col.size();
+            for (int k = 0; k < kBjRow; ++k) tr[t].col.push_back(0);
+        }
+        {
+            std::vector<uint4> by(total);
+            for (int b = 0; b < nb; ++b)
+                for (int sl = roff[b]; sl < roff[b + 1]; ++sl) by[sl] = out[roff[b] + rows_l[sl]];
+            if (factor_tables(A->fac, nb, roff, bia, bja, bdiag, rows_l, by, maxrow)) return -1;
         }
         // the solve's levels: each factor level cut into pieces of at most 32 slots (one per lane pair)
         auto split = [&](const std::vector<int> &blev, const std::vector<int> &lptr, std::vector<int> &sb,
@@ -1939,10 +2384,8 @@ static int build_bj(fvp_csr *A) {
         if (A->meta_l.upload(tr[0].meta.data(), tr[0].meta.size()) ||
             A->meta_u.upload(tr[1].meta.data(), tr[1].meta.size()) ||
             A->ebase_l.upload(tr[0].ebase.data(), nb + 1) || A->ebase_u.upload(tr[1].ebase.data(), nb + 1) ||
-            A->esrc_l.upload(tr[0].esrc.data(), tr[0].esrc.size()) ||
-            A->esrc_u.upload(tr[1].esrc.data(), tr[1].esrc.size()) ||
             A->col_l.upload(tr[0].col.data(), tr[0].col.size()) || A->col_u.upload(tr[1].col.data(), tr[1].col.size()) ||
-            A->dsrc.upload(dsr.data(), dsr.size()) || A->ov_ptr.upload(ovp.data(), nb + 1) ||
+            A->ov_ptr.upload(ovp.data(), nb + 1) ||
             A->ov_pos.upload(ovpos.data(), ovpos.size()) || A->ov_tri.upload(ovtri.data(), ovtri.size()) ||
             A->s_lev_l.upload(sbl.data(), nb + 1) || A->s_lev_u.upload(sbu.data(), nb + 1) ||
             A->s_lptr_l.upload(spl.data(), spl.size()) || A->s_lptr_u.upload(spu.data(), spu.size()))
@@ -1957,9 +2400,10 @@ static int build_bj(fvp_csr *A) {
         A->lds_max = 64 * 1024;
     // per-kernel attributes (shared by every matrix): allow the device maximum;
     // each build checks its own block against it
-    for (const void *f : {(const void *)bj_factor<double, true>, (const void *)bj_factor<double, false>,
+    for (const void *f : {(const void *)bj_factor<double, 1, true>, (const void *)bj_factor<double, 2, true>,
+                          (const void *)bj_factor<double, 4, true>, (const void *)bj_factor<float, 1, true>,
+                          (const void *)bj_factor<float, 2, true>, (const void *)bj_factor<float, 4, true>,
                           (const void *)bj_solve<double, false>, (const void *)bj_solve<double, true>,
-                          (const void *)bj_factor<float, true>, (const void *)bj_factor<float, false>,
                           (const void *)bj_solve<float, false>, (const void *)bj_solve<float, true>})
         (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, A->lds_max);
     A->nblk = nb;
@@ -2146,6 +2590,36 @@ static int schur_apply(fvp_csr *A, const double *x, double *y) {
     return 0;
 }
 
+// bj_factor's launch: the blocks' description, and the staged values' LDS bytes (0: in place)
+struct FactorArgs {
+    int nblk;
+    const int *roff, *ia, *src;
+    const double *a;
+    const FactorTab *tab;
+    const int *lev, *lptr;
+    int *flag;
+    size_t staged;
+    int npmax;  // most pieces of one block (staged form)
+};
+template <typename T, int NC>
+static void bj_factor_launch_nc(hipStream_t s, const FactorArgs &f, T *lu, T *vl, T *vu, T *vd) {
+    const FactorTab &t = *f.tab;
+    if (f.staged)
+        bj_factor<T, NC, true><<<f.nblk, kBjFactorThreads, f.staged, s>>>(f.roff, f.ia, f.src, f.a, t.slot.p, t.out.p,
+                                                                          t.piv.p, t.off.p, f.lev, f.lptr, lu, vl, vu,
+                                                                          vd, f.flag, f.npmax);
+    else
+        bj_factor<T, NC, false><<<f.nblk, kBjFactorThreads, 0, s>>>(f.roff, f.ia, f.src, f.a, t.slot.p, t.out.p,
+                                                                    t.piv.p, t.off.p, f.lev, f.lptr, lu, vl, vu, vd,
+                                                                    f.flag, 0);
+}
+template <typename T>
+static void bj_factor_launch(hipStream_t s, const FactorArgs &f, T *lu, T *vl, T *vu, T *vd) {
+    if (f.tab->nc == 1) bj_factor_launch_nc<T, 1>(s, f, lu, vl, vu, vd);
+    else if (f.tab->nc == 2) bj_factor_launch_nc<T, 2>(s, f, lu, vl, vu, vd);
+    else bj_factor_launch_nc<T, 4>(s, f, lu, vl, vu, vd);
+}
+
 static int precon_build_impl(fvp_csr *A, int type) {
     hipStream_t s = A->stream;
     const int n = A->n;
@@ -2166,38 +2640,35 @@ static int precon_build_impl(fvp_csr *A, int type) {
             if (rc) { A->ptype = -1; return rc; }
         }
         const size_t vb = type == FVP_PRECON_BJILU0 ? sizeof(double) : sizeof(float);
-        // values staged in LDS when two workgroups fit a CU (FVP_BJ_FACTOR_MODE 0 / 1
-        // forces in place / staged where it fits the workgroup: a tuning and test knob)
-        const size_t staged = (size_t)A->b_maxnz * vb;
-        bool stage = staged <= (size_t)A->lds_max / 2;
+        // Values staged in LDS wherever a block fits (rows past 32 entries in FP64
+        // spill registers in that form and stay in place).  Whole builds, staged
+        // against in place: 67 / 75 us (276 blocks of 512 rows, FP32), 200 / 307
+        // (1024 with one overlap layer, FP32), 323 / 365 (the same, FP64), 517 / 549
+        // (1000 blocks of 1024 with overlap, FP32); at worst 91 / 83 (276 blocks of
+        // 512, FP64).  FVP_BJ_FACTOR_MODE 0 / 1 forces in place / staged where it
+        // fits the workgroup: a tuning and test knob.
+        const size_t staged = (size_t)A->b_maxnz * vb + 8 * (size_t)((A->s_levmax_l + 2) / 2);
+        bool stage = staged <= (size_t)A->lds_max && !(A->fac.nc == 4 && vb == 8);
         if (const char *e = getenv("FVP_BJ_FACTOR_MODE")) stage = atoi(e) > 0 && staged <= (size_t)A->lds_max;
         A->factor_mode = stage ? 1 : 0;
-        const uint2 *frec = reinterpret_cast<const uint2 *>(A->fac_rec.p);
-#define FVP_BJ_FACTOR(TT, ST, LU)                                                                                 \
-    bj_factor<TT, ST><<<A->nblk, kBjFactorThreads, ST ? staged : 0, s>>>(                                         \
-        A->b_roff.p, A->b_ia.p, A->b_diag.p, A->b_src.p, A->a.p, frec, A->fac_pbase.p, A->fac_pair.p, A->b_lev_l.p, \
-        A->b_lptr_l.p, A->b_rows_l.p, LU, A->flag.p)
+        const FactorArgs fa{A->nblk, A->b_roff.p, A->b_ia.p, A->b_src.p, A->a.p, &A->fac, A->s_lev_l.p,
+                            A->s_lptr_l.p, A->flag.p, stage ? staged : 0, A->s_levmax_l};
+        const size_t nl = A->col_l.n, nu = A->col_u.n, nd = A->fac.slot.n;
+        // the packed arrays' padding stays zero: only the factor's entries are written
+        auto ensure = [&](auto &lu, auto &vl, auto &vu, auto &vd) {
+            if (!lu.p && lu.alloc(A->b_src.n)) return -1;
+            if (vl.p) return 0;
+            if (vl.alloc(nl) || vu.alloc(nu) || vd.alloc(nd)) return -1;
+            FVP_HIP(hipMemsetAsync(vl.p, 0, sizeof(*vl.p) * nl, s));
+            FVP_HIP(hipMemsetAsync(vu.p, 0, sizeof(*vu.p) * nu, s));
+            return 0;
+        };
         if (type == FVP_PRECON_BJILU0) {
-            if (stage) FVP_BJ_FACTOR(double, true, A->b_lu.p);
-            else FVP_BJ_FACTOR(double, false, A->b_lu.p);
+            if (ensure(A->b_lu, A->val_l, A->val_u, A->dinv)) return -1;
+            bj_factor_launch<double>(s, fa, A->b_lu.p, A->val_l.p, A->val_u.p, A->dinv.p);
         } else {
-            if (!A->b_lu32.p && A->b_lu32.alloc(A->b_lu.n)) return -1;
-            if (stage) FVP_BJ_FACTOR(float, true, A->b_lu32.p);
-            else FVP_BJ_FACTOR(float, false, A->b_lu32.p);
-        }
-#undef FVP_BJ_FACTOR
-        // packed solve values of the new factor
-        const long nl = (long)A->esrc_l.n, nu = (long)A->esrc_u.n, nd = (long)A->dsrc.n;
-        if (type == FVP_PRECON_BJILU0) {
-            if (!A->val_l.p && (A->val_l.alloc(nl) || A->val_u.alloc(nu) || A->dinv.alloc(nd))) return -1;
-            if (nl) bj_pack_vals<double><<<nblk(nl, 256), 256, 0, s>>>(nl, A->esrc_l.p, A->b_lu.p, A->val_l.p);
-            if (nu) bj_pack_vals<double><<<nblk(nu, 256), 256, 0, s>>>(nu, A->esrc_u.p, A->b_lu.p, A->val_u.p);
-            if (nd) bj_pack_vals<double><<<nblk(nd, 256), 256, 0, s>>>(nd, A->dsrc.p, A->b_lu.p, A->dinv.p);
-        } else {
-            if (!A->val32_l.p && (A->val32_l.alloc(nl) || A->val32_u.alloc(nu) || A->dinv32.alloc(nd))) return -1;
-            if (nl) bj_pack_vals<float><<<nblk(nl, 256), 256, 0, s>>>(nl, A->esrc_l.p, A->b_lu32.p, A->val32_l.p);
-            if (nu) bj_pack_vals<float><<<nblk(nu, 256), 256, 0, s>>>(nu, A->esrc_u.p, A->b_lu32.p, A->val32_u.p);
-            if (nd) bj_pack_vals<float><<<nblk(nd, 256), 256, 0, s>>>(nd, A->dsrc.p, A->b_lu32.p, A->dinv32.p);
+            if (ensure(A->b_lu32, A->val32_l, A->val32_u, A->dinv32)) return -1;
+            bj_factor_launch<float>(s, fa, A->b_lu32.p, A->val32_l.p, A->val32_u.p, A->dinv32.p);
         }
     } else if (type == FVP_PRECON_JACOBI) {
         if (A->jac.n != (size_t)n && A->jac.alloc(n)) return -1;
@@ -2216,7 +2687,14 @@ static int precon_build_impl(fvp_csr *A, int type) {
         }
         if (A->lu.n != (size_t)A->nnz && A->lu.alloc(A->nnz)) return -1;
         FVP_HIP(hipMemcpyAsync(A->lu.p, A->a.p, sizeof(double) * A->nnz, hipMemcpyDeviceToDevice, s));
-        for (size_t l = 0; l + 1 < A->lptr_h.size(); ++l) {
+        if (A->one) {
+            const int *fp = A->o_fptr.p;
+            double *vl = A->otri[0].val.p, *vu = A->otri[1].val.p;
+            bj_factor_launch<double>(s, FactorArgs{1, fp, A->ia.p, nullptr, nullptr, &A->ofac, fp + 2, fp + 4,
+                                                   A->flag.p, 0, 0},
+                                     A->lu.p, vl, vu, vu + (size_t)n * A->o_win);
+        }
+        for (size_t l = 0; !A->one && l + 1 < A->lptr_h.size(); ++l) {
             int cnt = A->lptr_h[l + 1] - A->lptr_h[l];
             ilu0_factor_level<<<nblk(cnt, 64), 64, 0, s>>>(cnt, A->lrows.p + A->lptr_h[l], A->ia.p, A->ja.p,
                                                            A->diag.p, A->lu.p, A->flag.p);
@@ -2231,13 +2709,29 @@ static int precon_build_impl(fvp_csr *A, int type) {
     return 0;
 }
 
-// y = M^-1 (x / xdiv) with xdiv optional (the block solves divide as they load);
-// yn2 (optional, at least nblk doubles): the block solves' partials of ||y||^2
+template <int KW, int TH>
+static void ilu0_one_launch_th(fvp_csr *A, const double *x, const double *xdiv, double *y, double *yn2) {
+    const IluTri &L = A->otri[0], &U = A->otri[1];
+    ilu0_solve<KW, TH><<<1, TH, A->o_lds, A->stream>>>(A->n, L.npieces, L.pptr.p, L.row.p, L.col.p, L.val.p,
+                                                       U.npieces, U.pptr.p, U.row.p, U.col.p, U.val.p, x, xdiv, y,
+                                                       yn2);
+}
+template <int KW>
+static void ilu0_one_launch(fvp_csr *A, const double *x, const double *xdiv, double *y, double *yn2) {
+    if (A->o_threads == 64) ilu0_one_launch_th<KW, 64>(A, x, xdiv, y, yn2);
+    else if (A->o_threads == 256) ilu0_one_launch_th<KW, 256>(A, x, xdiv, y, yn2);
+    else ilu0_one_launch_th<KW, 1024>(A, x, xdiv, y, yn2);
+}
+
+// y = M^-1 (x / xdiv) with xdiv optional (the block solves and the one-workgroup
+// ILU(0) divide as they load); yn2 (optional, at least nblk doubles): their
+// partials of ||y||^2
 static int precon_apply_impl(fvp_csr *A, const double *x, double *y, const double *xdiv, double *tmp,
                              double *yn2) {
     hipStream_t s = A->stream;
     const int n = A->n;
-    if (xdiv && A->ptype != FVP_PRECON_BJILU0 && A->ptype != FVP_PRECON_BJILU0_F32) {
+    const bool one = A->ptype == FVP_PRECON_ILU0 && A->one;
+    if (xdiv && A->ptype != FVP_PRECON_BJILU0 && A->ptype != FVP_PRECON_BJILU0_F32 && !one) {
         if (!tmp) { set_error("internal: scaled preconditioner solve needs a work vector"); return -1; }
         vdiv<<<nblk(n, 256), 256, 0, s>>>(n, x, xdiv, tmp);
         x = tmp;
@@ -2284,6 +2778,13 @@ static int precon_apply_impl(fvp_csr *A, const double *x, double *y, const doubl
         break;
     }
     case FVP_PRECON_ILU0: {
+        if (one) {
+            if (A->o_win == 4) ilu0_one_launch<4>(A, x, xdiv, y, yn2);
+            else if (A->o_win == 8) ilu0_one_launch<8>(A, x, xdiv, y, yn2);
+            else if (A->o_win == 16) ilu0_one_launch<16>(A, x, xdiv, y, yn2);
+            else ilu0_one_launch<32>(A, x, xdiv, y, yn2);
+            break;
+        }
         const int L = 8;
         for (size_t l = 0; l + 1 < A->lptr_h.size(); ++l) {
             int cnt = A->lptr_h[l + 1] - A->lptr_h[l];
@@ -2347,14 +2848,12 @@ extern "C" int fvp_csr_destroy(fvp_csr *A) {
     A->Hd.release(); A->gd.release(); A->csd.release(); A->snd.release(); A->yd.release(); A->Qk.release();
     if (A->hstat) (void)hipHostFree(A->hstat);
     for (hipEvent_t e : A->ev) (void)hipEventDestroy(e);
-    A->b_ia.release(); A->b_src.release(); A->b_diag.release(); A->b_ja.release(); A->b_lu.release(); A->b_lu32.release();
+    A->b_ia.release(); A->b_src.release(); A->b_lu.release(); A->b_lu32.release();
     A->b_roff.release(); A->b_rowid.release(); A->b_own.release(); A->b_zn2.release();
-    A->meta_l.release(); A->meta_u.release(); A->ebase_l.release(); A->ebase_u.release(); A->esrc_l.release();
-    A->esrc_u.release(); A->dsrc.release(); A->col_l.release(); A->col_u.release(); A->val_l.release();
+    A->meta_l.release(); A->meta_u.release(); A->ebase_l.release(); A->ebase_u.release();
+    A->col_l.release(); A->col_u.release(); A->val_l.release();
     A->val_u.release(); A->dinv.release(); A->val32_l.release(); A->val32_u.release(); A->dinv32.release();
-    A->b_lev_l.release(); A->b_lev_u.release(); A->b_lptr_l.release(); A->b_lptr_u.release();
-    A->b_rows_l.release(); A->b_rows_u.release();
-    A->fac_rec.release(); A->fac_pair.release(); A->fac_pbase.release();
+    A->fac.release(); A->ofac.release(); A->otri[0].release(); A->otri[1].release(); A->o_fptr.release();
     A->s_lev_l.release(); A->s_lev_u.release(); A->s_lptr_l.release(); A->s_lptr_u.release();
     A->ov_ptr.release(); A->ov_pos.release(); A->ov_tri.release();
     schur_free(A);
@@ -2452,7 +2951,7 @@ extern "C" int fvp_precon_values(fvp_csr *A, double *values_host) {
         return -1;
     } else if (A->ptype == FVP_PRECON_BJILU0 || A->ptype == FVP_PRECON_BJILU0_F32) {
         // scattered back to the full pattern, 0 off the blocks
-        std::vector<double> lu(A->b_lu.n);
+        std::vector<double> lu(A->b_src.n);
         std::vector<int> src(A->b_src.n);
         if (A->ptype == FVP_PRECON_BJILU0)
             FVP_HIP(hipMemcpy(lu.data(), A->b_lu.p, sizeof(double) * lu.size(), hipMemcpyDeviceToHost));
@@ -2807,16 +3306,18 @@ int precon_solve_div(fvp_ctx *c, const double *r, const double *rdiv, double *tm
     fvp_csr *A = c->jd->J;
     fvp_csr_set_stream(A, c->stream);
     const bool bj = A->ptype == FVP_PRECON_BJILU0 || A->ptype == FVP_PRECON_BJILU0_F32;
+    const bool one = A->ptype == FVP_PRECON_ILU0 && A->one;
+    const int np = bj ? A->nblk : one ? 1 : 0;
     double *part = nullptr;
-    if (zn2 && bj) {
-        if ((size_t)A->nblk > A->b_zn2.n && A->b_zn2.alloc(A->nblk)) return -1;
+    if (zn2 && np) {
+        if ((size_t)np > A->b_zn2.n && A->b_zn2.alloc(np)) return -1;
         part = A->b_zn2.p;
     }
     prof_mark(c, 2, 0);
     int rc = precon_apply_impl(A, r, z, rdiv, tmp, part);
     prof_mark(c, 2, 1);
     if (zn2) *zn2 = part;
-    if (zn2_count) *zn2_count = part ? A->nblk : 0;
+    if (zn2_count) *zn2_count = part ? np : 0;
     return rc;
 }
 }  // namespace fvp

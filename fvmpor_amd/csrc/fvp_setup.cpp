@@ -60,6 +60,8 @@ template struct DevBuf<double>;
 template struct DevBuf<unsigned short>;
 template struct DevBuf<float>;
 template struct DevBuf<long>;
+template struct DevBuf<uint2>;
+template struct DevBuf<uint4>;
 template struct DevBuf<unsigned>;
 
 static const int TRI_EDGE[3][2] = {{0, 1}, {1, 2}, {2, 0}};
