@@ -15,7 +15,15 @@ void set_error(const std::string &msg);
 
 constexpr int kMaxZones = 16;
 constexpr int kMaxTags = 1 << 16;
-constexpr int kTileNodes = 512;  // default nodes per tile of the tiled residual kernel
+constexpr int kTileNodes = 512;  // nodes per tile where the windows do not fit the LDS
+// Nodes per tile of the owner variant's windows.  Residual of 1 024 000 nodes in tiles
+// of 128 / 256 / 512: 127 / 106 / 108 us; 264 000: 41 / 41 / 44; 31 000: 16 / 18 / 22
+// (fewer tiles than CUs); 58 500 in 2D: 9.8 / 9.6 / 10.8.
+inline int default_tile_nodes(int n) { return n >= 65536 ? 256 : 128; }
+// Up to this many nodes the element kernel does the van Genuchten pass too: a launch
+// less (58 500 nodes in 2D: 9.7 against 11.6 us; 31 000 in 3D: 15.7 either way), where
+// larger problems pay more for evaluating the halo again (1 024 000: 135 against 106).
+constexpr int kFusedVgNodes = 65535;
 
 // Zone parameters passed by value to kernels: K_xx, K_yy, K_zz, phi, alpha, n, m, S_r, S_s.
 struct ZoneTable {
@@ -93,6 +101,11 @@ struct fvp_ctx {
     fvp::DevBuf<int> t_xptr, x_iptr, x_ilist, x_tgt;  // x_tgt: target node of each slot
     fvp::DevBuf<double> xf;
     long nexport = 0;
+    // owner variant from LDS windows (owner_lds): t_wptr / t_whalo hold each tile's halo,
+    // t_lconn the window-local nodes, x_ilist the export slot of each halo entry
+    bool owner_win = false, owner_vg = false;  // owner_vg: it does the van Genuchten pass too
+    fvp::DevBuf<int> x_inode;  // nodes with imports
+    int nimp = 0;
     fvp::DevBuf<int> t_wptr, t_whalo, t_vptr, t_tz;  // window halo nodes, visits, zones per tile
     fvp::DevBuf<unsigned short> t_lconn;             // 4 window-local node indices per visit
     int win_max = 0, ntz_max = 1;
@@ -158,6 +171,10 @@ int edge_areas(fvp_ctx *c);
 int residual_impl(fvp_ctx *c, double t, const double *psi, const double *psip, double *F, int averaging,
                   const JvArgs *jv = nullptr);
 int tile_kernel_attrs(fvp_ctx *c);
+constexpr int kOwnerStaticLds = 2048;         // owner_lds: zone tables and reductions
+constexpr size_t kOwnerLdsMax = 78 * 1024;    // its windows: two workgroups per CU
+size_t owner_window_lds(int dim, int wmax, int nr);
+int owner_window_code(int dim, int nr, int local, int rank);  // a corner's entry in t_lconn
 int upload_bc_values(fvp_ctx *c);
 int upload_dirichlet_values(fvp_ctx *c);
 void jac_free(fvp_ctx *c);

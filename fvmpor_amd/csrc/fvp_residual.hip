@@ -59,9 +59,55 @@ __device__ __forceinline__ void vg_eval(double h, const double *zp, double &Sw, 
     Sw = s; dSw = d; krw = k;
 }
 
-// One node per thread; the node's zones (its mask bits) are visited in a
-// per-lane loop with the zone parameters in LDS, so a wavefront pays for the
-// largest zone count of its nodes rather than for every zone any of them has.
+// Node i's zones (mask bits m, ascending): put(zone, rank among them, k_r) for
+// each; returns the CV-averaged capacity (without CAP: 0).
+template <bool CAP, typename Put>
+__device__ __forceinline__ double vg_node(int N, int i, double h, unsigned m, const double *zp,
+                                          const double *__restrict__ zw, double rho0, Put put) {
+    double phi = 0., Sw = 0., dSw = 0., Ss = 0.;
+    for (int r = 0; m; ++r) {
+        const int z = __ffs(m) - 1;
+        m &= m - 1;
+        const double *p = zp + 10 * z;
+        const double w = CAP ? zw[(size_t)z * N + i] : 0.;
+        double s, d, k;
+        vg_eval(h, p, s, d, k);
+        put(z, r, k);
+        if (CAP) {
+            phi += p[Z_PHI] * w;
+            Sw += s * w;
+            dSw += d * w;
+            Ss += p[Z_SS] * w;
+        }
+    }
+    return (phi * dSw + Ss * Sw) * rho0;
+}
+
+// The FD increment of J v from np partials of ||v||^2, in the fixed order of
+// jv_sigma_n2 (the same sigma bit for bit in every workgroup); red: one double
+// per wavefront.  Holds barriers; only thread 0's value is the increment.
+__device__ __forceinline__ double jv_sigma_block(const JvArgs &jv, double *red) {
+    // each lane's partials in order, four loads in flight at a time
+    double b = 0.;
+    const int bd = 256;
+    if (threadIdx.x < bd)
+        for (int k0 = threadIdx.x; k0 < jv.np; k0 += 4 * bd) {
+            double q[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) q[u] = k0 + u * bd < jv.np ? jv.part_v[k0 + u * bd] : 0.;
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (k0 + u * bd < jv.np) b += q[u];
+        }
+    b = block_sum(b, red);
+    return jv_sigma_of(jv.psi_n2[0], b);
+}
+
+// One node per thread, the zone parameters in LDS.  Nodes of several zones are set
+// aside in a list and done together afterwards: a per-lane loop over the zones made
+// every wavefront pay for the most zones any of its nodes has (1 024 000 nodes, a
+// quarter of them at layer boundaries: 41 us; 33 us with the list).  Bound by FP64
+// instructions (about 440 per node and zone).
 // JV with jv.np > 0: every workgroup reduces the np partials of ||v||^2 in the
 // fixed order of jv_sigma_n2 (the same sigma bit for bit) and workgroup 0
 // stores sigma for the finalisation, so no launch of its own is needed.
@@ -72,6 +118,10 @@ __global__ void __launch_bounds__(256) vg_kernel(int N, ZoneTable zt, double rho
                                                  double *__restrict__ nrec) {
     __shared__ double zp[kMaxZones * 10];
     __shared__ double red[4];
+    __shared__ int nlist;
+    __shared__ unsigned char list[256];
+    __shared__ double hlist[256];
+    if (threadIdx.x == 0) nlist = 0;
     if (threadIdx.x < 10 * zt.nz) zp[threadIdx.x] = zt.p[threadIdx.x / 10][threadIdx.x % 10];
     // the node's own inputs are loaded first: their latency overlaps sigma's reduction
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -81,21 +131,10 @@ __global__ void __launch_bounds__(256) vg_kernel(int N, ZoneTable zt, double rho
     unsigned m = live ? zmask[i] : 0u;
     double sg = 0.;
     if (JV && jv.np > 0) {
-        // each lane's partials in order, four loads in flight at a time
-        double b = 0.;
-        const int bd = blockDim.x;
-        for (int k0 = threadIdx.x; k0 < jv.np; k0 += 4 * bd) {
-            double q[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) q[u] = k0 + u * bd < jv.np ? jv.part_v[k0 + u * bd] : 0.;
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (k0 + u * bd < jv.np) b += q[u];
-        }
-        b = block_sum(b, red);  // ends with a barrier, so the zone table is in place
+        const double sigma = jv_sigma_block(jv, red);  // ends with a barrier, so the zone table is in place
         if (threadIdx.x == 0) {
-            red[0] = jv_sigma_of(jv.psi_n2[0], b);
-            if (blockIdx.x == 0) jv.sig_out[0] = red[0];
+            red[0] = sigma;
+            if (blockIdx.x == 0) jv.sig_out[0] = sigma;
         }
         __syncthreads();
         sg = red[0];
@@ -103,26 +142,28 @@ __global__ void __launch_bounds__(256) vg_kernel(int N, ZoneTable zt, double rho
         __syncthreads();
         if (JV) sg = jv.sig[0];
     }
-    if (!live) return;
     if (JV) h += sg * vi;
-    // the head of the node record the element kernel gathers (x, y, z are
-    // written once at set-up)
-    if (nrec) nrec[4 * (size_t)i + 3] = h;
-    double phi = 0., Sw = 0., dSw = 0., Ss = 0.;
-    while (m) {
-        const int z = __ffs(m) - 1;
-        m &= m - 1;
-        const double *p = zp + 10 * z;
-        const double w = zw[(size_t)z * N + i];
-        double s, d, k;
-        vg_eval(h, p, s, d, k);
-        kr[(size_t)z * N + i] = k;
-        phi += p[Z_PHI] * w;
-        Sw += s * w;
-        dSw += d * w;
-        Ss += p[Z_SS] * w;
+    auto evaluate = [&](int node, double hn, unsigned mn) {
+        cap[node] = vg_node<true>(N, node, hn, mn, zp, zw, rho0,
+                                  [&](int z, int, double k) { kr[(size_t)z * N + node] = k; });
+    };
+    if (live) {
+        // the head of the node record the element kernel gathers (x, y, z are
+        // written once at set-up)
+        if (nrec) nrec[4 * (size_t)i + 3] = h;
+        if (m & (m - 1)) {
+            const int k = atomicAdd(&nlist, 1);
+            list[k] = (unsigned char)threadIdx.x;
+            hlist[k] = h;
+        } else {
+            evaluate(i, h, m);
+        }
     }
-    cap[i] = (phi * dSw + Ss * Sw) * rho0;
+    __syncthreads();
+    if ((int)threadIdx.x < nlist) {
+        const int node = blockIdx.x * blockDim.x + list[threadIdx.x];
+        evaluate(node, hlist[threadIdx.x], zmask[node]);
+    }
 }
 
 __device__ __forceinline__ void load_pt(const double *__restrict__ xyz, int i, double &x, double &y, double &z) {
@@ -462,6 +503,251 @@ __global__ void __launch_bounds__(1024) owner_finalize(
     }
 }
 
+// t ? x : y for the sign-extended bit t (0 or ~0), on the two halves
+__device__ __forceinline__ double half_select(unsigned t, double x, double y) {
+    const long long a = __double_as_longlong(x), b = __double_as_longlong(y);
+    const unsigned lo = ((unsigned)a & t) | ((unsigned)b & ~t);
+    const unsigned hi = ((unsigned)(a >> 32) & t) | ((unsigned)(b >> 32) & ~t);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// The face fluxes of element_fluxes_vals<DIM, 0>, with fewer operations: gravity is
+// added to the head differences (so a hydrostatic element cancels before the
+// gradient is formed), rho0 / (d! (d + 1)) comes with the conductivities (kz), the
+// sign of det cancels, and node 0's gradient and flux are minus the others' sums.
+template <int DIM>
+__device__ __forceinline__ void upwind_fluxes(const NodeVals<DIM> &nv, const double *kz, double km, unsigned mask,
+                                              double (&f)[DIM + 1]) {
+    const double *px = nv.px, *py = nv.py, *pz = nv.pz, *h = nv.h;
+    double g[DIM + 1];
+    const double ux = px[1] - px[0], uy = py[1] - py[0], vx = px[2] - px[0], vy = py[2] - py[0];
+    if (DIM == 3) {
+        const double uz = pz[1] - pz[0], vz = pz[2] - pz[0];
+        const double wx = px[3] - px[0], wy = py[3] - py[0], wz = pz[3] - pz[0];
+        const double a1 = vy * wz - vz * wy, b1 = vz * wx - vx * wz, c1 = vx * wy - vy * wx;
+        const double a2 = wy * uz - wz * uy, b2 = wz * ux - wx * uz, c2 = wx * uy - wy * ux;
+        const double a3 = uy * vz - uz * vy, b3 = uz * vx - ux * vz, c3 = ux * vy - uy * vx;
+        const double det = ux * a1 + uy * b1 + uz * c1;
+        const double d1 = (h[1] - h[0]) + uz, d2 = (h[2] - h[0]) + vz, d3 = (h[3] - h[0]) + wz;
+        const double t = km / fabs(det);
+        const double qx = (d1 * a1 + d2 * a2 + d3 * a3) * (kz[0] * t);
+        const double qy = (d1 * b1 + d2 * b2 + d3 * b3) * (kz[1] * t);
+        const double qz = (d1 * c1 + d2 * c2 + d3 * c3) * (kz[2] * t);
+        g[1] = a1 * qx + b1 * qy + c1 * qz;
+        g[2] = a2 * qx + b2 * qy + c2 * qz;
+        g[DIM] = a3 * qx + b3 * qy + c3 * qz;
+        g[0] = -(g[1] + g[2] + g[DIM]);
+    } else {
+        const double det = ux * vy - uy * vx;
+        const double d1 = (h[1] - h[0]) + uy, d2 = (h[2] - h[0]) + vy;
+        const double t = km / fabs(det);
+        // gradients of N_1, N_2 times det: (vy, -vx), (-uy, ux)
+        const double qx = (d1 * vy - d2 * uy) * (kz[0] * t), qy = (d2 * ux - d1 * vx) * (kz[1] * t);
+        g[1] = vy * qx - vx * qy;
+        g[2] = ux * qy - uy * qx;
+        g[0] = -(g[1] + g[2]);
+    }
+#pragma unroll
+    for (int k = 0; k < DIM + 1; ++k) f[k] = 0.;
+#pragma unroll
+    for (int j = 0; j < (DIM == 2 ? 3 : 6); ++j) {
+        const int a = edge_a(j), b = edge_b(j);
+        const double kr = half_select((unsigned)((int)(mask << (31 - j)) >> 31), nv.k[a], nv.k[b]);
+        const double d = g[b] - g[a];
+        f[a] += kr * d;
+        f[b] -= kr * d;
+    }
+}
+
+// Element-owner residual from LDS windows.  A workgroup owns the nodes of one tile
+// and evaluates the tile's primary elements (lowest node in the tile), once each.
+// It stages one LDS record per node of those elements' window (owned nodes, then
+// the halo: higher nodes of other tiles): coordinates, head, flux sum and k_r per
+// rank of the node's zones.  Elements then need 18 streamed bytes each and take the
+// rest from LDS (per corner the record's place in 14 bits, the rank of the element's
+// zone there in 2).  Halo sums leave as one export per (tile, halo node), its slot
+// grouped by target node.  An owned node without imports is finished here; the
+// others' sums go to acc and owner_imports.
+// VG: the van Genuchten pass is part of the staging (owned nodes write the capacity,
+// halo nodes are evaluated again); otherwise k_r comes from vg_kernel.  Nodes of
+// several zones are set aside in a list and done afterwards, as there.
+// Bound by the LDS (268 cycles per 64 elements: 16-byte record reads and four sums)
+// and the phases' latency.  1 024 000 nodes, 512-node tiles: 76 us, with vg_kernel 33
+// and owner_imports 8 us more.  Gathering from memory through the L1 (owner_kernel,
+// kept for windows that do not fit) with a finalisation of its own: 120 + 41 + 33 us.
+constexpr int kRecBits = 14, kRecRanks = 4;
+
+// doubles per window record: DIM coordinates, head, sum, k_r per rank; odd, so that
+// records start in all banks
+__host__ __device__ inline int win_stride(int dim, int nr) { return (dim + 2 + nr) | 1; }
+
+template <int DIM, bool JV, bool VG, int TH>
+__global__ void __launch_bounds__(TH) owner_lds(
+    int N, int ntiles, int tile_nodes, int per_xcd, int wmax, int nr, ZoneTable zt, double rho0,
+    const uint8_t *__restrict__ ezone, const double *__restrict__ kmul, const uint8_t *__restrict__ emask,
+    const ushort4 *__restrict__ lconn, const double *__restrict__ xyz, const double *__restrict__ psi,
+    const uint8_t *__restrict__ zmask, const double *__restrict__ zw, const double *__restrict__ kr,
+    const int *__restrict__ eptr, const int *__restrict__ wptr, const int *__restrict__ whalo,
+    const int *__restrict__ xdst,
+    double *__restrict__ xf, const int *__restrict__ iptr, const int *__restrict__ bptr,
+    const int *__restrict__ bnode, const double *__restrict__ bval, const double *__restrict__ invV,
+    const double *__restrict__ psip, double *__restrict__ cap, double *__restrict__ acc_g, double *__restrict__ F,
+    JvArgs jv) {
+    constexpr int kH = DIM, kAcc = DIM + 1, kK = DIM + 2;
+    extern __shared__ __align__(16) double sm[];
+    __shared__ double zk[3 * kMaxZones], zp[VG ? 10 * kMaxZones : 1];
+    __shared__ double red[16];
+    __shared__ int nlist;
+    const int tile = per_xcd ? (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3) : blockIdx.x;
+    if (tile >= ntiles) return;  // uniform for the whole workgroup
+    const int lo = tile * tile_nodes, hi = min(N, lo + tile_nodes), nown = hi - lo;
+    const int w0 = wptr[tile], win = nown + wptr[tile + 1] - w0;
+    const int stride = win_stride(DIM, nr);
+    unsigned short *const list = reinterpret_cast<unsigned short *>(sm + wmax * stride);
+    const double c0 = rho0 / (DIM == 3 ? 24.0 : 6.0);
+    for (int k = threadIdx.x; k < 3 * zt.nz; k += TH) zk[k] = zt.p[k / 3][ZK_X + k % 3] * c0;
+    if (VG)
+        for (int k = threadIdx.x; k < 10 * zt.nz; k += TH) zp[k] = zt.p[k / 10][k % 10];
+    if (threadIdx.x == 0) nlist = 0;
+    double sig = 0.;
+    if (JV && VG && jv.np > 0) {
+        const double sigma = jv_sigma_block(jv, red);
+        if (threadIdx.x == 0) {
+            red[0] = sigma;
+            if (blockIdx.x == 0) jv.sig_out[0] = sigma;
+        }
+        __syncthreads();
+        sig = red[0];
+    } else {
+        __syncthreads();  // the zone tables
+        if (JV) sig = jv.sig[0];
+    }
+    auto node_of = [&](int i) { return i < nown ? lo + i : whalo[w0 + i - nown]; };
+    auto evaluate = [&](int i, int g, double h, unsigned m) {
+        double *const rec = sm + i * stride;
+        auto put = [&](int, int r, double k) { rec[kK + r] = k; };
+        if (i < nown) cap[g] = vg_node<true>(N, g, h, m, zp, zw, rho0, put);
+        else vg_node<false>(N, g, h, m, zp, zw, rho0, put);
+    };
+    for (int i = threadIdx.x; i < win; i += TH) {
+        const int g = node_of(i);
+        double h = psi[g];
+        if (JV) h += sig * jv.v[g];
+        const unsigned m = zmask[g];
+        double *const rec = sm + i * stride;
+        double x, y, z;
+        load_pt(xyz, g, x, y, z);
+        rec[0] = x;
+        rec[1] = y;
+        if (DIM == 3) rec[2] = z;
+        rec[kH] = h;
+        rec[kAcc] = 0.;
+        if (VG) {
+            if (m & (m - 1)) list[atomicAdd(&nlist, 1)] = (unsigned short)i;
+            else evaluate(i, g, h, m);
+        } else {
+            unsigned q = m;
+            for (int r = 0; q; ++r, q &= q - 1) rec[kK + r] = kr[(size_t)(__ffs(q) - 1) * N + g];
+        }
+    }
+    __syncthreads();
+    if (VG) {
+        for (int k = threadIdx.x; k < nlist; k += TH) {
+            const int i = list[k], g = node_of(i);
+            evaluate(i, g, sm[i * stride + kH], zmask[g]);
+        }
+        __syncthreads();
+    }
+    constexpr int NPE = DIM + 1;
+    const int e1 = eptr[tile + 1];
+    int e = eptr[tile] + threadIdx.x;
+    if (e < e1) {
+        // the next element's stream is in flight while this one is evaluated
+        ushort4 lc = lconn[e];
+        int z = ezone[e];
+        double km = kmul[e];
+        unsigned mask = emask[e];
+        for (; e < e1; e += TH) {
+            const int en = min(e + TH, e1 - 1);
+            const ushort4 ln = lconn[en];
+            const int zn = ezone[en];
+            const double kn = kmul[en];
+            const unsigned mn = emask[en];
+            const unsigned l[4] = {lc.x, lc.y, lc.z, lc.w};
+            NodeVals<DIM> nv;
+            double *rec[NPE];
+#pragma unroll
+            for (int q = 0; q < NPE; ++q) {
+                rec[q] = sm + (l[q] & ((1u << kRecBits) - 1));
+                nv.px[q] = rec[q][0];
+                nv.py[q] = rec[q][1];
+                nv.pz[q] = DIM == 3 ? rec[q][2] : 0.;
+                nv.h[q] = rec[q][kH];
+                nv.k[q] = rec[q][kK + (l[q] >> kRecBits)];
+            }
+            double f[NPE];
+            upwind_fluxes<DIM>(nv, zk + 3 * z, km, mask, f);
+#pragma unroll
+            for (int q = 0; q < NPE; ++q) atomicAdd(rec[q] + kAcc, f[q]);
+            lc = ln;
+            z = zn;
+            km = kn;
+            mask = mn;
+        }
+    }
+    __syncthreads();
+    for (int k = bptr[tile] + threadIdx.x; k < bptr[tile + 1]; k += TH)
+        sm[(bnode[k] - lo) * stride + kAcc] -= bval[k];
+    __syncthreads();
+    for (int i = threadIdx.x; i < nown; i += TH) {
+        const int g = lo + i;
+        const double a = sm[i * stride + kAcc];
+        if (iptr[g] != iptr[g + 1]) {
+            acc_g[g] = a;
+            continue;
+        }
+        if (JV) {
+            const double yp = psip[g] + jv.cj * (sig * jv.v[g]);
+            const double F1 = a * invV[g] - yp * cap[g];
+            F[g] = jv_scaled(jv, g, (F1 - jv.F0[g]) / sig);
+        } else
+            F[g] = a * invV[g] - psip[g] * cap[g];
+    }
+    for (int i = nown + threadIdx.x; i < win; i += TH) xf[xdst[w0 + i - nown]] = sm[i * stride + kAcc];
+}
+
+// The nodes with imports (inode, ascending): their own sums plus their slots in
+// order, then the finalisation.
+template <bool JV>
+__global__ void __launch_bounds__(256) owner_imports(int nimp, const int *__restrict__ inode,
+                                                     const double *__restrict__ acc, const int *__restrict__ iptr,
+                                                     const double *__restrict__ xf, const double *__restrict__ invV,
+                                                     const double *__restrict__ psip, const double *__restrict__ cap,
+                                                     double *__restrict__ F, JvArgs jv) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= nimp) return;
+    const int i = inode[k];
+    const int s0 = iptr[i], s1 = iptr[i + 1];
+    double a = acc[i];
+    const double iv = invV[i], p = psip[i], c = cap[i];
+    const double sig = JV ? jv.sig[0] : 0., v = JV ? jv.v[i] : 0., f0 = JV ? jv.F0[i] : 0.;
+    // four slots in flight at a time
+    for (int s = s0; s < s1; s += 4) {
+        double q[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) q[u] = xf[min(s + u, s1 - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (s + u < s1) a += q[u];
+    }
+    if (JV) {
+        const double yp = p + jv.cj * (sig * v);
+        const double F1 = a * iv - yp * c;
+        F[i] = jv_scaled(jv, i, (F1 - f0) / sig);
+    } else
+        F[i] = a * iv - p * c;
+}
+
 // LDS-staged owner-computes residual.  A workgroup owns tile_nodes nodes; it
 // stages the coordinates, heads and relative permeabilities of its window (owned
 // nodes plus the halo nodes its elements reach) in LDS with coalesced loads for
@@ -739,6 +1025,16 @@ __global__ void mask_kernel(int T, const int *__restrict__ eedge, const uint8_t 
 
 static inline int blocks(long n, int bs) { return (int)((n + bs - 1) / bs); }
 
+// Dynamic LDS of owner_lds for windows of wmax nodes with up to nr zones per node
+// (0: not used): the records have to fit the elements' 14 + 2 bits and half of the LDS
+// (two workgroups per CU).
+size_t owner_window_lds(int dim, int wmax, int nr) {
+    const long recs = (long)wmax * win_stride(dim, nr);
+    const size_t bytes = sizeof(double) * recs + 2 * (size_t)((wmax + 3) & ~3);
+    return nr <= kRecRanks && recs <= 1 << kRecBits && bytes <= kOwnerLdsMax ? bytes : 0;
+}
+int owner_window_code(int dim, int nr, int local, int rank) { return local * win_stride(dim, nr) | (rank << kRecBits); }
+
 // Allow the tile kernel's dynamic LDS beyond the default limit; fails cleanly if
 // the device cannot provide it.
 int tile_kernel_attrs(fvp_ctx *c) {
@@ -759,13 +1055,57 @@ int tile_kernel_attrs(fvp_ctx *c) {
     FVP_HIP(hipFuncSetAttribute((const void *)tile_lds_kernel<2, false>, hipFuncAttributeMaxDynamicSharedMemorySize, dyn));
     FVP_HIP(hipFuncSetAttribute((const void *)tile_lds_kernel<3, true>, hipFuncAttributeMaxDynamicSharedMemorySize, dyn));
     FVP_HIP(hipFuncSetAttribute((const void *)tile_lds_kernel<2, true>, hipFuncAttributeMaxDynamicSharedMemorySize, dyn));
+    for (const void *f : {(const void *)owner_lds<2, false, false, 256>, (const void *)owner_lds<2, false, true, 256>,
+                          (const void *)owner_lds<2, true, false, 256>, (const void *)owner_lds<2, true, true, 256>,
+                          (const void *)owner_lds<3, false, false, 256>, (const void *)owner_lds<3, false, true, 256>,
+                          (const void *)owner_lds<3, true, false, 256>, (const void *)owner_lds<3, true, true, 256>,
+                          (const void *)owner_lds<2, false, false, 512>, (const void *)owner_lds<2, false, true, 512>,
+                          (const void *)owner_lds<2, true, false, 512>, (const void *)owner_lds<2, true, true, 512>,
+                          (const void *)owner_lds<3, false, false, 512>, (const void *)owner_lds<3, false, true, 512>,
+                          (const void *)owner_lds<3, true, false, 512>, (const void *)owner_lds<3, true, true, 512>})
+        FVP_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds_max - kOwnerStaticLds));
     return 0;
+}
+
+template <int DIM, bool JV>
+static void launch_owner_lds(fvp_ctx *c, const double *psi, const double *psip, double *F, const JvArgs &jv) {
+    const int per = (c->ntiles + 7) / 8;
+    hipStream_t s = c->stream;
+    hipEvent_t ea, eb;
+    prof_pair(c, JV ? 3 : 0, &ea, &eb);
+    // 512 threads (31 000 nodes in tiles of 128: 15.7 us against 16.8 with 256; 1 024 000
+    // in tiles of 256: 106 against 122), 256 for the smallest tiles
+    const int threads = c->tile_nodes >= 128 ? 512 : 256;
+    const auto kernel = threads == 512 ? (c->owner_vg ? owner_lds<DIM, JV, true, 512> : owner_lds<DIM, JV, false, 512>)
+                                       : (c->owner_vg ? owner_lds<DIM, JV, true, 256> : owner_lds<DIM, JV, false, 256>);
+    hipExtLaunchKernelGGL(kernel, dim3(c->xcd_map ? per * 8 : c->ntiles), dim3(threads), c->tile_lds, s, ea,
+                          eb, 0, c->N, c->ntiles, c->tile_nodes, c->xcd_map ? per : 0, c->win_max, c->ntz_max, c->zt,
+                          c->rho0, (const uint8_t *)c->ezone.p, (const double *)c->kmul.p,
+                          (const uint8_t *)c->emask.p, (const ushort4 *)c->t_lconn.p, (const double *)c->xyz.p, psi,
+                          (const uint8_t *)c->zmask.p, (const double *)c->zw.p, (const double *)c->kr.p,
+                          (const int *)c->t_eptr.p, (const int *)c->t_wptr.p, (const int *)c->t_whalo.p, (const int *)c->x_ilist.p, c->xf.p,
+                          (const int *)c->x_iptr.p, (const int *)c->t_bptr.p, (const int *)c->bnode.p,
+                          (const double *)c->bval.p, (const double *)c->invV.p, psip, c->cap.p, c->acc.p, F, jv);
+    if (c->nimp)
+        owner_imports<JV><<<blocks(c->nimp, 256), 256, 0, s>>>(c->nimp, c->x_inode.p, c->acc.p, c->x_iptr.p, c->xf.p,
+                                                               c->invV.p, psip, c->cap.p, F, jv);
+    if (c->ndir)
+        dirichlet_kernel<JV><<<blocks(c->ndir, 256), 256, 0, s>>>(c->ndir, c->dnode.p, c->dval.p, psi, F, jv);
 }
 
 template <int DIM, bool JV>
 static void launch_tile(fvp_ctx *c, const double *psi, const double *psip, double *F, const JvArgs &jv) {
     const int per = (c->ntiles + 7) / 8;  // tiles per XCD: consecutive tiles share an XCD's L2
     hipStream_t s = c->stream;
+    if (c->owner_win) {
+        // the tiles read their halo's psi and v while others write F: a result in place
+        // of either goes through a work vector
+        auto meets = [&](const double *p) { return p && F < p + c->N && p < F + c->N; };
+        const bool in_place = meets(psi) || meets(jv.v);
+        launch_owner_lds<DIM, JV>(c, psi, psip, in_place ? c->tmp1.p : F, jv);
+        if (in_place) (void)hipMemcpyAsync(F, c->tmp1.p, sizeof(double) * c->N, hipMemcpyDeviceToDevice, s);
+        return;
+    }
     if (c->rvariant == FVP_RESIDUAL_OWNER) {
         const int N = c->N;
         // one workgroup per tile, wide enough that large tiles still fill the CUs; when
@@ -1055,12 +1395,14 @@ int residual_impl(fvp_ctx *c, double t, const double *psi, const double *psip, d
     }
     ++c->nres;
     prof_mark(c, 1, 0);
-    if (jv)
+    const bool fused = c->owner_win && c->owner_vg && !averaging;  // the element kernel does the van Genuchten pass
+    double *const nrec = c->rvariant == FVP_RESIDUAL_OWNER && !c->owner_win ? c->nrec.p : nullptr;
+    if (jv && !fused)
         vg_kernel<true><<<blocks(N, 256), 256, 0, s>>>(N, c->zt, c->rho0, psi, c->zmask.p, c->zw.p, c->kr.p,
-                                                        c->cap.p, *jv, c->nrec.p);
-    else
+                                                        c->cap.p, *jv, nrec);
+    else if (!fused)
         vg_kernel<false><<<blocks(N, 256), 256, 0, s>>>(N, c->zt, c->rho0, psi, c->zmask.p, c->zw.p, c->kr.p,
-                                                         c->cap.p, JvArgs(), c->rvariant == FVP_RESIDUAL_OWNER ? c->nrec.p : nullptr);
+                                                         c->cap.p, JvArgs(), nrec);
     if (!averaging) {
         // tiled paths (element fluxes with the boundary fluxes, then the finalisation)
         const JvArgs none;

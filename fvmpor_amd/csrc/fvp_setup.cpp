@@ -225,7 +225,77 @@ int build_tiles(fvp_ctx *c, int TILE) {
         // element-owner variant: contributions of a tile's elements to nodes of
         // other tiles are stored in export slots (numbered per tile, element order,
         // local node order) and gathered by their nodes in the finalisation
+        c->owner_win = false;
         if (!window) {
+            // LDS windows where every tile's fits: the halo of a tile's primary elements
+            // (all its nodes are past the tile), window-local connectivity, one export
+            // per (tile, halo node)
+            std::vector<int> owptr(nt + 1, 0), owhalo;
+            int owmax = 0, nr = 1;
+            std::vector<uint8_t> zm(N);
+            FVP_HIP(hipMemcpy(zm.data(), c->zmask.p, N, hipMemcpyDeviceToHost));
+            for (int i = 0; i < N; ++i) nr = std::max(nr, __builtin_popcount(zm[i]));
+            for (int t = 0; t < nt; ++t) {
+                const int lo = t * TILE, hi = std::min(N, lo + TILE);
+                const size_t h0 = owhalo.size();
+                long run = 0;
+                for (int e = eptr[t]; e < eptr[t + 1]; ++e) {
+                    const int4 q = conn4[e];
+                    const int n[4] = {q.x, q.y, q.z, q.w};
+                    if (run > 65535) { set_error("a residual tile exports more than 65535 contributions"); return -1; }
+                    for (int k = 0; k < npe; ++k)
+                        if (n[k] < lo || n[k] >= hi) {
+                            ++run;
+                            if (mark[n[k]] != t) { mark[n[k]] = t; owhalo.push_back(n[k]); }
+                        }
+                }
+                std::sort(owhalo.begin() + h0, owhalo.end());
+                owptr[t + 1] = (int)owhalo.size();
+                owmax = std::max(owmax, hi - lo + (int)(owhalo.size() - h0));
+            }
+            const size_t bytes = owner_window_lds(c->dim, owmax, nr);
+            c->owner_win = bytes > 0;
+            c->owner_vg = N <= kFusedVgNodes;
+            std::vector<int> iptr(N + 1, 0);
+            if (c->owner_win) {
+                std::vector<unsigned short> lc(4 * (size_t)T, 0);
+                for (int t = 0; t < nt; ++t) {
+                    const int lo = t * TILE, hi = std::min(N, lo + TILE);
+                    for (int j = owptr[t]; j < owptr[t + 1]; ++j) loc[owhalo[j]] = hi - lo + j - owptr[t];
+                    for (int e = eptr[t]; e < eptr[t + 1]; ++e) {
+                        const int4 q = conn4[e];
+                        const int n[4] = {q.x, q.y, q.z, q.w};
+                        for (int k = 0; k < npe; ++k) {
+                            const int l = n[k] < hi ? n[k] - lo : loc[n[k]];
+                            const int rank = __builtin_popcount(zm[n[k]] & ((1u << ez[e]) - 1));
+                            lc[4 * (size_t)e + k] = (unsigned short)owner_window_code(c->dim, nr, l, rank);
+                        }
+                    }
+                }
+                std::vector<int> xdst(owhalo.size()), inode;
+                for (int tn : owhalo) iptr[tn + 1]++;
+                for (int i = 0; i < N; ++i) {
+                    if (iptr[i + 1]) inode.push_back(i);
+                    iptr[i + 1] += iptr[i];
+                }
+                std::vector<int> fill(iptr.begin(), iptr.end() - 1);
+                for (size_t k = 0; k < owhalo.size(); ++k) xdst[k] = fill[owhalo[k]]++;
+                c->nexport = (long)owhalo.size();
+                c->nimp = (int)inode.size();
+                c->win_max = owmax;
+                c->ntz_max = nr;
+                c->tile_lds = bytes;
+                c->t_xoff.release(); c->t_xptr.release(); c->x_tgt.release();
+                if (c->t_wptr.upload(owptr.data(), nt + 1) || c->t_whalo.upload(owhalo.data(), owhalo.size()) ||
+                    c->t_lconn.upload(lc.data(), lc.size()) || c->x_iptr.upload(iptr.data(), N + 1) ||
+                    c->x_ilist.upload(xdst.data(), xdst.size()) || c->x_inode.upload(inode.data(), inode.size()) ||
+                    c->xf.alloc(std::max<size_t>(1, owhalo.size())))
+                    return -1;
+            }
+        }
+        if (!window && !c->owner_win) {
+            c->x_inode.release();
+            c->nimp = 0;
             std::vector<unsigned short> xoff(T);
             std::vector<int> xptr(nt + 1, 0), target;
             for (int t = 0; t < nt; ++t) {
@@ -256,10 +326,11 @@ int build_tiles(fvp_ctx *c, int TILE) {
                 c->x_iptr.upload(iptr.data(), N + 1) || c->x_ilist.upload(xdst.data(), xdst.size()) ||
                 c->x_tgt.upload(xtgt.data(), xtgt.size()) || c->xf.alloc(std::max<size_t>(1, target.size())))
                 return -1;
-        } else {
+        } else if (window) {
             c->t_xoff.release(); c->t_xptr.release(); c->x_iptr.release(); c->x_ilist.release(); c->xf.release();
-            c->x_tgt.release();
+            c->x_tgt.release(); c->x_inode.release();
             c->nexport = 0;
+            c->nimp = 0;
         }
     }
     c->tile_nodes = TILE;
@@ -585,7 +656,10 @@ extern "C" int fvp_create(const fvp_problem *p, int device, fvp_ctx **out) {
         c->ndir = (int)dn.size();
         if (c->dnode.upload(dn.data(), dn.size()) || upload_dirichlet_values(c)) return fail();
     }
-    if (build_tiles(c, c->tile_nodes) || edge_areas(c)) return fail();
+    if (build_tiles(c, default_tile_nodes(N))) return fail();
+    // node orders whose windows do not fit the LDS keep the larger tiles of the kernel that gathers
+    if (!c->owner_win && build_tiles(c, kTileNodes)) return fail();
+    if (edge_areas(c)) return fail();
     if (c->tmp1.alloc(N) || c->tmp2.alloc(N) || c->tmp3.alloc(N) || c->red.alloc(4096)) return fail();
     c->red_h.resize(4096);
     *out = c;
@@ -604,7 +678,7 @@ extern "C" int fvp_destroy(fvp_ctx *c) {
     c->dval.release(); c->t_wptr.release(); c->t_whalo.release(); c->t_vptr.release(); c->t_lconn.release();
     c->t_tz.release(); c->t_eptr.release(); c->t_hptr.release(); c->t_hlist.release(); c->t_bptr.release();
     c->t_dptr.release(); c->t_xoff.release(); c->t_xptr.release(); c->x_iptr.release(); c->x_ilist.release();
-    c->x_tgt.release();
+    c->x_tgt.release(); c->x_inode.release();
     c->xf.release(); c->eedge.release(); c->slot_ptr.release(); c->slot.release(); c->qface.release();
     c->ea.release(); c->eflux.release(); c->wf.release(); c->tmp1.release(); c->tmp2.release();
     c->tmp3.release(); c->red.release();
