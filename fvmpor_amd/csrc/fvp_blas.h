@@ -47,9 +47,10 @@ int host_wait(hipStream_t s, hipEvent_t ev);
 using Op = std::function<int(const double *, double *)>;
 // Restarted right-preconditioned GMRES on A x = b; W supplies the workspace.
 // x_zero: the caller has set x = 0, so the first residual is b itself (no
-// product with A).
+// product with A).  diag: M is the product with this vector, and is not called.
 int gmres_device(fvp_csr *W, hipStream_t s, long n, const Op &A, const Op &M, const double *b, double *x,
-                 const fvp_gmres_params *p, fvp_gmres_stats *st, bool x_zero = false);
+                 const fvp_gmres_params *p, fvp_gmres_stats *st, bool x_zero = false,
+                 const double *diag = nullptr);
 // the context's Jacobian handle (built on first use)
 fvp_csr *jacobian_handle(fvp_ctx *c);
 }  // namespace fvp

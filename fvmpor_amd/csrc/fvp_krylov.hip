@@ -20,6 +20,7 @@
 #include <array>
 #include <cmath>
 #include <complex>
+#include <cstring>
 #include <functional>
 #include <mutex>
 #include <numeric>
@@ -115,9 +116,9 @@ struct fvp_csr {
     int m_alloc = -1;
     DevBuf<double> Q, w, r, z, part, scal, hdev;
     DevBuf<double> Hd, gd, csd, snd, yd;    // Hessenberg (column-major, m+1 rows), Givens pairs, rhs, solution
-    double *hstat = nullptr;                // pinned host: per Arnoldi step {residual estimate, h_{j+1,j}}
+    double *hstat = nullptr;                // pinned host: slots of kSlot doubles, see GmresWork
+    double tag = 0;                         // last tag given to a slot's writer
     DevBuf<double> Qk;                      // deflated GMRES: the kept harmonic Ritz vectors
-    std::vector<hipEvent_t> ev;             // per Arnoldi step: its status copy has landed
     fvp_schur *sc = nullptr;                // Schur-complement preconditioner (FVP_PRECON_SCHUR)
 };
 
@@ -261,6 +262,10 @@ __global__ void vscale_inv_norm(long n, const double *__restrict__ src, const do
     if (i < n) dst[i] = src[i] * (1. / sqrt(nsq[0]));
 }
 
+// compiler-only ordering of one wavefront's LDS accesses (the LDS executes a
+// wavefront's accesses in issue order; no wait for outstanding memory loads)
+__device__ __forceinline__ void wave_lds_order() { asm volatile("" ::: "memory"); }
+
 constexpr int kChunk = 16;  // basis columns per Gram-Schmidt dot pass
 
 __device__ __forceinline__ double wave_reduce(double v) {
@@ -383,47 +388,6 @@ __global__ void __launch_bounds__(kThreads) axpy_norm(long n, double *__restrict
     block_partial(acc, part + blockIdx.x);
 }
 
-// The first pass's update and the second pass's dots in one read of the basis:
-// w -= Q[:, 0..NC) coef, then block partials of Q[:, c] . w (c < NC) and of
-// w . w (column NC) on the updated w.
-template <int NC>
-__global__ void __launch_bounds__(kThreads) axpy_mdot(long n, double *__restrict__ w, const double *__restrict__ Q,
-                                                      long ldq, const double *__restrict__ coef,
-                                                      double *__restrict__ part) {
-    double h[NC], acc[NC + 1];
-#pragma unroll
-    for (int c = 0; c < NC; ++c) h[c] = coef[c];
-#pragma unroll
-    for (int c = 0; c <= NC; ++c) acc[c] = 0.;
-    const long np = n >> 1;
-    for (long p = blockIdx.x * (long)blockDim.x + threadIdx.x; p < np; p += (long)gridDim.x * blockDim.x) {
-        double2 q[NC];
-#pragma unroll
-        for (int c = 0; c < NC; ++c) q[c] = reinterpret_cast<const double2 *>(Q + c * ldq)[p];
-        double2 a = reinterpret_cast<double2 *>(w)[p];
-        double sx = 0., sy = 0.;
-#pragma unroll
-        for (int c = 0; c < NC; ++c) { sx += h[c] * q[c].x; sy += h[c] * q[c].y; }
-        a.x -= sx;
-        a.y -= sy;
-        reinterpret_cast<double2 *>(w)[p] = a;
-#pragma unroll
-        for (int c = 0; c < NC; ++c) acc[c] += a.x * q[c].x + a.y * q[c].y;
-        acc[NC] += a.x * a.x + a.y * a.y;
-    }
-    if ((n & 1) && blockIdx.x == 0 && threadIdx.x == 0) {
-        double qt[NC], sx = 0.;
-#pragma unroll
-        for (int c = 0; c < NC; ++c) { qt[c] = Q[c * ldq + n - 1]; sx += h[c] * qt[c]; }
-        const double a = w[n - 1] - sx;
-        w[n - 1] = a;
-#pragma unroll
-        for (int c = 0; c < NC; ++c) acc[c] += a * qt[c];
-        acc[NC] += a * a;
-    }
-    block_partials<NC + 1>(acc, NC + 1, part);
-}
-
 using MdotLaunch = void (*)(hipStream_t, int, long, const double *, const double *, long, int, double *,
                            const double *);
 using AxpyLaunch = void (*)(hipStream_t, int, long, double *, const double *, long, const double *, double *,
@@ -438,15 +402,6 @@ static void axpy_launch(hipStream_t s, int nb, long n, double *w, const double *
                         double *part, const double *skip) {
     axpy_norm<NC><<<nb, kThreads, 0, s>>>(n, w, Q, ldq, coef, part, skip);
 }
-template <int NC>
-static void axpy_mdot_launch(hipStream_t s, int nb, long n, double *w, const double *Q, long ldq, const double *coef,
-                             double *part, const double *) {
-    axpy_mdot<NC><<<nb, kThreads, 0, s>>>(n, w, Q, ldq, coef, part);
-}
-template <int... I>
-static constexpr std::array<AxpyLaunch, sizeof...(I)> axpy_mdot_table(std::integer_sequence<int, I...>) {
-    return {&axpy_mdot_launch<I + 1>...};
-}
 template <int... I>
 static constexpr std::array<MdotLaunch, sizeof...(I)> mdot_table(std::integer_sequence<int, I...>) {
     return {&mdot_launch<I + 1>...};
@@ -458,7 +413,6 @@ static constexpr std::array<AxpyLaunch, sizeof...(I)> axpy_table(std::integer_se
 // per column count 1..kChunk
 static const auto kMdot = mdot_table(std::make_integer_sequence<int, kChunk>{});
 static const auto kAxpy = axpy_table(std::make_integer_sequence<int, kChunk>{});
-static const auto kAxpyMdot = axpy_mdot_table(std::make_integer_sequence<int, kChunk>{});
 
 // Selective reorthogonalisation (Kahan-Parlett "twice is enough"): a second
 // classical Gram-Schmidt pass when the first one cancelled more than half of
@@ -490,8 +444,8 @@ __host__ __device__ inline void drotg_dev(double *da, double *db, double *c, dou
 // set) and scales its slice of w into q_{j+1}.  Block 0 also sets the new
 // Hessenberg column j = h1 (+ h2 after a second pass) with h_{j+1,j} = ||w||,
 // applies the previous rotations and the new Givens rotation, rotates the
-// right-hand side g, and writes {|g_{j+1}|, h_{j+1,j}} to stat and, when hstat
-// is given (pinned host memory the device can write), there too.
+// right-hand side g, and writes {|g_{j+1}|, h_{j+1,j}} to stat and, when hslot
+// is given (pinned host memory the device can write), there too, then tag.
 // With npart, ||w||^2 is not reduced beforehand: every block sums the nb
 // partials of the single Gram-Schmidt pass itself, in reduce_cols' order (the
 // same value bit for bit, one launch fewer), and the slices are grid-strided.
@@ -503,7 +457,7 @@ __global__ void __launch_bounds__(256) arnoldi_finish(int j, int m, const double
                                                       const double *__restrict__ n2, const double *__restrict__ flag,
                                                       double *__restrict__ H, double *__restrict__ cs,
                                                       double *__restrict__ sn, double *__restrict__ g,
-                                                      double *__restrict__ stat, double *__restrict__ hstat, long n,
+                                                      double *__restrict__ stat, double *hslot, double tag, long n,
                                                       const double *__restrict__ w, double *__restrict__ q,
                                                       const double *__restrict__ npart = nullptr, int nb = 0) {
     __shared__ double lds[4];
@@ -553,25 +507,465 @@ __global__ void __launch_bounds__(256) arnoldi_finish(int j, int m, const double
     g[j + 1] = -sv * gj;
     stat[0] = fabs(g[j + 1]);
     stat[1] = hn;
-    if (hstat) {
-        hstat[0] = stat[0];
-        hstat[1] = hn;
+    if (hslot) {
+        hslot[0] = fabs(g[j + 1]);
+        hslot[1] = hn;
         __threadfence_system();
+        __hip_atomic_store(hslot + 2, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
-__global__ void gmres_cycle_init(double *__restrict__ g, int len, double beta) {
-    for (int i = threadIdx.x; i < len; i += blockDim.x) g[i] = i == 0 ? beta : 0.;
+// ---- Arnoldi steps of up to kGsCols basis columns in three launches --------------
+// gs_dots: block partials of Q^T w and w . w; gs_update: sums them (every
+// workgroup by itself), w -= Q h1, block partials of the second pass's dots and
+// of the updated w . w; gs_finish: sums those, the second update where the first
+// pass cancelled, q_{j+1}, the Hessenberg column and its rotations.  A reduction
+// launch of its own costs about as much as the pass it follows (192 000 rows, 10
+// columns: 6 us for the dots, 3 + 2 us for the launch that sums 10 x 512 numbers),
+// so the partials go to the next kernel, kGsNb workgroups x (NC + 1) columns,
+// 4 loads a lane; more workgroups would read more than the basis itself.
+// What bounds the three: the basis, read once each (twice with the second
+// update), and at 192 000 rows and below the latency of one round of loads per
+// thread, which is why every column's load is issued before the sums.
+// Per step of the Krylov solve of 191 771 rows, 21 steps (Jacobi): 65 -> 33 us.
+constexpr int kGsThreads = 512;
+constexpr int kGsNb = 256;   // workgroups: one per CU
+constexpr int kGsCols = 32;  // columns held in registers; longer bases go through mdot_kernel and axpy_norm
+constexpr int kGsWaves = kGsThreads / 64;
+static_assert(kGsNb * (kGsCols + 1) <= kGsBlocks * (kChunk + 1), "partials fit the workspace");
+
+static inline int gs_nb(long n) {
+    return (int)std::max(1L, std::min((long)kGsNb, ((n >> 1) + kGsThreads - 1) / kGsThreads));
 }
 
-// y = R^{-1} g on the first k rotated columns (back substitution)
-__global__ void gmres_backsolve(int k, int m, const double *__restrict__ H, const double *__restrict__ g,
-                                double *__restrict__ y) {
-    if (threadIdx.x != 0) return;
-    for (int i = k - 1; i >= 0; --i) {
-        double sum = g[i];
-        for (int l = i + 1; l < k; ++l) sum -= H[(size_t)l * (m + 1) + i] * y[l];
-        y[i] = sum / H[(size_t)i * (m + 1) + i];
+// Sums L columns over the wavefront: at each step a lane keeps one half of the
+// columns and gives the other to its partner, L / 2 + L / 4 + ... exchanges
+// instead of 6 L.  Returns column col's sum, if col < end (else the lane has none).
+template <int BIT, int L>
+__device__ __forceinline__ double fold_cols(const double (&v)[L], int &col, int &end) {
+    if constexpr (BIT == 0) {
+        static_assert(L == 1, "at most 64 columns");
+        return v[0];
+    } else if constexpr (L == 1) {
+        double k[1] = {v[0] + __shfl_xor(v[0], BIT, 64)};
+        return fold_cols<BIT / 2, 1>(k, col, end);
+    } else {
+        constexpr int H = (L + 1) / 2;
+        const bool up = threadIdx.x & BIT;
+        double k[H];
+#pragma unroll
+        for (int i = 0; i < H; ++i) {
+            const double lo = v[i], hi = i + H < L ? v[i + H] : 0.;
+            k[i] = (up ? hi : lo) + __shfl_xor(up ? lo : hi, BIT, 64);
+        }
+        if (up) col += H;
+        else end = end < col + H ? end : col + H;
+        return fold_cols<BIT / 2, H>(k, col, end);
+    }
+}
+
+// Block partials of K columns: part[c * nb + block]
+template <int K>
+__device__ __forceinline__ void gs_store(const double (&acc)[K], int nk, int nb, double *__restrict__ part) {
+    __shared__ double lds[kGsWaves][K];
+    int col = 0, end = K;
+    const double v = fold_cols<32, K>(acc, col, end);
+    if (col < end) lds[threadIdx.x >> 6][col] = v;
+    __syncthreads();
+    if ((int)threadIdx.x < nk) {
+        double t = 0.;
+#pragma unroll
+        for (int w = 0; w < kGsWaves; ++w) t += lds[w][threadIdx.x];
+        part[threadIdx.x * nb + blockIdx.x] = t;
+    }
+}
+
+// out[c] (LDS) = sum of column c's nb partials, c < K, in an order that depends
+// on nb alone: every workgroup gets the same values.  Ends with a barrier.
+template <int K>
+__device__ __forceinline__ void gs_sums(int nb, const double *__restrict__ part, double *out) {
+    constexpr int CW = (K + kGsWaves - 1) / kGsWaves, U = kGsNb / 64;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    double v[CW][U], s[CW];
+#pragma unroll
+    for (int i = 0; i < CW; ++i) {
+        const int c = wv + i * kGsWaves;
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[i][u] = c < K && lane + 64 * u < nb ? part[c * nb + lane + 64 * u] : 0.;
+    }
+#pragma unroll
+    for (int i = 0; i < CW; ++i) {
+        s[i] = 0.;
+#pragma unroll
+        for (int u = 0; u < U; ++u) s[i] += v[i][u];
+    }
+    int col = 0, end = CW;
+    const double t = fold_cols<32, CW>(s, col, end);
+    if (col < end && wv + col * kGsWaves < K) out[wv + col * kGsWaves] = t;
+    __syncthreads();
+}
+
+// a wavefront-uniform value in scalar registers
+__device__ __forceinline__ double uniform(double x) {
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(x)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(x)));
+}
+
+// Rows per load: pairs while the columns' loads in flight fit 64 registers,
+// then single rows
+template <int NC>
+using GsRow = std::conditional_t<(NC <= 16), double2, double>;
+__device__ __forceinline__ double gs_dot(double2 a, double2 b) { return a.x * b.x + a.y * b.y; }
+__device__ __forceinline__ double gs_dot(double a, double b) { return a * b; }
+__device__ __forceinline__ void gs_fma(double2 &s, double h, double2 q) { s.x += h * q.x; s.y += h * q.y; }
+__device__ __forceinline__ void gs_fma(double &s, double h, double q) { s += h * q; }
+__device__ __forceinline__ void gs_sub(double2 &a, double2 s) { a.x -= s.x; a.y -= s.y; }
+__device__ __forceinline__ void gs_sub(double &a, double s) { a -= s; }
+__device__ __forceinline__ double2 gs_scale(double2 a, double f) { return {a.x * f, a.y * f}; }
+__device__ __forceinline__ double gs_scale(double a, double f) { return a * f; }
+__device__ __forceinline__ double2 gs_mul(double2 a, double2 b) { return {a.x * b.x, a.y * b.y}; }
+__device__ __forceinline__ double gs_mul(double a, double b) { return a * b; }
+
+// Runs f on every row group of the grid and, with pairs, g on an odd last row.
+// The leading dimension of Q is even; w, the diagonal and the caller's vectors
+// end at n, so the odd row is read by itself.
+template <int NC>
+__device__ __forceinline__ long gs_groups(long n) { return NC <= 16 ? n >> 1 : n; }
+template <int NC>
+__device__ __forceinline__ bool gs_tail(long n) { return NC <= 16 && (n & 1) && blockIdx.x == 0 && threadIdx.x == 0; }
+
+template <int NC>
+__global__ void __launch_bounds__(kGsThreads) gs_dots(long n, const double *__restrict__ w,
+                                                      const double *__restrict__ Q, long ldq,
+                                                      double *__restrict__ part) {
+    using R = GsRow<NC>;
+    double acc[NC + 1];
+#pragma unroll
+    for (int c = 0; c <= NC; ++c) acc[c] = 0.;
+    const long np = gs_groups<NC>(n);
+    for (long p = blockIdx.x * (long)kGsThreads + threadIdx.x; p < np; p += (long)gridDim.x * kGsThreads) {
+        const R a = reinterpret_cast<const R *>(w)[p];
+        R q[NC];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) q[c] = reinterpret_cast<const R *>(Q + c * ldq)[p];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc[c] += gs_dot(a, q[c]);
+        acc[NC] += gs_dot(a, a);
+    }
+    if (gs_tail<NC>(n)) {
+        const double a = w[n - 1];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc[c] += a * Q[c * ldq + n - 1];
+        acc[NC] += a * a;
+    }
+    gs_store<NC + 1>(acc, NC + 1, gridDim.x, part);
+}
+
+// h1[0, NC] = the sums; twice: the second pass's dots too.  ctl[1] != 0: the
+// cycle has converged, nothing is done.
+template <int NC>
+__global__ void __launch_bounds__(kGsThreads) gs_update(long n, double *__restrict__ w,
+                                                        const double *__restrict__ Q, long ldq, int twice,
+                                                        const double *__restrict__ part, double *__restrict__ part2,
+                                                        double *__restrict__ h1, const double *__restrict__ ctl) {
+    using R = GsRow<NC>;
+    __shared__ double hs[NC + 1];
+    const long np = gs_groups<NC>(n), step = (long)gridDim.x * kGsThreads;
+    long p = blockIdx.x * (long)kGsThreads + threadIdx.x;
+    const double done = ctl[1];
+    R a{}, q[NC];
+    auto load = [&]() {
+        a = reinterpret_cast<const R *>(w)[p];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) q[c] = reinterpret_cast<const R *>(Q + c * ldq)[p];
+    };
+    if (p < np) load();
+    gs_sums<NC + 1>(gridDim.x, part, hs);
+    if (done != 0.) return;
+    if (blockIdx.x == 0 && (int)threadIdx.x <= NC) h1[threadIdx.x] = hs[threadIdx.x];
+    double h[NC], acc[NC + 1];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) h[c] = uniform(hs[c]);
+#pragma unroll
+    for (int c = 0; c <= NC; ++c) acc[c] = 0.;
+    while (p < np) {
+        R s{};
+#pragma unroll
+        for (int c = 0; c < NC; ++c) gs_fma(s, h[c], q[c]);
+        gs_sub(a, s);
+        reinterpret_cast<R *>(w)[p] = a;
+        if (twice) {
+#pragma unroll
+            for (int c = 0; c < NC; ++c) acc[c] += gs_dot(a, q[c]);
+        }
+        acc[NC] += gs_dot(a, a);
+        p += step;
+        if (p < np) load();
+    }
+    if (gs_tail<NC>(n)) {
+        double qt[NC], s = 0.;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) { qt[c] = Q[c * ldq + n - 1]; s += h[c] * qt[c]; }
+        const double at = w[n - 1] - s;
+        w[n - 1] = at;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc[c] += at * qt[c];
+        acc[NC] += at * at;
+    }
+    gs_store<NC + 1>(acc, NC + 1, gridDim.x, part2);
+}
+
+// Column j = NC - 1 of the Hessenberg matrix: the previous rotations, the new
+// one, the right-hand side g, {|g_{j+1}|, h_{j+1,j}} to stat and, when hslot is
+// given (pinned host memory), there too, then tag behind them; ctl[1] = 1 when
+// the cycle ends here by the host's own test.  By one wavefront: everything the
+// rotations' serial chain needs is loaded into the LDS at once.
+__device__ inline void gs_hessenberg(int j, int m, double hk, double hn, double thr, double *__restrict__ H,
+                                     double *__restrict__ cs, double *__restrict__ sn, double *__restrict__ g,
+                                     double *__restrict__ ctl, double *__restrict__ stat, double *hslot, double tag) {
+    __shared__ double hc[kGsCols + 1], cl[kGsCols], sl[kGsCols];
+    const int l = threadIdx.x & 63;
+    if (l <= j) hc[l] = hk;
+    if (l < j) { cl[l] = cs[l]; sl[l] = sn[l]; }
+    wave_lds_order();
+    if (l == 0) {
+        const double gj = g[j];
+        double a = hc[0];
+        for (int k = 0; k < j; ++k) {
+            const double b = hc[k + 1], c = cl[k], s = sl[k];
+            hc[k] = c * a + s * b;
+            a = c * b - s * a;
+        }
+        double b = hn, c, s, r = a;
+        drotg_dev(&r, &b, &c, &s);
+        cs[j] = c;
+        sn[j] = s;
+        hc[j] = c * a + s * hn;
+        g[j] = c * gj;
+        const double g1 = -s * gj, est = fabs(g1);
+        g[j + 1] = g1;
+        stat[0] = est;
+        stat[1] = hn;
+        if (est < thr || !(hn > 1e-16)) ctl[1] = 1.;
+        if (hslot) {
+            hslot[0] = est;
+            hslot[1] = hn;
+            __threadfence_system();
+            __hip_atomic_store(hslot + 2, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
+    wave_lds_order();
+    double *col = H + (size_t)j * (m + 1);
+    if (l <= j) col[l] = hc[l];
+    if (l == 0) col[j + 1] = 0.;
+}
+
+// End of step j = NC - 1.  mode: 0 never a second update, 1 where the first pass
+// cancelled more than half of ||w||^2, 2 always (Kahan-Parlett "twice is
+// enough").  The norm after the second update is ||w||^2 - ||h2||^2 (q's
+// orthonormal columns), whose rounding error is that of ||w||^2 as long as
+// ||h2||^2 is a small part of it; above 2^-10 of it (w lies in the basis' span to
+// rounding) the update is written unscaled, and the last workgroup to finish
+// takes its norm and scales it.  All workgroups but the last stream rows, that
+// one sets the Hessenberg column.  diag: z = diag q_{j+1} as well.
+template <int NC>
+__global__ void __launch_bounds__(kGsThreads) gs_finish(int mode, int m, long n, const double *__restrict__ w,
+                                                        double *__restrict__ Q, long ldq,
+                                                        double *__restrict__ part, const double *__restrict__ part2,
+                                                        const double *__restrict__ h1, double thr,
+                                                        double *__restrict__ H, double *__restrict__ cs,
+                                                        double *__restrict__ sn, double *__restrict__ g,
+                                                        double *__restrict__ ctl, double *__restrict__ stat,
+                                                        double *hslot, double tag, const double *__restrict__ diag,
+                                                        double *__restrict__ z) {
+    using R = GsRow<NC>;
+    __shared__ double hs[NC + 1];
+    const int nb = gridDim.x - 1, wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const double done = ctl[1], ww = h1[NC];
+    if (mode) {
+        gs_sums<NC + 1>(nb, part2, hs);
+    } else {
+        gs_sums<1>(nb, part2 + (size_t)NC * nb, hs + NC);
+    }
+    if (done != 0.) return;
+    const double n1 = uniform(hs[NC]);
+    const bool two = mode == 2 || (mode == 1 && n1 < 0.5 * ww);
+    double hh = 0.;
+    if (two)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) hh += hs[c] * hs[c];
+    const bool exact = two && !(hh <= n1 * (1. / 1024));
+    const double nn = two ? n1 - hh : n1;
+    if ((int)blockIdx.x == nb) {
+        if (!exact && wv == 0)
+            gs_hessenberg(NC - 1, m, lane < NC ? (two ? h1[lane] + hs[lane] : h1[lane]) : 0., sqrt(nn), thr, H, cs, sn,
+                          g, ctl, stat, hslot, tag);
+        return;
+    }
+    const double hn = sqrt(nn), f = exact ? 1. : hn > 0. ? 1. / hn : 0.;
+    double *__restrict__ qn = Q + (size_t)NC * ldq;
+    const long np = gs_groups<NC>(n), step = (long)nb * kGsThreads;
+    const long p0 = blockIdx.x * (long)kGsThreads + threadIdx.x;
+    double acc = 0.;
+    auto put = [&](auto *out, long p, auto a) {
+        using A = decltype(a);
+        acc += gs_dot(a, a);
+        a = gs_scale(a, f);
+        out[p] = a;
+        if (diag) reinterpret_cast<A *>(z)[p] = gs_mul(a, reinterpret_cast<const A *>(diag)[p]);
+    };
+    if (two) {
+        double h[NC];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) h[c] = uniform(hs[c]);
+        for (long p = p0; p < np; p += step) {
+            R a = reinterpret_cast<const R *>(w)[p], q[NC], s{};
+#pragma unroll
+            for (int c = 0; c < NC; ++c) q[c] = reinterpret_cast<const R *>(Q + c * ldq)[p];
+#pragma unroll
+            for (int c = 0; c < NC; ++c) gs_fma(s, h[c], q[c]);
+            gs_sub(a, s);
+            put(reinterpret_cast<R *>(qn), p, a);
+        }
+        if (gs_tail<NC>(n)) {
+            double s = 0.;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) s += h[c] * Q[c * ldq + n - 1];
+            put(qn, n - 1, w[n - 1] - s);
+        }
+    } else {
+        for (long p = p0; p < np; p += step) put(reinterpret_cast<R *>(qn), p, reinterpret_cast<const R *>(w)[p]);
+        if (gs_tail<NC>(n)) put(qn, n - 1, w[n - 1]);
+    }
+    if (!exact) return;
+    // part's first column is free here: gs_update has summed it
+    __shared__ int last;
+    {
+        double a1[1] = {acc};
+        gs_store<1>(a1, 1, nb, part);
+    }
+    __threadfence();
+    __syncthreads();
+    unsigned *ticket = reinterpret_cast<unsigned *>(ctl + 2);
+    if (threadIdx.x == 0) last = atomicAdd(ticket, 1u) == (unsigned)nb - 1;
+    __syncthreads();
+    if (!last) return;
+    __threadfence();
+    if (threadIdx.x == 0) *ticket = 0;
+    __shared__ double ex[kGsWaves];
+    const double pv = (int)threadIdx.x < nb ? __hip_atomic_load(part + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.;
+    const double ps = wave_reduce(pv);
+    if (lane == 0) ex[wv] = ps;
+    __syncthreads();
+    double en = 0.;
+#pragma unroll
+    for (int k = 0; k < kGsWaves; ++k) en += ex[k];
+    const double he = sqrt(en), fe = he > 0. ? 1. / he : 0.;
+    for (long i = threadIdx.x; i < n; i += kGsThreads) {
+        const double q = __hip_atomic_load(qn + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) * fe;
+        qn[i] = q;
+        if (diag) z[i] = q * diag[i];
+    }
+    if (wv == 0)
+        gs_hessenberg(NC - 1, m, lane < NC ? h1[lane] + hs[lane] : 0., he, thr, H, cs, sn, g, ctl, stat, hslot, tag);
+}
+
+struct GsStep {
+    void (*dots)(long, const double *, const double *, long, double *);
+    void (*update)(long, double *, const double *, long, int, const double *, double *, double *, const double *);
+    void (*finish)(int, int, long, const double *, double *, long, double *, const double *, const double *, double,
+                   double *, double *, double *, double *, double *, double *, double *, double, const double *,
+                   double *);
+};
+template <int... I>
+static constexpr std::array<GsStep, sizeof...(I)> gs_table(std::integer_sequence<int, I...>) {
+    return {GsStep{&gs_dots<I + 1>, &gs_update<I + 1>, &gs_finish<I + 1>}...};
+}
+static const auto kGs = gs_table(std::make_integer_sequence<int, kGsCols>{});
+
+// Start of a cycle: q_0 = r / beta (and z = diag q_0), g = beta e_1, the
+// control words cleared.
+__global__ void gs_start(long n, const double *__restrict__ r, const double *__restrict__ nsq, double beta,
+                         double *__restrict__ q, const double *__restrict__ diag, double *__restrict__ z,
+                         double *__restrict__ g, int len, double *__restrict__ ctl) {
+    long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
+    if (blockIdx.x == 0) {
+        for (int k = threadIdx.x; k < len; k += blockDim.x) g[k] = k == 0 ? beta : 0.;
+        if (threadIdx.x < 3) ctl[threadIdx.x] = 0.;
+    }
+    if (i >= n) return;
+    const double v = r[i] * (1. / sqrt(nsq[0]));
+    q[i] = v;
+    if (diag) z[i] = v * diag[i];
+}
+
+// r = b - r (or b, when zero), block partials of r . r and b . b
+__global__ void __launch_bounds__(kGsThreads) gs_residual(long n, int zero, const double *__restrict__ b,
+                                                          double *__restrict__ r, double *__restrict__ part) {
+    double acc[2] = {0., 0.};
+    for (long i = blockIdx.x * (long)kGsThreads + threadIdx.x; i < n; i += (long)gridDim.x * kGsThreads) {
+        const double bi = b[i], v = zero ? bi : bi - r[i];
+        r[i] = v;
+        acc[0] += v * v;
+        acc[1] += bi * bi;
+    }
+    gs_store<2>(acc, 2, gridDim.x, part);
+}
+
+// out[0, 2) = the two sums, to the host's slot as well, tag behind them
+__global__ void __launch_bounds__(kGsThreads) gs_norms(int nb, const double *__restrict__ part,
+                                                       double *__restrict__ out, double *hslot, double tag) {
+    __shared__ double s[2];
+    gs_sums<2>(nb, part, s);
+    if (threadIdx.x) return;
+    out[0] = s[0];
+    out[1] = s[1];
+    if (hslot) {
+        hslot[0] = s[0];
+        hslot[1] = s[1];
+        __threadfence_system();
+        __hip_atomic_store(hslot + 2, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+// End of a cycle: y = R^-1 g on the first k rotated columns, then out = Q y, or
+// with add x += diag (Q y) (diag null: x += Q y).  Every workgroup solves the
+// small triangle by itself, a lane per row, from the LDS (one thread reading
+// memory entry by entry took 23 us for 21 columns).
+__global__ void __launch_bounds__(256) gs_solution(long n, int k, int m, const double *__restrict__ H,
+                                                   const double *__restrict__ g, const double *__restrict__ Q,
+                                                   long ldq, const double *__restrict__ diag, int add,
+                                                   double *__restrict__ out) {
+    __shared__ double R[63 * 64 / 2], y[64];
+    for (int c = threadIdx.x >> 6; c < k; c += 4) {
+        const int l = threadIdx.x & 63;
+        if (l <= c) R[c * (c + 1) / 2 + l] = H[(size_t)c * (m + 1) + l];
+    }
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        const int l = threadIdx.x;
+        double v = l < k ? g[l] : 0.;
+        for (int c = k - 1; c >= 0; --c) {
+            const double *col = R + c * (c + 1) / 2;
+            const double yc = __shfl(v, c, 64) / col[c];
+            if (l < c) v -= col[l] * yc;
+            if (l == c) y[c] = yc;
+        }
+    }
+    __syncthreads();
+    for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += gridDim.x * 256L) {
+        double s = 0.;
+        int c = 0;
+        for (; c + 8 <= k; c += 8) {
+            double q[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) q[u] = Q[(c + u) * ldq + i];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) s += y[c + u] * q[u];
+        }
+        for (; c < k; ++c) s += y[c] * Q[c * ldq + i];
+        if (add) out[i] += diag ? s * diag[i] : s;
+        else out[i] = s;
     }
 }
 
@@ -632,10 +1026,6 @@ __global__ void vaxpby(long n, double a, const double *__restrict__ x, double b,
 // ---- block-Jacobi ILU(0): one workgroup per block of bs consecutive rows
 // (factorisation: bj_factor; the rows of one level run concurrently)
 constexpr int kBjFactorThreads = 512;
-
-// compiler-only ordering of one wavefront's LDS accesses (the LDS executes a
-// wavefront's accesses in issue order; no wait for outstanding memory loads)
-__device__ __forceinline__ void wave_lds_order() { asm volatile("" ::: "memory"); }
 
 // workgroup barrier for LDS data: waits for LDS accesses only, so global loads
 // issued ahead stay in flight across it
@@ -1565,6 +1955,8 @@ __global__ void schur_back(int nI, const int *__restrict__ irow, const int *__re
 }
 
 // ---- host helpers ---------------------------------------------------------------
+constexpr int kSlot = 4;  // doubles per host slot: two values, their tag, one spare
+
 static int ensure_work(fvp_csr *A, int m) {
     if (A->m_alloc >= m) return 0;
     long n = A->n;
@@ -1575,17 +1967,14 @@ static int ensure_work(fvp_csr *A, int m) {
         return -1;
     if (A->hstat) (void)hipHostFree(A->hstat);
     A->hstat = nullptr;
-    // per Arnoldi step {estimate, h_{j+1,j}}, then two scalar slots
-    if (hipHostMalloc((void **)&A->hstat, sizeof(double) * (2 * (m + 1) + 2), hipHostMallocDefault) != hipSuccess) {
+    const size_t bytes = sizeof(double) * kSlot * (m + 1);
+    if (hipHostMalloc((void **)&A->hstat, bytes, hipHostMallocCoherent) != hipSuccess) {
         A->hstat = nullptr;
         set_error("pinned host allocation failed");
         return -1;
     }
-    while ((int)A->ev.size() < m + 1) {
-        hipEvent_t e;
-        if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) { set_error("event creation failed"); return -1; }
-        A->ev.push_back(e);
-    }
+    std::memset(A->hstat, 0, bytes);
+    A->tag = 0;
     A->m_alloc = m;
     return 0;
 }
@@ -1620,29 +2009,52 @@ using Op = std::function<int(const double *, double *)>;
 // Restarted right-preconditioned GMRES (gmres.c:26-201) with the host kept off
 // the critical path: the Hessenberg column, the Givens rotations and the
 // residual estimate are updated on the device; each Arnoldi step's estimate is
-// copied to pinned host memory and read one step later, while the next step
+// written to pinned host memory and read one step later, while the next step
 // is already queued (a cycle that has converged runs one extra, discarded
-// step).  Classical Gram-Schmidt with a second pass only when the first one
+// step, of which the Gram-Schmidt updates return at once).  Classical
+// Gram-Schmidt with a second pass only when the first one
 // cancelled more than half of ||w||^2 (reorthogonalise = 1), always (2) or
 // never (0).  A cycle ends early once the estimate meets tol * ||b||.
 // Device and host memory of one GMRES solve: the basis Q (gs_ldq(n) x (m+1)),
 // work vectors w, r, z (gs_ldq(n) each), reduction partials part
 // (kGsBlocks x (kChunk+1)), scalars sc (16), per-step coefficients hdev
 // (2 (m+2) + 2), the Hessenberg matrix Hd ((m+1) x m), Givens pairs, rhs and
-// solution; hstat (host, 2 (m+1)) receives each step's {estimate, h_{j+1,j}}.
-// With ev (one event per step) the host reads step j-1 while step j runs;
-// without, each step's pair is read right after the step (same control flow
+// solution; hstat (host, kSlot (m+1)): slot j receives step j's {estimate,
+// h_{j+1,j}}, slot m the squared norms {||r||^2, ||b||^2}.
+// With tag hstat is pinned memory that the kernels write, a tag last (counted
+// up, so that no slot ever holds the awaited tag beforehand), and the host polls
+// the tag: an event per step costs the stream a barrier packet each.  Without,
+// each step's pair is copied and read right after the step (same control flow
 // and results, one synchronisation per step).
+// diag: the preconditioner is this diagonal, and the kernels that write a basis
+// vector write z = diag q as well.
 struct GmresWork {
     double *Q, *w, *r, *z, *part, *sc, *hdev, *Hd, *gd, *csd, *snd, *yd;
     double *hstat;
-    const hipEvent_t *ev;
-    bool hmapped;  // hstat is pinned host memory the kernels write directly
-    // with hmapped: two pinned scalar slots for ||r||^2 and ||b||^2, and the
-    // event the host polls for them (hipMemcpyAsync and a blocking wait otherwise)
-    double *hscal;
-    hipEvent_t hev;
+    double *tag;
+    const double *diag;
 };
+
+// Waits for tag in a slot.  A queue that ends (or fails) without having written
+// it is an error; asked for only now and then, since the query itself costs more
+// than the reads.
+static int slot_wait(hipStream_t s, const double *slot, double tag) {
+    auto there = [&]() {
+        double v;
+        __atomic_load(slot + 2, &v, __ATOMIC_ACQUIRE);
+        return v == tag;
+    };
+    for (long k = 1; !there(); ++k) {
+        if (k & 0xfffff) continue;
+        const hipError_t e = hipStreamQuery(s);
+        if (e == hipErrorNotReady) continue;
+        FVP_HIP(e);
+        if (there()) break;
+        set_error("GMRES: the queue ended without its status");
+        return -1;
+    }
+    return 0;
+}
 
 // doubles of a GmresWork carved from one device buffer (each piece 256-byte aligned)
 static size_t gmres_work_doubles(long n, int m) {
@@ -1676,13 +2088,13 @@ static int gmres_core(const GmresWork &W, hipStream_t s, long n, const Op &A, co
                       double *x, const fvp_gmres_params *p, fvp_gmres_stats *st, bool x_zero = false);
 
 int gmres_device(fvp_csr *W, hipStream_t s, long n, const Op &A, const Op &M, const double *b, double *x,
-                 const fvp_gmres_params *p, fvp_gmres_stats *st, bool x_zero) {
+                 const fvp_gmres_params *p, fvp_gmres_stats *st, bool x_zero, const double *diag) {
     const int m = p->dim_krylov;
     if (m < 1 || m > 63) { set_error("dim_krylov must be 1..63"); return -1; }
     if (p->reorthogonalise < 0 || p->reorthogonalise > 2) { set_error("reorthogonalise must be 0, 1 or 2"); return -1; }
     if (ensure_work(W, m)) return -1;
     GmresWork wk{W->Q.p, W->w.p, W->r.p, W->z.p, W->part.p, W->scal.p, W->hdev.p, W->Hd.p, W->gd.p, W->csd.p,
-                 W->snd.p, W->yd.p, W->hstat, W->ev.data(), true, W->hstat + 2 * (m + 1), W->ev[m]};
+                 W->snd.p, W->yd.p, W->hstat, &W->tag, diag};
     return gmres_core(wk, s, n, A, M, b, x, p, st, x_zero);
 }
 
@@ -1692,35 +2104,33 @@ static int gmres_core(const GmresWork &W, hipStream_t s, long n, const Op &A, co
     double *Q = W.Q, *w = W.w, *r = W.r, *z = W.z, *part = W.part, *sc = W.sc;
     // h1, h2: first / second pass coefficients (j+1 dots, then ||w||^2); stat: {estimate, h_{j+1,j}}
     double *h1 = W.hdev, *h2 = W.hdev + (m + 2), *stat = W.hdev + 2 * (m + 2);
-    // device scalars: sc[0] ||r||^2, sc[1] ||b||^2, sc[2] first-pass ||w||^2 after projection,
-    // sc[3] second-pass ||w||^2, sc[4] reorthogonalisation flag
-    double *n1 = sc + 2, *n2 = sc + 3, *flag = sc + 4;
+    // device scalars: sc[0] ||r||^2, sc[1] ||b||^2; for bases past kGsCols columns sc[2] first-pass ||w||^2
+    // after projection, sc[3] second-pass ||w||^2, sc[4] reorthogonalisation flag; ctl[1], ctl[2] as gs_finish has them
+    double *n1 = sc + 2, *n2 = sc + 3, *flag = sc + 4, *ctl = sc + 4;
     const long ldq = gs_ldq(n);
-    const int mode = p->reorthogonalise;
+    const int mode = p->reorthogonalise, nb = gs_nb(n);
+    // the second pass's partials: the other half of part, or r (free during a cycle) where they need more
+    constexpr int kHalf = kGsNb / 2 * (kGsCols + 1);
+    double *part2 = nb <= kGsNb / 2 ? part + kHalf : r;
     fvp_gmres_stats stats{0, 0, 0, 0., 0.};
     double hn2[2] = {0., 0.};
-    // r = b - A x; ||r||, ||b|| with one synchronisation
-    if (x_zero) {
-        vcopy<<<nblk(n, 256), 256, 0, s>>>(n, b, r);
-    } else {
-        if (A(x, r)) return -1;
-        vrsub<<<nblk(n, 256), 256, 0, s>>>(n, b, r);
-    }
-    // ||r||^2 and ||b||^2 to the host (pinned slots and a polled event when
-    // there are, a copy and a blocking wait otherwise)
-    auto fetch = [&](int cnt) -> int {
-        if (W.hscal) {
-            if (host_wait(s, W.hev)) return -1;
-            for (int k = 0; k < cnt; ++k) hn2[k] = W.hscal[k];
-            return 0;
+    // queues r = b - r (x_zero: r = b) and waits for ||r||^2 and ||b||^2
+    auto residual = [&](int zero) -> int {
+        gs_residual<<<nb, kGsThreads, 0, s>>>(n, zero, b, r, part);
+        double *slot = W.hstat + (size_t)kSlot * m;
+        gs_norms<<<1, kGsThreads, 0, s>>>(nb, part, sc, W.tag ? slot : nullptr, W.tag ? ++*W.tag : 0.);
+        FVP_HIP(hipGetLastError());
+        if (W.tag) {
+            if (slot_wait(s, slot, *W.tag)) return -1;
+        } else {
+            FVP_HIP(hipMemcpyAsync(slot, sc, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
+            FVP_HIP(hipStreamSynchronize(s));
         }
-        FVP_HIP(hipMemcpyAsync(hn2, sc, cnt * sizeof(double), hipMemcpyDeviceToHost, s));
-        FVP_HIP(hipStreamSynchronize(s));
+        for (int k = 0; k < 2; ++k) hn2[k] = slot[k];
         return 0;
     };
-    dot_async(s, n, r, r, part, sc, W.hscal);
-    dot_async(s, n, b, b, part, sc + 1, W.hscal ? W.hscal + 1 : nullptr);
-    if (fetch(2)) return -1;
+    if (!x_zero && A(x, r)) return -1;
+    if (residual(x_zero)) return -1;
     double beta = std::sqrt(hn2[0]), normb = std::sqrt(hn2[1]);
     double error = normb > 0 ? beta / normb : 0.;
     if (beta == 0. || error < p->tol) {
@@ -1728,73 +2138,71 @@ static int gmres_core(const GmresWork &W, hipStream_t s, long n, const Op &A, co
         if (st) *st = stats;
         return 0;
     }
+    const double thr = p->tol * normb;
     int restarts = 0, converged = 0, total = 0;
-    vscale_inv_norm<<<nblk(n, 256), 256, 0, s>>>(n, r, sc, Q);  // q0 = r / beta
+    double step_tag = 0.;  // of the step before
     while (restarts <= p->max_restarts && !converged) {
-        gmres_cycle_init<<<1, 64, 0, s>>>(W.gd, m + 1, beta);
+        gs_start<<<nblk(n, 256), 256, 0, s>>>(n, r, sc, beta, Q, W.diag, z, W.gd, m + 1, ctl);
         int k = m;
         for (int j = 0; j <= m; ++j) {
+            const double prev_tag = step_tag;
             if (j < m) {  // queue Arnoldi step j
                 const double *qj = Q + (size_t)j * ldq;
-                if (M) { if (M(qj, z)) return -1; if (A(z, w)) return -1; }
+                double *slot = W.tag ? W.hstat + (size_t)kSlot * j : nullptr;
+                if (W.tag) step_tag = ++*W.tag;
+                if (W.diag) { if (A(z, w)) return -1; }
+                else if (M) { if (M(qj, z)) return -1; if (A(z, w)) return -1; }
                 else if (A(qj, w)) return -1;
-                // first pass: h1 = Q^T w, ||w||^2 -> h1[j+1]; w -= Q h1, ||w||^2 -> n1
-                multidot(s, n, w, Q, ldq, j + 1, part, h1, nullptr);
-                if (mode && j + 1 <= kChunk) {
-                    // first pass's update fused with the second pass's dots (h2, and
-                    // ||w||^2 after the first pass into n1 = h2[j + 1]); the second
-                    // update only when the first pass cancelled (flag)
-                    kAxpyMdot[j](s, gs_blocks(n), n, w, Q, ldq, h1, part, nullptr);
-                    reduce_cols<<<j + 2, kThreads, 0, s>>>(gs_blocks(n), part, h2, 0, nullptr,
-                                                           mode == 2 ? nullptr : h1 + j + 1, flag);
-                    multiaxpy(s, n, w, Q, ldq, j + 1, h2, part, n2, flag);
+                if (j < kGsCols) {
+                    const GsStep &g = kGs[j];
+                    g.dots<<<nb, kGsThreads, 0, s>>>(n, w, Q, ldq, part);
+                    g.update<<<nb, kGsThreads, 0, s>>>(n, w, Q, ldq, mode != 0, part, part2, h1, ctl);
+                    g.finish<<<nb + 1, kGsThreads, 0, s>>>(mode, m, n, w, Q, ldq, part, part2, h1, thr, W.Hd, W.csd,
+                                                           W.snd, W.gd, ctl, stat, slot, step_tag, W.diag, z);
                 } else {
-                    // single pass: arnoldi_finish reduces ||w||^2 itself
+                    // first pass: h1 = Q^T w, ||w||^2 -> h1[j+1]; w -= Q h1, ||w||^2 -> n1
+                    // (single pass: arnoldi_finish reduces ||w||^2 itself)
+                    multidot(s, n, w, Q, ldq, j + 1, part, h1, nullptr);
                     multiaxpy(s, n, w, Q, ldq, j + 1, h1, part, mode ? n1 : nullptr, nullptr);
                     if (mode) {
                         reorth_decide<<<1, 64, 0, s>>>(h1 + j + 1, n1, mode, flag);
                         multidot(s, n, w, Q, ldq, j + 1, part, h2, flag);
                         multiaxpy(s, n, w, Q, ldq, j + 1, h2, part, n2, flag);
                     }
+                    double *qn = Q + (size_t)(j + 1) * ldq;
+                    arnoldi_finish<<<std::min(nblk(n, 256), kFinishBlocks), 256, 0, s>>>(
+                        j, m, h1, h2, n1, n2, mode ? flag : nullptr, W.Hd, W.csd, W.snd, W.gd, stat, slot, step_tag, n,
+                        w, qn, mode ? nullptr : part, gs_blocks(n));
+                    if (W.diag) vmul<<<nblk(n, 256), 256, 0, s>>>(n, qn, W.diag, z);
                 }
-                const bool fused = mode && j + 1 <= kChunk;  // ||w||^2 after the first pass in h2[j + 1]
-                arnoldi_finish<<<std::min(nblk(n, 256), kFinishBlocks), 256, 0, s>>>(
-                    j, m, h1, h2, fused ? h2 + j + 1 : n1, n2, mode ? flag : nullptr, W.Hd, W.csd, W.snd, W.gd, stat,
-                    W.hmapped ? W.hstat + 2 * j : nullptr, n, w, Q + (size_t)(j + 1) * ldq, mode ? nullptr : part,
-                    gs_blocks(n));
-                if (!W.hmapped)
-                    FVP_HIP(hipMemcpyAsync(W.hstat + 2 * j, stat, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
-                if (W.ev) FVP_HIP(hipEventRecord(W.ev[j], s));
-                else FVP_HIP(hipStreamSynchronize(s));
                 FVP_HIP(hipGetLastError());
+                if (!W.tag) {
+                    FVP_HIP(hipMemcpyAsync(W.hstat + (size_t)kSlot * j, stat, 2 * sizeof(double),
+                                           hipMemcpyDeviceToHost, s));
+                    FVP_HIP(hipStreamSynchronize(s));
+                }
             }
             if (j > 0) {  // read step j-1 (while step j runs, when pipelined)
-                if (W.ev) {  // polled: a blocking wait would wake up late
-                    hipError_t e;
-                    while ((e = hipEventQuery(W.ev[j - 1])) == hipErrorNotReady) {
-                    }
-                    FVP_HIP(e);
-                }
+                const double *slot = W.hstat + (size_t)kSlot * (j - 1);
+                if (W.tag && slot_wait(s, slot, prev_tag)) return -1;
                 ++total;
-                const double est = W.hstat[2 * (j - 1)], hn = W.hstat[2 * (j - 1) + 1];
-                if (est < p->tol * normb || !(hn > 1e-16)) { k = j; break; }
+                const double est = slot[0], hn = slot[1];
+                if (est < thr || !(hn > 1e-16)) { k = j; break; }
             }
         }
-        gmres_backsolve<<<1, 64, 0, s>>>(k, m, W.Hd, W.gd, W.yd);
-        lincomb<<<nblk(n, 256), 256, 0, s>>>(n, w, Q, ldq, k, W.yd);
-        if (M) { if (M(w, z)) return -1; }
-        else vcopy<<<nblk(n, 256), 256, 0, s>>>(n, w, z);
-        vadd<<<nblk(n, 256), 256, 0, s>>>(n, z, x);
+        const bool own = M && !W.diag;  // M is a call of its own
+        gs_solution<<<std::min(nblk(n, 256), kFinishBlocks), 256, 0, s>>>(n, k, m, W.Hd, W.gd, Q, ldq, W.diag, !own,
+                                                                         own ? w : x);
+        if (own) {
+            if (M(w, z)) return -1;
+            vadd<<<nblk(n, 256), 256, 0, s>>>(n, z, x);
+        }
         if (A(x, r)) return -1;
-        vrsub<<<nblk(n, 256), 256, 0, s>>>(n, b, r);
-        dot_async(s, n, r, r, part, sc, W.hscal);
-        if (fetch(1)) return -1;
+        if (residual(0)) return -1;
         beta = std::sqrt(hn2[0]);
         error = beta / normb;
         if (error < p->tol) converged = 1;
         else ++restarts;
-        if (!converged && restarts <= p->max_restarts)
-            vscale_inv_norm<<<nblk(n, 256), 256, 0, s>>>(n, r, sc, Q);
     }
     stats.restarts = converged ? restarts : restarts - 1;
     stats.iterations = total;
@@ -2847,7 +3255,6 @@ extern "C" int fvp_csr_destroy(fvp_csr *A) {
     A->z.release(); A->part.release(); A->scal.release(); A->hdev.release();
     A->Hd.release(); A->gd.release(); A->csd.release(); A->snd.release(); A->yd.release(); A->Qk.release();
     if (A->hstat) (void)hipHostFree(A->hstat);
-    for (hipEvent_t e : A->ev) (void)hipEventDestroy(e);
     A->b_ia.release(); A->b_src.release(); A->b_lu.release(); A->b_lu32.release();
     A->b_roff.release(); A->b_rowid.release(); A->b_own.release(); A->b_zn2.release();
     A->meta_l.release(); A->meta_u.release(); A->ebase_l.release(); A->ebase_u.release();
@@ -2968,6 +3375,9 @@ extern "C" int fvp_precon_values(fvp_csr *A, double *values_host) {
     return 0;
 }
 
+// the preconditioner's diagonal, where it is one
+static const double *diagonal_of(const fvp_csr *A) { return A->ptype == FVP_PRECON_JACOBI ? A->jac.p : nullptr; }
+
 extern "C" int fvp_gmres_csr(fvp_csr *A, const double *b, double *x, const fvp_gmres_params *p,
                              fvp_gmres_stats *st) {
     if (!A || !b || !x || !p) { set_error("null argument"); return -1; }
@@ -2976,7 +3386,7 @@ extern "C" int fvp_gmres_csr(fvp_csr *A, const double *b, double *x, const fvp_g
     Op op = [A](const double *in, double *out) { return csr_gemv_impl(A, 1.0, in, 0.0, out); };
     Op pc;
     if (A->ptype != FVP_PRECON_NONE) pc = [A](const double *in, double *out) { return precon_apply_impl(A, in, out); };
-    return gmres_device(A, A->stream, A->n, op, pc, b, x, p, st);
+    return gmres_device(A, A->stream, A->n, op, pc, b, x, p, st, false, diagonal_of(A));
 }
 
 extern "C" int fvp_gmres_csr_deflated(fvp_csr *A, const double *b, double *x, const fvp_gmres_params *p, int k,
@@ -3045,10 +3455,9 @@ extern "C" int fvp_gmres_csr_noalloc(fvp_csr *A, const double *b, double *x, con
     const long small = (long)(need - (size_t)(wk.sc - base));
     zero_fill<<<(int)std::min(1024L, (small + 255) / 256), 256, 0, A->stream>>>(small, wk.sc);
     FVP_HIP(hipGetLastError());
-    double hstat[2 * 64];
+    double hstat[kSlot * 64];
     wk.hstat = hstat;  // pageable: each step's pair is copied and read synchronously
-    wk.ev = nullptr;
-    wk.hmapped = false;
+    wk.diag = diagonal_of(A);
     Op op = [A](const double *in, double *out) { return csr_gemv_impl(A, 1.0, in, 0.0, out); };
     Op pc;
     if (A->ptype != FVP_PRECON_NONE) pc = [A](const double *in, double *out) { return precon_apply_impl(A, in, out); };
@@ -3382,5 +3791,5 @@ extern "C" int fvp_newton_gmres(fvp_ctx *c, double t, const double *psi, const d
     Op op = [=](const double *in, double *out) { return fvp_jv(c, t, psi, psip, F0, c_j, in, out); };
     Op pc;
     if (W->ptype > 0) pc = [W](const double *in, double *out) { return precon_apply_impl(W, in, out); };
-    return gmres_device(W, c->stream, c->N, op, pc, b, x, p, st);
+    return gmres_device(W, c->stream, c->N, op, pc, b, x, p, st, false, diagonal_of(W));
 }
