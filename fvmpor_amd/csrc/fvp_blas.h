@@ -36,21 +36,23 @@ __host__ __device__ inline double jv_sigma_of(double psi_n2, double v_n2) {
 }
 
 // out[0] (device) = x . y; part must hold 512 doubles.  Asynchronous on s.
-// hout (optional): pinned host memory that receives the value as well.
-int dot_async(hipStream_t s, long n, const double *x, const double *y, double *part, double *out,
-              double *hout = nullptr);
-// Waits until the work queued on s so far has finished: records ev behind it
-// and polls the event.  Scalars that kernels stored to pinned host memory are
-// then readable; the poll avoids the wake-up latency of a blocking wait.
-int host_wait(hipStream_t s, hipEvent_t ev);
-
+int dot_async(hipStream_t s, long n, const double *x, const double *y, double *part, double *out);
 using Op = std::function<int(const double *, double *)>;
+// x = 0 to begin with: the first residual is b itself, its squared norm known
+// on the host and on the device
+struct GmresZero {
+    double norm2;
+    const double *d_norm2;
+};
 // Restarted right-preconditioned GMRES on A x = b; W supplies the workspace.
-// x_zero: the caller has set x = 0, so the first residual is b itself (no
-// product with A).  diag: M is the product with this vector, and is not called.
+// zero (optional): the caller has set x = 0, so no product with A begins the
+// solve.  diag (optional): M is the product with this vector, and is not called.
 int gmres_device(fvp_csr *W, hipStream_t s, long n, const Op &A, const Op &M, const double *b, double *x,
-                 const fvp_gmres_params *p, fvp_gmres_stats *st, bool x_zero = false,
+                 const fvp_gmres_params *p, fvp_gmres_stats *st, const GmresZero *zero = nullptr,
                  const double *diag = nullptr);
+// while GMRES queues an Arnoldi step on W: the device word that its products
+// and solves may leave early on (else null)
+const double *gmres_skip(const fvp_csr *W);
 // the context's Jacobian handle (built on first use)
 fvp_csr *jacobian_handle(fvp_ctx *c);
 }  // namespace fvp

@@ -7,6 +7,7 @@
 
 #include "fvp_blas.h"
 #include "fvp_internal.h"
+#include "fvp_sums.h"
 
 namespace fvp {
 
@@ -24,10 +25,9 @@ __global__ void __launch_bounds__(kRedThreads) dot_partial(long n, const double 
     if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
-// out[0] = sum of np partials (fixed order: deterministic); hout (optional,
-// pinned host memory) gets it too
+// out[0] = sum of np partials (fixed order: deterministic)
 __global__ void __launch_bounds__(kRedThreads) sum_partials(int np, const double *__restrict__ part,
-                                                           double *__restrict__ out, double *__restrict__ hout) {
+                                                           double *__restrict__ out) {
     __shared__ double lds[kRedThreads / 64];
     // each lane's partials in order, four loads in flight at a time
     double s = 0.;
@@ -41,13 +41,7 @@ __global__ void __launch_bounds__(kRedThreads) sum_partials(int np, const double
             if (i0 + u * bd < np) s += q[u];
     }
     s = block_sum(s, lds);
-    if (threadIdx.x == 0) {
-        out[0] = s;
-        if (hout) {
-            hout[0] = s;
-            __threadfence_system();
-        }
-    }
+    if (threadIdx.x == 0) out[0] = s;
 }
 
 // FD increment sigma = sqrt(eps) * ||psi|| / ||v|| from two squared norms
@@ -91,19 +85,48 @@ __global__ void jv_finish(long n, const double *__restrict__ sig, const double *
 
 static inline int nblk(long n, int bs) { return (int)((n + bs - 1) / bs); }
 
-int dot_async(hipStream_t s, long n, const double *x, const double *y, double *part, double *out, double *hout) {
+int dot_async(hipStream_t s, long n, const double *x, const double *y, double *part, double *out) {
     dot_partial<<<kRedBlocks, kRedThreads, 0, s>>>(n, x, y, part);
-    sum_partials<<<1, kRedThreads, 0, s>>>(kRedBlocks, part, out, hout);
+    sum_partials<<<1, kRedThreads, 0, s>>>(kRedBlocks, part, out);
     FVP_HIP(hipGetLastError());
     return 0;
 }
 
-int host_wait(hipStream_t s, hipEvent_t ev) {
-    FVP_HIP(hipEventRecord(ev, s));
-    hipError_t e;
-    while ((e = hipEventQuery(ev)) == hipErrorNotReady) {
+int HostSlots::alloc(int slots) {
+    release();
+    const size_t bytes = sizeof(double) * kSlot * slots;
+    if (hipHostMalloc((void **)&p, bytes, hipHostMallocCoherent) != hipSuccess) {
+        p = nullptr;
+        set_error("pinned host allocation failed");
+        return -1;
     }
-    FVP_HIP(e);
+    std::fill(p, p + (size_t)kSlot * slots, 0.);
+    tag = 0.;
+    return 0;
+}
+
+void HostSlots::release() {
+    if (p) (void)hipHostFree(p);
+    p = nullptr;
+}
+
+// A queue that ends (or fails) without having written the tag is an error; asked
+// for only now and then, since the query costs more than the reads.
+int slot_wait(hipStream_t s, const double *slot, double tag) {
+    auto there = [&]() {
+        double v;
+        __atomic_load(slot + kSlot - 1, &v, __ATOMIC_ACQUIRE);
+        return v == tag;
+    };
+    for (long k = 1; !there(); ++k) {
+        if (k & 0xfffff) continue;
+        const hipError_t e = hipStreamQuery(s);
+        if (e == hipErrorNotReady) continue;
+        FVP_HIP(e);
+        if (there()) break;
+        set_error("the queue ended without its result");
+        return -1;
+    }
     return 0;
 }
 
@@ -114,7 +137,7 @@ using namespace fvp;
 namespace fvp {
 int jv_impl(fvp_ctx *c, double t, const double *psi, const double *psip, const double *F0, double c_j,
             const double *v, double *Jv, const double *psi_n2, const double *osc, const double *v_n2,
-            int v_count) {
+            int v_count, const double *skip) {
     hipStream_t s = c->stream;
     const long N = c->N;
     double *part = c->red.p;  // [0, 512) psi partials, [512, 1024) v partials, [1024] sigma
@@ -134,7 +157,7 @@ int jv_impl(fvp_ctx *c, double t, const double *psi, const double *psip, const d
     FVP_HIP(hipGetLastError());
     if (!c->averaging) {  // perturbation and difference quotient fused into the residual kernels
         JvArgs jv;
-        jv.v = v; jv.sig = part + 2 * kRedBlocks; jv.F0 = F0; jv.cj = c_j; jv.osc = osc;
+        jv.v = v; jv.sig = part + 2 * kRedBlocks; jv.F0 = F0; jv.cj = c_j; jv.osc = osc; jv.skip = skip;
         if (fold) {
             jv.psi_n2 = psi_n2; jv.part_v = v_n2; jv.np = v_count; jv.sig_out = part + 2 * kRedBlocks;
         }

@@ -22,6 +22,7 @@
 
 #include "fvp_blas.h"
 #include "fvp_internal.h"
+#include "fvp_sums.h"
 
 using fvp::DevBuf;
 using fvp::set_error;
@@ -40,9 +41,8 @@ struct fvp_integrator {
     int slot[NHIST];
     double th[NHIST];
     int nh = 0;
-    DevBuf<double> yp, ewt, y, ypn, ypred, ypred2, G, b, delta, beta, tmp, part, scal;
-    double *hscal = nullptr;   // pinned host: the norms the step logic reads
-    hipEvent_t hev = nullptr;  // marks the kernels that wrote them
+    DevBuf<double> yp, ewt, y, ypn, ypred, G, b, delta, beta, tmp, part, scal;
+    fvp::HostSlots hscal;           // the norms the step logic reads
     double h = 0., ss = 20., cj_setup = -1.;
     int k = 1, steps_at_k = 0, steps_since_setup = 0;
     bool need_setup = true;
@@ -96,19 +96,98 @@ __global__ void ewt_kernel(long n, double rtol, double atol, const double *__res
     if (i < n) w[i] = 1.0 / (rtol * fabs(y[i]) + atol);
 }
 
-__global__ void mul_kernel(long n, const double *__restrict__ a, const double *__restrict__ b, double *__restrict__ o) {
-    long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    if (i < n) o[i] = a[i] * b[i];
-}
-
 __global__ void div_kernel(long n, const double *__restrict__ a, const double *__restrict__ b, double *__restrict__ o) {
     long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
     if (i < n) o[i] = a[i] / b[i];
 }
 
-__global__ void axpby_kernel(long n, double a, const double *__restrict__ x, double b, double *__restrict__ y) {
-    long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    if (i < n) y[i] = a * x[i] + b * y[i];
+// ---- the vector work of a step, one launch between two kernels of the solver -------
+// Small problems are bound by launches and by the host's waits (31 000 nodes: about
+// 4 us for a launch that the queue is waiting for, 15 us for a copy or an event), large
+// ones by the vectors' bytes, so that each of these reads a vector once for all that
+// is made of it.  8 steps on 31 000 nodes: 5.7 -> 3.2 ms with these in place of one
+// launch per vector operation and a wait per norm.
+
+// Start of an attempt: the predictor (also the first iterate), beta and y' = cj y + beta
+__global__ void step_predict(long n, int mp, Coef8 cp, int mb, Coef8 cb, double cj, double *__restrict__ ypred,
+                             double *__restrict__ beta, double *__restrict__ y, double *__restrict__ yp) {
+    const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    double s = 0., b = 0., d = 0.;
+    for (int q = 0; q < mp; ++q) s += cp.v[q] * cp.x[q][i];
+    for (int q = 0; q < mb; ++q) b += cb.v[q] * cb.x[q][i];
+    d += cj * s;
+    d += b;
+    ypred[i] = s;
+    beta[i] = b;
+    y[i] = s;
+    yp[i] = d;
+}
+
+// Newton's linear system: b = -ewt G, delta = 0; partials of ||b||^2 and ||y||^2
+__global__ void __launch_bounds__(kGsThreads) newton_rhs(long n, const double *__restrict__ G,
+                                                         const double *__restrict__ ewt, const double *__restrict__ y,
+                                                         double *__restrict__ b, double *__restrict__ delta,
+                                                         double *__restrict__ part) {
+    double acc[2] = {0., 0.};
+    for (long i = blockIdx.x * (long)kGsThreads + threadIdx.x; i < n; i += (long)gridDim.x * kGsThreads) {
+        const double v = G[i] * ewt[i], yi = y[i];
+        b[i] = -v;
+        delta[i] = 0.;
+        acc[0] += v * v;
+        acc[1] += yi * yi;
+    }
+    gs_store<2>(acc, 2, gridDim.x, part);
+}
+
+// Newton update y += delta and its y' = cj y + beta; partials of the weighted squares
+// of delta, of the error estimate y - ypred and, with m2 > 0, of the next lower order's
+// y - sum c2 x2 (the estimates are read only where the iteration ends here)
+__global__ void __launch_bounds__(kGsThreads) newton_update(long n, const double *__restrict__ delta,
+                                                            const double *__restrict__ ewt, double cj,
+                                                            const double *__restrict__ beta,
+                                                            const double *__restrict__ ypred, int m2, Coef8 c2,
+                                                            double *__restrict__ y, double *__restrict__ yp,
+                                                            double *__restrict__ part) {
+    double acc[3] = {0., 0., 0.};
+    for (long i = blockIdx.x * (long)kGsThreads + threadIdx.x; i < n; i += (long)gridDim.x * kGsThreads) {
+        const double d = delta[i], w = ewt[i], yn = d + y[i];
+        double s = 0., p = 0.;
+        s += cj * yn;
+        s += beta[i];
+        y[i] = yn;
+        yp[i] = s;
+        const double e0 = d * w, e1 = (yn - ypred[i]) * w;
+        for (int q = 0; q < m2; ++q) p += c2.v[q] * c2.x[q][i];
+        const double e2 = (yn - p) * w;
+        acc[0] += e0 * e0;
+        acc[1] += e1 * e1;
+        acc[2] += e2 * e2;
+    }
+    gs_store<3>(acc, 3, gridDim.x, part);
+}
+
+// An accepted step: the history's new vector, its derivative and the error weights
+__global__ void step_accept(long n, double rtol, double atol, const double *__restrict__ y,
+                            const double *__restrict__ ypn, double *__restrict__ hist, double *__restrict__ yp,
+                            double *__restrict__ ewt) {
+    const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const double v = y[i];
+    hist[i] = v;
+    yp[i] = ypn[i];
+    ewt[i] = 1.0 / (rtol * fabs(v) + atol);
+}
+
+// partials of the weighted squares of v
+__global__ void __launch_bounds__(kGsThreads) weighted_sq(long n, const double *__restrict__ v,
+                                                          const double *__restrict__ ewt, double *__restrict__ part) {
+    double acc[1] = {0.};
+    for (long i = blockIdx.x * (long)kGsThreads + threadIdx.x; i < n; i += (long)gridDim.x * kGsThreads) {
+        const double x = v[i] * ewt[i];
+        acc[0] += x * x;
+    }
+    gs_store<1>(acc, 1, gridDim.x, part);
 }
 
 // yp0 = F / ahh where ahh != 0 and the row is not Dirichlet, else 0 (Physics::initialise)
@@ -201,42 +280,32 @@ __global__ void __launch_bounds__(256) seg_sq(const int *__restrict__ seg, const
     if (threadIdx.x == 0) out[g] = lds[0] + lds[1] + lds[2] + lds[3];
 }
 
-// out[0] = max over instances of sqrt(sum / size), out[1] = total sum; the
-// same to hout (pinned host memory)
-__global__ void seg_fold(int nseg, const int *__restrict__ seg, const double *__restrict__ sums,
-                         double *__restrict__ out, double *__restrict__ hout) {
+// max over instances of sqrt(sum / size) to the host's slot
+__global__ void seg_fold(int nseg, const int *__restrict__ seg, const double *__restrict__ sums, double *slot,
+                         double tag) {
     if (threadIdx.x != 0) return;
-    double mx = 0., tot = 0.;
-    for (int g = 0; g < nseg; ++g) {
-        mx = fmax(mx, sqrt(sums[g] / (seg[g + 1] - seg[g])));
-        tot += sums[g];
-    }
-    out[0] = mx;
-    out[1] = tot;
-    hout[0] = mx;
-    hout[1] = tot;
-    __threadfence_system();
+    double mx = 0.;
+    for (int g = 0; g < nseg; ++g) mx = fmax(mx, sqrt(sums[g] / (seg[g + 1] - seg[g])));
+    slot[0] = mx;
+    slot_post(slot, tag);
 }
 
 // Weighted RMS norm ||v||_WRMS with the error weights (the maximum over the
-// instances of an ensemble); l2 (optional) gets the plain 2-norm of v * ewt.
-// The norm's last kernel stores it to pinned host memory; a failed wait gives
-// NaN (every test on it fails; the error is recorded).
-static double wrms(fvp_integrator *I, const double *v, double *l2 = nullptr) {
+// instances of an ensemble).  The norm's last kernel stores it to pinned host
+// memory; a failed wait gives NaN (every test on it fails; the error is recorded).
+static double wrms(fvp_integrator *I, const double *v) {
     hipStream_t s = I->c->stream;
-    const double *r = I->hscal;
+    double *r = I->hscal.p;
+    const double tag = ++I->hscal.tag;
     if (I->nseg > 1) {
         seg_sq<<<I->nseg, 256, 0, s>>>(I->seg.p, v, I->ewt.p, I->seg_sum.p);
-        seg_fold<<<1, 64, 0, s>>>(I->nseg, I->seg.p, I->seg_sum.p, I->scal.p, I->hscal);
-        if (host_wait(s, I->hev)) return std::nan("");
-        if (l2) *l2 = std::sqrt(r[1]);
-        return r[0];
+        seg_fold<<<1, 64, 0, s>>>(I->nseg, I->seg.p, I->seg_sum.p, r, tag);
+        return slot_wait(s, r, tag) ? std::nan("") : r[0];
     }
-    mul_kernel<<<nb(I->N), 256, 0, s>>>(I->N, v, I->ewt.p, I->tmp.p);
-    dot_async(s, I->N, I->tmp.p, I->tmp.p, I->part.p, I->scal.p, I->hscal);
-    if (host_wait(s, I->hev)) return std::nan("");
-    if (l2) *l2 = std::sqrt(r[0]);
-    return std::sqrt(r[0] / I->N);
+    const int np = gs_nb(I->N);
+    weighted_sq<<<np, kGsThreads, 0, s>>>(I->N, v, I->ewt.p, I->part.p);
+    gs_post<1><<<1, kGsThreads, 0, s>>>(np, I->part.p, I->scal.p, r, tag);
+    return slot_wait(s, r, tag) ? std::nan("") : std::sqrt(r[0] / I->N);
 }
 
 static void lincomb(fvp_integrator *I, int m, const double *c, const double *const *x, double *out) {
@@ -272,19 +341,19 @@ static void bdf_weights(const double *tau, int k, double *a) {
 
 static const double *H(fvp_integrator *I, int i) { return I->hist[I->slot[i]].p; }
 
-// predicted y at tau[0] of degree q (needs q+1 history points); q < 0: y_n + h y'_n
-static void predict(fvp_integrator *I, const double *tau, int q, double *out) {
+// terms of the predicted y at tau[0] of degree q (needs q+1 history points); q < 1: y_n + h y'_n
+static int predictor(fvp_integrator *I, const double *tau, int q, Coef8 &cf) {
+    cf = Coef8{};
     if (q < 1 || I->nh < q + 1) {
-        double c2[2] = {1., tau[0] - tau[1]};
-        const double *x2[2] = {H(I, 0), I->yp.p};
-        lincomb(I, 2, c2, x2, out);
-        return;
+        cf.v[0] = 1.;
+        cf.x[0] = H(I, 0);
+        cf.v[1] = tau[0] - tau[1];
+        cf.x[1] = I->yp.p;
+        return 2;
     }
-    double w[NHIST];
-    const double *x[NHIST];
-    predictor_weights(tau, q, w);
-    for (int i = 0; i <= q; ++i) x[i] = H(I, i);
-    lincomb(I, q + 1, w, x, out);
+    predictor_weights(tau, q, cf.v);
+    for (int i = 0; i <= q; ++i) cf.x[i] = H(I, i);
+    return q + 1;
 }
 
 // One attempt: 0 accepted, 1 error test failed, 2 Newton / linear failure, <0 fatal
@@ -297,25 +366,15 @@ static int attempt(fvp_integrator *I, double h, int k, double *err_k, double *er
     for (int i = 0; i < I->nh; ++i) tau[i + 1] = I->th[i];
     const double t = tau[0];
     const int q = std::min(k, I->nh - 1);  // predictor degree
-    predict(I, tau, q, I->ypred.p);
+    Coef8 cp, cb{};
+    const int mp = predictor(I, tau, q, cp);
     double a[NHIST];
     bdf_weights(tau, k, a);
     const double cj = a[0];
     // beta = sum_{i>=1} a_i y_{n+1-i}
-    {
-        double w[NHIST];
-        const double *x[NHIST];
-        for (int i = 1; i <= k; ++i) { w[i - 1] = a[i]; x[i - 1] = H(I, i - 1); }
-        lincomb(I, k, w, x, I->beta.p);
-    }
-    FVP_HIP(hipMemcpyAsync(I->y.p, I->ypred.p, sizeof(double) * N, hipMemcpyDeviceToDevice, s));
-    // y' = cj y + beta
-    auto deriv = [&]() {
-        double c2[2] = {cj, 1.};
-        const double *x2[2] = {I->y.p, I->beta.p};
-        lincomb(I, 2, c2, x2, I->ypn.p);
-    };
-    deriv();
+    for (int i = 1; i <= k; ++i) { cb.v[i - 1] = a[i]; cb.x[i - 1] = H(I, i - 1); }
+    step_predict<<<nb(N), 256, 0, s>>>(N, mp, cp, k, cb, cj, I->ypred.p, I->beta.p, I->y.p, I->ypn.p);
+    FVP_HIP(hipGetLastError());
     if (fvp::residual_impl(c, t, I->y.p, I->ypn.p, I->G.p, c->averaging)) return -1;
     I->learn_took = false;
     bool learn = I->mp && !I->learn_block;
@@ -391,24 +450,28 @@ static int attempt(fvp_integrator *I, double h, int k, double *err_k, double *er
     const double tol_abs = I->p.lin_factor * I->p.newton_tol * std::sqrt((double)(I->nseg > 1 ? I->seg_min : N));
     double oldnrm = 0.;
     bool conv = false;
+    // the error estimate of the next lower order, where there is one
+    const bool lower = k >= 2 && I->nh >= k;
+    Coef8 c2{};
+    const int m2 = lower ? predictor(I, tau, k - 1, c2) : 0;
+    const int np = gs_nb(N);
+    double sums[3] = {0., 0., 0.};  // of the last update
     for (int m = 0; m < I->p.max_newton; ++m) {
-        if (m > 0) {
-            deriv();
-            if (fvp::residual_impl(c, t, I->y.p, I->ypn.p, I->G.p, c->averaging)) return -1;
-        }
-        // b = -ewt * G ; solve (S J) delta = S (-G), right precond M S^-1
-        mul_kernel<<<nb(N), 256, 0, s>>>(N, I->G.p, I->ewt.p, I->b.p);
-        axpby_kernel<<<nb(N), 256, 0, s>>>(N, 0., I->b.p, -1., I->b.p);
-        FVP_HIP(hipMemsetAsync(I->delta.p, 0, sizeof(double) * N, s));
-        double bn = 0.;
-        (void)wrms(I, I->G.p, &bn);
+        if (m > 0 && fvp::residual_impl(c, t, I->y.p, I->ypn.p, I->G.p, c->averaging)) return -1;
+        // solve (S J) delta = S (-G), right precond M S^-1; ||y||^2 once for the Newton
+        // iterate (the FD increment of every J v of this solve)
+        double *const hs = I->hscal.p, *const bn2 = I->scal.p + 3, *const yn2 = I->scal.p + 4;
+        newton_rhs<<<np, kGsThreads, 0, s>>>(N, I->G.p, I->ewt.p, I->y.p, I->b.p, I->delta.p, I->part.p);
+        double tag = ++I->hscal.tag;
+        gs_post<2><<<1, kGsThreads, 0, s>>>(np, I->part.p, bn2, hs, tag);
+        FVP_HIP(hipGetLastError());
+        if (slot_wait(s, hs, tag)) return -1;
+        const fvp::GmresZero zero{hs[0], bn2};
+        const double bn = std::sqrt(zero.norm2);
         fvp_gmres_params gp{I->p.dim_krylov, I->p.max_restarts, I->p.reorthogonalise, bn > 0 ? tol_abs / bn : 1.};
         fvp_gmres_stats gs{};
         const double *yv = I->y.p, *ypv = I->ypn.p, *Gv = I->G.p, *ew = I->ewt.p;
         double *tmpv = I->tmp.p;
-        // ||y||^2 once for the Newton iterate (the FD increment of every J v of this solve)
-        double *yn2 = I->scal.p + 4;
-        if (dot_async(s, N, yv, yv, I->part.p, yn2)) return -1;
         // S J: the error weights scale the J v rows inside the residual kernels.
         // GMRES applies J to the vector the preconditioner solve has just written
         // (its ||z||^2 partials come with it); any other input is reduced afresh.
@@ -421,7 +484,7 @@ static int attempt(fvp_integrator *I, double h, int k, double *err_k, double *er
             const bool fresh = in == ls->z && ls->zn2;
             ls->z = nullptr;
             return fvp::jv_impl(c, t, yv, ypv, Gv, cj, in, out, yn2, ew, fresh ? ls->zn2 : nullptr,
-                                fresh ? ls->count : 0);
+                                fresh ? ls->count : 0, fvp::gmres_skip(W));
         };
         Op M;
         if (I->p.precon_type != FVP_PRECON_NONE)
@@ -436,7 +499,7 @@ static int attempt(fvp_integrator *I, double h, int k, double *err_k, double *er
                 div_kernel<<<nb(N), 256, 0, s>>>(N, in, ew, out);
                 return 0;
             };
-        int rc = fvp::gmres_device(W, s, N, A, M, I->b.p, I->delta.p, &gp, &gs, true);
+        int rc = fvp::gmres_device(W, s, N, A, M, I->b.p, I->delta.p, &gp, &gs, &zero);
         I->st.gmres_iters += gs.iterations;
         if (rc < 0) return -1;
         // a linear solve that stopped short of its tolerance still gives a Newton
@@ -447,9 +510,20 @@ static int attempt(fvp_integrator *I, double h, int k, double *err_k, double *er
         // J v is formed at the current c_j, so the Newton update is taken as
         // solved; IDA scales by 2/(1+c_j ratio) only for a stored (stale)
         // iteration matrix, not for its matrix-free SPGMR solve
-        axpby_kernel<<<nb(N), 256, 0, s>>>(N, 1., I->delta.p, 1., I->y.p);
+        newton_update<<<np, kGsThreads, 0, s>>>(N, I->delta.p, I->ewt.p, cj, I->beta.p, I->ypred.p, m2, c2, I->y.p,
+                                                I->ypn.p, I->part.p);
         ++I->st.newton_iters;
-        double delnrm = wrms(I, I->delta.p);
+        double delnrm;
+        if (I->nseg > 1) {
+            delnrm = wrms(I, I->delta.p);
+        } else {
+            tag = ++I->hscal.tag;
+            gs_post<3><<<1, kGsThreads, 0, s>>>(np, I->part.p, I->scal.p, hs, tag);
+            FVP_HIP(hipGetLastError());
+            if (slot_wait(s, hs, tag)) return -1;
+            std::copy(hs, hs + 3, sums);
+            delnrm = std::sqrt(sums[0] / N);
+        }
         if (m == 0) {
             oldnrm = delnrm;
             if (delnrm <= 1e-4 * I->p.newton_tol || I->ss * delnrm <= I->p.newton_tol) { conv = true; break; }
@@ -463,24 +537,22 @@ static int attempt(fvp_integrator *I, double h, int k, double *err_k, double *er
         }
     }
     if (!conv) return 2;
-    deriv();
     if (I->rec_targ) learn_target<<<nb(N), 256, 0, s>>>(N, I->y.p, I->ypred.p, I->ewt.p, I->rec_targ);
     // local error estimate from the predictor-corrector difference
-    {
-        double c2[2] = {1., -1.};
-        const double *x2[2] = {I->y.p, I->ypred.p};
-        lincomb(I, 2, c2, x2, I->b.p);
-    }
     double fac = (q >= 1 && I->nh >= q + 1) ? h / (tau[0] - tau[q + 1]) : 1.0;
-    *err_k = wrms(I, I->b.p) * fac;
+    auto estimate = [&](double sum, int mx, const double *cx, const double *const *xx) {
+        if (I->nseg <= 1) return std::sqrt(sum / N);
+        double cf[8] = {1.};
+        const double *x[8] = {I->y.p};
+        for (int i = 0; i < mx; ++i) { cf[i + 1] = -cx[i]; x[i + 1] = xx[i]; }
+        lincomb(I, mx + 1, cf, x, I->b.p);
+        return wrms(I, I->b.p);
+    };
+    const double one = 1.;
+    const double *const yq = I->ypred.p;
+    *err_k = estimate(sums[1], 1, &one, &yq) * fac;
     *err_km1 = 1e300;
-    if (k >= 2 && I->nh >= k) {
-        predict(I, tau, k - 1, I->ypred2.p);
-        double c2[2] = {1., -1.};
-        const double *x2[2] = {I->y.p, I->ypred2.p};
-        lincomb(I, 2, c2, x2, I->b.p);
-        *err_km1 = wrms(I, I->b.p) * h / (tau[0] - tau[k]);
-    }
+    if (lower) *err_km1 = estimate(sums[2], m2, c2.v, c2.x) * h / (tau[0] - tau[k]);
     return *err_k <= 1.0 ? 0 : 1;
 }
 
@@ -491,10 +563,10 @@ static int accept(fvp_integrator *I, double h) {
     for (int i = NHIST - 1; i > 0; --i) { I->slot[i] = I->slot[i - 1]; I->th[i] = I->th[i - 1]; }
     I->slot[0] = oldest;
     I->th[0] = I->th[1] + h;
-    FVP_HIP(hipMemcpyAsync(I->hist[oldest].p, I->y.p, sizeof(double) * I->N, hipMemcpyDeviceToDevice, s));
-    FVP_HIP(hipMemcpyAsync(I->yp.p, I->ypn.p, sizeof(double) * I->N, hipMemcpyDeviceToDevice, s));
+    step_accept<<<nb(I->N), 256, 0, s>>>(I->N, I->p.rtol, I->p.atol, I->y.p, I->ypn.p, I->hist[oldest].p, I->yp.p,
+                                         I->ewt.p);
+    FVP_HIP(hipGetLastError());
     I->nh = std::min(I->nh + 1, NHIST);
-    ewt_kernel<<<nb(I->N), 256, 0, s>>>(I->N, I->p.rtol, I->p.atol, H(I, 0), I->ewt.p);
     ++I->st.steps;
     ++I->steps_since_setup;
     I->st.t = I->th[0];
@@ -583,21 +655,13 @@ extern "C" int fvp_integrator_create(fvp_ctx *c, const fvp_integrator_params *p,
         I->th[i] = t0;
     }
     if (I->yp.alloc(N) || I->ewt.alloc(N) || I->y.alloc(N) || I->ypn.alloc(N) || I->ypred.alloc(N) ||
-        I->ypred2.alloc(N) || I->G.alloc(N) || I->b.alloc(N) || I->delta.alloc(N) || I->beta.alloc(N) ||
-        I->tmp.alloc(N) || I->part.alloc(512) || I->scal.alloc(8)) {
+        I->G.alloc(N) || I->b.alloc(N) || I->delta.alloc(N) || I->beta.alloc(N) ||
+        I->tmp.alloc(N) || I->part.alloc(3 * kGsNb) || I->scal.alloc(8)) {
         fvp_integrator_destroy(I);
         return -1;
     }
-    if (hipHostMalloc((void **)&I->hscal, sizeof(double) * 8, hipHostMallocDefault) != hipSuccess) {
-        I->hscal = nullptr;
+    if (I->hscal.alloc(1)) {
         fvp_integrator_destroy(I);
-        set_error("pinned host allocation failed");
-        return -1;
-    }
-    if (hipEventCreateWithFlags(&I->hev, hipEventDisableTiming) != hipSuccess) {
-        I->hev = nullptr;
-        fvp_integrator_destroy(I);
-        set_error("event creation failed");
         return -1;
     }
     hipStream_t s = c->stream;
@@ -620,14 +684,13 @@ extern "C" int fvp_integrator_create(fvp_ctx *c, const fvp_integrator_params *p,
 extern "C" int fvp_integrator_destroy(fvp_integrator *I) {
     if (!I) return 0;
     for (int i = 0; i < NHIST; ++i) I->hist[i].release();
-    I->yp.release(); I->ewt.release(); I->y.release(); I->ypn.release(); I->ypred.release(); I->ypred2.release();
+    I->yp.release(); I->ewt.release(); I->y.release(); I->ypn.release(); I->ypred.release();
     I->G.release(); I->b.release(); I->delta.release(); I->beta.release(); I->tmp.release(); I->part.release();
     I->scal.release();
     I->seg.release(); I->seg_sum.release();
     I->stat.release(); I->feat.release(); I->ylearn.release(); I->y2.release(); I->ypn2.release();
     I->G2.release();
-    if (I->hscal) (void)hipHostFree(I->hscal);
-    if (I->hev) (void)hipEventDestroy(I->hev);
+    I->hscal.release();
     delete I;
     return 0;
 }

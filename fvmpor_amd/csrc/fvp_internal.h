@@ -147,15 +147,16 @@ struct JvArgs {
     const double *psi_n2 = nullptr, *part_v = nullptr;
     double *sig_out = nullptr;
     int np = 0;
+    const double *skip = nullptr;  // optional: a nonzero word ends the element kernels early
 };
 // J v with options for the integrator's scaled solve: psi_n2 (device scalar,
 // or null) is ||psi||^2 computed once for the Newton iterate; v_n2 (or null)
 // holds v_count partial sums of ||v||^2 already formed by the solve that wrote
-// v (used only with psi_n2); osc (or null) scales the result row-wise.
-// fvp_jv is the plain form.
+// v (used only with psi_n2); osc (or null) scales the result row-wise; skip (or
+// null): see JvArgs.  fvp_jv is the plain form.
 int jv_impl(fvp_ctx *c, double t, const double *psi, const double *psip, const double *F0, double c_j,
             const double *v, double *Jv, const double *psi_n2, const double *osc, const double *v_n2 = nullptr,
-            int v_count = 0);
+            int v_count = 0, const double *skip = nullptr);
 // element-local FD Jacobian into J (nnz values); the arrays as in fvp_jacdata
 int fd_jacobian_elem(fvp_ctx *c, double cj, const double *psi, const double *psip, const double *shift, double *ys,
                      double *kr2, double *cap2, double *contrib, const long *cptr, const int *srank, const int *ia,

@@ -31,6 +31,7 @@
 #include "fvp_blas.h"
 #include "fvp_dense.h"
 #include "fvp_internal.h"
+#include "fvp_sums.h"
 
 using fvp::DevBuf;
 using fvp::set_error;
@@ -116,8 +117,9 @@ struct fvp_csr {
     int m_alloc = -1;
     DevBuf<double> Q, w, r, z, part, scal, hdev;
     DevBuf<double> Hd, gd, csd, snd, yd;    // Hessenberg (column-major, m+1 rows), Givens pairs, rhs, solution
-    double *hstat = nullptr;                // pinned host: slots of kSlot doubles, see GmresWork
-    double tag = 0;                         // last tag given to a slot's writer
+    fvp::HostSlots hstat;                        // GMRES, see GmresWork
+    fvp::HostSlots hflag;                        // factorisation: the pivot flag
+    const double *skip = nullptr;           // while GMRES queues a step: its word that ends the cycle
     DevBuf<double> Qk;                      // deflated GMRES: the kept harmonic Ritz vectors
     fvp_schur *sc = nullptr;                // Schur-complement preconditioner (FVP_PRECON_SCHUR)
 };
@@ -151,12 +153,14 @@ template <int LANES>
 __global__ void __launch_bounds__(256) csr_gemv_kernel(int n, const int *__restrict__ ia, const int *__restrict__ ja,
                                                        const double *__restrict__ a, double alpha,
                                                        const double *__restrict__ x, double beta,
-                                                       double *__restrict__ y) {
+                                                       double *__restrict__ y, const double *skip) {
+    const double over = skip_word(skip);
     int tid = blockIdx.x * blockDim.x + threadIdx.x;
     int row = tid / LANES, lane = tid % LANES;
     double s = 0.;
-    if (row < n)
-        for (int k = ia[row] + lane; k < ia[row + 1]; k += LANES) s += a[k] * x[ja[k]];
+    const int k0 = row < n ? ia[row] : 0, k1 = row < n ? ia[row + 1] : 0;
+    if (over != 0.) return;
+    for (int k = k0 + lane; k < k1; k += LANES) s += a[k] * x[ja[k]];
 #pragma unroll
     for (int off = LANES / 2; off > 0; off >>= 1) s += __shfl_down(s, off, LANES);
     if (row < n && lane == 0) y[row] = beta == 0. ? alpha * s : alpha * s + beta * y[row];
@@ -226,6 +230,15 @@ __global__ void jacobi_build(int n, const int *__restrict__ ia, const int *__res
     while (pos < ia[i + 1] && ja[pos] < i) pos++;
     if (pos == ia[i + 1] || ja[pos] != i || a[pos] == 0.) { atomicOr(flag, 1); J[i] = 0.; return; }
     J[i] = 1. / a[pos];
+}
+
+// the pivot flag to the host's slot (a copy and a blocking wait cost about
+// 15 us after the kernel), cleared for the next factorisation
+__global__ void flag_post(int *__restrict__ flag, double *slot, double tag) {
+    if (threadIdx.x) return;
+    slot[0] = flag[0];
+    flag[0] = 0;
+    slot_post(slot, tag);
 }
 
 __global__ void vmul(long n, const double *__restrict__ a, const double *__restrict__ b, double *__restrict__ c) {
@@ -510,8 +523,7 @@ __global__ void __launch_bounds__(256) arnoldi_finish(int j, int m, const double
     if (hslot) {
         hslot[0] = fabs(g[j + 1]);
         hslot[1] = hn;
-        __threadfence_system();
-        __hip_atomic_store(hslot + 2, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        slot_post(hslot, tag);
     }
 }
 
@@ -528,82 +540,8 @@ __global__ void __launch_bounds__(256) arnoldi_finish(int j, int m, const double
 // update), and at 192 000 rows and below the latency of one round of loads per
 // thread, which is why every column's load is issued before the sums.
 // Per step of the Krylov solve of 191 771 rows, 21 steps (Jacobi): 65 -> 33 us.
-constexpr int kGsThreads = 512;
-constexpr int kGsNb = 256;   // workgroups: one per CU
 constexpr int kGsCols = 32;  // columns held in registers; longer bases go through mdot_kernel and axpy_norm
-constexpr int kGsWaves = kGsThreads / 64;
 static_assert(kGsNb * (kGsCols + 1) <= kGsBlocks * (kChunk + 1), "partials fit the workspace");
-
-static inline int gs_nb(long n) {
-    return (int)std::max(1L, std::min((long)kGsNb, ((n >> 1) + kGsThreads - 1) / kGsThreads));
-}
-
-// Sums L columns over the wavefront: at each step a lane keeps one half of the
-// columns and gives the other to its partner, L / 2 + L / 4 + ... exchanges
-// instead of 6 L.  Returns column col's sum, if col < end (else the lane has none).
-template <int BIT, int L>
-__device__ __forceinline__ double fold_cols(const double (&v)[L], int &col, int &end) {
-    if constexpr (BIT == 0) {
-        static_assert(L == 1, "at most 64 columns");
-        return v[0];
-    } else if constexpr (L == 1) {
-        double k[1] = {v[0] + __shfl_xor(v[0], BIT, 64)};
-        return fold_cols<BIT / 2, 1>(k, col, end);
-    } else {
-        constexpr int H = (L + 1) / 2;
-        const bool up = threadIdx.x & BIT;
-        double k[H];
-#pragma unroll
-        for (int i = 0; i < H; ++i) {
-            const double lo = v[i], hi = i + H < L ? v[i + H] : 0.;
-            k[i] = (up ? hi : lo) + __shfl_xor(up ? lo : hi, BIT, 64);
-        }
-        if (up) col += H;
-        else end = end < col + H ? end : col + H;
-        return fold_cols<BIT / 2, H>(k, col, end);
-    }
-}
-
-// Block partials of K columns: part[c * nb + block]
-template <int K>
-__device__ __forceinline__ void gs_store(const double (&acc)[K], int nk, int nb, double *__restrict__ part) {
-    __shared__ double lds[kGsWaves][K];
-    int col = 0, end = K;
-    const double v = fold_cols<32, K>(acc, col, end);
-    if (col < end) lds[threadIdx.x >> 6][col] = v;
-    __syncthreads();
-    if ((int)threadIdx.x < nk) {
-        double t = 0.;
-#pragma unroll
-        for (int w = 0; w < kGsWaves; ++w) t += lds[w][threadIdx.x];
-        part[threadIdx.x * nb + blockIdx.x] = t;
-    }
-}
-
-// out[c] (LDS) = sum of column c's nb partials, c < K, in an order that depends
-// on nb alone: every workgroup gets the same values.  Ends with a barrier.
-template <int K>
-__device__ __forceinline__ void gs_sums(int nb, const double *__restrict__ part, double *out) {
-    constexpr int CW = (K + kGsWaves - 1) / kGsWaves, U = kGsNb / 64;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    double v[CW][U], s[CW];
-#pragma unroll
-    for (int i = 0; i < CW; ++i) {
-        const int c = wv + i * kGsWaves;
-#pragma unroll
-        for (int u = 0; u < U; ++u) v[i][u] = c < K && lane + 64 * u < nb ? part[c * nb + lane + 64 * u] : 0.;
-    }
-#pragma unroll
-    for (int i = 0; i < CW; ++i) {
-        s[i] = 0.;
-#pragma unroll
-        for (int u = 0; u < U; ++u) s[i] += v[i][u];
-    }
-    int col = 0, end = CW;
-    const double t = fold_cols<32, CW>(s, col, end);
-    if (col < end && wv + col * kGsWaves < K) out[wv + col * kGsWaves] = t;
-    __syncthreads();
-}
 
 // a wavefront-uniform value in scalar registers
 __device__ __forceinline__ double uniform(double x) {
@@ -750,8 +688,7 @@ __device__ inline void gs_hessenberg(int j, int m, double hk, double hn, double 
         if (hslot) {
             hslot[0] = est;
             hslot[1] = hn;
-            __threadfence_system();
-            __hip_atomic_store(hslot + 2, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+            slot_post(hslot, tag);
         }
     }
     wave_lds_order();
@@ -899,33 +836,17 @@ __global__ void gs_start(long n, const double *__restrict__ r, const double *__r
     if (diag) z[i] = v * diag[i];
 }
 
-// r = b - r (or b, when zero), block partials of r . r and b . b
-__global__ void __launch_bounds__(kGsThreads) gs_residual(long n, int zero, const double *__restrict__ b,
+// r = b - r, block partials of r . r and b . b
+__global__ void __launch_bounds__(kGsThreads) gs_residual(long n, const double *__restrict__ b,
                                                           double *__restrict__ r, double *__restrict__ part) {
     double acc[2] = {0., 0.};
     for (long i = blockIdx.x * (long)kGsThreads + threadIdx.x; i < n; i += (long)gridDim.x * kGsThreads) {
-        const double bi = b[i], v = zero ? bi : bi - r[i];
+        const double bi = b[i], v = bi - r[i];
         r[i] = v;
         acc[0] += v * v;
         acc[1] += bi * bi;
     }
     gs_store<2>(acc, 2, gridDim.x, part);
-}
-
-// out[0, 2) = the two sums, to the host's slot as well, tag behind them
-__global__ void __launch_bounds__(kGsThreads) gs_norms(int nb, const double *__restrict__ part,
-                                                       double *__restrict__ out, double *hslot, double tag) {
-    __shared__ double s[2];
-    gs_sums<2>(nb, part, s);
-    if (threadIdx.x) return;
-    out[0] = s[0];
-    out[1] = s[1];
-    if (hslot) {
-        hslot[0] = s[0];
-        hslot[1] = s[1];
-        __threadfence_system();
-        __hip_atomic_store(hslot + 2, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
 }
 
 // End of a cycle: y = R^-1 g on the first k rotated columns, then out = Q y, or
@@ -1567,8 +1488,9 @@ __global__ void __launch_bounds__(64) bj_solve(const int *__restrict__ roff, con
                                                int maxrows, int ovmax, int levmax_l, int levmax_u,
                                                const double *__restrict__ x,
                                                const double *__restrict__ xdiv, double *__restrict__ y,
-                                               double *__restrict__ yn2) {
+                                               double *__restrict__ yn2, const double *skip) {
     extern __shared__ double smem[];
+    const double over = skip_word(skip);
     const int b = blockIdx.x;
     const int base = roff[b];
     const int cnt = roff[b + 1] - base;
@@ -1631,6 +1553,7 @@ __global__ void __launch_bounds__(64) bj_solve(const int *__restrict__ roff, con
     if (nsl > 0) bj_meta_store(mq, ms, nsl, threadIdx.x);
     bj_meta_stage(meta_l + sl0, ms, nsl, threadIdx.x + 64 * kBjMeta);
     wave_lds_order();
+    if (over != 0.) return;
     bj_sweep<T, false, OVG>(v, vd, nl, lpl, ms, val_l + ebase_l[b], col_l + ebase_l[b], nullptr, ovp);
     // U's meta words replace L's (the sweep's LDS accesses execute in order;
     // loading them during L's sweep instead was measured no faster)
@@ -1742,8 +1665,9 @@ __global__ void __launch_bounds__(TH) ilu0_solve(int n, int npl, const int *__re
                                                  const unsigned short *__restrict__ col_u,
                                                  const double *__restrict__ val_u, const double *__restrict__ x,
                                                  const double *__restrict__ xdiv, double *__restrict__ y,
-                                                 double *__restrict__ yn2) {
+                                                 double *__restrict__ yn2, const double *skip) {
     extern __shared__ double smem[];
+    const double over = skip_word(skip);
     double *v = smem, *spare = v + n + threadIdx.x;
     int *pl = reinterpret_cast<int *>(v + n + TH), *pu = pl + npl + 1;
     for (int k = threadIdx.x; k <= npl; k += TH) pl[k] = ppl[k];
@@ -1762,6 +1686,7 @@ __global__ void __launch_bounds__(TH) ilu0_solve(int n, int npl, const int *__re
             if (i0 + TH * u < n) v[i0 + TH * u] = xdiv ? q[u] / d[u] : q[u];
     }
     __syncthreads();
+    if (over != 0.) return;
     ilu0_sweep<KW, TH, false>(v, spare, npl, pl, row_l, col_l, val_l, nullptr);
     __syncthreads();
     ilu0_sweep<KW, TH, true>(v, spare, npu, pu, row_u, col_u, val_u, val_u + (size_t)n * KW);
@@ -1955,8 +1880,6 @@ __global__ void schur_back(int nI, const int *__restrict__ irow, const int *__re
 }
 
 // ---- host helpers ---------------------------------------------------------------
-constexpr int kSlot = 4;  // doubles per host slot: two values, their tag, one spare
-
 static int ensure_work(fvp_csr *A, int m) {
     if (A->m_alloc >= m) return 0;
     long n = A->n;
@@ -1965,16 +1888,7 @@ static int ensure_work(fvp_csr *A, int m) {
         A->Hd.alloc((size_t)(m + 1) * m) || A->gd.alloc(m + 1) || A->csd.alloc(m) || A->snd.alloc(m) ||
         A->yd.alloc(m))
         return -1;
-    if (A->hstat) (void)hipHostFree(A->hstat);
-    A->hstat = nullptr;
-    const size_t bytes = sizeof(double) * kSlot * (m + 1);
-    if (hipHostMalloc((void **)&A->hstat, bytes, hipHostMallocCoherent) != hipSuccess) {
-        A->hstat = nullptr;
-        set_error("pinned host allocation failed");
-        return -1;
-    }
-    std::memset(A->hstat, 0, bytes);
-    A->tag = 0;
+    if (A->hstat.alloc(m + 1)) return -1;
     A->m_alloc = m;
     return 0;
 }
@@ -2011,7 +1925,7 @@ using Op = std::function<int(const double *, double *)>;
 // residual estimate are updated on the device; each Arnoldi step's estimate is
 // written to pinned host memory and read one step later, while the next step
 // is already queued (a cycle that has converged runs one extra, discarded
-// step, of which the Gram-Schmidt updates return at once).  Classical
+// step, whose kernels return once they have read that).  Classical
 // Gram-Schmidt with a second pass only when the first one
 // cancelled more than half of ||w||^2 (reorthogonalise = 1), always (2) or
 // never (0).  A cycle ends early once the estimate meets tol * ||b||.
@@ -2026,35 +1940,17 @@ using Op = std::function<int(const double *, double *)>;
 // the tag: an event per step costs the stream a barrier packet each.  Without,
 // each step's pair is copied and read right after the step (same control flow
 // and results, one synchronisation per step).
+// skip: set, while a step is queued, to the device word that the end of the
+// cycle makes nonzero: the products and solves that look at it leave early.
 // diag: the preconditioner is this diagonal, and the kernels that write a basis
 // vector write z = diag q as well.
 struct GmresWork {
     double *Q, *w, *r, *z, *part, *sc, *hdev, *Hd, *gd, *csd, *snd, *yd;
     double *hstat;
     double *tag;
+    const double **skip;
     const double *diag;
 };
-
-// Waits for tag in a slot.  A queue that ends (or fails) without having written
-// it is an error; asked for only now and then, since the query itself costs more
-// than the reads.
-static int slot_wait(hipStream_t s, const double *slot, double tag) {
-    auto there = [&]() {
-        double v;
-        __atomic_load(slot + 2, &v, __ATOMIC_ACQUIRE);
-        return v == tag;
-    };
-    for (long k = 1; !there(); ++k) {
-        if (k & 0xfffff) continue;
-        const hipError_t e = hipStreamQuery(s);
-        if (e == hipErrorNotReady) continue;
-        FVP_HIP(e);
-        if (there()) break;
-        set_error("GMRES: the queue ended without its status");
-        return -1;
-    }
-    return 0;
-}
 
 // doubles of a GmresWork carved from one device buffer (each piece 256-byte aligned)
 static size_t gmres_work_doubles(long n, int m) {
@@ -2085,21 +1981,25 @@ static GmresWork gmres_work_carve(double *base, long n, int m) {
 }
 
 static int gmres_core(const GmresWork &W, hipStream_t s, long n, const Op &A, const Op &M, const double *b,
-                      double *x, const fvp_gmres_params *p, fvp_gmres_stats *st, bool x_zero = false);
+                      double *x, const fvp_gmres_params *p, fvp_gmres_stats *st, const GmresZero *zero = nullptr);
+
+const double *gmres_skip(const fvp_csr *W) { return W->skip; }
 
 int gmres_device(fvp_csr *W, hipStream_t s, long n, const Op &A, const Op &M, const double *b, double *x,
-                 const fvp_gmres_params *p, fvp_gmres_stats *st, bool x_zero, const double *diag) {
+                 const fvp_gmres_params *p, fvp_gmres_stats *st, const GmresZero *zero, const double *diag) {
     const int m = p->dim_krylov;
     if (m < 1 || m > 63) { set_error("dim_krylov must be 1..63"); return -1; }
     if (p->reorthogonalise < 0 || p->reorthogonalise > 2) { set_error("reorthogonalise must be 0, 1 or 2"); return -1; }
     if (ensure_work(W, m)) return -1;
     GmresWork wk{W->Q.p, W->w.p, W->r.p, W->z.p, W->part.p, W->scal.p, W->hdev.p, W->Hd.p, W->gd.p, W->csd.p,
-                 W->snd.p, W->yd.p, W->hstat, &W->tag, diag};
-    return gmres_core(wk, s, n, A, M, b, x, p, st, x_zero);
+                 W->snd.p, W->yd.p, W->hstat.p, &W->hstat.tag, &W->skip, diag};
+    const int rc = gmres_core(wk, s, n, A, M, b, x, p, st, zero);
+    W->skip = nullptr;
+    return rc;
 }
 
 static int gmres_core(const GmresWork &W, hipStream_t s, long n, const Op &A, const Op &M, const double *b,
-                      double *x, const fvp_gmres_params *p, fvp_gmres_stats *st, bool x_zero) {
+                      double *x, const fvp_gmres_params *p, fvp_gmres_stats *st, const GmresZero *zero) {
     const int m = p->dim_krylov;
     double *Q = W.Q, *w = W.w, *r = W.r, *z = W.z, *part = W.part, *sc = W.sc;
     // h1, h2: first / second pass coefficients (j+1 dots, then ||w||^2); stat: {estimate, h_{j+1,j}}
@@ -2114,11 +2014,11 @@ static int gmres_core(const GmresWork &W, hipStream_t s, long n, const Op &A, co
     double *part2 = nb <= kGsNb / 2 ? part + kHalf : r;
     fvp_gmres_stats stats{0, 0, 0, 0., 0.};
     double hn2[2] = {0., 0.};
-    // queues r = b - r (x_zero: r = b) and waits for ||r||^2 and ||b||^2
-    auto residual = [&](int zero) -> int {
-        gs_residual<<<nb, kGsThreads, 0, s>>>(n, zero, b, r, part);
+    // queues r = b - r and waits for ||r||^2 and ||b||^2
+    auto residual = [&]() -> int {
+        gs_residual<<<nb, kGsThreads, 0, s>>>(n, b, r, part);
         double *slot = W.hstat + (size_t)kSlot * m;
-        gs_norms<<<1, kGsThreads, 0, s>>>(nb, part, sc, W.tag ? slot : nullptr, W.tag ? ++*W.tag : 0.);
+        gs_post<2><<<1, kGsThreads, 0, s>>>(nb, part, sc, W.tag ? slot : nullptr, W.tag ? ++*W.tag : 0.);
         FVP_HIP(hipGetLastError());
         if (W.tag) {
             if (slot_wait(s, slot, *W.tag)) return -1;
@@ -2129,8 +2029,8 @@ static int gmres_core(const GmresWork &W, hipStream_t s, long n, const Op &A, co
         for (int k = 0; k < 2; ++k) hn2[k] = slot[k];
         return 0;
     };
-    if (!x_zero && A(x, r)) return -1;
-    if (residual(x_zero)) return -1;
+    if (zero) hn2[0] = hn2[1] = zero->norm2;
+    else if (A(x, r) || residual()) return -1;
     double beta = std::sqrt(hn2[0]), normb = std::sqrt(hn2[1]);
     double error = normb > 0 ? beta / normb : 0.;
     if (beta == 0. || error < p->tol) {
@@ -2141,8 +2041,9 @@ static int gmres_core(const GmresWork &W, hipStream_t s, long n, const Op &A, co
     const double thr = p->tol * normb;
     int restarts = 0, converged = 0, total = 0;
     double step_tag = 0.;  // of the step before
+    bool x_zero = zero;  // x is still zero, the residual still b
     while (restarts <= p->max_restarts && !converged) {
-        gs_start<<<nblk(n, 256), 256, 0, s>>>(n, r, sc, beta, Q, W.diag, z, W.gd, m + 1, ctl);
+        gs_start<<<nblk(n, 256), 256, 0, s>>>(n, x_zero ? b : r, x_zero ? zero->d_norm2 : sc, beta, Q, W.diag, z, W.gd, m + 1, ctl);
         int k = m;
         for (int j = 0; j <= m; ++j) {
             const double prev_tag = step_tag;
@@ -2150,6 +2051,7 @@ static int gmres_core(const GmresWork &W, hipStream_t s, long n, const Op &A, co
                 const double *qj = Q + (size_t)j * ldq;
                 double *slot = W.tag ? W.hstat + (size_t)kSlot * j : nullptr;
                 if (W.tag) step_tag = ++*W.tag;
+                if (W.skip) *W.skip = j < kGsCols ? ctl + 1 : nullptr;
                 if (W.diag) { if (A(z, w)) return -1; }
                 else if (M) { if (M(qj, z)) return -1; if (A(z, w)) return -1; }
                 else if (A(qj, w)) return -1;
@@ -2190,15 +2092,17 @@ static int gmres_core(const GmresWork &W, hipStream_t s, long n, const Op &A, co
                 if (est < thr || !(hn > 1e-16)) { k = j; break; }
             }
         }
+        if (W.skip) *W.skip = nullptr;
         const bool own = M && !W.diag;  // M is a call of its own
         gs_solution<<<std::min(nblk(n, 256), kFinishBlocks), 256, 0, s>>>(n, k, m, W.Hd, W.gd, Q, ldq, W.diag, !own,
                                                                          own ? w : x);
         if (own) {
-            if (M(w, z)) return -1;
-            vadd<<<nblk(n, 256), 256, 0, s>>>(n, z, x);
+            if (M(w, x_zero ? x : z)) return -1;
+            if (!x_zero) vadd<<<nblk(n, 256), 256, 0, s>>>(n, z, x);
         }
+        x_zero = false;
         if (A(x, r)) return -1;
-        if (residual(0)) return -1;
+        if (residual()) return -1;
         beta = std::sqrt(hn2[0]);
         error = beta / normb;
         if (error < p->tol) converged = 1;
@@ -2424,7 +2328,7 @@ namespace fvp {
 static int csr_gemv_impl(fvp_csr *A, double alpha, const double *x, double beta, double *y) {
     const int L = 8;
     csr_gemv_kernel<L><<<nblk((long)A->n * L, 256), 256, 0, A->stream>>>(A->n, A->ia.p, A->ja.p, A->a.p, alpha, x,
-                                                                         beta, y);
+                                                                         beta, y, A->skip);
     FVP_HIP(hipGetLastError());
     return 0;
 }
@@ -3037,8 +2941,11 @@ static int precon_build_impl(fvp_csr *A, int type) {
         set_error("invalid preconditioner type");
         return -1;
     }
-    if (!A->flag.p && A->flag.alloc(1)) return -1;
-    FVP_HIP(hipMemsetAsync(A->flag.p, 0, sizeof(int), s));
+    if (!A->flag.p) {  // cleared here and by every flag_post
+        if (A->flag.alloc(1)) return -1;
+        FVP_HIP(hipMemsetAsync(A->flag.p, 0, sizeof(int), s));
+    }
+    if (!A->hflag.p && A->hflag.alloc(1)) return -1;
     if (type == FVP_PRECON_SCHUR) {
         int rc = schur_factor(A);
         if (rc) { A->ptype = -1; return rc; }
@@ -3108,11 +3015,11 @@ static int precon_build_impl(fvp_csr *A, int type) {
                                                            A->diag.p, A->lu.p, A->flag.p);
         }
     }
+    const double tag = ++A->hflag.tag;
+    flag_post<<<1, 64, 0, s>>>(A->flag.p, A->hflag.p, tag);
     FVP_HIP(hipGetLastError());
-    int flag = 0;
-    FVP_HIP(hipMemcpyAsync(&flag, A->flag.p, sizeof(int), hipMemcpyDeviceToHost, s));
-    FVP_HIP(hipStreamSynchronize(s));
-    if (flag) { set_error("zero pivot in preconditioner factorisation"); A->ptype = -1; return FVP_ERR_PIVOT; }
+    if (slot_wait(s, A->hflag.p, tag)) return -1;
+    if (A->hflag.p[0] != 0.) { set_error("zero pivot in preconditioner factorisation"); A->ptype = -1; return FVP_ERR_PIVOT; }
     A->ptype = type;
     return 0;
 }
@@ -3122,7 +3029,7 @@ static void ilu0_one_launch_th(fvp_csr *A, const double *x, const double *xdiv, 
     const IluTri &L = A->otri[0], &U = A->otri[1];
     ilu0_solve<KW, TH><<<1, TH, A->o_lds, A->stream>>>(A->n, L.npieces, L.pptr.p, L.row.p, L.col.p, L.val.p,
                                                        U.npieces, U.pptr.p, U.row.p, U.col.p, U.val.p, x, xdiv, y,
-                                                       yn2);
+                                                       yn2, A->skip);
 }
 template <int KW>
 static void ilu0_one_launch(fvp_csr *A, const double *x, const double *xdiv, double *y, double *yn2) {
@@ -3169,7 +3076,7 @@ static int precon_apply_impl(fvp_csr *A, const double *x, double *y, const doubl
                                               ml, A->ebase_l.p, VL, A->col_l.p, A->s_lev_u.p, A->s_lptr_u.p, mu, \
                                               A->ebase_u.p, VU, A->col_u.p, DI, A->ov_ptr.p, A->ov_pos.p,         \
                                               A->ov_tri.p, A->b_maxrows, A->ov_max, A->s_levmax_l,       \
-                                              A->s_levmax_u, x, xdiv, y, yn2)
+                                              A->s_levmax_u, x, xdiv, y, yn2, A->skip)
         if (f64) {
             if (ovg) FVP_BJ_SOLVE(double, true, A->val_l.p, A->val_u.p, A->dinv.p);
             else FVP_BJ_SOLVE(double, false, A->val_l.p, A->val_u.p, A->dinv.p);
@@ -3254,7 +3161,8 @@ extern "C" int fvp_csr_destroy(fvp_csr *A) {
     A->lrows.release(); A->urows.release(); A->flag.release(); A->Q.release(); A->w.release(); A->r.release();
     A->z.release(); A->part.release(); A->scal.release(); A->hdev.release();
     A->Hd.release(); A->gd.release(); A->csd.release(); A->snd.release(); A->yd.release(); A->Qk.release();
-    if (A->hstat) (void)hipHostFree(A->hstat);
+    A->hstat.release();
+    A->hflag.release();
     A->b_ia.release(); A->b_src.release(); A->b_lu.release(); A->b_lu32.release();
     A->b_roff.release(); A->b_rowid.release(); A->b_own.release(); A->b_zn2.release();
     A->meta_l.release(); A->meta_u.release(); A->ebase_l.release(); A->ebase_u.release();
@@ -3386,7 +3294,7 @@ extern "C" int fvp_gmres_csr(fvp_csr *A, const double *b, double *x, const fvp_g
     Op op = [A](const double *in, double *out) { return csr_gemv_impl(A, 1.0, in, 0.0, out); };
     Op pc;
     if (A->ptype != FVP_PRECON_NONE) pc = [A](const double *in, double *out) { return precon_apply_impl(A, in, out); };
-    return gmres_device(A, A->stream, A->n, op, pc, b, x, p, st, false, diagonal_of(A));
+    return gmres_device(A, A->stream, A->n, op, pc, b, x, p, st, nullptr, diagonal_of(A));
 }
 
 extern "C" int fvp_gmres_csr_deflated(fvp_csr *A, const double *b, double *x, const fvp_gmres_params *p, int k,
@@ -3788,8 +3696,10 @@ extern "C" int fvp_newton_gmres(fvp_ctx *c, double t, const double *psi, const d
     if (jac_init(c)) return -1;
     fvp_csr *W = c->jd->J;
     fvp_csr_set_stream(W, c->stream);
-    Op op = [=](const double *in, double *out) { return fvp_jv(c, t, psi, psip, F0, c_j, in, out); };
+    Op op = [=](const double *in, double *out) {
+        return jv_impl(c, t, psi, psip, F0, c_j, in, out, nullptr, nullptr, nullptr, 0, W->skip);
+    };
     Op pc;
     if (W->ptype > 0) pc = [W](const double *in, double *out) { return precon_apply_impl(W, in, out); };
-    return gmres_device(W, c->stream, c->N, op, pc, b, x, p, st, false, diagonal_of(W));
+    return gmres_device(W, c->stream, c->N, op, pc, b, x, p, st, nullptr, diagonal_of(W));
 }

@@ -26,6 +26,7 @@
 
 #include "fvp_blas.h"
 #include "fvp_internal.h"
+#include "fvp_sums.h"
 
 namespace fvp {
 
@@ -604,6 +605,7 @@ __global__ void __launch_bounds__(TH) owner_lds(
     const int w0 = wptr[tile], win = nown + wptr[tile + 1] - w0;
     const int stride = win_stride(DIM, nr);
     unsigned short *const list = reinterpret_cast<unsigned short *>(sm + wmax * stride);
+    const double over = JV ? skip_word(jv.skip) : 0.;
     const double c0 = rho0 / (DIM == 3 ? 24.0 : 6.0);
     for (int k = threadIdx.x; k < 3 * zt.nz; k += TH) zk[k] = zt.p[k / 3][ZK_X + k % 3] * c0;
     if (VG)
@@ -651,6 +653,7 @@ __global__ void __launch_bounds__(TH) owner_lds(
         }
     }
     __syncthreads();
+    if (JV && over != 0.) return;
     if (VG) {
         for (int k = threadIdx.x; k < nlist; k += TH) {
             const int i = list[k], g = node_of(i);
@@ -724,10 +727,12 @@ __global__ void __launch_bounds__(256) owner_imports(int nimp, const int *__rest
                                                      const double *__restrict__ xf, const double *__restrict__ invV,
                                                      const double *__restrict__ psip, const double *__restrict__ cap,
                                                      double *__restrict__ F, JvArgs jv) {
+    const double over = JV ? skip_word(jv.skip) : 0.;
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= nimp) return;
     const int i = inode[k];
     const int s0 = iptr[i], s1 = iptr[i + 1];
+    if (over != 0.) return;
     double a = acc[i];
     const double iv = invV[i], p = psip[i], c = cap[i];
     const double sig = JV ? jv.sig[0] : 0., v = JV ? jv.v[i] : 0., f0 = JV ? jv.F0[i] : 0.;
