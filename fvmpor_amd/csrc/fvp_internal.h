@@ -157,10 +157,22 @@ struct JvArgs {
 int jv_impl(fvp_ctx *c, double t, const double *psi, const double *psip, const double *F0, double c_j,
             const double *v, double *Jv, const double *psi_n2, const double *osc, const double *v_n2 = nullptr,
             int v_count = 0, const double *skip = nullptr);
-// element-local FD Jacobian into J (nnz values); the arrays as in fvp_jacdata
-int fd_jacobian_elem(fvp_ctx *c, double cj, const double *psi, const double *psip, const double *shift, double *ys,
-                     double *kr2, double *cap2, double *contrib, const long *cptr, const int *srank, const int *ia,
-                     const int *dpos, double *J, long nnz, bool fp32 = false);
+// The element-local FD Jacobian's inputs, work arrays and tables (device pointers).
+// A visit is a row in one of its elements: vec4 place npe e + i in contrib.
+struct FdJacobian {
+    double eps, h, cj;
+    const double *psi, *psip, *ewt;
+    double *shift, *dterm, *rec;  // per node; rec: 16 bytes per zone and node
+    double *contrib;              // 4 values per visit
+    int rows, max_visits;         // rows per workgroup of fd_gather, most visits of one
+    const int *vptr, *visit;      // per workgroup its visits
+    const unsigned *cptr;         // per entry its first code; bit 31: a diagonal
+    const uint16_t *code;         // 4 x visit within the workgroup + k; null: code32
+    const int *code32;            // place in contrib
+    const int *ia, *dpos;
+    double *J;
+};
+int fd_jacobian_elem(fvp_ctx *c, const FdJacobian &fd, bool fp32);
 // z = M^-1 (r / rdiv) with the context's preconditioner (tmp: a work vector of
 // N).  With zn2 given, the block-Jacobi solves also leave partial sums of
 // ||z||^2: *zn2 points at them and *zn2_count is their number (null and 0 for

@@ -3384,14 +3384,12 @@ struct fvp_jacdata {
     std::vector<int> eptr;             // colour -> entries
     DevBuf<int> cols, erow, epos, ecol;
     DevBuf<double> shift, ys, yps, Fs;
-    // element-local quotients: the contribution of (element e, row node i,
-    // moved node k) goes to srank[16 e + 4 i + k], so that each entry's
-    // contributions lie contiguous in [cptr2[p], cptr2[p + 1]) in element
-    // order; per row its diagonal entry; k_r and capacity with every node
-    // moved by its shift
-    DevBuf<long> cptr2;
-    DevBuf<int> srank, dpos;
-    DevBuf<double> contrib, kr2, cap2;
+    // element-local quotients, see FdJacobian; per row its diagonal entry
+    DevBuf<int> vptr, visit, code32, dpos;
+    DevBuf<unsigned> cptr2;
+    DevBuf<uint16_t> code;
+    int rows = 0, max_visits = 0;
+    DevBuf<double> contrib, rec, dterm;
 };
 
 namespace fvp {
@@ -3421,6 +3419,85 @@ __global__ void fd_scatter(int cnt, const int *__restrict__ erow, const int *__r
     if (k >= cnt) return;
     int r = erow[k];
     J[epos[k]] = (F0[r] - Fs[r]) / shift[ecol[k]];
+}
+
+// Tables of fd_gather: each entry's quotients in element order, as places in
+// the visits of its workgroup of rows.  A workgroup takes 64 rows (a box: about
+// 1500 visits, 24 KB in FP32), fewer where their visits need more than kFdLds in
+// FP64; where even 8 do, the codes are places in contrib and nothing is staged.
+constexpr size_t kFdLds = 64 * 1024;
+static int fd_tables(fvp_ctx *c, fvp_jacdata *jd, const std::vector<int4> &conn, const std::vector<int> &ia,
+                     const std::vector<int> &ja) {
+    const int N = c->N, T = c->T, npe = c->npe;
+    const long nnz = ia[N];
+    if ((long)16 * T > INT32_MAX) { set_error("too many elements for the FD Jacobian slots"); return -1; }
+    auto at = [&](int row, int col) {
+        return (int)(std::lower_bound(ja.begin() + ia[row], ja.begin() + ia[row + 1], col) - ja.begin());
+    };
+    // visits by row, element order within; each entry's number of quotients
+    std::vector<int> rv(N + 1, 0), visit((size_t)npe * T), local((size_t)npe * T), pos((size_t)npe * npe * T), dpos(N);
+    std::vector<unsigned> cp(nnz + 1, 0);
+    for (int e = 0; e < T; ++e) {
+        const int n[4] = {conn[e].x, conn[e].y, conn[e].z, conn[e].w};
+        for (int i = 0; i < npe; ++i) {
+            ++rv[n[i] + 1];
+            for (int k = 0; k < npe; ++k) {
+                const int p = at(n[i], n[k]);
+                pos[((size_t)e * npe + i) * npe + k] = p;
+                ++cp[p + 1];
+            }
+        }
+    }
+    for (int i = 0; i < N; ++i) { rv[i + 1] += rv[i]; dpos[i] = at(i, i); }
+    for (long p = 0; p < nnz; ++p) cp[p + 1] += cp[p];
+    {
+        std::vector<int> fill(rv.begin(), rv.end() - 1);
+        for (int e = 0; e < T; ++e) {
+            const int n[4] = {conn[e].x, conn[e].y, conn[e].z, conn[e].w};
+            for (int i = 0; i < npe; ++i) {
+                const int v = fill[n[i]]++;
+                visit[v] = e * npe + i;
+                local[(size_t)e * npe + i] = v;
+            }
+        }
+    }
+    const int limit = (int)(kFdLds / (4 * sizeof(double)));
+    auto most = [&](int rows) {
+        int m = 0;
+        for (int r = 0; r < N; r += rows) m = std::max(m, rv[std::min(N, r + rows)] - rv[r]);
+        return m;
+    };
+    int rows = 64;
+    while (rows > 8 && most(rows) > limit) rows /= 2;
+    jd->max_visits = most(rows);
+    const bool staged = jd->max_visits <= limit;
+    if (!staged) rows = 64;
+    jd->rows = rows;
+    std::vector<uint16_t> code;
+    std::vector<int> code32, vptr;
+    (staged ? code.resize(cp[nnz]) : code32.resize(cp[nnz]));
+    {
+        std::vector<unsigned> fill(cp.begin(), cp.end() - 1);
+        for (int e = 0; e < T; ++e) {
+            const int n[4] = {conn[e].x, conn[e].y, conn[e].z, conn[e].w};
+            for (int i = 0; i < npe; ++i)
+                for (int k = 0; k < npe; ++k) {
+                    const size_t v = (size_t)e * npe + i;
+                    const unsigned to = fill[pos[v * npe + k]]++;
+                    if (staged) code[to] = (uint16_t)(4 * (local[v] - rv[n[i] / rows * rows]) + k);
+                    else code32[to] = (int)(4 * v + k);
+                }
+        }
+    }
+    for (int r = 0; r < N; r += rows) vptr.push_back(rv[r]);
+    vptr.push_back(rv[N]);
+    for (int i = 0; i < N; ++i) cp[dpos[i]] |= 1u << 31;
+    if (staged ? jd->code.upload(code.data(), code.size()) || jd->visit.upload(visit.data(), visit.size()) ||
+                     jd->vptr.upload(vptr.data(), vptr.size())
+               : jd->code32.upload(code32.data(), code32.size()))
+        return -1;
+    return jd->cptr2.upload(cp.data(), cp.size()) || jd->dpos.upload(dpos.data(), N) ||
+           jd->contrib.alloc((size_t)4 * npe * T) || jd->rec.alloc(2 * (size_t)c->nz * N) || jd->dterm.alloc(N);
 }
 
 // Node adjacency over element pairs (preconditioner_dss.cpp:107-142) and the
@@ -3460,35 +3537,7 @@ static int jac_init(fvp_ctx *c) {
     if (csr_create_impl(c->device, N, ia.data(), ja.data(), &jd->J)) { delete jd; return -1; }
     fvp_csr_set_stream(jd->J, c->stream);
     {
-        // each entry's contribution slots, counting-sorted by entry (element order within)
-        const long nnz = ia[N];
-        std::vector<int> pos((size_t)npe * npe * T), dpos(N), srank(16 * (size_t)T, 0);
-        std::vector<long> cp(nnz + 1, 0);
-        auto at = [&](int row, int col) {
-            return (int)(std::lower_bound(ja.begin() + ia[row], ja.begin() + ia[row + 1], col) - ja.begin());
-        };
-        for (int e = 0; e < T; ++e) {
-            const int n[4] = {conn[e].x, conn[e].y, conn[e].z, conn[e].w};
-            for (int i = 0; i < npe; ++i)
-                for (int k = 0; k < npe; ++k) {
-                    const int p = at(n[i], n[k]);
-                    pos[((size_t)e * npe + i) * npe + k] = p;
-                    ++cp[p + 1];
-                }
-        }
-        for (long p = 0; p < nnz; ++p) cp[p + 1] += cp[p];
-        {
-            std::vector<long> fill(cp.begin(), cp.end() - 1);
-            for (int e = 0; e < T; ++e)
-                for (int i = 0; i < npe; ++i)
-                    for (int k = 0; k < npe; ++k)
-                        srank[16 * (size_t)e + 4 * i + k] = (int)fill[pos[((size_t)e * npe + i) * npe + k]]++;
-        }
-        for (int i = 0; i < N; ++i) dpos[i] = at(i, i);
-        if ((long)16 * T > INT32_MAX) { set_error("too many elements for the FD Jacobian slots"); fvp_csr_destroy(jd->J); delete jd; return -1; }
-        if (jd->cptr2.upload(cp.data(), cp.size()) || jd->srank.upload(srank.data(), srank.size()) ||
-            jd->dpos.upload(dpos.data(), N) || jd->contrib.alloc((size_t)npe * npe * T) ||
-            jd->kr2.alloc((size_t)c->nz * N) || jd->cap2.alloc(N)) {
+        if (fd_tables(c, jd, conn, ia, ja)) {
             fvp_csr_destroy(jd->J);
             delete jd;
             return -1;
@@ -3571,8 +3620,8 @@ void jac_free(fvp_ctx *c) {
     fvp_csr_destroy(jd->J);
     jd->cols.release(); jd->erow.release(); jd->epos.release(); jd->ecol.release();
     jd->shift.release(); jd->ys.release(); jd->yps.release(); jd->Fs.release();
-    jd->cptr2.release(); jd->srank.release(); jd->dpos.release(); jd->contrib.release();
-    jd->kr2.release(); jd->cap2.release();
+    jd->cptr2.release(); jd->vptr.release(); jd->visit.release(); jd->code.release(); jd->code32.release();
+    jd->dpos.release(); jd->contrib.release(); jd->rec.release(); jd->dterm.release();
     delete jd;
     c->jd = nullptr;
 }
@@ -3589,14 +3638,14 @@ extern "C" int fvp_precon_setup(fvp_ctx *c, double t, double c_j, double h, cons
     fvp_csr_set_stream(jd->J, s);
     const int N = c->N;
     const double eps = 1.4901161193847656e-08;  // sqrt(2^-52)
-    shift_kernel<<<nblk(N, 256), 256, 0, s>>>(N, eps, h, psi, psip, ewt, jd->shift.p);
     if (!c->averaging && c->jac_mode == FVP_JACOBIAN_ELEMENT) {
-        if (fd_jacobian_elem(c, c_j, psi, psip, jd->shift.p, jd->ys.p, jd->kr2.p, jd->cap2.p, jd->contrib.p,
-                             jd->cptr2.p, jd->srank.p, jd->J->ia.p, jd->dpos.p, jd->J->a.p, jd->J->nnz,
-                             type == FVP_PRECON_BJILU0_F32))
-            return -1;
+        const FdJacobian fd{eps, h, c_j, psi, psip, ewt, jd->shift.p, jd->dterm.p, jd->rec.p, jd->contrib.p,
+                            jd->rows, jd->max_visits, jd->vptr.p, jd->visit.p, jd->cptr2.p, jd->code.p, jd->code32.p,
+                            jd->J->ia.p, jd->dpos.p, jd->J->a.p};
+        if (fd_jacobian_elem(c, fd, type == FVP_PRECON_BJILU0_F32)) return -1;
         return precon_build_impl(jd->J, type);
     }
+    shift_kernel<<<nblk(N, 256), 256, 0, s>>>(N, eps, h, psi, psip, ewt, jd->shift.p);
     if (colour_init(c)) return -1;
     vcopy<<<nblk(N, 256), 256, 0, s>>>(N, psi, jd->ys.p);
     vcopy<<<nblk(N, 256), 256, 0, s>>>(N, psip, jd->yps.p);

@@ -1143,26 +1143,91 @@ static void launch_tile(fvp_ctx *c, const double *psi, const double *psip, doubl
     if (eb) (void)hipEventRecord(eb, s);
 }
 
+// The node side of the element-local Jacobian, one pass: the increment of each node
+// (IDA's), k_r and capacity at the base state and with the node moved by its
+// increment, and what the elements gather of them: per zone and node one 16-byte
+// record, {V^-1, k_r, k_r moved, dk_r / shift} in FP32 or the two k_r in FP64; the
+// diagonal's capacity term -psi' a_hh(psi) moved with psi_i and psi'_i + c_j shift_i.
+// Nodes of several zones are set aside as in vg_kernel.  Bound by FP64 instructions
+// (two evaluations per node and zone).  141 000 nodes: 25 us, where five launches
+// (increments, base, sum, moved, capacity term) took 42, and the elements' four
+// 8-byte gathers per node become one of 16.
+template <typename C>
+__global__ void __launch_bounds__(256) fd_nodes(int N, ZoneTable zt, double rho0, FdJacobian fd,
+                                                const uint8_t *__restrict__ zmask, const double *__restrict__ zw,
+                                                const double *__restrict__ invV, double *__restrict__ kr,
+                                                double *__restrict__ cap, double *__restrict__ nrec) {
+    __shared__ double zp[kMaxZones * 10];
+    __shared__ int nlist;
+    __shared__ unsigned char list[256];
+    if (threadIdx.x == 0) nlist = 0;
+    if (threadIdx.x < 10 * zt.nz) zp[threadIdx.x] = zt.p[threadIdx.x / 10][threadIdx.x % 10];
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    __syncthreads();
+    auto evaluate = [&](int g, unsigned m, bool multi) {
+        const double y = fd.psi[g], yp = fd.psip[g];
+        const double sh = fd.eps * fmax(fabs(y), fmax(fabs(fd.h * yp), 1.0 / fd.ewt[g]));
+        const float w = (float)invV[g];
+        double one = 0.;
+        const double c0 = vg_node<true>(N, g, y, m, zp, zw, rho0, [&](int z, int, double k) {
+            one = k;
+            if (multi) kr[(size_t)z * N + g] = k;
+        });
+        const double c1 = vg_node<true>(N, g, y + sh, m, zp, zw, rho0, [&](int z, int, double k1) {
+            const double k0 = multi ? kr[(size_t)z * N + g] : one;
+            if constexpr (sizeof(C) == 4)
+                reinterpret_cast<float4 *>(fd.rec)[(size_t)z * N + g] = make_float4(w, (float)k0, (float)k1, (float)((k1 - k0) / sh));
+            else
+                reinterpret_cast<double2 *>(fd.rec)[(size_t)z * N + g] = make_double2(k0, k1);
+        });
+        cap[g] = c0;
+        fd.dterm[g] = ((yp + fd.cj * sh) * c1 - yp * c0) / sh;
+        fd.shift[g] = sh;
+        nrec[4 * (size_t)g + 3] = y;
+    };
+    if (i < N) {
+        const unsigned m = zmask[i];
+        if (m & (m - 1)) list[atomicAdd(&nlist, 1)] = (unsigned char)threadIdx.x;
+        else evaluate(i, m, false);
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < nlist) {
+        const int g = blockIdx.x * 256 + list[threadIdx.x];
+        evaluate(g, zmask[g], true);
+    }
+}
+
+// node values of an element from the packed records (x, y, z, head: two 16-byte loads)
+template <int DIM>
+__device__ __forceinline__ void load_geometry(const ElemRec &rec, const double *__restrict__ nrec,
+                                              NodeVals<DIM> &nv) {
+    const int n[4] = {rec.c4.x, rec.c4.y, rec.c4.z, rec.c4.w};
+#pragma unroll
+    for (int k = 0; k < DIM + 1; ++k) {
+        const double2 *r = reinterpret_cast<const double2 *>(nrec + 4 * (size_t)n[k]);
+        const double2 a = r[0], b = r[1];
+        nv.px[k] = a.x; nv.py[k] = a.y; nv.pz[k] = b.x; nv.h[k] = b.y;
+    }
+}
+
 // Element-local finite-difference Jacobian, -(dF/dpsi + c_j dF/dpsi') with
 // the coloured method's increments (shift) and upwind bits: every element is
 // evaluated at the base state and once per node with that node's head moved
 // by its shift (k_r from the second van Genuchten pass, kr2), and
 // (f_base - f_moved) V^-1 / shift for (row node i, moved node k) is stored at
-// contrib[srank[16 e + 4 i + k]], where the entries' contributions lie
-// contiguous and in element order; fd_gather_t sums each entry's range (no
-// atomics, so the Jacobian is repeatable bit for bit).  The
-// capacity term and the Dirichlet rows are set by fd_node_kernel and
-// fd_dirichlet.  The residual is a sum of element terms, so these are the
+// contrib[4 (npe e + i) + k], an element's quotients in one piece; fd_gather
+// sums each entry's (in a fixed order without atomics, so the Jacobian is
+// repeatable bit for bit) and adds fd_nodes' capacity term to the diagonal.  The
+// Dirichlet rows are set by fd_dirichlet.  The residual is a sum of element terms, so these are the
 // coloured quotients up to the rounding of the sums.
 template <int DIM>
 __global__ void __launch_bounds__(256) fd_elem_kernel(int T, int N, ZoneTable zt, double rho0,
                                                       const int4 *__restrict__ conn, const uint8_t *__restrict__ ezone,
                                                       const double *__restrict__ kmul, const uint8_t *__restrict__ emask,
-                                                      const double *__restrict__ nrec, const double *__restrict__ kr,
-                                                      const double *__restrict__ kr2, const double *__restrict__ shift,
+                                                      const double *__restrict__ nrec, const double2 *__restrict__ kk,
+                                                      const double *__restrict__ shift,
                                                       const double *__restrict__ invV,
-                                                      const int *__restrict__ srank,
-                                                      double *__restrict__ contrib) {
+                                                      double2 *__restrict__ contrib) {
     __shared__ double zk[3 * kMaxZones];
     if (threadIdx.x < 3 * zt.nz) zk[threadIdx.x] = zt.p[threadIdx.x / 3][ZK_X + threadIdx.x % 3];
     __syncthreads();
@@ -1170,26 +1235,38 @@ __global__ void __launch_bounds__(256) fd_elem_kernel(int T, int N, ZoneTable zt
     if (e >= T) return;
     const ElemRec rec = load_elem<0>(e, conn, ezone, kmul, emask, nullptr);
     NodeVals<DIM> nv;
-    load_nodes_rec<DIM>(rec, N, nrec, kr, nv);
-    int n[4];
+    load_geometry<DIM>(rec, nrec, nv);
+    int n[4] = {rec.c4.x, rec.c4.y, rec.c4.z, rec.c4.w};
+    double w[DIM + 1], sh[DIM + 1], km[DIM + 1], d[DIM + 1][4];
+#pragma unroll
+    for (int i = 0; i < DIM + 1; ++i) {
+        const double2 k2 = kk[(size_t)rec.z * N + n[i]];
+        nv.k[i] = k2.x;
+        km[i] = k2.y;
+        w[i] = invV[n[i]];
+        sh[i] = shift[n[i]];
+        d[i][3] = 0.;
+    }
     double f0[4];
     element_fluxes_vals<DIM, 0>(e, rec, nv, zk, rho0, nullptr, n, f0);
-    const double *k2 = kr2 + (size_t)rec.z * N;
-    double w[DIM + 1];
-#pragma unroll
-    for (int i = 0; i < DIM + 1; ++i) w[i] = invV[n[i]];
 #pragma unroll
     for (int k = 0; k < DIM + 1; ++k) {
-        const double sk = shift[n[k]], hk = nv.h[k], kk = nv.k[k];
+        const double sk = sh[k], hk = nv.h[k], k0 = nv.k[k];
         nv.h[k] = hk + sk;
-        nv.k[k] = k2[n[k]];
+        nv.k[k] = km[k];
         int n1[4];
         double f1[4];
         element_fluxes_vals<DIM, 0>(e, rec, nv, zk, rho0, nullptr, n1, f1);
         nv.h[k] = hk;
-        nv.k[k] = kk;
+        nv.k[k] = k0;
 #pragma unroll
-        for (int i = 0; i < DIM + 1; ++i) contrib[srank[16 * (size_t)e + 4 * i + k]] = (f0[i] - f1[i]) * w[i] / sk;
+        for (int i = 0; i < DIM + 1; ++i) d[i][k] = (f0[i] - f1[i]) * w[i] / sk;
+    }
+    double2 *const out = contrib + 2 * (DIM + 1) * (size_t)e;
+#pragma unroll
+    for (int i = 0; i < DIM + 1; ++i) {
+        out[2 * i] = make_double2(d[i][0], d[i][1]);
+        out[2 * i + 1] = make_double2(d[i][2], d[i][3]);
     }
 }
 
@@ -1203,17 +1280,17 @@ __global__ void __launch_bounds__(256) fd_elem_kernel(int T, int N, ZoneTable zt
 // in FP64 from the two van Genuchten passes), so nothing cancels and FP32
 // carries the quotient to its rounding; the geometry is built once per
 // element, relative to its first node.  Same increments, same upwind bits,
-// same contribution slots as fd_elem_kernel.
+// same places as fd_elem_kernel.  787 000 elements: 27 us; scattering the 16
+// quotients to their entries, one 4-byte store each, took 67 (bound by the L2's
+// requests).
 template <int DIM>
 __global__ void __launch_bounds__(256) fd_elem_kernel32(int T, int N, ZoneTable zt, double rho0,
                                                         const int4 *__restrict__ conn,
                                                         const uint8_t *__restrict__ ezone,
                                                         const double *__restrict__ kmul,
                                                         const uint8_t *__restrict__ emask,
-                                                        const double *__restrict__ nrec, const double *__restrict__ kr,
-                                                        const double *__restrict__ kr2, const double *__restrict__ shift,
-                                                        const double *__restrict__ invV, const int *__restrict__ srank,
-                                                        float *__restrict__ contrib) {
+                                                        const double *__restrict__ nrec, const float4 *__restrict__ kk,
+                                                        float4 *__restrict__ contrib) {
     constexpr int NPE = DIM + 1;
     constexpr int NED = DIM == 2 ? 3 : 6;
     __shared__ float zk[3 * kMaxZones];
@@ -1223,8 +1300,14 @@ __global__ void __launch_bounds__(256) fd_elem_kernel32(int T, int N, ZoneTable 
     if (e >= T) return;
     const ElemRec rec = load_elem<0>(e, conn, ezone, kmul, emask, nullptr);
     NodeVals<DIM> nv;
-    load_nodes_rec<DIM>(rec, N, nrec, kr, nv);
+    load_geometry<DIM>(rec, nrec, nv);
     const int n[4] = {rec.c4.x, rec.c4.y, rec.c4.z, rec.c4.w};
+    float w[NPE], kb[NPE], km1[NPE], dkr[NPE];
+#pragma unroll
+    for (int i = 0; i < NPE; ++i) {
+        const float4 q = kk[(size_t)rec.z * N + n[i]];
+        w[i] = q.x; kb[i] = q.y; km1[i] = q.z; dkr[i] = q.w;
+    }
     float G[NPE][3], det;
     if (DIM == 3) {
         const float ux = (float)(nv.px[1] - nv.px[0]), uy = (float)(nv.py[1] - nv.py[0]), uz = (float)(nv.pz[1] - nv.pz[0]);
@@ -1262,24 +1345,17 @@ __global__ void __launch_bounds__(256) fd_elem_kernel32(int T, int N, ZoneTable 
     for (int k = 0; k < NPE; ++k) g[k] = G[k][0] * qx + G[k][1] * qy + G[k][2] * qz;
     const float sc = (det > 0.f ? 1.f : -1.f) / (DIM == 3 ? 24.f : 6.f);
     const float r0 = (float)rho0;
-    const double *k2 = kr2 + (size_t)rec.z * N;
-    float w[NPE], kb[NPE], dkr[NPE];
+    float out[NPE][4];
 #pragma unroll
-    for (int i = 0; i < NPE; ++i) {
-        w[i] = (float)invV[n[i]];
-        kb[i] = (float)nv.k[i];
-    }
+    for (int i = 0; i < NPE; ++i) out[i][3] = 0.f;
 #pragma unroll
     for (int k = 0; k < NPE; ++k) {
-        const double sk = shift[n[k]], k1 = k2[n[k]];
-        dkr[k] = (float)((k1 - nv.k[k]) / sk);
         // d(grad h)/dh_k = G[k] / det, so dq/dh_k = K (G[k] / det) (no gravity term)
         const float dqx = G[k][0] * inv * Kx, dqy = G[k][1] * inv * Ky, dqz = G[k][2] * inv * Kz;
         float dg[NPE];
 #pragma unroll
         for (int m = 0; m < NPE; ++m) dg[m] = G[m][0] * dqx + G[m][1] * dqy + G[m][2] * dqz;
         float d[4] = {0.f, 0.f, 0.f, 0.f};
-        const float kmv = (float)k1;
 #pragma unroll
         for (int j = 0; j < NED; ++j) {
             const int a = edge_a(j), b = edge_b(j);
@@ -1287,45 +1363,103 @@ __global__ void __launch_bounds__(256) fd_elem_kernel32(int T, int N, ZoneTable 
             const int u = up_a ? a : b;
             const float flux = sc * (g[b] - g[a]);
             const float dflux = sc * (dg[b] - dg[a]);
-            const float kr1 = u == k ? kmv : (up_a ? kb[a] : kb[b]);
+            const float kr1 = u == k ? km1[k] : (up_a ? kb[a] : kb[b]);
             const float dM = r0 * ((u == k ? dkr[k] : 0.f) * flux + kr1 * dflux);
             d[a] += dM;  // (f0 - f1) / s_k at a: f[a] -= M
             d[b] -= dM;
         }
 #pragma unroll
-        for (int i = 0; i < NPE; ++i) contrib[srank[16 * (size_t)e + 4 * i + k]] = d[i] * w[i];
+        for (int i = 0; i < NPE; ++i) out[i][k] = d[i] * w[i];
     }
+#pragma unroll
+    for (int i = 0; i < NPE; ++i)
+        contrib[NPE * (size_t)e + i] = make_float4(out[i][0], out[i][1], out[i][2], out[i][3]);
 }
 
-// J[p] = sum of entry p's contributions contrib[cptr[p] .. cptr[p + 1]) in
-// element order, accumulated in FP64 (FP32 or FP64 contributions); the loads
-// go out kEdgeBatch at a time so that they are in flight together.
-template <typename C>
-__global__ void fd_gather_t(long nnz, const long *__restrict__ cptr, const C *__restrict__ contrib,
-                            double *__restrict__ J) {
-    const long p = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    if (p >= nnz) return;
-    const long q0 = cptr[p], q1 = cptr[p + 1];
-    double s = 0.;
-    for (long qb = q0; qb < q1; qb += kEdgeBatch) {
-        C c[kEdgeBatch];
+// The entries of a block of rows: per entry the sum of its quotients, accumulated in
+// FP64 in a fixed order, the capacity term added on the diagonal.  A row's quotients
+// lie four to an element (its visit); the block's visits are staged in the LDS with
+// 16- or 32-byte loads, which both the requests and the lines are few for, and the
+// entries pick their 2-byte codes (visit, place) there.  Diagonals have a quotient of
+// every visit, so kDiagLanes lanes share one.  Without STAGED (more visits than the
+// LDS holds) the codes are places in contrib.  787 000 elements, 2 million entries,
+// FP32: 37 us (46 with 256 threads and no loads ahead of the barrier); bound by the
+// latency of its chain of loads (entry, code; visit, quotients) and then the bytes.
+constexpr int kFdThreads = 512;
+constexpr int kDiagLanes = 8;  // x 64 rows
+template <typename C, bool STAGED>
+__global__ void __launch_bounds__(kFdThreads) fd_gather(int N, FdJacobian fd) {
+    using V = std::conditional_t<sizeof(C) == 4, float4, double4>;
+    extern __shared__ __align__(16) char fd_lds[];
+    constexpr unsigned kDiag = 1u << 31;
+    const V *const contrib = reinterpret_cast<const V *>(fd.contrib);
+    const C *const q = STAGED ? reinterpret_cast<const C *>(fd_lds) : reinterpret_cast<const C *>(fd.contrib);
+    const int r0 = blockIdx.x * fd.rows, r1 = min(N, r0 + fd.rows), p1 = fd.ia[r1];
+    // an entry's codes [k0, k1), every step-th from k0 + l; the first kEdgeBatch of them
+    struct Codes {
+        unsigned k0, k1;
+        int at[kEdgeBatch];
+    };
+    auto place = [&](unsigned k) { return STAGED ? (int)fd.code[k] : fd.code32[k]; };
+    auto fetch = [&](int p, unsigned l, unsigned step, Codes &e) {
+        e.k0 = fd.cptr[p];
+        e.k1 = fd.cptr[p + 1] & ~kDiag;
+        const unsigned k = (e.k0 & ~kDiag) + l;
 #pragma unroll
-        for (int u = 0; u < kEdgeBatch; ++u) c[u] = qb + u < q1 ? contrib[qb + u] : C(0);
+        for (int u = 0; u < kEdgeBatch; ++u) e.at[u] = place(min(k + u * step, e.k1 - 1));
+    };
+    auto sum = [&](const Codes &e, unsigned l, unsigned step) {
+        double s = 0.;
+        unsigned k = (e.k0 & ~kDiag) + l;
+        int at[kEdgeBatch];
 #pragma unroll
-        for (int u = 0; u < kEdgeBatch; ++u)
-            if (qb + u < q1) s += (double)c[u];
+        for (int u = 0; u < kEdgeBatch; ++u) at[u] = e.at[u];
+        while (k < e.k1) {
+            C c[kEdgeBatch];
+#pragma unroll
+            for (int u = 0; u < kEdgeBatch; ++u) c[u] = q[at[u]];
+#pragma unroll
+            for (int u = 0; u < kEdgeBatch; ++u)
+                if (k + u * step < e.k1) s += (double)c[u];
+            k += kEdgeBatch * step;
+            if (k >= e.k1) break;
+#pragma unroll
+            for (int u = 0; u < kEdgeBatch; ++u) at[u] = place(min(k + u * step, e.k1 - 1));
+        }
+        return s;
+    };
+    int p = fd.ia[r0] + threadIdx.x;
+    const int r = r0 + threadIdx.x / kDiagLanes, pd = fd.dpos[min(r, r1 - 1)], l = threadIdx.x % kDiagLanes;
+    Codes e{}, d;
+    if (p < p1) fetch(p, 0, 1, e);
+    fetch(pd, l, kDiagLanes, d);
+    if (STAGED) {
+        const int v0 = fd.vptr[blockIdx.x], nv = fd.vptr[blockIdx.x + 1] - v0;
+        constexpr int kU = 4;
+        for (int k0 = threadIdx.x; k0 < nv; k0 += kFdThreads * kU) {
+            int at[kU];
+            V c[kU];
+#pragma unroll
+            for (int u = 0; u < kU; ++u) at[u] = fd.visit[v0 + min(k0 + kFdThreads * u, nv - 1)];
+#pragma unroll
+            for (int u = 0; u < kU; ++u) c[u] = contrib[at[u]];
+#pragma unroll
+            for (int u = 0; u < kU; ++u)
+                if (k0 + kFdThreads * u < nv) reinterpret_cast<V *>(fd_lds)[k0 + kFdThreads * u] = c[u];
+        }
+        __syncthreads();
     }
-    J[p] = s;
-}
-
-// diagonal: the capacity term -psi' a_hh(psi) moved with psi_i and psi'_i + c_j shift_i
-__global__ void fd_node_kernel(int N, double cj, const double *__restrict__ psip, const double *__restrict__ shift,
-                               const double *__restrict__ cap, const double *__restrict__ cap2,
-                               const int *__restrict__ dpos, double *__restrict__ J) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    const double sh = shift[i];
-    J[dpos[i]] += ((psip[i] + cj * sh) * cap2[i] - psip[i] * cap[i]) / sh;
+    double s = sum(d, l, kDiagLanes);
+#pragma unroll
+    for (int m = 1; m < kDiagLanes; m *= 2) s += __shfl_xor(s, m, 64);
+    if (l == 0 && r < r1) fd.J[pd] = s + fd.dterm[r];
+    while (p < p1) {
+        Codes n{};
+        if (p + kFdThreads < p1) fetch(p + kFdThreads, 0, 1, n);
+        if (!(e.k0 & kDiag)) fd.J[p] = sum(e, 0, 1);
+        e = n;
+        p += kFdThreads;
+    }
 }
 
 // Dirichlet rows F = psi_D - psi: zero off the diagonal, the quotient on it
@@ -1339,52 +1473,35 @@ __global__ void fd_dirichlet(int nd, const int *__restrict__ dnode, const double
     J[dpos[i]] = ((dval[k] - psi[i]) - (dval[k] - (psi[i] + shift[i]))) / shift[i];
 }
 
-__global__ void fd_add(long n, const double *__restrict__ a, const double *__restrict__ b, double *__restrict__ c) {
-    const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    if (i < n) c[i] = a[i] + b[i];
-}
-
-int fd_jacobian_elem(fvp_ctx *c, double cj, const double *psi, const double *psip, const double *shift, double *ys,
-                     double *kr2, double *cap2, double *contrib, const long *cptr, const int *srank, const int *ia,
-                     const int *dpos, double *J, long nnz, bool fp32) {
+template <typename C>
+static void fd_launch(fvp_ctx *c, const FdJacobian &fd) {
     hipStream_t s = c->stream;
     const int N = c->N, T = c->T;
-    // base state: k_r, capacity and the node records' heads
-    vg_kernel<false><<<blocks(N, 256), 256, 0, s>>>(N, c->zt, c->rho0, psi, c->zmask.p, c->zw.p, c->kr.p, c->cap.p,
-                                                     JvArgs(), c->nrec.p);
-    // every node moved by its shift (each node is moved once, in its own column)
-    fd_add<<<blocks(N, 256), 256, 0, s>>>(N, psi, shift, ys);
-    vg_kernel<false><<<blocks(N, 256), 256, 0, s>>>(N, c->zt, c->rho0, ys, c->zmask.p, c->zw.p, kr2, cap2, JvArgs(),
-                                                     nullptr);
-    if (fp32) {
-        float *c32 = reinterpret_cast<float *>(contrib);
-        if (c->dim == 3)
-            fd_elem_kernel32<3><<<blocks(T, 256), 256, 0, s>>>(T, N, c->zt, c->rho0, (const int4 *)c->conn.p,
-                                                                (const uint8_t *)c->ezone.p, c->kmul.p,
-                                                                (const uint8_t *)c->emask.p, c->nrec.p, c->kr.p, kr2,
-                                                                shift, c->invV.p, srank, c32);
-        else
-            fd_elem_kernel32<2><<<blocks(T, 256), 256, 0, s>>>(T, N, c->zt, c->rho0, (const int4 *)c->conn.p,
-                                                                (const uint8_t *)c->ezone.p, c->kmul.p,
-                                                                (const uint8_t *)c->emask.p, c->nrec.p, c->kr.p, kr2,
-                                                                shift, c->invV.p, srank, c32);
-        fd_gather_t<float><<<blocks(nnz, 256), 256, 0, s>>>(nnz, cptr, c32, J);
+    fd_nodes<C><<<blocks(N, 256), 256, 0, s>>>(N, c->zt, c->rho0, fd, c->zmask.p, c->zw.p, c->invV.p, c->kr.p, c->cap.p,
+                                              c->nrec.p);
+    const int4 *conn = (const int4 *)c->conn.p;
+    const uint8_t *ezone = c->ezone.p, *emask = c->emask.p;
+    if constexpr (sizeof(C) == 4) {
+        const auto elem = c->dim == 3 ? fd_elem_kernel32<3> : fd_elem_kernel32<2>;
+        elem<<<blocks(T, 256), 256, 0, s>>>(T, N, c->zt, c->rho0, conn, ezone, c->kmul.p, emask, c->nrec.p,
+                                            (const float4 *)fd.rec, (float4 *)fd.contrib);
     } else {
-        if (c->dim == 3)
-            fd_elem_kernel<3><<<blocks(T, 256), 256, 0, s>>>(T, N, c->zt, c->rho0, (const int4 *)c->conn.p,
-                                                              (const uint8_t *)c->ezone.p, c->kmul.p,
-                                                              (const uint8_t *)c->emask.p, c->nrec.p, c->kr.p, kr2,
-                                                              shift, c->invV.p, srank, contrib);
-        else
-            fd_elem_kernel<2><<<blocks(T, 256), 256, 0, s>>>(T, N, c->zt, c->rho0, (const int4 *)c->conn.p,
-                                                              (const uint8_t *)c->ezone.p, c->kmul.p,
-                                                              (const uint8_t *)c->emask.p, c->nrec.p, c->kr.p, kr2,
-                                                              shift, c->invV.p, srank, contrib);
-        fd_gather_t<double><<<blocks(nnz, 256), 256, 0, s>>>(nnz, cptr, contrib, J);
+        const auto elem = c->dim == 3 ? fd_elem_kernel<3> : fd_elem_kernel<2>;
+        elem<<<blocks(T, 256), 256, 0, s>>>(T, N, c->zt, c->rho0, conn, ezone, c->kmul.p, emask, c->nrec.p,
+                                            (const double2 *)fd.rec, fd.shift, c->invV.p, (double2 *)fd.contrib);
     }
-    fd_node_kernel<<<blocks(N, 256), 256, 0, s>>>(N, cj, psip, shift, c->cap.p, cap2, dpos, J);
+    if (fd.code)
+        fd_gather<C, true><<<blocks(N, fd.rows), kFdThreads, 4 * sizeof(C) * (size_t)fd.max_visits, s>>>(N, fd);
+    else
+        fd_gather<C, false><<<blocks(N, fd.rows), kFdThreads, 0, s>>>(N, fd);
     if (c->ndir)
-        fd_dirichlet<<<blocks(c->ndir, 256), 256, 0, s>>>(c->ndir, c->dnode.p, c->dval.p, psi, shift, ia, dpos, J);
+        fd_dirichlet<<<blocks(c->ndir, 256), 256, 0, s>>>(c->ndir, c->dnode.p, c->dval.p, fd.psi, fd.shift, fd.ia,
+                                                          fd.dpos, fd.J);
+}
+
+int fd_jacobian_elem(fvp_ctx *c, const FdJacobian &fd, bool fp32) {
+    if (fp32) fd_launch<float>(c, fd);
+    else fd_launch<double>(c, fd);
     FVP_HIP(hipGetLastError());
     return 0;
 }
