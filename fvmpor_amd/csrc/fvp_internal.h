@@ -112,13 +112,13 @@ struct fvp_ctx {
     size_t tile_lds = 0;
     // time-step upwinding
     int averaging = 1;             // 1: all edge weights 0.5
-    fvp::DevBuf<int> eedge;        // T x ned global edge of each local edge
+    fvp::DevBuf<int> eedge;        // ned x T global edge of each local edge
     fvp::DevBuf<int> slot_ptr;     // NE + 1
-    fvp::DevBuf<int> slot;         // T x ned (e*ned + j) sorted by (edge, element)
-    fvp::DevBuf<double> qface;     // T x ned averaged q.n per (element, local edge), back->front
+    fvp::DevBuf<int> slot;         // ned x T places (j*T + e) sorted by (edge, element)
+    fvp::DevBuf<double> qface;     // ned x T averaged q.n per (local edge, element), back->front
     fvp::DevBuf<double> ea;        // NE: summed area of the edge's CV faces (geometry, set-up)
     fvp::DevBuf<double> eflux;     // NE
-    fvp::DevBuf<double> wf;        // NE front weight
+    fvp::DevBuf<uint8_t> front;    // NE: the front node is upwind (averaging == 0)
     // scratch for Jv / reductions
     fvp::DevBuf<double> tmp1, tmp2, tmp3;
     fvp::DevBuf<double> red;       // reduction partials

@@ -511,32 +511,29 @@ extern "C" int fvp_create(const fvp_problem *p, int device, fvp_ctx **out) {
         }
         slot_ptr.push_back((int)ns);
         c->NE = ne + 1;
-        // move the per-element tables to the sorted element order; slots keep their
-        // (edge, original element) order, the order the reference sums CV faces in
+        // move the per-element tables to the sorted element order, one array per local
+        // edge; slots keep their (edge, original element) order, the order the reference
+        // sums CV faces in
         std::vector<int> eedge_n(ns), slot_n(ns);
         std::vector<uint8_t> orient_n(T);
         for (int e = 0; e < T; ++e) {
             const int o = eperm[e];
             orient_n[e] = orient[o];
-            for (int j = 0; j < ned; ++j) eedge_n[(size_t)e * ned + j] = eedge[(size_t)o * ned + j];
+            for (int j = 0; j < ned; ++j) eedge_n[(size_t)j * T + e] = eedge[(size_t)o * ned + j];
         }
         for (size_t r = 0; r < ns; ++r) {
             int o = slot[r] / ned, j = slot[r] % ned;
-            slot_n[r] = einv[o] * ned + j;
+            slot_n[r] = j * T + einv[o];
         }
         if (c->eedge.upload(eedge_n.data(), ns) || c->slot.upload(slot_n.data(), ns) ||
             c->slot_ptr.upload(slot_ptr.data(), slot_ptr.size()) || c->eorient.upload(orient_n.data(), T))
             return fail();
     }
     if (c->emask.alloc(T) || c->qface.alloc((size_t)T * ned) || c->ea.alloc(c->NE) || c->eflux.alloc(c->NE) ||
-        c->wf.alloc(c->NE))
+        c->front.alloc(c->NE))
         return fail();
     FVP_HIP(hipMemset(c->emask.p, 0, T));
     FVP_HIP(hipMemset(c->eflux.p, 0, sizeof(double) * c->NE));
-    {
-        std::vector<double> half(c->NE, 0.5);
-        FVP_HIP(hipMemcpy(c->wf.p, half.data(), sizeof(double) * c->NE, hipMemcpyHostToDevice));
-    }
     c->averaging = 1;
 
     // ---- boundary CV faces aggregated per (node, tag)
@@ -680,7 +677,7 @@ extern "C" int fvp_destroy(fvp_ctx *c) {
     c->t_dptr.release(); c->t_xoff.release(); c->t_xptr.release(); c->x_iptr.release(); c->x_ilist.release();
     c->x_tgt.release(); c->x_inode.release();
     c->xf.release(); c->eedge.release(); c->slot_ptr.release(); c->slot.release(); c->qface.release();
-    c->ea.release(); c->eflux.release(); c->wf.release(); c->tmp1.release(); c->tmp2.release();
+    c->ea.release(); c->eflux.release(); c->front.release(); c->tmp1.release(); c->tmp2.release();
     c->tmp3.release(); c->red.release();
     if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
     delete c;
