@@ -30,10 +30,59 @@
 
 namespace fvp {
 
-// Host twin of the reference's saturation kernel (fvmpor.h:302-343), same operation order.
 // a J v row, scaled by the optional row weights of the integrator's scaled solve
 __device__ __forceinline__ double jv_scaled(const JvArgs &jv, int i, double d) {
     return jv.osc ? d * jv.osc[i] : d;
+}
+
+// ln x and e^x for vg_eval.  The van Genuchten pass is bound by FP64 instructions, and
+// the library's pair takes about 125 of them; these take 50, to 0.92 and 1.05 ulp
+// (no worse in k_r, S and dS/dh, whose errors come from the arguments' rounding).
+// 1 024 000 nodes: vg_kernel 33 us with the library's, 26 with these.
+// ln: x = 2^k m with m in [sqrt(1/2), sqrt(2)), f = m - 1, s = f / (2 + f), and from
+// ln m = 2 atanh s = 2 s + s R, 2 s = f - s f: ln m = f - s (f - R), R = s^2 P(s^2),
+// P the Chebyshev fit of degree 6 to the atanh series (1.6e-18).  0 gives -inf, below NaN.
+__device__ __forceinline__ double vg_log(double x) {
+    double m = __builtin_amdgcn_frexp_mant(x);
+    int k = __builtin_amdgcn_frexp_exp(x);
+    const bool low = m < 0.70710678118654752;
+    m = low ? m + m : m;
+    k = low ? k - 1 : k;
+    const double f = m - 1., d = m + 1.;
+    double r = __builtin_amdgcn_rcp(d);
+    r = fma(r, fma(-d, r, 1.), r);
+    r = fma(r, fma(-d, r, 1.), r);
+    const double s = f * r, t = s * s, kd = k;
+    double p = 0.14616449685043406;
+    p = fma(p, t, 0.15331721600556042);
+    p = fma(p, t, 0.18182889125261723);
+    p = fma(p, t, 0.2222221113479508);
+    p = fma(p, t, 0.28571428625975487);
+    p = fma(p, t, 0.39999999999899505);
+    p = fma(p, t, 0.666666666666667);
+    // ln 2 in two parts, the first times any k exact
+    const double c = fma(kd, -1.9082149292705877e-10, s * (f - t * p));
+    const double y = fma(kd, 0.6931471803691238, f - c);
+    return x > 0. ? y : x == 0. ? -__builtin_inf() : __builtin_nan("");
+}
+
+// e^x = 2^k e^r, r = x - k ln 2 in two parts, e^r = 1 + (r + r^2 P(r)), P the Chebyshev
+// fit of degree 9 on |r| <= ln 2 / 2 (1.3e-17).  Overflows to inf, underflows to 0.
+__device__ __forceinline__ double vg_exp(double x) {
+    x = x < -750. ? -750. : x > 720. ? 720. : x;
+    const double kd = rint(x * 1.4426950408889634);
+    const double r = fma(kd, -1.9082149292705877e-10, fma(kd, -0.6931471803691238, x));
+    double p = 2.5100375832561234e-08;
+    p = fma(p, r, 2.7620075879983367e-07);
+    p = fma(p, r, 2.7557268480310024e-06);
+    p = fma(p, r, 2.4801521322368692e-05);
+    p = fma(p, r, 0.00019841269863040545);
+    p = fma(p, r, 0.0013888888917196719);
+    p = fma(p, r, 0.008333333333330065);
+    p = fma(p, r, 0.041666666666624164);
+    p = fma(p, r, 0.16666666666666669);
+    p = fma(p, r, 0.5000000000000001);
+    return __builtin_amdgcn_ldexp(1. + fma(r * r, p, r), (int)kd);
 }
 
 __device__ __forceinline__ void vg_eval(double h, const double *zp, double &Sw, double &dSw, double &krw) {
@@ -42,16 +91,16 @@ __device__ __forceinline__ void vg_eval(double h, const double *zp, double &Sw, 
     // exp(p ln x) on the already-rounded base (a few ulp from pow, which keeps
     // extra precision internally and costs about twice as much in FP64).
     const double nVG = zp[Z_N], mVG = zp[Z_M], S_r = zp[Z_SR];
-    double d = exp(nVG * log(-zp[Z_ALPHA] * h));  // a = (alpha |h|)^n
+    double d = vg_exp(nVG * vg_log(-zp[Z_ALPHA] * h));  // a = (alpha |h|)^n
     double s = d + 1.;                            // b
     double k = -1. / s;
     d /= s;
-    s = exp(-mVG * log(s));                       // Se = b^-m
+    s = vg_exp(-mVG * vg_log(s));                       // Se = b^-m
     d *= s;
     d /= h;
     d *= -(1 - S_r) * (nVG - 1);
     k += 1.;
-    k = exp(mVG * log(k));                        // (1 - 1/b)^m
+    k = vg_exp(mVG * vg_log(k));                        // (1 - 1/b)^m
     k -= 1.;
     k = k * k;
     k *= sqrt(s);
@@ -107,8 +156,8 @@ __device__ __forceinline__ double jv_sigma_block(const JvArgs &jv, double *red) 
 // One node per thread, the zone parameters in LDS.  Nodes of several zones are set
 // aside in a list and done together afterwards: a per-lane loop over the zones made
 // every wavefront pay for the most zones any of its nodes has (1 024 000 nodes, a
-// quarter of them at layer boundaries: 41 us; 33 us with the list).  Bound by FP64
-// instructions (about 440 per node and zone).
+// quarter of them at layer boundaries, with the library's ln and e^x: 41 us; 33 us with
+// the list).  Bound by FP64 instructions.
 // JV with jv.np > 0: every workgroup reduces the np partials of ||v||^2 in the
 // fixed order of jv_sigma_n2 (the same sigma bit for bit) and workgroup 0
 // stores sigma for the finalisation, so no launch of its own is needed.
@@ -595,7 +644,7 @@ __device__ __forceinline__ void upwind_fluxes(const NodeVals<DIM> &nv, const dou
 // halo nodes are evaluated again); otherwise k_r comes from vg_kernel.  Nodes of
 // several zones are set aside in a list and done afterwards, as there.
 // Bound by the LDS (268 cycles per 64 elements: 16-byte record reads and four sums)
-// and the phases' latency.  1 024 000 nodes, 512-node tiles: 76 us, with vg_kernel 33
+// and the phases' latency.  1 024 000 nodes, 512-node tiles: 76 us, with vg_kernel 26
 // and owner_imports 8 us more.  Gathering from memory through the L1 (owner_kernel,
 // kept for windows that do not fit) with a finalisation of its own: 120 + 41 + 33 us.
 constexpr int kRecBits = 14, kRecRanks = 4;
@@ -1188,7 +1237,7 @@ static void launch_tile(fvp_ctx *c, const double *psi, const double *psip, doubl
 // record, {V^-1, k_r, k_r moved, dk_r / shift} in FP32 or the two k_r in FP64; the
 // diagonal's capacity term -psi' a_hh(psi) moved with psi_i and psi'_i + c_j shift_i.
 // Nodes of several zones are set aside as in vg_kernel.  Bound by FP64 instructions
-// (two evaluations per node and zone).  141 000 nodes: 25 us, where five launches
+// (two evaluations per node and zone).  141 000 nodes: 19 us, where five launches
 // (increments, base, sum, moved, capacity term) took 42, and the elements' four
 // 8-byte gathers per node become one of 16.
 template <typename C>

@@ -83,3 +83,41 @@ def test_residual_and_jv(which):
         ctx.synchronize()
         assert np.abs(w.cpu().numpy() - Jc).max() <= 1e-6 * np.abs(Jc).max(), tile
         assert _rel(x.cpu().numpy(), Fc, scale) <= TOL, tile
+
+
+@pytest.mark.parametrize("soil", ["clay", "loam", "sandy_loam", "sand"])
+def test_capacity_over_the_range_of_heads(soil):
+    """The soil law from saturation to a dry head of 1e5 m, and at the edges of
+    ln and e^x: against the same law in extended precision.  Its relative error
+    is that of the exponents, |n ln(alpha |h|)| <= 40 times 2^-53 and a few like
+    it, below 2e-14; 1e-13 is allowed."""
+    import torch
+    from fvmpor_amd.lib import Context
+    from fvmpor_amd.problems import SOIL_CLASSES, slice2d_problem
+    base = slice2d_problem(nx=41, ny=26)
+    alpha, nv, tr, ts = SOIL_CLASSES[soil]
+    zone = np.array([[1.0, 1.0, 1.0, ts, alpha, nv, tr / ts, 1e-5]])
+    prob = dataclasses.replace(base, zones=zone)
+    ctx = Context(prob)
+    n = prob.mesh.n_nodes
+    psi = -np.logspace(-12, 5, n)
+    psi[:8] = [0.0, -0.0, 1.0, -5e-324, -1e-300, -1e-100, -1.0 / alpha, -1e-17]
+    dev = device()
+    tp, cap = torch.tensor(psi, device=dev), torch.zeros(n, dtype=torch.float64, device=dev)
+    F = torch.zeros_like(cap)
+    torch.cuda.synchronize()
+    ctx.residual(0.0, tp, torch.zeros_like(cap), F)
+    ctx.capacity(cap)
+    torch.cuda.synchronize()
+    h = np.where(psi < 0, psi, -1.0).astype(np.longdouble)
+    a, nl, sr = np.longdouble(alpha), np.longdouble(nv), np.longdouble(tr / ts)
+    m = 1 - 1 / nl
+    d = (a * -h) ** nl
+    se = (1 + d) ** -m
+    ds = -(1 - sr) * (nl - 1) * (d / (1 + d)) * se / h
+    sw = np.where(psi < 0, sr + (1 - sr) * se, 1)
+    want = (ts * np.where(psi < 0, ds, 0) + np.longdouble(1e-5) * sw) * 1000
+    # the node's zone weight sums the shares of its elements: 1 to rounding
+    err = np.abs(cap.cpu().numpy() - want) / np.abs(want)
+    print(soil, err.max())
+    assert err.max() < 1e-13
