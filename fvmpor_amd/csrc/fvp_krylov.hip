@@ -59,6 +59,22 @@ struct IluTri {
     void release() { pptr.release(); row.release(); col.release(); val.release(); }
 };
 
+// Packed layout of the block solve (see bj_solve), per triangle: the levels of at most
+// 64 slots, win entries per slot, their columns (two per word) and the row; out: where
+// the factorisation puts a row (see factor_tables), place: the entries of a row of
+// several slots
+struct BjPack {
+    int win = 0, levmax_l = 0, levmax_u = 0;
+    fvp::DevBuf<int> lev_l, lptr_l, lev_u, lptr_u;
+    fvp::DevBuf<unsigned> col_l, col_u, place;
+    fvp::DevBuf<unsigned short> row_l, row_u;
+    fvp::DevBuf<uint4> out;
+    void release() {
+        lev_l.release(); lptr_l.release(); lev_u.release(); lptr_u.release();
+        col_l.release(); col_u.release(); place.release(); row_l.release(); row_u.release(); out.release();
+    }
+};
+
 struct fvp_csr {
     int device = 0;
     hipStream_t stream = nullptr, own_stream = nullptr;
@@ -86,39 +102,30 @@ struct fvp_csr {
     DevBuf<int> b_ia, b_src;                // row pointers into the block arrays, source entry
     DevBuf<double> b_lu;
     DevBuf<float> b_lu32;                   // FP32 factor (FVP_PRECON_BJILU0_F32)
-    FactorTab fac;                          // block factorisation (bj_factor), its slots the s_lptr_l order
+    FactorTab fac;                          // block factorisation (bj_factor), its slots the blocks' level order
     // global ILU(0) in one workgroup: its factor tables, and per triangle the
     // solve's pieces and padded row windows (see ilu0_solve)
     bool one = false;
     FactorTab ofac;
     DevBuf<int> o_fptr;                     // {0, n}, {0, pieces}, then the factorisation's pieces of slots
     IluTri otri[2];
-    int o_threads = 64, o_win = 0;
+    int o_threads = 64, o_fthreads = 512, o_win = 0;  // threads of the solve and of the factorisation
     size_t o_lds = 0;
-    // the solve's levels: the factor's levels cut into pieces of at most 32 rows
-    DevBuf<int> s_lev_l, s_lev_u, s_lptr_l, s_lptr_u;
-    int s_levmax_l = 0, s_levmax_u = 0;
-    int s_maxslots = 0;                     // most slots of one block's triangle
-    // packed solve layout per triangle (see bj_solve): per slot its meta word
-    // pair, per block its entry base, per entry its local column (0-valued
-    // entries pad odd rows) and the current factor's value, which bj_factor
-    // writes; per U slot the inverted diagonal
-    DevBuf<unsigned> meta_l, meta_u;
-    DevBuf<long> ebase_l, ebase_u;
-    DevBuf<unsigned short> col_l, col_u;
+    DevBuf<int> f_lev[2], f_lptr[2];        // the factorisation's level pieces for 512 and 1024 threads
+    int f_levmax[2] = {0, 0};
+    // packed solve layouts, FP64's and FP32's (the same one where their windows are);
+    // values, which bj_factor writes (the rest stays zero), and per U slot the inverted
+    // diagonal
+    BjPack pack[2];
+    int pack32 = 0;
     DevBuf<double> val_l, val_u, dinv;
     DevBuf<float> val32_l, val32_u, dinv32;
-    // per block its overflow entries (row parts past kBjRow): packed position and triangle
-    DevBuf<int> ov_ptr;
-    DevBuf<long> ov_pos;
-    DevBuf<uint8_t> ov_tri;
-    int ov_max = 0;
     // workspace
     int m_alloc = -1;
     DevBuf<double> Q, w, r, z, part, scal, hdev;
     DevBuf<double> Hd, gd, csd, snd, yd;    // Hessenberg (column-major, m+1 rows), Givens pairs, rhs, solution
-    fvp::HostSlots hstat;                        // GMRES, see GmresWork
-    fvp::HostSlots hflag;                        // factorisation: the pivot flag
+    fvp::HostSlots hstat;                   // GMRES, see GmresWork
+    fvp::HostSlots hflag;                   // factorisation: the pivot flag
     const double *skip = nullptr;           // while GMRES queues a step: its word that ends the cycle
     DevBuf<double> Qk;                      // deflated GMRES: the kept harmonic Ritz vectors
     fvp_schur *sc = nullptr;                // Schur-complement preconditioner (FVP_PRECON_SCHUR)
@@ -946,7 +953,6 @@ __global__ void vaxpby(long n, double a, const double *__restrict__ x, double b,
 
 // ---- block-Jacobi ILU(0): one workgroup per block of bs consecutive rows
 // (factorisation: bj_factor; the rows of one level run concurrently)
-constexpr int kBjFactorThreads = 512;
 
 // workgroup barrier for LDS data: waits for LDS accesses only, so global loads
 // issued ahead stay in flight across it
@@ -969,11 +975,23 @@ __device__ __forceinline__ void lds_barrier() {
 // a wavefront has are skipped four at a time.  The pattern gives per L entry
 // (i, k) the position of u_kk, and per entry j of row i one byte: the distance
 // from u_kk to u_kj in row k, or 0.  Eight bytes (eight L entries) are one load
-// per lane.  141k-node box, FP32, 1024-row blocks, one overlap layer: 110 us,
-// packing of the solve's copies included; pairs read, modified and written in
+// per lane.  141k-node box, FP32, 1024-row blocks, one overlap layer: 86 us
+// with 1024 threads, 110 with 512, the solve's packed copies written as well; pairs read, modified and written in
 // memory one L entry after another, and a packing pass, took 500 + 25 us.
 // STAGED: the block's values are held in LDS; otherwise in place in memory.
 constexpr int kBjGroup = 16;
+// Threads: 512 or, for rows of up to 16 entries, 1024 (32 or 64 rows of a level at once;
+// longer rows' registers leave room for 512).  Both leave 16 wavefronts a CU, so 1024
+// halve the blocks in flight: taken where the pieces of levels they save are worth it,
+// with 1.2 for a piece's cost against 512's.  Blocks of 1024 rows with an overlap
+// layer, FP32, 138 of them: 110 us with 512 threads, 86 with 1024; 281 blocks of 512 rows
+// without overlap: 54 against 70.
+static int bj_factor_threads(int nc, long blocks, size_t lds, long lds_max, int pieces512, int pieces1024) {
+    if (nc > 1) return 512;
+    const long cus = 256, fit = lds ? std::max(1L, lds_max / (long)lds) : 2;
+    const long r512 = (blocks + cus * std::min(2L, fit) - 1) / (cus * std::min(2L, fit)), r1024 = (blocks + cus - 1) / cus;
+    return 1.2 * (double)r1024 * pieces1024 <= (double)r512 * pieces512 ? 1024 : 512;
+}
 constexpr int kAhead = 2;  // offset words of eight L entries loaded a level ahead
 
 // x of lane K of each 16-lane row, in every lane of that row
@@ -993,11 +1011,20 @@ __device__ __forceinline__ double row_bcast(double x) {
 }
 
 // What a row needs besides the other rows' values, loaded a level ahead.
+// The layout of the solve's packed copies: win values per slot; place: where
+// the entries of a row of several slots go (out.w > 0), from out.w - 1 on; all within
+// the block, whose first slots are ptr[lev[b]] of the solve's levels (null: 0)
+struct FacOut {
+    unsigned win;
+    const unsigned *place;
+    const int *lev_l, *ptr_l, *lev_u, *ptr_u;
+};
+
 template <typename T, int NC>
 struct FacRow {
     int s0, len, d;           // first entry, entries, L entries
     unsigned tab, l0;         // its first offset word, its first L entry
-    uint4 out;                // where the solve's packed copies of its L part, its U part and its pivot go
+    unsigned at[NC];          // place of each entry in the solve's packed copies
     T a[NC];                  // this lane's entries
     unsigned piv;             // pivot position of L entry `lane`
     unsigned off[2 * kAhead][NC];  // distances, four L entries a word, 0: none
@@ -1006,13 +1033,18 @@ struct FacRow {
 template <typename T, int NC>
 __device__ __forceinline__ void fac_row_load(FacRow<T, NC> &w, uint4 m, uint4 out, int gl,
                                              const unsigned *__restrict__ piv, const uint2 *__restrict__ off,
-                                             const T *val) {
+                                             const FacOut &fo, const T *val) {
     w.s0 = (int)m.x;
     w.len = (int)(m.y & 0xffu);
     w.d = (int)((m.y >> 8) & 0xffu);
     w.tab = m.z;
     w.l0 = m.w;
-    w.out = out;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        const int e = gl + kBjGroup * c;
+        w.at[c] = e < w.d ? out.x * fo.win + e : e > w.d ? out.y * fo.win + (e - w.d - 1) : out.y;
+        if (out.w && e < w.len && e != w.d) w.at[c] = fo.place[out.w - 1 + e];
+    }
     const int nch = (w.len + kBjGroup - 1) / kBjGroup;
 #pragma unroll
     for (int c = 0; c < NC; ++c) w.a[c] = gl + kBjGroup * c < w.len ? val[w.s0 + gl + kBjGroup * c] : T(0);
@@ -1109,7 +1141,8 @@ __device__ __forceinline__ void fac_row(FacRow<T, NC> &w, int gl, const unsigned
 // (a zero pivot sets the flag).
 template <typename T, int NC>
 __device__ __forceinline__ void fac_row_store(const FacRow<T, NC> &w, int gl, T *val, T *__restrict__ vl,
-                                              T *__restrict__ vu, T *__restrict__ vd, int *__restrict__ flag) {
+                                              T *__restrict__ vu, T *__restrict__ vd,
+                                              int *__restrict__ flag) {
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
         const int e = gl + kBjGroup * c;
@@ -1120,36 +1153,41 @@ __device__ __forceinline__ void fac_row_store(const FacRow<T, NC> &w, int gl, T 
         }
         if (e < w.len) {
             val[w.s0 + e] = v;
-            T *const p = e < w.d ? vl + w.out.x + e : e > w.d ? vu + w.out.y + (e - w.d - 1) : vd + w.out.z;
-            *p = v;
+            (e < w.d ? vl : e > w.d ? vu : vd)[w.at[c]] = v;
         }
     }
 }
 
 // One workgroup per block b: values ia[roff[b]] ... ia[roff[b + 1]] of lu, the
-// slots of its level pieces (at most kBjFactorThreads / kBjGroup each)
+// slots of its level pieces (at most TH / kBjGroup each)
 // lptr[blev[b]] ... lptr[blev[b + 1]].  src null: lu already holds the values to
 // factor.  vl, vu, vd: the solve's packed L, U and inverted diagonal.  STAGED: values and piece pointers (npmax + 1 ints) in LDS, so that a
 // barrier waits for LDS accesses only and rows are loaded kRing levels ahead.
-template <typename T, int NC, bool STAGED>
-__global__ void __launch_bounds__(kBjFactorThreads) bj_factor(
+template <typename T, int NC, bool STAGED, int TH>
+__global__ void __launch_bounds__(TH) bj_factor(
     const int *__restrict__ roff, const int *__restrict__ ia, const int *__restrict__ src,
     const double *__restrict__ a, const uint4 *__restrict__ slot, const uint4 *__restrict__ sout,
     const unsigned *__restrict__ piv, const uint2 *__restrict__ off, const int *__restrict__ blev,
     const int *__restrict__ lptr, T *lu, T *__restrict__ vl, T *__restrict__ vu, T *__restrict__ vd,
-    int *__restrict__ flag, int npmax) {
+    FacOut fo, int *__restrict__ flag, int npmax) {
     extern __shared__ double smem[];
     const int b = blockIdx.x;
     const int z0 = ia[roff[b]], nzb = ia[roff[b + 1]] - z0;
     const int l0 = blev[b], nl = blev[b + 1] - l0;
+    if (fo.ptr_l) {
+        const size_t sl = fo.ptr_l[fo.lev_l[b]], su = fo.ptr_u[fo.lev_u[b]];
+        vl += sl * fo.win;
+        vu += su * fo.win;
+        vd += su;
+    }
     int *pp = reinterpret_cast<int *>(smem);
     T *val = STAGED ? reinterpret_cast<T *>(smem + (npmax + 2) / 2) : lu + z0;
     if (src)
-        for (int k = threadIdx.x; k < nzb; k += kBjFactorThreads) val[k] = (T)a[src[z0 + k]];
+        for (int k = threadIdx.x; k < nzb; k += TH) val[k] = (T)a[src[z0 + k]];
     else if (STAGED)
-        for (int k = threadIdx.x; k < nzb; k += kBjFactorThreads) val[k] = lu[z0 + k];
+        for (int k = threadIdx.x; k < nzb; k += TH) val[k] = lu[z0 + k];
     if (STAGED)
-        for (int k = threadIdx.x; k <= nl; k += kBjFactorThreads) pp[k] = lptr[l0 + k];
+        for (int k = threadIdx.x; k <= nl; k += TH) pp[k] = lptr[l0 + k];
     else
         __threadfence_block();
     __syncthreads();
@@ -1176,7 +1214,7 @@ __global__ void __launch_bounds__(kBjFactorThreads) bj_factor(
             o[q] = sout[sl];
         }
 #pragma unroll
-        for (int q = 0; q < kRing; ++q) fac_row_load(w[q], m[q], o[q], gl, piv, off, val);
+        for (int q = 0; q < kRing; ++q) fac_row_load(w[q], m[q], o[q], gl, piv, off, fo, val);
 #pragma unroll
         for (int q = 0; q < kRing; ++q) {
             const int sl = slot_of(q + kRing, have1[q]);
@@ -1190,7 +1228,7 @@ __global__ void __launch_bounds__(kBjFactorThreads) bj_factor(
                     fac_row(w[q], gl, piv, off, val);
                     if (have[q]) fac_row_store(w[q], gl, val, vl, vu, vd, flag);
                 }
-                fac_row_load(w[q], m[q], o[q], gl, piv, off, val);
+                fac_row_load(w[q], m[q], o[q], gl, piv, off, fo, val);
                 have[q] = have1[q];
                 const int sl = slot_of(lb + q + 2 * kRing, have1[q]);
                 m[q] = slot[sl];
@@ -1198,16 +1236,16 @@ __global__ void __launch_bounds__(kBjFactorThreads) bj_factor(
                 lds_barrier();
             }
         }
-        for (int k = threadIdx.x; k < nzb; k += kBjFactorThreads) lu[z0 + k] = val[k];
+        for (int k = threadIdx.x; k < nzb; k += TH) lu[z0 + k] = val[k];
     } else {
         bool have, have1, have2;
         FacRow<T, NC> w;
         const int sl0 = slot_of(0, have), sl1 = slot_of(1, have1);
-        fac_row_load(w, slot[sl0], sout[sl0], gl, piv, off, val);
+        fac_row_load(w, slot[sl0], sout[sl0], gl, piv, off, fo, val);
         uint4 m1 = slot[sl1], o1 = sout[sl1];
         for (int l = 0; l < nl; ++l) {
             FacRow<T, NC> nx;
-            fac_row_load(nx, m1, o1, gl, piv, off, val);
+            fac_row_load(nx, m1, o1, gl, piv, off, fo, val);
             const int sl = slot_of(l + 2, have2);
             const uint4 m2 = slot[sl], o2 = sout[sl];
             if (__any(have)) {
@@ -1225,228 +1263,117 @@ __global__ void __launch_bounds__(kBjFactorThreads) bj_factor(
     }
 }
 
-// Solve: one wavefront per block.  Only the block's solution, its overflow
-// entries and its level pointers live in LDS (so that every block of the
-// matrix is resident at once and the CU interleaves their dependency chains).
-// The factor streams from a level-ordered packed copy per triangle: the row
-// parts one after another (each padded to an even length), so the bytes read
-// are the factor's own.  Per row part (a "slot", level order) a meta word pair
-// gives its start and its overflow offset, its row and its length.  A lane
-// pair takes a slot: the pair reads the fixed window of kBjRow entries
-// starting at the slot's start, one half each (past the row's length the
-// window runs into the following rows, which the level uses anyway, and is
-// masked); the halves' sums meet by a swap within the pair, and the even lane
-// subtracts the entries past kBjRow (from LDS) and stores the row.  So a level
-// of up to 32 slots costs one half window of instructions per lane.  T is the
-// factor's arithmetic type (double, or float for the FP32 preconditioner); x
-// and y stay FP64.
-constexpr int kBjRow = 12;
-#ifndef BJ_AHEAD_F32
-#define BJ_AHEAD_F32 8
-#endif
-#ifndef BJ_AHEAD_F64
-#define BJ_AHEAD_F64 4
-#endif
-
-constexpr int kBjHalf = kBjRow / 2;  // window entries per lane of a pair
-
-template <typename T>
+// Solve: one wavefront per block.  Only the block's solution and its level
+// pointers live in LDS (so that every block of the matrix is resident at once
+// and the CU interleaves their dependency chains).  The factor streams from a
+// level-ordered packed copy per triangle, which bj_factor writes: slots of W
+// entries, zero past the row's length (their column is the row itself), one lane
+// each, up to 64 a level.  A row of more than W entries takes further slots in
+// earlier levels, for the entries whose rows are final there: each subtracts its
+// share from v[r] (with d = 1 in U).  T is the factor's arithmetic type (double, or
+// float for the FP32 preconditioner); x and y stay FP64.
+// What bounds it is one wavefront's instruction issue and LDS latency per level, and
+// for large matrices the factor's bytes.  Rows end to end, a lane pair to a row and
+// windows of 12 entries (levels of 32, starts and lengths from the LDS, two selects an
+// entry) needed 71 vector instructions a level and twice the levels where those are
+// wide.  With a tetrahedral box's rows (at most 7 entries a triangle, 10 next to
+// other blocks), one overlap layer, us: 144 000 rows in blocks of 1024, FP64 51 -> 32,
+// FP32 49 -> 32; 614 000 in blocks of 512, FP64 49 -> 42, FP32 46 -> 39; in two
+// dimensions 23 000 in blocks of 1024, 43 -> 25 both.
+// W: in FP64 8, or 4 where nine rows in ten fit that; in FP32 the least of 4, 8 and 12
+// that all rows fit (12 beyond): a row's sum is kept in the order of the form before
+// (entries 0 to 5, then 6 to 11), which FP32 would show.
+template <typename T, int W>
 struct BjWin {
-    T a[kBjHalf];
-    unsigned c[kBjHalf / 2];  // local columns, two per word
-    unsigned m0, m1;          // meta words
-    T d;                      // inverted diagonal (U)
-    bool have;
+    T a[W];
+    unsigned c[W / 2];  // local columns, two per word
+    unsigned r;
+    T d;                // inverted diagonal (U)
+    bool mine;
 };
 
-// x plus the other lane of the pair (lanes 2i, 2i+1): a DPP quad permutation
-// [1, 0, 3, 2], so both lanes get the same sum
-__device__ __forceinline__ float pair_sum(float x) {
-    const int y = __builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xF, 0xF, false);
-    return x + __int_as_float(y);
-}
-__device__ __forceinline__ double pair_sum(double x) {
-    const long long b = __double_as_longlong(x);
-    const int lo = __builtin_amdgcn_mov_dpp((int)(unsigned)b, 0xB1, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), 0xB1, 0xF, 0xF, false);
-    return x + __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
-}
-struct BjMeta {
-    unsigned m0, m1;  // start (low 16) | overflow offset (high 16); row (low 16) | length (high 16)
-    int s;            // slot
-    bool have;
-};
-
-template <typename T, bool UPPER>
-__device__ __forceinline__ void bj_win_load(BjWin<T> &w, const BjMeta &m, int half, const T *__restrict__ val,
-                                            const unsigned short *__restrict__ col, const T *__restrict__ dinv) {
-    // this lane's half of the window: even start, so pairs stay aligned
-    const long k = (long)(m.m0 & 0xffffu) + half * kBjHalf;
-    if (sizeof(T) == 4) {
-        const uint2 *p = reinterpret_cast<const uint2 *>(val + k);
+// slot s of the block's
+template <typename T, int W, bool UPPER>
+__device__ __forceinline__ void bj_win_load(BjWin<T, W> &w, unsigned s, bool mine, const T *__restrict__ val,
+                                            const unsigned *__restrict__ col, const unsigned short *__restrict__ row,
+                                            const T *__restrict__ dinv) {
+    if constexpr (sizeof(T) == 4) {
+        const float4 *p = reinterpret_cast<const float4 *>(val + W * s);
 #pragma unroll
-        for (int i = 0; i < kBjHalf / 2; ++i) {
-            const uint2 q = p[i];
-            w.a[2 * i] = (T)__uint_as_float(q.x);
-            w.a[2 * i + 1] = (T)__uint_as_float(q.y);
+        for (int i = 0; i < W / 4; ++i) {
+            const float4 q = p[i];
+            w.a[4 * i] = q.x; w.a[4 * i + 1] = q.y; w.a[4 * i + 2] = q.z; w.a[4 * i + 3] = q.w;
         }
     } else {
-        const double2 *p = reinterpret_cast<const double2 *>(val + k);
+        const double2 *p = reinterpret_cast<const double2 *>(val + W * s);
 #pragma unroll
-        for (int i = 0; i < kBjHalf / 2; ++i) {
+        for (int i = 0; i < W / 2; ++i) {
             const double2 q = p[i];
-            w.a[2 * i] = (T)q.x;
-            w.a[2 * i + 1] = (T)q.y;
+            w.a[2 * i] = q.x; w.a[2 * i + 1] = q.y;
         }
     }
-    const unsigned *pc = reinterpret_cast<const unsigned *>(col + k);
+    const uint2 *pc = reinterpret_cast<const uint2 *>(col + W / 2 * s);
 #pragma unroll
-    for (int i = 0; i < kBjHalf / 2; ++i) w.c[i] = pc[i];
-    w.m0 = m.m0;
-    w.m1 = m.m1;
-    w.d = UPPER ? dinv[m.s] : T(0);
-    w.have = m.have;
-}
-
-// Each lane of the pair sums its half window (bj_win_partial); the even lane
-// then finishes the row (bj_win_finish): s = v[r] - (both halves) - (entries
-// past kBjRow, in column order), times the inverted diagonal for U.  Every
-// lane takes part in the pair sum (lanes without a slot read a valid clamped
-// slot and store nothing).
-// The half window's partial sum; vr: v[r], read with the window's columns
-// (rows of one level do not depend on each other, so v[r] is final here).
-template <typename T>
-__device__ __forceinline__ T bj_win_partial(const BjWin<T> &w, int half, const T *v, T &vr) {
-    const int r = (int)(w.m1 & 0xffffu), kn = (int)(w.m1 >> 16);
-    T p = T(0);
-#pragma unroll
-    for (int u = 0; u < kBjHalf; ++u) {
-        // past the row's length the window holds the following rows' entries
-        // (possibly of another block): masked to 0 * v[r]
-        const int ug = half * kBjHalf + u;
-        const unsigned cw = w.c[u / 2];
-        const int c = ug < kn ? (int)((u & 1) ? (cw >> 16) : (cw & 0xffffu)) : r;
-        const T a = ug < kn ? w.a[u] : T(0);
-        p += a * v[c];
+    for (int i = 0; i < W / 4; ++i) {
+        const uint2 q = pc[i];
+        w.c[2 * i] = q.x; w.c[2 * i + 1] = q.y;
     }
-    vr = v[r];
-    return p;
-}
-
-// OVG: the overflow entries are read from the packed arrays in memory (blocks
-// whose overflow lists do not fit the LDS) instead of from LDS
-template <typename T, bool UPPER, bool OVG>
-__device__ __forceinline__ void bj_win_finish(const BjWin<T> &w, int half, T p, T vr, T *v, T *vd,
-                                              const uint4 *ovp, const T *__restrict__ val,
-                                              const unsigned short *__restrict__ col) {
-    const int r = (int)(w.m1 & 0xffffu), kn = (int)(w.m1 >> 16);
-    // every lane forms and stores s (lanes without a row store to their own
-    // spare slot vd), so v[r]'s read stays with the window's reads
-    const bool mine = w.have && !half;
-    T s = vr - pair_sum(p);
-    if (mine && kn > kBjRow) {
-        if (OVG) {  // overflow entries straight after the window in the packed arrays
-            const int k0 = (int)(w.m0 & 0xffffu);
-            for (int k = k0 + kBjRow; k < k0 + kn; ++k) s -= val[k] * v[col[k]];
-        } else {
-            const int oo = (int)(w.m0 >> 16);
-            for (int k = oo; k < oo + kn - kBjRow; ++k) {
-                const uint4 q = ovp[k];
-                T a;
-                if (sizeof(T) == 4) a = (T)__uint_as_float(q.x);
-                else a = (T)__longlong_as_double((long long)(((unsigned long long)q.y << 32) | q.x));
-                s -= a * v[q.z];
-            }
-        }
-    }
-    if (UPPER) s *= w.d;  // inverted diagonal
-    *(mine ? v + r : vd) = s;
+    w.r = row[s];
+    w.d = UPPER ? dinv[s] : T(0);
+    w.mine = mine;
 }
 
 // levels loaded ahead: deep enough to cover a memory round trip with the short
-// per-level arithmetic; FP64 windows are larger, so fewer of them fit the registers
-template <typename T>
-constexpr int bj_ahead() { return sizeof(T) == 4 ? BJ_AHEAD_F32 : BJ_AHEAD_F64; }
+// per-level arithmetic, as far as the registers go
+template <typename T, int W>
+constexpr int bj_ahead() { return sizeof(T) == 4 ? (W == 12 ? 5 : 8) : W == 4 ? 7 : 4; }
 
-// Staging a triangle's meta words (its ns slots from meta) in LDS: one round
-// is kBjMeta loads per lane, all in flight together, so a block of up to
-// 64 * kBjMeta slots per triangle waits out one memory latency.
-constexpr int kBjMeta = 32;
-__device__ __forceinline__ void bj_meta_load(uint2 (&q)[kBjMeta], const uint2 *__restrict__ meta, int ns, int k0) {
-#pragma unroll
-    for (int i = 0; i < kBjMeta; ++i) q[i] = meta[min(k0 + 64 * i, ns - 1)];
-}
-__device__ __forceinline__ void bj_meta_store(const uint2 (&q)[kBjMeta], uint2 *ms, int ns, int k0) {
-#pragma unroll
-    for (int i = 0; i < kBjMeta; ++i)
-        if (k0 + 64 * i < ns) ms[k0 + 64 * i] = q[i];
-}
-// the slots from k0 (this lane's first) on, round by round
-__device__ __forceinline__ void bj_meta_stage(const uint2 *__restrict__ meta, uint2 *ms, int ns, int k0) {
-    for (; k0 < ns; k0 += 64 * kBjMeta) {
-        uint2 q[kBjMeta];
-        bj_meta_load(q, meta, ns, k0);
-        bj_meta_store(q, ms, ns, k0);
-    }
-}
-
-// One triangle of one block: lane pair t/2 takes the (t/2)-th slot of each
-// level (the solve's levels hold at most 32 slots).  The triangle's meta words
-// are staged in LDS (ms, slot lp[0] first) before the sweep, so a level's
-// window addresses come from LDS and only the windows themselves are loads in
-// flight: kA levels ahead, one window per lane and level, each consumed by the
-// same unrolled stage that issued it kA stages earlier (no loop-carried
-// register holds a pending load, so the compiler's wait counts keep all kA
-// levels in flight).  No global load with a data-dependent count is issued
-// inside the level loop, and every pass runs all kA levels (those past the
-// last have no lane with work).
-template <typename T, bool UPPER, bool OVG>
-__device__ __forceinline__ void bj_sweep(T *v, T *vd, int nl, const int *lp, const uint2 *ms,
-                                         const T *__restrict__ val, const unsigned short *__restrict__ col,
-                                         const T *__restrict__ dinv, const uint4 *ovp) {
-    const int t = threadIdx.x;
+// One triangle of one block: lane t takes the t-th slot of each level (lp: the
+// levels' slots within the block).  The windows are loads in flight, kA levels
+// ahead, one per lane and level, each consumed by the same unrolled stage that
+// issued it kA stages earlier (no loop-carried register holds a pending load, so
+// the compiler's wait counts keep all kA levels in flight).  Every pass runs all
+// kA levels (those past the last have no lane with work).  Every lane forms and
+// stores s, lanes without a slot to their own spare place vd, so that v[r]'s read
+// stays with the window's (rows of one level do not depend on each other, so it
+// is final here).
+template <typename T, int W, bool UPPER>
+__device__ __forceinline__ void bj_sweep(T *v, T *vd, int nl, const int *lp, const T *__restrict__ val,
+                                         const unsigned *__restrict__ col, const unsigned short *__restrict__ row,
+                                         const T *__restrict__ dinv) {
     if (nl <= 0) return;
-    constexpr int kA = bj_ahead<T>();
-    const int s0 = lp[0];
-    const int q = t >> 1, half = t & 1;
-    // a level's slot range, then this lane's slot and its meta words
-    auto level_range = [&](int l, int &p0, int &cnt) {
-        const int lc = min(l, nl - 1);
-        p0 = lp[lc];
-        cnt = lp[lc + 1] - p0;
+    constexpr int kA = bj_ahead<T, W>();
+    auto load = [&](BjWin<T, W> &w, int l, int p0, int p1) {
+        const int s = p0 + (int)threadIdx.x;
+        bj_win_load<T, W, UPPER>(w, min(s, p1 - 1), l < nl && s < p1, val, col, row, dinv);
     };
-    auto slot_meta = [&](int l, int p0, int cnt, BjMeta &m) {
-        m.s = p0 + min(q, cnt - 1);
-        const uint2 mq = ms[m.s - s0];
-        m.m0 = mq.x;
-        m.m1 = mq.y;
-        m.have = l < nl && q < cnt;
-    };
-    BjWin<T> wr[kA];
+    BjWin<T, W> wr[kA];
 #pragma unroll
     for (int d = 0; d < kA; ++d) {
-        int p0, cnt;
-        level_range(d, p0, cnt);
-        BjMeta m;
-        slot_meta(d, p0, cnt, m);
-        bj_win_load<T, UPPER>(wr[d], m, half, val, col, dinv);
+        const int lc = min(d, nl - 1);
+        load(wr[d], d, lp[lc], lp[lc + 1]);
         wave_lds_order();
     }
-    // Per stage three LDS round trips overlap: level lb + d + kA's range is
-    // read with the update's values, its meta words while the update's sums
-    // are formed; the window of that level is issued last.
+    // Level lb + d + kA's range is read with the update's values; its window is
+    // issued last.
     for (int lb = 0; lb < nl; lb += kA) {
 #pragma unroll
         for (int d = 0; d < kA; ++d) {
-            const int ln = lb + d + kA;
-            int p0, cnt;
-            level_range(ln, p0, cnt);
-            T vr;
-            const T p = bj_win_partial<T>(wr[d], half, v, vr);
-            BjMeta m;
-            slot_meta(ln, p0, cnt, m);
-            bj_win_finish<T, UPPER, OVG>(wr[d], half, p, vr, v, vd, ovp, val, col);
-            bj_win_load<T, UPPER>(wr[d], m, half, val, col, dinv);  // level ln
+            const int ln = lb + d + kA, lc = min(ln, nl - 1);
+            const int p0 = lp[lc], p1 = lp[lc + 1];
+            const BjWin<T, W> &w = wr[d];
+            constexpr int kFirst = sizeof(T) == 4 ? 6 : W / 2;
+            T q0 = T(0), q1 = T(0);
+#pragma unroll
+            for (int u = 0; u < W; ++u) {
+                const T x = v[(u & 1) ? w.c[u / 2] >> 16 : w.c[u / 2] & 0xffffu];
+                if (u < kFirst) q0 += w.a[u] * x;
+                else q1 += w.a[u] * x;
+            }
+            T s = v[w.r] - (q0 + q1);
+            if (UPPER) s *= w.d;
+            *(w.mine ? v + w.r : vd) = s;
+            load(wr[d], ln, p0, p1);
             // one wavefront: the LDS executes its accesses in order, so only
             // the compiler must keep them in program order
             wave_lds_order();
@@ -1455,13 +1382,9 @@ __device__ __forceinline__ void bj_sweep(T *v, T *vd, int nl, const int *lp, con
 }
 
 // LDS bytes of one block's solve: the solution (T x maxrows) and a spare
-// slot per lane (T x 64), the block's
-// overflow entries (16 bytes each; none with OVG), its L and U level pointers,
-// the meta words of one triangle's slots
-__host__ __device__ inline size_t bj_solve_lds(size_t tsize, int maxrows, int ovmax, int levl, int levu,
-                                                int maxslots) {
-    return ((tsize * (size_t)(maxrows + 64) + 15) & ~(size_t)15) + 16 * (size_t)ovmax +
-           ((4 * (size_t)(levl + levu + 2) + 7) & ~(size_t)7) + 8 * (size_t)maxslots;
+// place per lane (T x 64), its L and U level pointers
+__host__ __device__ inline size_t bj_solve_lds(size_t tsize, int maxrows, int levl, int levu) {
+    return ((tsize * (size_t)(maxrows + 64) + 7) & ~(size_t)7) + 4 * (size_t)(levl + levu + 2);
 }
 
 // rowid: global row of each local row (nullptr: block b's rows are the
@@ -1470,25 +1393,20 @@ __host__ __device__ inline size_t bj_solve_lds(size_t tsize, int maxrows, int ov
 // block, so that every block of the matrix is resident at once.  (Staging the
 // whole block in LDS was measured slower: it limits the resident blocks, and
 // one wavefront stages too slowly.)  Per triangle: solve levels blev (per
-// block) into lptr (per level, into the level-ordered slots, at most 32 per
-// level), per slot its meta word pair, the packed values and local columns
-// from the block's entry base ebase, U's inverted diagonals; the block's
-// overflow entries are the packed entries at ov_pos[ov_ptr[b] ..).
-template <typename T, bool OVG>
+// block) into lptr (per level, into the level-ordered slots, at most 64 per
+// level), the slots' values, columns and rows, U's inverted diagonals.
+template <typename T, int W>
 __global__ void __launch_bounds__(64) bj_solve(const int *__restrict__ roff, const int *__restrict__ rowid,
                                                const int *__restrict__ own, const int *__restrict__ blev_l,
-                                               const int *__restrict__ lptr_l, const uint2 *__restrict__ meta_l,
-                                               const long *__restrict__ ebase_l, const T *__restrict__ val_l,
-                                               const unsigned short *__restrict__ col_l,
+                                               const int *__restrict__ lptr_l, const T *__restrict__ val_l,
+                                               const unsigned *__restrict__ col_l,
+                                               const unsigned short *__restrict__ row_l,
                                                const int *__restrict__ blev_u, const int *__restrict__ lptr_u,
-                                               const uint2 *__restrict__ meta_u, const long *__restrict__ ebase_u,
-                                               const T *__restrict__ val_u, const unsigned short *__restrict__ col_u,
-                                               const T *__restrict__ dinv, const int *__restrict__ ov_ptr,
-                                               const long *__restrict__ ov_pos, const unsigned char *__restrict__ ov_tri,
-                                               int maxrows, int ovmax, int levmax_l, int levmax_u,
-                                               const double *__restrict__ x,
-                                               const double *__restrict__ xdiv, double *__restrict__ y,
-                                               double *__restrict__ yn2, const double *skip) {
+                                               const T *__restrict__ val_u, const unsigned *__restrict__ col_u,
+                                               const unsigned short *__restrict__ row_u,
+                                               const T *__restrict__ dinv, int maxrows,
+                                               const double *__restrict__ x, const double *__restrict__ xdiv,
+                                               double *__restrict__ y, double *__restrict__ yn2, const double *skip) {
     extern __shared__ double smem[];
     const double over = skip_word(skip);
     const int b = blockIdx.x;
@@ -1496,16 +1414,15 @@ __global__ void __launch_bounds__(64) bj_solve(const int *__restrict__ roff, con
     const int cnt = roff[b + 1] - base;
     char *lds = reinterpret_cast<char *>(smem);
     T *v = reinterpret_cast<T *>(lds);
-    // v: the block's rows, then one spare slot per lane
+    // v: the block's rows, then one spare place per lane
     T *vd = v + maxrows + threadIdx.x;
-    uint4 *ovp = reinterpret_cast<uint4 *>(lds + ((sizeof(T) * (size_t)(maxrows + 64) + 15) & ~(size_t)15));
     const int l0 = blev_l[b], nl = blev_l[b + 1] - l0;
     const int u0 = blev_u[b], nu = blev_u[b + 1] - u0;
-    // L's meta words: the first round's loads are issued here, ahead of
-    // staging x, and stored to the LDS after it
-    const int sl0 = nl > 0 ? lptr_l[l0] : 0, nsl = nl > 0 ? lptr_l[l0 + nl] - sl0 : 0;
-    uint2 mq[kBjMeta];
-    if (nsl > 0) bj_meta_load(mq, meta_l + sl0, nsl, threadIdx.x);
+    const long sl = lptr_l[l0], su = lptr_u[u0];  // the block's first slots
+    int *lpl = reinterpret_cast<int *>(lds + ((sizeof(T) * (size_t)(maxrows + 64) + 7) & ~(size_t)7));
+    int *lpu = lpl + nl + 1;
+    for (int k = threadIdx.x; k <= nl; k += 64) lpl[k] = lptr_l[l0 + k] - (int)sl;
+    for (int k = threadIdx.x; k <= nu; k += 64) lpu[k] = lptr_u[u0 + k] - (int)su;
     // stage x (optionally scaled by 1 / xdiv) in batches of kBjStage rows per
     // lane, so that a batch's gathers are in flight together
     constexpr int kBjStage = 16;
@@ -1528,38 +1445,10 @@ __global__ void __launch_bounds__(64) bj_solve(const int *__restrict__ roff, con
             if (r < cnt) v[r] = (T)(xdiv ? xv[k] / dv[k] : xv[k]);
         }
     }
-    // overflow entries: value bits, local column
-    const int ob = ov_ptr[b], on = OVG ? 0 : ov_ptr[b + 1] - ob;
-    if (OVG) ovmax = 0;
-    for (int k = threadIdx.x; k < on; k += 64) {
-        const long e = ov_pos[ob + k];
-        const bool up = ov_tri[ob + k];
-        const T a = up ? val_u[e] : val_l[e];
-        unsigned lo, hi = 0u;
-        if (sizeof(T) == 4) lo = __float_as_uint((float)a);
-        else {
-            const unsigned long long u = (unsigned long long)__double_as_longlong((double)a);
-            lo = (unsigned)u;
-            hi = (unsigned)(u >> 32);
-        }
-        ovp[k] = make_uint4(lo, hi, (unsigned)(up ? col_u[e] : col_l[e]), 0u);
-    }
-    int *lpl = reinterpret_cast<int *>(ovp + ovmax);
-    int *lpu = lpl + nl + 1;
-    uint2 *ms = reinterpret_cast<uint2 *>(reinterpret_cast<char *>(lpl) +
-                                          ((4 * (size_t)(levmax_l + levmax_u + 2) + 7) & ~(size_t)7));
-    for (int k = threadIdx.x; k <= nl; k += 64) lpl[k] = lptr_l[l0 + k];
-    for (int k = threadIdx.x; k <= nu; k += 64) lpu[k] = lptr_u[u0 + k];
-    if (nsl > 0) bj_meta_store(mq, ms, nsl, threadIdx.x);
-    bj_meta_stage(meta_l + sl0, ms, nsl, threadIdx.x + 64 * kBjMeta);
     wave_lds_order();
     if (over != 0.) return;
-    bj_sweep<T, false, OVG>(v, vd, nl, lpl, ms, val_l + ebase_l[b], col_l + ebase_l[b], nullptr, ovp);
-    // U's meta words replace L's (the sweep's LDS accesses execute in order;
-    // loading them during L's sweep instead was measured no faster)
-    if (nu > 0) bj_meta_stage(meta_u + lpu[0], ms, lpu[nu] - lpu[0], threadIdx.x);
-    wave_lds_order();
-    bj_sweep<T, true, OVG>(v, vd, nu, lpu, ms, val_u + ebase_u[b], col_u + ebase_u[b], dinv, ovp);
+    bj_sweep<T, W, false>(v, vd, nl, lpl, val_l + W * sl, col_l + W / 2 * sl, row_l + sl, nullptr);
+    bj_sweep<T, W, true>(v, vd, nu, lpu, val_u + W * su, col_u + W / 2 * su, row_u + su, dinv + su);
     const int olo = own[2 * b], ohi = own[2 * b + 1];
     double q = 0.;
     for (int r0 = olo + threadIdx.x; r0 < ohi; r0 += 64 * kBjStage) {
@@ -1592,13 +1481,13 @@ __global__ void __launch_bounds__(64) bj_solve(const int *__restrict__ roff, con
 // pieces ahead; the chain per piece is one batch of LDS reads, the row's sum and
 // one LDS store.  One wavefront needs no barrier (the LDS runs its accesses in
 // order); wider workgroups meet at one per piece.  A 4 141-node slice (141 levels
-// per triangle) takes 52 us, and its factorisation 282 us; one launch per level
+// per triangle) takes 52 us, and its factorisation 205 us; one launch per level
 // and triangle (the form that matrices outside these limits keep) took 707 to
 // 1075 us, and 1500 us.  The chain bounds it: 0.18 us per level.
 // kOneWidth: rows per level, on average over both triangles, up to which one
 // workgroup is used: a launch per level costs 2.5 us in the solve and 10 us in
-// the factorisation, one workgroup 0.2 us per piece of up to 1024 rows and 2 us
-// per 32 rows of a level.
+// the factorisation, one workgroup 0.2 us per piece of up to 1024 rows and 1.5
+// us per 64 rows of a level.
 constexpr long kOneWidth = 256;
 
 template <int KW>
@@ -2372,13 +2261,13 @@ static int build_levels(fvp_csr *A, const std::vector<int> &diag) {
 
 // The tables of bj_factor: roff, bia, bja, bdiag describe the blocks (local
 // columns, entry positions over all blocks), rows the local rows as slots in
-// level order (block b's slots are [roff[b], roff[b + 1])), out per slot the
-// places of its packed L part, U part and pivot; no row is longer than 64
-// entries.
+// level order (block b's slots are [roff[b], roff[b + 1])), out per slot its
+// slots in the solve's L (x) and U (y), counted within the block, and w as in FacOut; no row is longer than
+// 64 entries.
 template <typename Col, typename Row>
 static int factor_tables(FactorTab &F, int nb, const std::vector<int> &roff, const std::vector<int> &bia,
                          const std::vector<Col> &bja, const std::vector<int> &bdiag, const std::vector<Row> &rows,
-                         const std::vector<uint4> &out, int maxrow) {
+                         int maxrow) {
     const int total = roff[nb];
     std::vector<uint4> slot(total);
     std::vector<unsigned> piv;
@@ -2420,7 +2309,7 @@ static int factor_tables(FactorTab &F, int nb, const std::vector<int> &roff, con
     if (piv.empty()) piv.push_back(0u);
     if (off.empty()) off.resize(8 * kBjGroup, (unsigned char)0);
     F.nc = maxrow <= kBjGroup ? 1 : maxrow <= 2 * kBjGroup ? 2 : 4;
-    return F.slot.upload(slot.data(), slot.size()) || F.out.upload(out.data(), out.size()) || F.piv.upload(piv.data(), piv.size()) ||
+    return F.slot.upload(slot.data(), slot.size()) || F.piv.upload(piv.data(), piv.size()) ||
            F.off.upload(reinterpret_cast<const uint2 *>(off.data()), off.size() / 8);
 }
 
@@ -2447,7 +2336,7 @@ static int build_one(fvp_csr *A, const std::vector<int> &diag, const std::vector
     const int win = maxtri <= 4 ? 4 : maxtri <= 8 ? 8 : maxtri <= 16 ? 16 : 32;
     if (maxrow > 64 || maxtri > win || n > 65536) return 0;
     // wide levels are worth a launch each (the whole device on one level); one
-    // workgroup takes kBjFactorThreads / kBjGroup rows of a level at a time
+    // workgroup's factorisation takes 32 or 64 rows of a level at a time
     const long levels = (long)(A->lptr_h.size() - 1 + A->uptr_h.size() - 1);
     if (2L * n > kOneWidth * levels) return 0;
     // threads: the count that makes the sweep's pieces cheapest (a piece's cost
@@ -2469,7 +2358,7 @@ static int build_one(fvp_csr *A, const std::vector<int> &diag, const std::vector
     }
     if (pieces[0].empty()) return 0;
     A->o_win = win;
-    std::vector<uint4> out(n);  // by row at first, then by slot of L's level order
+    std::vector<uint4> out(n, make_uint4(0u, 0u, 0u, 0u));  // by row at first, then by slot of L's level order
     for (int t = 0; t < 2; ++t) {
         const std::vector<int> &order = t ? urows : lrows;
         std::vector<unsigned> row(n);
@@ -2481,8 +2370,7 @@ static int build_one(fvp_csr *A, const std::vector<int> &diag, const std::vector
                 const size_t q = (size_t)sl * win + k;
                 col[q] = (unsigned short)(k0 + k < k1 ? A->ja_h[k0 + k] : i);
             }
-            (t ? out[i].y : out[i].x) = (unsigned)(sl * win);
-            if (t) out[i].z = (unsigned)sl;
+            (t ? out[i].y : out[i].x) = (unsigned)sl;
         }
         IluTri &T = A->otri[t];
         T.npieces = (int)pieces[t].size() - 1;
@@ -2494,12 +2382,15 @@ static int build_one(fvp_csr *A, const std::vector<int> &diag, const std::vector
     }
     std::vector<uint4> by(n);
     for (int sl = 0; sl < n; ++sl) by[sl] = out[lrows[sl]];
-    std::vector<int> fp;
-    level_pieces(A->lptr_h, kBjFactorThreads / kBjGroup, fp);
+    std::vector<int> fp, fp1024;
+    level_pieces(A->lptr_h, 512 / kBjGroup, fp);
+    level_pieces(A->lptr_h, 1024 / kBjGroup, fp1024);
+    A->o_fthreads = bj_factor_threads(maxrow <= kBjGroup ? 1 : 2, 1, 0, 0, (int)fp.size() - 1, (int)fp1024.size() - 1);
+    if (A->o_fthreads == 1024) fp.swap(fp1024);
     const int head[4] = {0, n, 0, (int)fp.size() - 1};
     fp.insert(fp.begin(), head, head + 4);
     if (A->o_fptr.upload(fp.data(), fp.size()) ||
-        factor_tables(A->ofac, 1, {0, n}, A->ia_h, A->ja_h, diag, lrows, by, maxrow))
+        factor_tables(A->ofac, 1, {0, n}, A->ia_h, A->ja_h, diag, lrows, maxrow) || A->ofac.out.upload(by.data(), n))
         return -1;
     for (const void *f :
          {(const void *)ilu0_solve<4, 64>, (const void *)ilu0_solve<8, 64>, (const void *)ilu0_solve<16, 64>,
@@ -2508,6 +2399,124 @@ static int build_one(fvp_csr *A, const std::vector<int> &diag, const std::vector
           (const void *)ilu0_solve<8, 1024>, (const void *)ilu0_solve<16, 1024>, (const void *)ilu0_solve<32, 1024>})
         (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, A->lds_max);
     A->one = true;
+    return 0;
+}
+
+// The solve's packed layout with windows of W entries for the blocks roff, bia, bja,
+// bdiag (as in factor_tables), rows_l their rows in the factorisation's order
+static int build_pack(BjPack &P, int W, int nb, const std::vector<int> &roff, const std::vector<int> &bia,
+                      const std::vector<unsigned short> &bja, const std::vector<int> &bdiag,
+                      const std::vector<unsigned short> &rows_l) {
+    const int total = roff[nb];
+    P.win = W;
+    std::vector<int> lev;
+    std::vector<uint4> out(total, make_uint4(0u, 0u, 0u, 0u));  // by row at first, then by slot of L's level order
+    std::vector<unsigned> place;
+    struct Slot {
+        int row, n;     // local row, entries
+        int first;      // in `order`
+        bool main;
+    };
+    std::vector<int> order, at, count, step;
+    std::vector<Slot> slots;
+    for (int tri = 0; tri < 2; ++tri) {
+        std::vector<unsigned> col;
+        std::vector<unsigned short> srow;
+        std::vector<int> sb(nb + 1, 0), sp(1, 0);
+        int &levmax = tri ? P.levmax_u : P.levmax_l;
+        levmax = 0;
+        for (int b = 0; b < nb; ++b) {
+            const int base = roff[b], cnt = roff[b + 1] - base;
+            lev.assign(cnt, 0);
+            order.clear();
+            slots.clear();
+            step.clear();
+            // rows in dependency order: the row's entries by level, the last W in its own
+            // slot; a row of further slots waits until each can precede the next
+            for (int q = 0; q < cnt; ++q) {
+                const int r = tri ? cnt - 1 - q : q, i = base + r;
+                const int k0 = tri ? bdiag[i] + 1 : bia[i], n = (tri ? bia[i + 1] : bdiag[i]) - k0;
+                const int f = (int)order.size();
+                for (int k = 0; k < n; ++k) order.push_back(k0 + k);
+                int l = 0;
+                if (n > W)
+                    std::stable_sort(order.begin() + f, order.end(), [&](int x, int y) { return lev[bja[x]] < lev[bja[y]]; });
+                for (int k = 0; k < n; ++k) l = std::max(l, lev[bja[order[f + k]]] + 1);
+                for (int j = 1, e = n - W; e > 0; ++j, e -= W) l = std::max(l, lev[bja[order[f + e - 1]]] + 1 + j);
+                lev[r] = l;
+                slots.push_back({r, std::min(n, W), f + std::max(0, n - W), true});
+                step.push_back(l);
+            }
+            int nl = 0;
+            for (int s : step) nl = std::max(nl, s + 1);
+            count.assign(nl + 1, 0);
+            for (int s : step) ++count[s];
+            for (int q = 0; q < cnt; ++q) {  // the further slots, where there is room
+                const Slot m = slots[q];
+                const int r = m.row, i = base + r, n = tri ? bia[i + 1] - bdiag[i] - 1 : bdiag[i] - bia[i];
+                int hi = step[q];
+                for (int e = n - W; e > 0; e -= W) {
+                    const int f0 = m.first - (n - W) + std::max(0, e - W), ne = std::min(e, W);
+                    // not before its rows are final, nor so early that the slots before it are
+                    int lo = lev[bja[order[f0 + ne - 1]]] + 1;
+                    for (int k = e - W, j = 1; k > 0; k -= W, ++j)
+                        lo = std::max(lo, lev[bja[order[m.first - (n - W) + k - 1]]] + 1 + j);
+                    int best = hi - 1;  // the latest level with a free lane in its last piece
+                    for (int s = hi - 1; s >= lo; --s)
+                        if (count[s] % 64) { best = s; break; }
+                    hi = best;
+                    slots.push_back({r, ne, f0, false});
+                    step.push_back(hi);
+                    ++count[hi];
+                }
+            }
+            // level by level, pieces of at most 64
+            at.assign(nl + 1, 0);
+            for (int l = 0; l < nl; ++l) at[l + 1] = at[l] + count[l];
+            const int s0 = (int)srow.size();
+            for (int l = 0; l < nl; ++l)
+                for (int p = at[l]; p < at[l + 1]; p += 64) sp.push_back(s0 + std::min(p + 64, at[l + 1]));
+            sb[b + 1] = (int)sp.size() - 1;
+            levmax = std::max(levmax, sb[b + 1] - sb[b]);
+            srow.resize(s0 + slots.size());
+            col.resize((size_t)srow.size() * (W / 2));
+            std::vector<int> by(slots.size());
+            for (size_t q = 0; q < slots.size(); ++q) {
+                const Slot &m = slots[q];
+                const int sl = s0 + at[step[q]]++;
+                by[q] = sl;
+                srow[sl] = (unsigned short)m.row;
+                unsigned short c[12];
+                for (int k = 0; k < W; ++k) c[k] = k < m.n ? bja[order[m.first + k]] : (unsigned short)m.row;
+                for (int k = 0; k < W; k += 2) col[(size_t)sl * (W / 2) + k / 2] = c[k] | (unsigned)c[k + 1] << 16;
+                if (m.main) (tri ? out[base + m.row].y : out[base + m.row].x) = (unsigned)(sl - s0);
+            }
+            // rows of several slots in either triangle: each entry's place
+            for (size_t q = 0; q < slots.size(); ++q) {
+                const Slot &m = slots[q];
+                const int i = base + m.row, len = bia[i + 1] - bia[i];
+                const bool several = std::max(bdiag[i] - bia[i], bia[i + 1] - bdiag[i] - 1) > W;
+                if (!several) continue;
+                if (!out[i].w) {
+                    out[i].w = (unsigned)place.size() + 1;
+                    place.resize(place.size() + len, 0);
+                }
+                for (int k = 0; k < m.n; ++k)
+                    place[out[i].w - 1 + (order[m.first + k] - bia[i])] = (unsigned)((by[q] - s0) * W + k);
+            }
+        }
+        if ((tri ? P.col_u : P.col_l).upload(col.data(), col.size()) ||
+            (tri ? P.row_u : P.row_l).upload(srow.data(), srow.size()) ||
+            (tri ? P.lev_u : P.lev_l).upload(sb.data(), nb + 1) ||
+            (tri ? P.lptr_u : P.lptr_l).upload(sp.data(), sp.size()))
+            return -1;
+    }
+    {
+        std::vector<uint4> by(total);
+        for (int b = 0; b < nb; ++b)
+            for (int sl = roff[b]; sl < roff[b + 1]; ++sl) by[sl] = out[roff[b] + rows_l[sl]];
+        if (P.out.upload(by.data(), by.size()) || P.place.upload(place.data(), place.size())) return -1;
+    }
     return 0;
 }
 
@@ -2562,8 +2571,8 @@ static int build_bj(fvp_csr *A) {
         roff[b + 1] = roff[b] + cnt;
     }
     const int total = roff[nb];
-    std::vector<int> blev_l(nb + 1, 0), blev_u(nb + 1, 0), lptr_l(1, 0), lptr_u(1, 0);
-    std::vector<unsigned short> rows_l, rows_u;
+    std::vector<int> blev_l(nb + 1, 0), lptr_l(1, 0);
+    std::vector<unsigned short> rows_l(total);
     std::vector<int> lev;
     int maxnz = 0, maxrow = 0, maxrows = 0;
     for (int b = 0; b < nb; ++b) {
@@ -2571,36 +2580,23 @@ static int build_bj(fvp_csr *A) {
         maxrows = std::max(maxrows, cnt);
         maxnz = std::max(maxnz, bia[base + cnt] - bia[base]);
         for (int r = 0; r < cnt; ++r) maxrow = std::max(maxrow, bia[base + r + 1] - bia[base + r]);
+        // the factorisation's levels
         lev.assign(cnt, 0);
-        auto group = [&](bool lower, std::vector<int> &lptr, std::vector<unsigned short> &rows) {
-            int nl = 0;
-            if (lower) {
-                for (int r = 0; r < cnt; ++r) {
-                    int i = base + r, l = 0;
-                    for (int k = bia[i]; k < bdiag[i]; ++k) l = std::max(l, lev[bja[k]] + 1);
-                    lev[r] = l;
-                    nl = std::max(nl, l + 1);
-                }
-            } else {
-                for (int r = cnt - 1; r >= 0; --r) {
-                    int i = base + r, l = 0;
-                    for (int k = bdiag[i] + 1; k < bia[i + 1]; ++k) l = std::max(l, lev[bja[k]] + 1);
-                    lev[r] = l;
-                    nl = std::max(nl, l + 1);
-                }
-            }
-            std::vector<int> c(nl + 1, 0);
-            for (int r = 0; r < cnt; ++r) c[lev[r] + 1]++;
-            for (int l = 0; l < nl; ++l) c[l + 1] += c[l];
-            const int off = (int)rows.size();
-            rows.resize(off + cnt);
-            std::vector<int> fill(c.begin(), c.end() - 1);
-            for (int r = 0; r < cnt; ++r) rows[off + fill[lev[r]]++] = (unsigned short)r;
-            for (int l = 0; l < nl; ++l) lptr.push_back(off + c[l + 1]);
-            return nl;
-        };
-        blev_l[b + 1] = blev_l[b] + group(true, lptr_l, rows_l);
-        blev_u[b + 1] = blev_u[b] + group(false, lptr_u, rows_u);
+        int nl = 0;
+        for (int r = 0; r < cnt; ++r) {
+            const int i = base + r;
+            int l = 0;
+            for (int k = bia[i]; k < bdiag[i]; ++k) l = std::max(l, lev[bja[k]] + 1);
+            lev[r] = l;
+            nl = std::max(nl, l + 1);
+        }
+        std::vector<int> c(nl + 1, 0);
+        for (int r = 0; r < cnt; ++r) c[lev[r] + 1]++;
+        for (int l = 0; l < nl; ++l) c[l + 1] += c[l];
+        std::vector<int> fill(c.begin(), c.end() - 1);
+        for (int r = 0; r < cnt; ++r) rows_l[base + fill[lev[r]]++] = (unsigned short)r;
+        for (int l = 0; l < nl; ++l) lptr_l.push_back(base + c[l + 1]);
+        blev_l[b + 1] = blev_l[b] + nl;
     }
     if (maxrow > 64) { set_error("block-Jacobi ILU(0) supports rows of at most 64 block entries"); return -1; }
     if (maxnz > 65535) { set_error("block-Jacobi ILU(0): more than 65535 entries in one block"); return -1; }
@@ -2614,95 +2610,31 @@ static int build_bj(fvp_csr *A) {
     A->b_lu32.release();
     {
         // packed solve layout (see bj_solve)
-        std::vector<int> ovp(nb + 1, 0);
-        std::vector<long> ovpos;
-        std::vector<uint8_t> ovtri;
-        std::vector<uint4> out(total);  // by row at first, then by slot of L's level order
-        long ndiag = 0;
-        struct Tri {
-            std::vector<unsigned> meta;
-            std::vector<long> ebase;
-            std::vector<unsigned short> col;
-        } tr[2];
-        for (int t = 0; t < 2; ++t) tr[t].ebase.assign(nb + 1, 0);
-        int ovmax = 0;
-        for (int b = 0; b < nb; ++b) {
-            const int base = roff[b];
-            int nov = 0;
-            for (int tri = 0; tri < 2; ++tri) {
-                Tri &T = tr[tri];
-                const long eb = (long)T.col.size();
-                T.ebase[b] = eb;
-                const std::vector<int> &lptr = tri ? lptr_u : lptr_l;
-                const std::vector<int> &blev = tri ? blev_u : blev_l;
-                const std::vector<unsigned short> &rows = tri ? rows_u : rows_l;
-                for (int sl = lptr[blev[b]]; sl < lptr[blev[b + 1]]; ++sl) {
-                    const int r = rows[sl];
-                    const int i = base + r;
-                    const int k0 = tri ? bdiag[i] + 1 : bia[i], k1 = tri ? bia[i + 1] : bdiag[i];
-                    const int kn = k1 - k0;
-                    const long kl = (long)T.col.size() - eb;
-                    if (kl > 65535 || nov > 65535) {
-                        set_error("block-Jacobi ILU(0): more than 65535 entries in one block triangle");
-                        return -1;
-                    }
-                    T.meta.push_back((unsigned)kl | ((unsigned)nov << 16));
-                    T.meta.push_back((unsigned)r | ((unsigned)kn << 16));
-                    (tri ? out[i].y : out[i].x) = (unsigned)T.col.size();
-                    if (tri) out[i].z = (unsigned)ndiag++;
-                    for (int k = k0; k < k1; ++k) {
-                        if (k - k0 >= kBjRow) {
-                            ovpos.push_back((long)T.col.size());
-                            ovtri.push_back((uint8_t)tri);
-                            ++nov;
-                        }
-                        T.col.push_back(bja[k]);
-                    }
-                    if (kn & 1) T.col.push_back((unsigned short)r);
-                }
-            }
-            ovp[b + 1] = ovp[b] + nov;
-            ovmax = std::max(ovmax, nov);
+        long small = 0;
+        int longest = 0;
+        for (int i = 0; i < total; ++i) {
+            const int l = bdiag[i] - bia[i], u = bia[i + 1] - bdiag[i] - 1;
+            small += (l <= 4) + (u <= 4);
+            longest = std::max({longest, l, u});
         }
-        for (int t = 0; t < 2; ++t) {  // the last windows read up to kBjRow entries past the end
-            tr[t].ebase[nb] = (long)tr[t].col.size();
-            for (int k = 0; k < kBjRow; ++k) tr[t].col.push_back(0);
-        }
-        {
-            std::vector<uint4> by(total);
-            for (int b = 0; b < nb; ++b)
-                for (int sl = roff[b]; sl < roff[b + 1]; ++sl) by[sl] = out[roff[b] + rows_l[sl]];
-            if (factor_tables(A->fac, nb, roff, bia, bja, bdiag, rows_l, by, maxrow)) return -1;
-        }
-        // the solve's levels: each factor level cut into pieces of at most 32 slots (one per lane pair)
-        auto split = [&](const std::vector<int> &blev, const std::vector<int> &lptr, std::vector<int> &sb,
-                         std::vector<int> &sp, int &levmax) {
-            sb.assign(nb + 1, 0);
-            sp.assign(1, 0);
-            levmax = 0;
+        const int win[2] = {small >= 9 * (2 * (long)total) / 10 ? 4 : 8, longest <= 4 ? 4 : longest <= 8 ? 8 : 12};
+        A->pack32 = win[1] != win[0];
+        for (int f32 = 0; f32 <= A->pack32; ++f32)
+            if (build_pack(A->pack[f32], win[f32], nb, roff, bia, bja, bdiag, rows_l)) return -1;
+        if (factor_tables(A->fac, nb, roff, bia, bja, bdiag, rows_l, maxrow)) return -1;
+        // the factor's levels in pieces of one slot per lane group
+        for (int w = 0; w < 2; ++w) {
+            const int width = (w ? 1024 : 512) / kBjGroup;
+            std::vector<int> fb(nb + 1, 0), fp(1, 0);
+            A->f_levmax[w] = 0;
             for (int b = 0; b < nb; ++b) {
-                for (int l = blev[b]; l < blev[b + 1]; ++l)
-                    for (int p = lptr[l]; p < lptr[l + 1]; p += 32) sp.push_back(std::min(p + 32, lptr[l + 1]));
-                sb[b + 1] = (int)sp.size() - 1;
-                levmax = std::max(levmax, sb[b + 1] - sb[b]);
+                for (int l = blev_l[b]; l < blev_l[b + 1]; ++l)
+                    for (int p = lptr_l[l]; p < lptr_l[l + 1]; p += width) fp.push_back(std::min(p + width, lptr_l[l + 1]));
+                fb[b + 1] = (int)fp.size() - 1;
+                A->f_levmax[w] = std::max(A->f_levmax[w], fb[b + 1] - fb[b]);
             }
-        };
-        std::vector<int> sbl, spl, sbu, spu;
-        split(blev_l, lptr_l, sbl, spl, A->s_levmax_l);
-        split(blev_u, lptr_u, sbu, spu, A->s_levmax_u);
-        A->s_maxslots = 0;
-        for (int b = 0; b < nb; ++b)
-            A->s_maxslots = std::max({A->s_maxslots, spl[sbl[b + 1]] - spl[sbl[b]], spu[sbu[b + 1]] - spu[sbu[b]]});
-        if (A->meta_l.upload(tr[0].meta.data(), tr[0].meta.size()) ||
-            A->meta_u.upload(tr[1].meta.data(), tr[1].meta.size()) ||
-            A->ebase_l.upload(tr[0].ebase.data(), nb + 1) || A->ebase_u.upload(tr[1].ebase.data(), nb + 1) ||
-            A->col_l.upload(tr[0].col.data(), tr[0].col.size()) || A->col_u.upload(tr[1].col.data(), tr[1].col.size()) ||
-            A->ov_ptr.upload(ovp.data(), nb + 1) ||
-            A->ov_pos.upload(ovpos.data(), ovpos.size()) || A->ov_tri.upload(ovtri.data(), ovtri.size()) ||
-            A->s_lev_l.upload(sbl.data(), nb + 1) || A->s_lev_u.upload(sbu.data(), nb + 1) ||
-            A->s_lptr_l.upload(spl.data(), spl.size()) || A->s_lptr_u.upload(spu.data(), spu.size()))
-            return -1;
-        A->ov_max = ovmax;
+            if (A->f_lev[w].upload(fb.data(), nb + 1) || A->f_lptr[w].upload(fp.data(), fp.size())) return -1;
+        }
         A->val_l.release(); A->val_u.release(); A->dinv.release();
         A->val32_l.release(); A->val32_u.release(); A->dinv32.release();
     }
@@ -2712,11 +2644,13 @@ static int build_bj(fvp_csr *A) {
         A->lds_max = 64 * 1024;
     // per-kernel attributes (shared by every matrix): allow the device maximum;
     // each build checks its own block against it
-    for (const void *f : {(const void *)bj_factor<double, 1, true>, (const void *)bj_factor<double, 2, true>,
-                          (const void *)bj_factor<double, 4, true>, (const void *)bj_factor<float, 1, true>,
-                          (const void *)bj_factor<float, 2, true>, (const void *)bj_factor<float, 4, true>,
-                          (const void *)bj_solve<double, false>, (const void *)bj_solve<double, true>,
-                          (const void *)bj_solve<float, false>, (const void *)bj_solve<float, true>})
+    for (const void *f : {(const void *)bj_factor<double, 1, true, 512>, (const void *)bj_factor<double, 1, true, 1024>,
+                          (const void *)bj_factor<double, 2, true, 512>, (const void *)bj_factor<double, 4, true, 512>,
+                          (const void *)bj_factor<float, 1, true, 512>, (const void *)bj_factor<float, 1, true, 1024>,
+                          (const void *)bj_factor<float, 2, true, 512>, (const void *)bj_factor<float, 4, true, 512>,
+                          (const void *)bj_solve<double, 4>, (const void *)bj_solve<double, 8>,
+                          (const void *)bj_solve<float, 4>, (const void *)bj_solve<float, 8>,
+                          (const void *)bj_solve<float, 12>})
         (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, A->lds_max);
     A->nblk = nb;
     A->bj = true;
@@ -2910,26 +2844,25 @@ struct FactorArgs {
     const FactorTab *tab;
     const int *lev, *lptr;
     int *flag;
+    FacOut out;
+    const uint4 *sout;
     size_t staged;
     int npmax;  // most pieces of one block (staged form)
+    int threads;
 };
-template <typename T, int NC>
+template <typename T, int NC, int TH>
 static void bj_factor_launch_nc(hipStream_t s, const FactorArgs &f, T *lu, T *vl, T *vu, T *vd) {
     const FactorTab &t = *f.tab;
-    if (f.staged)
-        bj_factor<T, NC, true><<<f.nblk, kBjFactorThreads, f.staged, s>>>(f.roff, f.ia, f.src, f.a, t.slot.p, t.out.p,
-                                                                          t.piv.p, t.off.p, f.lev, f.lptr, lu, vl, vu,
-                                                                          vd, f.flag, f.npmax);
-    else
-        bj_factor<T, NC, false><<<f.nblk, kBjFactorThreads, 0, s>>>(f.roff, f.ia, f.src, f.a, t.slot.p, t.out.p,
-                                                                    t.piv.p, t.off.p, f.lev, f.lptr, lu, vl, vu, vd,
-                                                                    f.flag, 0);
+    const auto kernel = f.staged ? bj_factor<T, NC, true, TH> : bj_factor<T, NC, false, TH>;
+    kernel<<<f.nblk, TH, f.staged, s>>>(f.roff, f.ia, f.src, f.a, t.slot.p, f.sout, t.piv.p, t.off.p, f.lev, f.lptr, lu,
+                                        vl, vu, vd, f.out, f.flag, f.npmax);
 }
 template <typename T>
 static void bj_factor_launch(hipStream_t s, const FactorArgs &f, T *lu, T *vl, T *vu, T *vd) {
-    if (f.tab->nc == 1) bj_factor_launch_nc<T, 1>(s, f, lu, vl, vu, vd);
-    else if (f.tab->nc == 2) bj_factor_launch_nc<T, 2>(s, f, lu, vl, vu, vd);
-    else bj_factor_launch_nc<T, 4>(s, f, lu, vl, vu, vd);
+    if (f.tab->nc == 1 && f.threads == 1024) bj_factor_launch_nc<T, 1, 1024>(s, f, lu, vl, vu, vd);
+    else if (f.tab->nc == 1) bj_factor_launch_nc<T, 1, 512>(s, f, lu, vl, vu, vd);
+    else if (f.tab->nc == 2) bj_factor_launch_nc<T, 2, 512>(s, f, lu, vl, vu, vd);
+    else bj_factor_launch_nc<T, 4, 512>(s, f, lu, vl, vu, vd);
 }
 
 static int precon_build_impl(fvp_csr *A, int type) {
@@ -2960,20 +2893,27 @@ static int precon_build_impl(fvp_csr *A, int type) {
         // against in place: 67 / 75 us (276 blocks of 512 rows, FP32), 200 / 307
         // (1024 with one overlap layer, FP32), 323 / 365 (the same, FP64), 517 / 549
         // (1000 blocks of 1024 with overlap, FP32); at worst 91 / 83 (276 blocks of
-        // 512, FP64).  FVP_BJ_FACTOR_MODE 0 / 1 forces in place / staged where it
-        // fits the workgroup: a tuning and test knob.
-        const size_t staged = (size_t)A->b_maxnz * vb + 8 * (size_t)((A->s_levmax_l + 2) / 2);
+        // 512, FP64), all with 512 threads.  FVP_BJ_FACTOR_MODE 0 / 1 forces in place /
+        // staged where it fits the workgroup: a tuning and test knob.
+        const size_t staged = (size_t)A->b_maxnz * vb + 8 * (size_t)((A->f_levmax[0] + 2) / 2);
         bool stage = staged <= (size_t)A->lds_max && !(A->fac.nc == 4 && vb == 8);
         if (const char *e = getenv("FVP_BJ_FACTOR_MODE")) stage = atoi(e) > 0 && staged <= (size_t)A->lds_max;
         A->factor_mode = stage ? 1 : 0;
-        const FactorArgs fa{A->nblk, A->b_roff.p, A->b_ia.p, A->b_src.p, A->a.p, &A->fac, A->s_lev_l.p,
-                            A->s_lptr_l.p, A->flag.p, stage ? staged : 0, A->s_levmax_l};
-        const size_t nl = A->col_l.n, nu = A->col_u.n, nd = A->fac.slot.n;
+        const int th = bj_factor_threads(A->fac.nc, A->nblk, stage ? staged : 0, A->lds_max, A->f_levmax[0], A->f_levmax[1]);
+        const int w = th == 1024;
+        const BjPack &P = A->pack[vb == 4 ? A->pack32 : 0];
+        const FactorArgs fa{A->nblk, A->b_roff.p, A->b_ia.p, A->b_src.p, A->a.p, &A->fac, A->f_lev[w].p,
+                            A->f_lptr[w].p, A->flag.p,
+                            FacOut{(unsigned)P.win, P.place.p, P.lev_l.p, P.lptr_l.p, P.lev_u.p, P.lptr_u.p},
+                            P.out.p, stage ? staged : 0, A->f_levmax[w], th};
+        const size_t nl = P.row_l.n * P.win, nu = P.row_u.n * P.win, nd = P.row_u.n;
         // the packed arrays' padding stays zero: only the factor's entries are written
         auto ensure = [&](auto &lu, auto &vl, auto &vu, auto &vd) {
             if (!lu.p && lu.alloc(A->b_src.n)) return -1;
             if (vl.p) return 0;
-            if (vl.alloc(nl) || vu.alloc(nu) || vd.alloc(nd)) return -1;
+            // ... and a slot without a diagonal keeps d = 1
+            const std::vector<std::decay_t<decltype(*vd.p)>> ones(nd, 1);
+            if (vl.alloc(nl) || vu.alloc(nu) || vd.upload(ones.data(), nd)) return -1;
             FVP_HIP(hipMemsetAsync(vl.p, 0, sizeof(*vl.p) * nl, s));
             FVP_HIP(hipMemsetAsync(vu.p, 0, sizeof(*vu.p) * nu, s));
             return 0;
@@ -3006,7 +2946,8 @@ static int precon_build_impl(fvp_csr *A, int type) {
             const int *fp = A->o_fptr.p;
             double *vl = A->otri[0].val.p, *vu = A->otri[1].val.p;
             bj_factor_launch<double>(s, FactorArgs{1, fp, A->ia.p, nullptr, nullptr, &A->ofac, fp + 2, fp + 4,
-                                                   A->flag.p, 0, 0},
+                                                   A->flag.p, FacOut{(unsigned)A->o_win, nullptr, nullptr, nullptr, nullptr, nullptr},
+                                                   A->ofac.out.p, 0, 0, A->o_fthreads},
                                      A->lu.p, vl, vu, vu + (size_t)n * A->o_win);
         }
         for (size_t l = 0; !A->one && l + 1 < A->lptr_h.size(); ++l) {
@@ -3063,26 +3004,23 @@ static int precon_apply_impl(fvp_csr *A, const double *x, double *y, const doubl
     case FVP_PRECON_BJILU0_F32: {
         const bool f64 = A->ptype == FVP_PRECON_BJILU0;
         const size_t ts = f64 ? sizeof(double) : sizeof(float);
-        size_t lds = bj_solve_lds(ts, A->b_maxrows, A->ov_max, A->s_levmax_l, A->s_levmax_u, A->s_maxslots);
-        const bool ovg = lds > (size_t)A->lds_max;  // overflow lists too long for the LDS: read them in memory
-        if (ovg) lds = bj_solve_lds(ts, A->b_maxrows, 0, A->s_levmax_l, A->s_levmax_u, A->s_maxslots);
+        const BjPack &P = A->pack[f64 ? 0 : A->pack32];
+        const size_t lds = bj_solve_lds(ts, A->b_maxrows, P.levmax_l, P.levmax_u);
         if (lds > (size_t)A->lds_max) {
             set_error("block-Jacobi ILU(0): a block's solution does not fit the LDS");
             return -1;
         }
-        const uint2 *ml = reinterpret_cast<const uint2 *>(A->meta_l.p), *mu = reinterpret_cast<const uint2 *>(A->meta_u.p);
-#define FVP_BJ_SOLVE(TT, OV, VL, VU, DI)                                                                          \
-    bj_solve<TT, OV><<<A->nblk, 64, lds, s>>>(A->b_roff.p, A->b_rowid.p, A->b_own.p, A->s_lev_l.p, A->s_lptr_l.p, \
-                                              ml, A->ebase_l.p, VL, A->col_l.p, A->s_lev_u.p, A->s_lptr_u.p, mu, \
-                                              A->ebase_u.p, VU, A->col_u.p, DI, A->ov_ptr.p, A->ov_pos.p,         \
-                                              A->ov_tri.p, A->b_maxrows, A->ov_max, A->s_levmax_l,       \
-                                              A->s_levmax_u, x, xdiv, y, yn2, A->skip)
+#define FVP_BJ_SOLVE(TT, W, VL, VU, DI)                                                                            \
+    bj_solve<TT, W><<<A->nblk, 64, lds, s>>>(A->b_roff.p, A->b_rowid.p, A->b_own.p, P.lev_l.p, P.lptr_l.p, VL,     \
+                                             P.col_l.p, P.row_l.p, P.lev_u.p, P.lptr_u.p, VU, P.col_u.p, P.row_u.p, \
+                                             DI, A->b_maxrows, x, xdiv, y, yn2, A->skip)
         if (f64) {
-            if (ovg) FVP_BJ_SOLVE(double, true, A->val_l.p, A->val_u.p, A->dinv.p);
-            else FVP_BJ_SOLVE(double, false, A->val_l.p, A->val_u.p, A->dinv.p);
+            if (P.win == 8) FVP_BJ_SOLVE(double, 8, A->val_l.p, A->val_u.p, A->dinv.p);
+            else FVP_BJ_SOLVE(double, 4, A->val_l.p, A->val_u.p, A->dinv.p);
         } else {
-            if (ovg) FVP_BJ_SOLVE(float, true, A->val32_l.p, A->val32_u.p, A->dinv32.p);
-            else FVP_BJ_SOLVE(float, false, A->val32_l.p, A->val32_u.p, A->dinv32.p);
+            if (P.win == 12) FVP_BJ_SOLVE(float, 12, A->val32_l.p, A->val32_u.p, A->dinv32.p);
+            else if (P.win == 8) FVP_BJ_SOLVE(float, 8, A->val32_l.p, A->val32_u.p, A->dinv32.p);
+            else FVP_BJ_SOLVE(float, 4, A->val32_l.p, A->val32_u.p, A->dinv32.p);
         }
 #undef FVP_BJ_SOLVE
         break;
@@ -3165,12 +3103,10 @@ extern "C" int fvp_csr_destroy(fvp_csr *A) {
     A->hflag.release();
     A->b_ia.release(); A->b_src.release(); A->b_lu.release(); A->b_lu32.release();
     A->b_roff.release(); A->b_rowid.release(); A->b_own.release(); A->b_zn2.release();
-    A->meta_l.release(); A->meta_u.release(); A->ebase_l.release(); A->ebase_u.release();
-    A->col_l.release(); A->col_u.release(); A->val_l.release();
+    A->pack[0].release(); A->pack[1].release(); A->val_l.release();
     A->val_u.release(); A->dinv.release(); A->val32_l.release(); A->val32_u.release(); A->dinv32.release();
     A->fac.release(); A->ofac.release(); A->otri[0].release(); A->otri[1].release(); A->o_fptr.release();
-    A->s_lev_l.release(); A->s_lev_u.release(); A->s_lptr_l.release(); A->s_lptr_u.release();
-    A->ov_ptr.release(); A->ov_pos.release(); A->ov_tri.release();
+    for (int w = 0; w < 2; ++w) { A->f_lev[w].release(); A->f_lptr[w].release(); }
     schur_free(A);
     if (A->own_stream) (void)hipStreamDestroy(A->own_stream);
     delete A;

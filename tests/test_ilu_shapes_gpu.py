@@ -42,6 +42,15 @@ def _grid(nx, ny, nz=1, diagonals=True):
     return sp.coo_matrix((np.ones(len(r)), (r, c)), shape=(i.size, i.size))
 
 
+def _hubs(n, first, count, width, extra=0):
+    """Rows first, first + 1, ... that couple to `width` rows before `first` each (all of one level, or a chain
+    with extra = 1): more entries of one level than a solve window holds."""
+    r = np.repeat(np.arange(first, first + count), width)
+    c = np.concatenate([np.arange(k % 3, k % 3 + width) for k in range(count)])
+    P = sp.coo_matrix((np.ones(len(r)), (r, c)), shape=(n, n))
+    return P + _band(n, 1) if extra else P
+
+
 SHAPES = {
     "one row": sp.coo_matrix((1, 1)),
     "diagonal": sp.coo_matrix((700, 700)),                 # a single level wider than a workgroup's pieces
@@ -50,6 +59,8 @@ SHAPES = {
     "row of 9 L entries": _band(130, 9),
     "row of 17 L entries": _band(90, 17),
     "rows of 63 entries": _band(140, 31),                  # four registers, 31 L entries
+    "rows with 30 entries of one level": _hubs(150, 40, 20, 30),
+    "a chain and rows of 20 entries": _hubs(700, 60, 7, 20, extra=1),  # windows of 4, a few rows of several
     "wide grid": _grid(97, 3, diagonals=False),
     "grid of 64-wide levels": _grid(65, 130),
     "box": _grid(13, 11, 9),
