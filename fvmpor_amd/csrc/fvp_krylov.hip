@@ -156,20 +156,50 @@ namespace fvp {
 constexpr int kThreads = 256;
 
 // ---- kernels ------------------------------------------------------------------
-template <int LANES>
+// y = alpha A x + beta y.  A workgroup's kGemvRows rows are one contiguous range of
+// entries: its threads load them entry by entry (whole lines, four values of x in flight
+// each) into the LDS, a chunk of 16 a row at a time, and four lanes to a row sum them
+// from there.  What bounds it is the latency of row pointer -> column -> x, then its
+// bytes (4.5 TB/s at 524 288 rows of 14.6).  Against eight lanes to a row straight from
+// memory: 191 771 rows of 14.6 11.3 -> 9.3 us, 524 288 of 14.6 26.9 -> 21.0, 600 000 of
+// 7 18.2 -> 17.0, 4 141 of 6.9 4.8 -> 4.0.  Rows per workgroup 32 / 64 / 128: 10.9 / 9.3 /
+// 9.1 us, 24.4 / 21.0 / 21.5, 24.1 / 17.0 / 17.0, 4.5 / 4.0 / 4.5.
+constexpr int kGemvRows = 64;
 __global__ void __launch_bounds__(256) csr_gemv_kernel(int n, const int *__restrict__ ia, const int *__restrict__ ja,
                                                        const double *__restrict__ a, double alpha,
                                                        const double *__restrict__ x, double beta,
                                                        double *__restrict__ y, const double *skip) {
+    constexpr int R = kGemvRows, L = 256 / R, U = R / 16, CH = 256 * U;
+    __shared__ double qa[CH], qx[CH];
     const double over = skip_word(skip);
-    int tid = blockIdx.x * blockDim.x + threadIdx.x;
-    int row = tid / LANES, lane = tid % LANES;
-    double s = 0.;
-    const int k0 = row < n ? ia[row] : 0, k1 = row < n ? ia[row + 1] : 0;
+    const int r0 = blockIdx.x * R, row = r0 + threadIdx.x / L, lane = threadIdx.x % L;
+    const int b0 = ia[r0], len = ia[min(n, r0 + R)] - b0;
+    const int k1 = (row < n ? ia[row + 1] : b0 + len) - b0;
+    int k = (row < n ? ia[row] : b0 + len) - b0 + lane;
     if (over != 0.) return;
-    for (int k = k0 + lane; k < k1; k += LANES) s += a[k] * x[ja[k]];
+    double s = 0.;
+    for (int c0 = 0; c0 < len; c0 += CH) {
+        int j[U];
+        double va[U], vx[U];
 #pragma unroll
-    for (int off = LANES / 2; off > 0; off >>= 1) s += __shfl_down(s, off, LANES);
+        for (int u = 0; u < U; ++u) {
+            const int e = b0 + min(c0 + 256 * u + (int)threadIdx.x, len - 1);
+            j[u] = ja[e];
+            va[u] = a[e];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) vx[u] = x[j[u]];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            qa[256 * u + threadIdx.x] = va[u];
+            qx[256 * u + threadIdx.x] = vx[u];
+        }
+        __syncthreads();
+        for (const int end = min(k1, c0 + CH); k < end; k += L) s += qa[k - c0] * qx[k - c0];
+        __syncthreads();
+    }
+#pragma unroll
+    for (int off = L / 2; off > 0; off >>= 1) s += __shfl_down(s, off, L);
     if (row < n && lane == 0) y[row] = beta == 0. ? alpha * s : alpha * s + beta * y[row];
 }
 
@@ -2215,9 +2245,8 @@ using namespace fvp;
 namespace fvp {
 
 static int csr_gemv_impl(fvp_csr *A, double alpha, const double *x, double beta, double *y) {
-    const int L = 8;
-    csr_gemv_kernel<L><<<nblk((long)A->n * L, 256), 256, 0, A->stream>>>(A->n, A->ia.p, A->ja.p, A->a.p, alpha, x,
-                                                                         beta, y, A->skip);
+    csr_gemv_kernel<<<nblk(A->n, kGemvRows), 256, 0, A->stream>>>(A->n, A->ia.p, A->ja.p, A->a.p, alpha, x, beta, y,
+                                                                 A->skip);
     FVP_HIP(hipGetLastError());
     return 0;
 }
