@@ -68,6 +68,8 @@ struct fvp_ctx {
     fvp::DevBuf<double> xyz;     // N x 3
     fvp::DevBuf<double> invV;    // 1 / CV volume
     fvp::DevBuf<uint8_t> zmask;  // bit z: node touches zone z
+    fvp::DevBuf<int> mznode;     // the nmz nodes that touch several zones, ascending
+    int nmz = 0;
     fvp::DevBuf<double> zw;      // nz x N SCV-volume fraction of zone z in CV i
     fvp::DevBuf<double> kr;      // nz x N relative permeability per (zone, node)
     fvp::DevBuf<double> cap;     // N capacity coefficient ahh

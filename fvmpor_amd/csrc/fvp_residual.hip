@@ -38,7 +38,7 @@ __device__ __forceinline__ double jv_scaled(const JvArgs &jv, int i, double d) {
 // ln x and e^x for vg_eval.  The van Genuchten pass is bound by FP64 instructions, and
 // the library's pair takes about 125 of them; these take 50, to 0.92 and 1.05 ulp
 // (no worse in k_r, S and dS/dh, whose errors come from the arguments' rounding).
-// 1 024 000 nodes: vg_kernel 33 us with the library's, 26 with these.
+// 1 024 000 nodes: vg_kernel 33 us with the library's, 24 to 26 with these.
 // ln: x = 2^k m with m in [sqrt(1/2), sqrt(2)), f = m - 1, s = f / (2 + f), and from
 // ln m = 2 atanh s = 2 s + s R, 2 s = f - s f: ln m = f - s (f - R), R = s^2 P(s^2),
 // P the Chebyshev fit of degree 6 to the atanh series (1.6e-18).  0 gives -inf, below NaN.
@@ -153,32 +153,34 @@ __device__ __forceinline__ double jv_sigma_block(const JvArgs &jv, double *red) 
     return jv_sigma_of(jv.psi_n2[0], b);
 }
 
-// One node per thread, the zone parameters in LDS.  Nodes of several zones are set
-// aside in a list and done together afterwards: a per-lane loop over the zones made
-// every wavefront pay for the most zones any of its nodes has (1 024 000 nodes, a
-// quarter of them at layer boundaries, with the library's ln and e^x: 41 us; 33 us with
-// the list).  Bound by FP64 instructions.
+// One node per thread, the zone parameters in LDS.  Nodes of several zones are left to
+// the first workgroups, which take them from a list (mznode, made at set-up): a per-lane
+// loop over the zones made every wavefront pay for the most zones any of its nodes has
+// (1 024 000 nodes, a quarter of them at layer boundaries: 41 us with the library's ln
+// and e^x; 33 us with a list of the workgroup's own nodes, 24 with the ln and e^x
+// above, 21 from one list, without the second phase of few lanes behind a barrier).
+// Bound by FP64 instructions and the latency around them.
 // JV with jv.np > 0: every workgroup reduces the np partials of ||v||^2 in the
 // fixed order of jv_sigma_n2 (the same sigma bit for bit) and workgroup 0
 // stores sigma for the finalisation, so no launch of its own is needed.
 template <bool JV>
-__global__ void __launch_bounds__(256) vg_kernel(int N, ZoneTable zt, double rho0, const double *__restrict__ psi,
+__global__ void __launch_bounds__(256) vg_kernel(int N, int nmz, const int *__restrict__ mznode, ZoneTable zt,
+                                                 double rho0, const double *__restrict__ psi,
                                                  const uint8_t *__restrict__ zmask, const double *__restrict__ zw,
                                                  double *__restrict__ kr, double *__restrict__ cap, JvArgs jv,
                                                  double *__restrict__ nrec) {
     __shared__ double zp[kMaxZones * 10];
     __shared__ double red[4];
-    __shared__ int nlist;
-    __shared__ unsigned char list[256];
-    __shared__ double hlist[256];
-    if (threadIdx.x == 0) nlist = 0;
     if (threadIdx.x < 10 * zt.nz) zp[threadIdx.x] = zt.p[threadIdx.x / 10][threadIdx.x % 10];
     // the node's own inputs are loaded first: their latency overlaps sigma's reduction
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool live = i < N;
+    const int mzb = (nmz + 255) / 256;
+    const bool several = (int)blockIdx.x < mzb;
+    int i = ((int)blockIdx.x - (several ? 0 : mzb)) * 256 + threadIdx.x;
+    bool live = i < (several ? nmz : N);
+    if (several) i = live ? mznode[i] : 0;
     double h = live ? psi[i] : 0.;
     const double vi = JV && live ? jv.v[i] : 0.;
-    unsigned m = live ? zmask[i] : 0u;
+    const unsigned m = live ? zmask[i] : 0u;
     double sg = 0.;
     if (JV && jv.np > 0) {
         const double sigma = jv_sigma_block(jv, red);  // ends with a barrier, so the zone table is in place
@@ -192,28 +194,12 @@ __global__ void __launch_bounds__(256) vg_kernel(int N, ZoneTable zt, double rho
         __syncthreads();
         if (JV) sg = jv.sig[0];
     }
+    if (!live || (!several && (m & (m - 1)))) return;
     if (JV) h += sg * vi;
-    auto evaluate = [&](int node, double hn, unsigned mn) {
-        cap[node] = vg_node<true>(N, node, hn, mn, zp, zw, rho0,
-                                  [&](int z, int, double k) { kr[(size_t)z * N + node] = k; });
-    };
-    if (live) {
-        // the head of the node record the element kernel gathers (x, y, z are
-        // written once at set-up)
-        if (nrec) nrec[4 * (size_t)i + 3] = h;
-        if (m & (m - 1)) {
-            const int k = atomicAdd(&nlist, 1);
-            list[k] = (unsigned char)threadIdx.x;
-            hlist[k] = h;
-        } else {
-            evaluate(i, h, m);
-        }
-    }
-    __syncthreads();
-    if ((int)threadIdx.x < nlist) {
-        const int node = blockIdx.x * blockDim.x + list[threadIdx.x];
-        evaluate(node, hlist[threadIdx.x], zmask[node]);
-    }
+    // the head of the node record the element kernel gathers (x, y, z are
+    // written once at set-up)
+    if (nrec) nrec[4 * (size_t)i + 3] = h;
+    cap[i] = vg_node<true>(N, i, h, m, zp, zw, rho0, [&](int z, int, double k) { kr[(size_t)z * N + i] = k; });
 }
 
 __device__ __forceinline__ void load_pt(const double *__restrict__ xyz, int i, double &x, double &y, double &z) {
@@ -644,7 +630,7 @@ __device__ __forceinline__ void upwind_fluxes(const NodeVals<DIM> &nv, const dou
 // halo nodes are evaluated again); otherwise k_r comes from vg_kernel.  Nodes of
 // several zones are set aside in a list and done afterwards, as there.
 // Bound by the LDS (268 cycles per 64 elements: 16-byte record reads and four sums)
-// and the phases' latency.  1 024 000 nodes, 512-node tiles: 76 us, with vg_kernel 26
+// and the phases' latency.  1 024 000 nodes, 512-node tiles: 76 us, with vg_kernel 21
 // and owner_imports 8 us more.  Gathering from memory through the L1 (owner_kernel,
 // kept for windows that do not fit) with a finalisation of its own: 120 + 41 + 33 us.
 constexpr int kRecBits = 14, kRecRanks = 4;
@@ -1117,6 +1103,12 @@ __global__ void mask_kernel(int T, const int *__restrict__ eedge, const uint8_t 
 }
 
 static inline int blocks(long n, int bs) { return (int)((n + bs - 1) / bs); }
+
+template <bool JV>
+static void launch_vg(fvp_ctx *c, const double *psi, const JvArgs &jv, double *nrec) {
+    vg_kernel<JV><<<blocks(c->nmz, 256) + blocks(c->N, 256), 256, 0, c->stream>>>(
+        c->N, c->nmz, c->mznode.p, c->zt, c->rho0, psi, c->zmask.p, c->zw.p, c->kr.p, c->cap.p, jv, nrec);
+}
 
 // Dynamic LDS of owner_lds for windows of wmax nodes with up to nr zones per node
 // (0: not used): the records have to fit the elements' 14 + 2 bits and half of the LDS
@@ -1608,11 +1600,9 @@ int residual_impl(fvp_ctx *c, double t, const double *psi, const double *psip, d
     const bool fused = c->owner_win && c->owner_vg && !averaging;  // the element kernel does the van Genuchten pass
     double *const nrec = c->rvariant == FVP_RESIDUAL_OWNER && !c->owner_win ? c->nrec.p : nullptr;
     if (jv && !fused)
-        vg_kernel<true><<<blocks(N, 256), 256, 0, s>>>(N, c->zt, c->rho0, psi, c->zmask.p, c->zw.p, c->kr.p,
-                                                        c->cap.p, *jv, nrec);
+        launch_vg<true>(c, psi, *jv, nrec);
     else if (!fused)
-        vg_kernel<false><<<blocks(N, 256), 256, 0, s>>>(N, c->zt, c->rho0, psi, c->zmask.p, c->zw.p, c->kr.p,
-                                                         c->cap.p, JvArgs(), nrec);
+        launch_vg<false>(c, psi, JvArgs(), nrec);
     if (!averaging) {
         // tiled paths (element fluxes with the boundary fluxes, then the finalisation)
         const JvArgs none;
@@ -1732,8 +1722,7 @@ extern "C" int fvp_begin_step(fvp_ctx *c, double t, const double *psi, const dou
     (void)t; (void)psip;
     const int N = c->N, T = c->T;
     // k_r at the state, then the averaged-weight face fluxes summed per edge
-    vg_kernel<false><<<blocks(N, 256), 256, 0, s>>>(N, c->zt, c->rho0, psi, c->zmask.p, c->zw.p, c->kr.p, c->cap.p,
-                                                     JvArgs(), c->nrec.p);
+    launch_vg<false>(c, psi, JvArgs(), c->nrec.p);
     const auto faces = c->dim == 3 ? face_flux_kernel<3> : face_flux_kernel<2>;
     faces<<<blocks(T, 256), 256, 0, s>>>(T, N, c->zt, c->conn.p, c->ezone.p, c->kmul.p, c->eorient.p, c->nrec.p,
                                          c->kr.p, c->qface.p);

@@ -459,8 +459,12 @@ extern "C" int fvp_create(const fvp_problem *p, int device, fvp_ctx **out) {
         }
     }
     if (c->nz > 8) { set_error("more than 8 zones need a wider zone mask"); return fail(); }
+    std::vector<int> several;
+    for (int i = 0; i < N; ++i)
+        if (zmask[i] & (zmask[i] - 1)) several.push_back(i);
+    c->nmz = (int)several.size();
     if (c->invV.upload(invV.data(), N) || c->zw.upload(zw.data(), zw.size()) ||
-        c->zmask.upload(zmask.data(), N))
+        c->zmask.upload(zmask.data(), N) || c->mznode.upload(several.data(), several.size()))
         return fail();
     if (c->kr.alloc((size_t)c->nz * N) || c->cap.alloc(N) || c->acc.alloc(N)) return fail();
     {
@@ -670,7 +674,7 @@ extern "C" int fvp_destroy(fvp_ctx *c) {
     jac_free(c);
     prof_release(c);
     c->conn.release(); c->ezone.release(); c->emask.release(); c->eorient.release(); c->kmul.release();
-    c->xyz.release(); c->invV.release(); c->zmask.release(); c->zw.release(); c->kr.release();
+    c->xyz.release(); c->invV.release(); c->zmask.release(); c->mznode.release(); c->zw.release(); c->kr.release();
     c->cap.release(); c->nrec.release(); c->acc.release(); c->bnode.release(); c->bval.release(); c->dnode.release();
     c->dval.release(); c->t_wptr.release(); c->t_whalo.release(); c->t_vptr.release(); c->t_lconn.release();
     c->t_tz.release(); c->t_eptr.release(); c->t_hptr.release(); c->t_hlist.release(); c->t_bptr.release();
