@@ -1228,53 +1228,47 @@ static void launch_tile(fvp_ctx *c, const double *psi, const double *psip, doubl
 // increment, and what the elements gather of them: per zone and node one 16-byte
 // record, {V^-1, k_r, k_r moved, dk_r / shift} in FP32 or the two k_r in FP64; the
 // diagonal's capacity term -psi' a_hh(psi) moved with psi_i and psi'_i + c_j shift_i.
-// Nodes of several zones are set aside as in vg_kernel.  Bound by FP64 instructions
-// (two evaluations per node and zone).  141 000 nodes: 19 us, where five launches
-// (increments, base, sum, moved, capacity term) took 42, and the elements' four
-// 8-byte gathers per node become one of 16.
+// Nodes of several zones come first, from the list, as in vg_kernel.  Bound by FP64
+// instructions (two evaluations per node and zone) and the latency around them: a
+// workgroup's own list behind a barrier, and inputs loaded once the zones were known,
+// took 19 us on 141 000 nodes, this 13; five launches (increments, base, sum, moved,
+// capacity term) took 42, and the elements' four 8-byte gathers per node become one of 16.
 template <typename C>
-__global__ void __launch_bounds__(256) fd_nodes(int N, ZoneTable zt, double rho0, FdJacobian fd,
-                                                const uint8_t *__restrict__ zmask, const double *__restrict__ zw,
-                                                const double *__restrict__ invV, double *__restrict__ kr,
-                                                double *__restrict__ cap, double *__restrict__ nrec) {
+__global__ void __launch_bounds__(256) fd_nodes(int N, int nmz, const int *__restrict__ mznode, ZoneTable zt,
+                                                double rho0, FdJacobian fd, const uint8_t *__restrict__ zmask,
+                                                const double *__restrict__ zw, const double *__restrict__ invV,
+                                                double *__restrict__ kr, double *__restrict__ cap,
+                                                double *__restrict__ nrec) {
     __shared__ double zp[kMaxZones * 10];
-    __shared__ int nlist;
-    __shared__ unsigned char list[256];
-    if (threadIdx.x == 0) nlist = 0;
     if (threadIdx.x < 10 * zt.nz) zp[threadIdx.x] = zt.p[threadIdx.x / 10][threadIdx.x % 10];
-    const int i = blockIdx.x * 256 + threadIdx.x;
+    const int mzb = (nmz + 255) / 256;
+    const bool several = (int)blockIdx.x < mzb;
+    int g = ((int)blockIdx.x - (several ? 0 : mzb)) * 256 + threadIdx.x;
+    const bool live = g < (several ? nmz : N);
+    if (several) g = live ? mznode[g] : 0;
+    else if (!live) g = 0;
+    const unsigned m = zmask[g];
+    const double y = fd.psi[g], yp = fd.psip[g], ew = fd.ewt[g], iv = invV[g];
     __syncthreads();
-    auto evaluate = [&](int g, unsigned m, bool multi) {
-        const double y = fd.psi[g], yp = fd.psip[g];
-        const double sh = fd.eps * fmax(fabs(y), fmax(fabs(fd.h * yp), 1.0 / fd.ewt[g]));
-        const float w = (float)invV[g];
-        double one = 0.;
-        const double c0 = vg_node<true>(N, g, y, m, zp, zw, rho0, [&](int z, int, double k) {
-            one = k;
-            if (multi) kr[(size_t)z * N + g] = k;
-        });
-        const double c1 = vg_node<true>(N, g, y + sh, m, zp, zw, rho0, [&](int z, int, double k1) {
-            const double k0 = multi ? kr[(size_t)z * N + g] : one;
-            if constexpr (sizeof(C) == 4)
-                reinterpret_cast<float4 *>(fd.rec)[(size_t)z * N + g] = make_float4(w, (float)k0, (float)k1, (float)((k1 - k0) / sh));
-            else
-                reinterpret_cast<double2 *>(fd.rec)[(size_t)z * N + g] = make_double2(k0, k1);
-        });
-        cap[g] = c0;
-        fd.dterm[g] = ((yp + fd.cj * sh) * c1 - yp * c0) / sh;
-        fd.shift[g] = sh;
-        nrec[4 * (size_t)g + 3] = y;
-    };
-    if (i < N) {
-        const unsigned m = zmask[i];
-        if (m & (m - 1)) list[atomicAdd(&nlist, 1)] = (unsigned char)threadIdx.x;
-        else evaluate(i, m, false);
-    }
-    __syncthreads();
-    if ((int)threadIdx.x < nlist) {
-        const int g = blockIdx.x * 256 + list[threadIdx.x];
-        evaluate(g, zmask[g], true);
-    }
+    if (!live || (!several && (m & (m - 1)))) return;
+    const double sh = fd.eps * fmax(fabs(y), fmax(fabs(fd.h * yp), 1.0 / ew));
+    const float w = (float)iv;
+    double one = 0.;
+    const double c0 = vg_node<true>(N, g, y, m, zp, zw, rho0, [&](int z, int, double k) {
+        one = k;
+        if (several) kr[(size_t)z * N + g] = k;
+    });
+    const double c1 = vg_node<true>(N, g, y + sh, m, zp, zw, rho0, [&](int z, int, double k1) {
+        const double k0 = several ? kr[(size_t)z * N + g] : one;
+        if constexpr (sizeof(C) == 4)
+            reinterpret_cast<float4 *>(fd.rec)[(size_t)z * N + g] = make_float4(w, (float)k0, (float)k1, (float)((k1 - k0) / sh));
+        else
+            reinterpret_cast<double2 *>(fd.rec)[(size_t)z * N + g] = make_double2(k0, k1);
+    });
+    cap[g] = c0;
+    fd.dterm[g] = ((yp + fd.cj * sh) * c1 - yp * c0) / sh;
+    fd.shift[g] = sh;
+    nrec[4 * (size_t)g + 3] = y;
 }
 
 // node values of an element from the packed records (x, y, z, head: two 16-byte loads)
@@ -1557,8 +1551,9 @@ template <typename C>
 static void fd_launch(fvp_ctx *c, const FdJacobian &fd) {
     hipStream_t s = c->stream;
     const int N = c->N, T = c->T;
-    fd_nodes<C><<<blocks(N, 256), 256, 0, s>>>(N, c->zt, c->rho0, fd, c->zmask.p, c->zw.p, c->invV.p, c->kr.p, c->cap.p,
-                                              c->nrec.p);
+    fd_nodes<C><<<blocks(c->nmz, 256) + blocks(N, 256), 256, 0, s>>>(N, c->nmz, c->mznode.p, c->zt, c->rho0, fd,
+                                                                    c->zmask.p, c->zw.p, c->invV.p, c->kr.p, c->cap.p,
+                                                                    c->nrec.p);
     const int4 *conn = (const int4 *)c->conn.p;
     const uint8_t *ezone = c->ezone.p, *emask = c->emask.p;
     if constexpr (sizeof(C) == 4) {
