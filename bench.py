@@ -412,7 +412,7 @@ def main():
     # accumulates 8 B per node and streams conn, K, class, upwind bits per tet; the window kernel is the
     # whole residual but the van Genuchten pass
     kbytes = 48 * N + 26 * T if owner else bf
-    kname = "owner_kernel<3> (residual element fluxes)" if owner else "tile_lds_kernel<3> (residual)"
+    kname = "owner_lds<3> (residual element fluxes)" if owner else "tile_lds_kernel<3> (residual)"
     ek_avg_s = ek_ms / max(ek_n, 1) * 1e-3
     achieved = kbytes / ek_avg_s / 1e9
     traffic = measured_traffic(N, T, launch)

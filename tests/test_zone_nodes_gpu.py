@@ -75,3 +75,32 @@ def test_residual_and_jv(count):
         ctx.synchronize()
         assert _rel(F.cpu().numpy(), Fc, op.flux_scale()) <= TOL, tile
         assert np.abs(Jv.cpu().numpy() - Jc).max() <= 1e-6 * np.abs(Jc).max(), tile
+
+
+@pytest.mark.parametrize("count", [0, 255, 257, 500])
+def test_jacobian_forms_agree(count):
+    """The element-local Jacobian, whose node pass has the same list, against the coloured form: the bar of
+    test_jacobian_shapes_gpu.py, 1e-4 of a row's largest entry (the quotients' rounding noise)."""
+    import torch
+    from fvmpor_amd.lib import Context, JACOBIAN_COLOURED, JACOBIAN_ELEMENT, PRECON_JACOBI, PRECON_BJILU0_F32
+    prob = _problem(count)
+    ctx = Context(prob)
+    psi, psip = _state(prob, 3)
+    y, yp = (torch.tensor(a, device=device()) for a in (psi, psip))
+    F0, ewt = torch.empty_like(y), 1.0 / (1e-6 * y.abs() + 1e-6)
+    torch.cuda.synchronize()
+    ctx.begin_step(0.0, y, yp)
+    ctx.residual(0.0, y, yp, F0)
+    n, conn = prob.mesh.n_nodes, prob.mesh.conn.astype(np.int64)
+    key = np.unique(np.concatenate([conn[:, a] * n + conn[:, b] for a in range(3) for b in range(3)]))
+    J = ctx.jacobian()
+    vals = []
+    for mode, precon in ((JACOBIAN_COLOURED, PRECON_JACOBI), (JACOBIAN_ELEMENT, PRECON_JACOBI),
+                         (JACOBIAN_ELEMENT, PRECON_BJILU0_F32)):
+        ctx.set_jacobian_mode(mode)
+        assert ctx.precon_setup(0.0, 12.0, 0.05, y, yp, F0, ewt, precon) == 0
+        vals.append(J.get_values(len(key)))
+    rows, rowmax = key // n, np.zeros(n)
+    np.maximum.at(rowmax, rows, np.abs(vals[0]))
+    for v in vals[1:]:
+        assert (np.abs(v - vals[0]) / rowmax[rows]).max() < 1e-4
