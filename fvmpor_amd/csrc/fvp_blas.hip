@@ -25,6 +25,24 @@ __global__ void __launch_bounds__(kRedThreads) dot_partial(long n, const double 
     if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
+// the same for ||psi||^2 (part) and ||v||^2 (part + kRedBlocks) in one launch
+__global__ void __launch_bounds__(kRedThreads) norms_partial(long n, const double *__restrict__ psi,
+                                                            const double *__restrict__ v, double *__restrict__ part) {
+    __shared__ double lds[kRedThreads / 64];
+    double a = 0., b = 0.;
+    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
+        const double x = psi[i], y = v[i];
+        a += x * x;
+        b += y * y;
+    }
+    a = block_sum(a, lds);
+    b = block_sum(b, lds);
+    if (threadIdx.x == 0) {
+        part[blockIdx.x] = a;
+        part[kRedBlocks + blockIdx.x] = b;
+    }
+}
+
 // out[0] = sum of np partials (fixed order: deterministic)
 __global__ void __launch_bounds__(kRedThreads) sum_partials(int np, const double *__restrict__ part,
                                                            double *__restrict__ out) {
@@ -141,28 +159,29 @@ int jv_impl(fvp_ctx *c, double t, const double *psi, const double *psip, const d
     hipStream_t s = c->stream;
     const long N = c->N;
     double *part = c->red.p;  // [0, 512) psi partials, [512, 1024) v partials, [1024] sigma
-    // partials of ||v||^2 from the solve that wrote v: the fused residual
-    // kernels' van Genuchten pass forms sigma itself
-    const bool fold = psi_n2 && v_n2 && !c->averaging;
-    if (!fold && psi_n2 && v_n2) {
-        jv_sigma_n2<<<1, kRedThreads, 0, s>>>(v_count, psi_n2, v_n2, part + 2 * kRedBlocks);
-    } else if (!fold && psi_n2) {
+    const double *pv = part + kRedBlocks;
+    int np = kRedBlocks;
+    if (psi_n2 && v_n2) {  // from the solve that wrote v
+        pv = v_n2;
+        np = v_count;
+    } else if (psi_n2) {
         dot_partial<<<kRedBlocks, kRedThreads, 0, s>>>(N, v, v, part + kRedBlocks);
-        jv_sigma_n2<<<1, kRedThreads, 0, s>>>(kRedBlocks, psi_n2, part + kRedBlocks, part + 2 * kRedBlocks);
-    } else if (!fold) {
-        dot_partial<<<kRedBlocks, kRedThreads, 0, s>>>(N, v, v, part + kRedBlocks);
-        dot_partial<<<kRedBlocks, kRedThreads, 0, s>>>(N, psi, psi, part);
-        jv_sigma<<<1, kRedThreads, 0, s>>>(kRedBlocks, part, part + kRedBlocks, part + 2 * kRedBlocks);
+    } else {
+        norms_partial<<<kRedBlocks, kRedThreads, 0, s>>>(N, psi, v, part);
     }
     FVP_HIP(hipGetLastError());
-    if (!c->averaging) {  // perturbation and difference quotient fused into the residual kernels
+    if (!c->averaging) {
+        // perturbation and difference quotient fused into the residual kernels, the first
+        // of which forms sigma from the partials.  J v by itself, 515 747 nodes: 70.2
+        // us with a launch per norm and one for sigma, 68.5 so
         JvArgs jv;
         jv.v = v; jv.sig = part + 2 * kRedBlocks; jv.F0 = F0; jv.cj = c_j; jv.osc = osc; jv.skip = skip;
-        if (fold) {
-            jv.psi_n2 = psi_n2; jv.part_v = v_n2; jv.np = v_count; jv.sig_out = part + 2 * kRedBlocks;
-        }
+        jv.psi_n2 = psi_n2; jv.part_psi = psi_n2 ? nullptr : part; jv.part_v = pv; jv.np = np;
+        jv.sig_out = part + 2 * kRedBlocks;
         return residual_impl(c, t, psi, psip, Jv, 0, &jv);
     }
+    if (psi_n2) jv_sigma_n2<<<1, kRedThreads, 0, s>>>(np, psi_n2, pv, part + 2 * kRedBlocks);
+    else jv_sigma<<<1, kRedThreads, 0, s>>>(np, part, pv, part + 2 * kRedBlocks);
     jv_perturb<<<nblk(N, 256), 256, 0, s>>>(N, part + 2 * kRedBlocks, c_j, psi, psip, v, c->tmp1.p, c->tmp2.p);
     FVP_HIP(hipGetLastError());
     if (residual_impl(c, t, c->tmp1.p, c->tmp2.p, c->tmp3.p, c->averaging)) return -1;

@@ -143,10 +143,10 @@ struct JvArgs {
     const double *v = nullptr, *sig = nullptr, *F0 = nullptr;
     const double *osc = nullptr;  // optional: J v scaled row-wise by osc
     double cj = 0.;
-    // optional (np > 0): the van Genuchten pass forms sigma itself from
-    // ||psi||^2 (psi_n2) and np partials of ||v||^2 and writes it to sig_out
-    // (== sig) for the kernels after it
-    const double *psi_n2 = nullptr, *part_v = nullptr;
+    // optional (np > 0): the van Genuchten pass forms sigma itself from np partials
+    // of ||v||^2 and ||psi||^2 (psi_n2) or np partials of it (part_psi), and writes
+    // it to sig_out (== sig) for the kernels after it
+    const double *psi_n2 = nullptr, *part_psi = nullptr, *part_v = nullptr;
     double *sig_out = nullptr;
     int np = 0;
     const double *skip = nullptr;  // optional: a nonzero word ends the element kernels early

@@ -133,24 +133,42 @@ __device__ __forceinline__ double vg_node(int N, int i, double h, unsigned m, co
     return (phi * dSw + Ss * Sw) * rho0;
 }
 
-// The FD increment of J v from np partials of ||v||^2, in the fixed order of
-// jv_sigma_n2 (the same sigma bit for bit in every workgroup); red: one double
-// per wavefront.  Holds barriers; only thread 0's value is the increment.
+// The FD increment of J v from np partials of ||v||^2 and, where given, of ||psi||^2,
+// summed in the order of jv_sigma and jv_sigma_n2 (the same sigma bit for bit in every
+// workgroup and thread); red: eight doubles.  Holds one barrier (five, a block sum per
+// norm and a broadcast, took 17.1 us instead of 16.9 in vg_kernel, 515 747 nodes).
 __device__ __forceinline__ double jv_sigma_block(const JvArgs &jv, double *red) {
     // each lane's partials in order, four loads in flight at a time
-    double b = 0.;
     const int bd = 256;
-    if (threadIdx.x < bd)
-        for (int k0 = threadIdx.x; k0 < jv.np; k0 += 4 * bd) {
-            double q[4];
+    auto sum = [&](const double *part) {
+        double b = 0.;
+        if (threadIdx.x < bd)
+            for (int k0 = threadIdx.x; k0 < jv.np; k0 += 4 * bd) {
+                double q[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) q[u] = k0 + u * bd < jv.np ? jv.part_v[k0 + u * bd] : 0.;
+                for (int u = 0; u < 4; ++u) q[u] = k0 + u * bd < jv.np ? part[k0 + u * bd] : 0.;
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (k0 + u * bd < jv.np) b += q[u];
-        }
-    b = block_sum(b, red);
-    return jv_sigma_of(jv.psi_n2[0], b);
+                for (int u = 0; u < 4; ++u)
+                    if (k0 + u * bd < jv.np) b += q[u];
+            }
+        return b;
+    };
+    double b = sum(jv.part_v), a = jv.part_psi ? sum(jv.part_psi) : 0.;
+    b = wave_sum(b);
+    if (jv.part_psi) a = wave_sum(a);
+    const int waves = bd / 64, w = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0 && w < waves) {
+        red[w] = b;
+        red[waves + w] = a;
+    }
+    const double n2 = jv.part_psi ? 0. : jv.psi_n2[0];
+    __syncthreads();
+    b = a = 0.;
+    for (int k = 0; k < waves; ++k) {
+        b += red[k];
+        a += red[waves + k];
+    }
+    return jv_sigma_of(jv.part_psi ? a : n2, b);
 }
 
 // One node per thread, the zone parameters in LDS.  Nodes of several zones are left to
@@ -161,8 +179,9 @@ __device__ __forceinline__ double jv_sigma_block(const JvArgs &jv, double *red) 
 // above, 21 from one list, without the second phase of few lanes behind a barrier).
 // Bound by FP64 instructions and the latency around them.
 // JV with jv.np > 0: every workgroup reduces the np partials of ||v||^2 in the
-// fixed order of jv_sigma_n2 (the same sigma bit for bit) and workgroup 0
-// stores sigma for the finalisation, so no launch of its own is needed.
+// fixed order of jv_sigma_n2 (the same sigma bit for bit), those of ||psi||^2
+// too where they come as partials, and workgroup 0 stores sigma for the
+// finalisation, so no launch of its own is needed.
 template <bool JV>
 __global__ void __launch_bounds__(256) vg_kernel(int N, int nmz, const int *__restrict__ mznode, ZoneTable zt,
                                                  double rho0, const double *__restrict__ psi,
@@ -170,7 +189,7 @@ __global__ void __launch_bounds__(256) vg_kernel(int N, int nmz, const int *__re
                                                  double *__restrict__ kr, double *__restrict__ cap, JvArgs jv,
                                                  double *__restrict__ nrec) {
     __shared__ double zp[kMaxZones * 10];
-    __shared__ double red[4];
+    __shared__ double red[8];
     if (threadIdx.x < 10 * zt.nz) zp[threadIdx.x] = zt.p[threadIdx.x / 10][threadIdx.x % 10];
     // the node's own inputs are loaded first: their latency overlaps sigma's reduction
     const int mzb = (nmz + 255) / 256;
@@ -183,13 +202,8 @@ __global__ void __launch_bounds__(256) vg_kernel(int N, int nmz, const int *__re
     const unsigned m = live ? zmask[i] : 0u;
     double sg = 0.;
     if (JV && jv.np > 0) {
-        const double sigma = jv_sigma_block(jv, red);  // ends with a barrier, so the zone table is in place
-        if (threadIdx.x == 0) {
-            red[0] = sigma;
-            if (blockIdx.x == 0) jv.sig_out[0] = sigma;
-        }
-        __syncthreads();
-        sg = red[0];
+        sg = jv_sigma_block(jv, red);  // holds a barrier, so the zone table is in place
+        if (threadIdx.x == 0 && blockIdx.x == 0) jv.sig_out[0] = sg;
     } else {
         __syncthreads();
         if (JV) sg = jv.sig[0];
@@ -670,13 +684,8 @@ __global__ void __launch_bounds__(TH) owner_lds(
     if (threadIdx.x == 0) nlist = 0;
     double sig = 0.;
     if (JV && VG && jv.np > 0) {
-        const double sigma = jv_sigma_block(jv, red);
-        if (threadIdx.x == 0) {
-            red[0] = sigma;
-            if (blockIdx.x == 0) jv.sig_out[0] = sigma;
-        }
-        __syncthreads();
-        sig = red[0];
+        sig = jv_sigma_block(jv, red);  // holds a barrier
+        if (threadIdx.x == 0 && blockIdx.x == 0) jv.sig_out[0] = sig;
     } else {
         __syncthreads();  // the zone tables
         if (JV) sig = jv.sig[0];
