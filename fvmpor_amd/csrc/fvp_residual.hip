@@ -41,7 +41,9 @@ __device__ __forceinline__ double jv_scaled(const JvArgs &jv, int i, double d) {
 // 1 024 000 nodes: vg_kernel 33 us with the library's, 24 to 26 with these.
 // ln: x = 2^k m with m in [sqrt(1/2), sqrt(2)), f = m - 1, s = f / (2 + f), and from
 // ln m = 2 atanh s = 2 s + s R, 2 s = f - s f: ln m = f - s (f - R), R = s^2 P(s^2),
-// P the Chebyshev fit of degree 6 to the atanh series (1.6e-18).  0 gives -inf, below NaN.
+// P the Chebyshev fit of degree 6 to the atanh series (1.6e-18); the published scheme of
+// fdlibm's log with a polynomial of its own.  0 gives -inf, below NaN, inf gives inf (a
+// head so dry that (alpha |h|)^n overflows: S = S_r, k_r = 0).
 __device__ __forceinline__ double vg_log(double x) {
     double m = __builtin_amdgcn_frexp_mant(x);
     int k = __builtin_amdgcn_frexp_exp(x);
@@ -63,7 +65,7 @@ __device__ __forceinline__ double vg_log(double x) {
     // ln 2 in two parts, the first times any k exact
     const double c = fma(kd, -1.9082149292705877e-10, s * (f - t * p));
     const double y = fma(kd, 0.6931471803691238, f - c);
-    return x > 0. ? y : x == 0. ? -__builtin_inf() : __builtin_nan("");
+    return x > 0. ? (x < __builtin_inf() ? y : x) : x == 0. ? -__builtin_inf() : __builtin_nan("");
 }
 
 // e^x = 2^k e^r, r = x - k ln 2 in two parts, e^r = 1 + (r + r^2 P(r)), P the Chebyshev
