@@ -657,9 +657,10 @@ extern "C" int fvp_create(const fvp_problem *p, int device, fvp_ctx **out) {
         c->ndir = (int)dn.size();
         if (c->dnode.upload(dn.data(), dn.size()) || upload_dirichlet_values(c)) return fail();
     }
-    if (build_tiles(c, default_tile_nodes(N))) return fail();
-    // node orders whose windows do not fit the LDS keep the larger tiles of the kernel that gathers
-    if (!c->owner_win && build_tiles(c, kTileNodes)) return fail();
+    // node orders whose windows do not fit the LDS keep the larger tiles of the kernel that
+    // gathers; so does a hub of so many elements that a small tile's exports pass 16 bits
+    const bool windows = !build_tiles(c, default_tile_nodes(N)) && c->owner_win;
+    if (!windows && build_tiles(c, kTileNodes)) return fail();
     if (edge_areas(c)) return fail();
     if (c->tmp1.alloc(N) || c->tmp2.alloc(N) || c->tmp3.alloc(N) || c->red.alloc(4096)) return fail();
     c->red_h.resize(4096);
