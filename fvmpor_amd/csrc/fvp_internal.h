@@ -93,6 +93,7 @@ struct fvp_ctx {
     std::vector<double> delev_h;   // elevation of each Dirichlet node (y in 2D, z in 3D)
     // node tiles of the residual kernel (see fvp_setup.cpp)
     int ntiles = 0, tile_nodes = fvp::kTileNodes, xcd_map = 1;  // tile size, XCD-grouped tile order
+    int made_tile = fvp::kTileNodes;  // the tile size that set-up chose
     int rvariant = FVP_RESIDUAL_OWNER;  // residual kernel variant
     long tile_elems = 0;            // element visits per residual (primary + halo)
     fvp::DevBuf<int> t_eptr, t_hptr, t_hlist, t_bptr, t_dptr;

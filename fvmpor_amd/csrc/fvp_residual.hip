@@ -22,7 +22,9 @@
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
+#include <vector>
 
 #include "fvp_blas.h"
 #include "fvp_internal.h"
@@ -1825,7 +1827,8 @@ extern "C" int fvp_set_residual_launch(fvp_ctx *c, int variant, int tile_nodes, 
 
 // Launch-shape autotuner for the residual: every (tile size, XCD grouping)
 // candidate that fits the LDS is built and timed with HIP events over a few
-// upwinded residual evaluations at the given state; the fastest is kept.
+// upwinded residual evaluations at the given state; the fastest is kept.  The
+// tile sizes that the context was made with and has now are candidates too.
 extern "C" int fvp_autotune(fvp_ctx *c, double t, const double *psi, const double *psip, int *variant,
                             int *tile_nodes, int *xcd_map, double *best_us) {
     if (!c || !psi || !psip) { set_error("null argument"); return -1; }
@@ -1835,7 +1838,9 @@ extern "C" int fvp_autotune(fvp_ctx *c, double t, const double *psi, const doubl
     hipEvent_t e0, e1;
     FVP_HIP(hipEventCreate(&e0));
     FVP_HIP(hipEventCreate(&e1));
-    const int tiles[] = {256, 512, 1024, 2048};
+    std::vector<int> tiles = {256, 512, 1024, 2048};
+    for (int tn : {c->made_tile, c->tile_nodes})
+        if (std::find(tiles.begin(), tiles.end(), tn) == tiles.end()) tiles.push_back(tn);
     int best_t = c->tile_nodes, best_x = c->xcd_map, best_v = c->rvariant;
     double best = 1e300;
     const int reps = 10;

@@ -661,6 +661,7 @@ extern "C" int fvp_create(const fvp_problem *p, int device, fvp_ctx **out) {
     // gathers; so does a hub of so many elements that a small tile's exports pass 16 bits
     const bool windows = !build_tiles(c, default_tile_nodes(N)) && c->owner_win;
     if (!windows && build_tiles(c, kTileNodes)) return fail();
+    c->made_tile = c->tile_nodes;
     if (edge_areas(c)) return fail();
     if (c->tmp1.alloc(N) || c->tmp2.alloc(N) || c->tmp3.alloc(N) || c->red.alloc(4096)) return fail();
     c->red_h.resize(4096);
