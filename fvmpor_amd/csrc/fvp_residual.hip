@@ -1803,6 +1803,11 @@ extern "C" int fvp_profile_get(fvp_ctx *c, int kind, double *total_ms, long *cou
     return 0;
 }
 
+extern "C" int fvp_default_tile_nodes(const fvp_ctx *c) {
+    if (!c) { set_error("null context"); return -1; }
+    return c->made_tile;
+}
+
 extern "C" int fvp_set_residual_launch(fvp_ctx *c, int variant, int tile_nodes, int xcd_map) {
     if (!c) { set_error("null context"); return -1; }
     if (variant != FVP_RESIDUAL_OWNER && variant != FVP_RESIDUAL_WINDOW) { set_error("unknown residual variant"); return -1; }

@@ -56,6 +56,7 @@ SIGNATURES = {
     "fvp_set_jacobian_mode": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int]),
     "fvp_precon_overlap": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int]),
     "fvp_set_residual_launch": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int]),
+    "fvp_default_tile_nodes": (ctypes.c_int, [ctypes.c_void_p]),
     "fvp_autotune": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_double, ctypes.c_void_p, ctypes.c_void_p, _c_int_p,
                                     _c_int_p, _c_int_p, _c_dbl_p]),
     "fvp_integrator_set_segments": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, _c_int_p]),
@@ -378,7 +379,11 @@ def _ctx_set_block_rows(self, rows):
     _check(lib().fvp_set_block_rows(self.h, int(rows)), "fvp_set_block_rows")
 
 
-def _ctx_set_residual_launch(self, variant=0, tile_nodes=512, xcd_map=1):
+def _ctx_set_residual_launch(self, variant=0, tile_nodes=None, xcd_map=1):
+    """tile_nodes None: the size the context was made with, 512 for the window variant."""
+    if tile_nodes is None:
+        tile_nodes = 512 if variant == RESIDUAL_WINDOW else _check(lib().fvp_default_tile_nodes(self.h),
+                                                                   "fvp_default_tile_nodes")
     _check(lib().fvp_set_residual_launch(self.h, int(variant), int(tile_nodes), int(xcd_map)),
            "fvp_set_residual_launch")
 

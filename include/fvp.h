@@ -332,6 +332,7 @@ int fvp_integrator_get_stats(const fvp_integrator *I, fvp_integrator_stats *st);
 #define FVP_RESIDUAL_OWNER 0
 #define FVP_RESIDUAL_WINDOW 1
 int fvp_set_residual_launch(fvp_ctx *ctx, int variant, int tile_nodes, int xcd_map);
+int fvp_default_tile_nodes(const fvp_ctx *ctx); /* the size the context was made with */
 int fvp_autotune(fvp_ctx *ctx, double t, const double *psi, const double *psip, int *variant, int *tile_nodes,
                  int *xcd_map, double *best_us);
 

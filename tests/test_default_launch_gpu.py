@@ -63,3 +63,14 @@ def test_the_autotuner_times_it():
     assert pick["variant"] == 0 and pick["tile_nodes"] == 128 and 0.0 < pick["residual_us"] < 1e6, pick
     # a node sums 129 elements or 880, in any order: their rounding is below 1e-13 of the largest sum
     assert np.abs(residual() - before).max() <= 1e-12 * np.abs(before).max()
+
+
+def test_a_launch_without_a_tile_size_is_it():
+    ctx, psi, psip, residual = _context()
+    before = residual()
+    for tile in (64, None):
+        if tile:
+            ctx.set_residual_launch(0, tile)
+        else:
+            ctx.set_residual_launch()
+        assert np.abs(residual() - before).max() <= 1e-12 * np.abs(before).max()
