@@ -1,9 +1,12 @@
 // Sparse linear algebra and the Newton-Krylov inner loop on gfx950.
 //
-//  * CSR SpMV: 8 lanes per row, shuffle reduction (rows hold ~7 (2D) to ~15 (3D) entries).
+//  * CSR SpMV: the entries of 64 rows by whole lines into the LDS, four lanes to a
+//    row (rows hold ~7 (2D) to ~15 (3D) entries).
 //  * ILU(0): level-scheduled factorisation and triangular solves.  Levels come
 //    from the dependency DAG of L (forward) and U (backward); rows of a level
-//    are independent and run as one launch.
+//    are independent.  Matrices whose solution fits the LDS take one launch for
+//    all levels, larger ones a launch per level.
+//  * Block-Jacobi ILU(0): a workgroup factors a block, a wavefront solves it.
 //  * Jacobi: inverse diagonal.
 //  * GMRES: right-preconditioned, restarted (gmres.c:26-201) with classical
 //    Gram-Schmidt fused into one multi-dot and one multi-axpy pass per sweep
@@ -123,7 +126,7 @@ struct fvp_csr {
     // workspace
     int m_alloc = -1;
     DevBuf<double> Q, w, r, z, part, scal, hdev;
-    DevBuf<double> Hd, gd, csd, snd, yd;    // Hessenberg (column-major, m+1 rows), Givens pairs, rhs, solution
+    DevBuf<double> Hd, gd, csd, snd;        // Hessenberg (column-major, m+1 rows), rhs, Givens pairs
     fvp::HostSlots hstat;                   // GMRES, see GmresWork
     fvp::HostSlots hflag;                   // factorisation: the pivot flag
     const double *skip = nullptr;           // while GMRES queues a step: its word that ends the cycle
@@ -303,13 +306,6 @@ __global__ void vrsub(long n, const double *__restrict__ b, double *__restrict__
 __global__ void vadd(long n, const double *__restrict__ x, double *__restrict__ y) {
     long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
     if (i < n) y[i] += x[i];
-}
-
-// dst = src / sqrt(nsq[0])
-__global__ void vscale_inv_norm(long n, const double *__restrict__ src, const double *__restrict__ nsq,
-                                double *__restrict__ dst) {
-    long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    if (i < n) dst[i] = src[i] * (1. / sqrt(nsq[0]));
 }
 
 // compiler-only ordering of one wavefront's LDS accesses (the LDS executes a
@@ -927,15 +923,9 @@ __global__ void __launch_bounds__(256) gs_solution(long n, int k, int m, const d
     }
 }
 
-// out[c] (+)= sum over blocks of part[c * nb + block]
-// With flag set, the block of the last column (||w||^2 after a first
-// Gram-Schmidt pass) also decides the second pass: flag = 1 when that norm
-// fell below half of ww[0] (||w||^2 before the pass), or always when ww is null.
+// out[c] = sum over blocks of part[c * nb + block]; skip: see mdot_kernel
 __global__ void __launch_bounds__(kThreads) reduce_cols(int nb, const double *__restrict__ part,
-                                                        double *__restrict__ out, int accumulate,
-                                                        const double *__restrict__ skip,
-                                                        const double *__restrict__ ww = nullptr,
-                                                        double *__restrict__ flag = nullptr) {
+                                                        double *__restrict__ out, const double *__restrict__ skip) {
     if (skip && skip[0] == 0.) return;
     __shared__ double lds[kThreads / 64];
     int c = blockIdx.x;
@@ -958,12 +948,10 @@ __global__ void __launch_bounds__(kThreads) reduce_cols(int nb, const double *__
     if (threadIdx.x == 0) {
         double v = 0.;
         for (int k = 0; k < (int)(blockDim.x >> 6); ++k) v += lds[k];
-        out[c] = accumulate ? out[c] + v : v;
-        if (flag && c == (int)gridDim.x - 1) flag[0] = (!ww || v < 0.5 * ww[0]) ? 1. : 0.;
+        out[c] = v;
     }
 }
 
-// w += sign * sum_c coef[c] Q[:, c]
 // out = sum_c y[c] Q[:, c]  (y on the device)
 __global__ void lincomb(long n, double *__restrict__ out, const double *__restrict__ Q, long ldq, int nc,
                         const double *__restrict__ y) {
@@ -1040,7 +1028,6 @@ __device__ __forceinline__ double row_bcast(double x) {
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// What a row needs besides the other rows' values, loaded a level ahead.
 // The layout of the solve's packed copies: win values per slot; place: where
 // the entries of a row of several slots go (out.w > 0), from out.w - 1 on; all within
 // the block, whose first slots are ptr[lev[b]] of the solve's levels (null: 0)
@@ -1050,6 +1037,7 @@ struct FacOut {
     const int *lev_l, *ptr_l, *lev_u, *ptr_u;
 };
 
+// What a row needs besides the other rows' values, loaded a level ahead.
 template <typename T, int NC>
 struct FacRow {
     int s0, len, d;           // first entry, entries, L entries
@@ -1804,8 +1792,7 @@ static int ensure_work(fvp_csr *A, int m) {
     long n = A->n;
     if (A->Q.alloc((size_t)gs_ldq(n) * (m + 1)) || A->w.alloc(n) || A->r.alloc(n) || A->z.alloc(n) ||
         A->part.alloc((size_t)kGsBlocks * (kChunk + 1)) || A->scal.alloc(16) || A->hdev.alloc(2 * (m + 2) + 2) ||
-        A->Hd.alloc((size_t)(m + 1) * m) || A->gd.alloc(m + 1) || A->csd.alloc(m) || A->snd.alloc(m) ||
-        A->yd.alloc(m))
+        A->Hd.alloc((size_t)(m + 1) * m) || A->gd.alloc(m + 1) || A->csd.alloc(m) || A->snd.alloc(m))
         return -1;
     if (A->hstat.alloc(m + 1)) return -1;
     A->m_alloc = m;
@@ -1821,7 +1808,7 @@ static void multidot(hipStream_t s, long n, const double *w, const double *Q, lo
         const int k = std::min(kChunk, nc - c0);
         const int last = c0 + k == nc;
         kMdot[k - 1](s, nb, n, w, Q + c0 * ldq, ldq, last, part, skip);
-        reduce_cols<<<k + last, kThreads, 0, s>>>(nb, part, out + c0, 0, skip);
+        reduce_cols<<<k + last, kThreads, 0, s>>>(nb, part, out + c0, skip);
     }
 }
 
@@ -1834,7 +1821,7 @@ static void multiaxpy(hipStream_t s, long n, double *w, const double *Q, long ld
         const int k = std::min(kChunk, nc - c0);
         kAxpy[k - 1](s, nb, n, w, Q + c0 * ldq, ldq, coef + c0, part, skip);
     }
-    if (norm2) reduce_cols<<<1, kThreads, 0, s>>>(nb, part, norm2, 0, skip);
+    if (norm2) reduce_cols<<<1, kThreads, 0, s>>>(nb, part, norm2, skip);
 }
 
 using Op = std::function<int(const double *, double *)>;
@@ -1851,8 +1838,8 @@ using Op = std::function<int(const double *, double *)>;
 // Device and host memory of one GMRES solve: the basis Q (gs_ldq(n) x (m+1)),
 // work vectors w, r, z (gs_ldq(n) each), reduction partials part
 // (kGsBlocks x (kChunk+1)), scalars sc (16), per-step coefficients hdev
-// (2 (m+2) + 2), the Hessenberg matrix Hd ((m+1) x m), Givens pairs, rhs and
-// solution; hstat (host, kSlot (m+1)): slot j receives step j's {estimate,
+// (2 (m+2) + 2), the Hessenberg matrix Hd ((m+1) x m), Givens pairs and rhs;
+// hstat (host, kSlot (m+1)): slot j receives step j's {estimate,
 // h_{j+1,j}}, slot m the squared norms {||r||^2, ||b||^2}.
 // With tag hstat is pinned memory that the kernels write, a tag last (counted
 // up, so that no slot ever holds the awaited tag beforehand), and the host polls
@@ -1864,7 +1851,7 @@ using Op = std::function<int(const double *, double *)>;
 // diag: the preconditioner is this diagonal, and the kernels that write a basis
 // vector write z = diag q as well.
 struct GmresWork {
-    double *Q, *w, *r, *z, *part, *sc, *hdev, *Hd, *gd, *csd, *snd, *yd;
+    double *Q, *w, *r, *z, *part, *sc, *hdev, *Hd, *gd, *csd, *snd;
     double *hstat;
     double *tag;
     const double **skip;
@@ -1876,7 +1863,7 @@ static size_t gmres_work_doubles(long n, int m) {
     auto up = [](size_t v) { return (v + 31) & ~(size_t)31; };
     const size_t ldq = (size_t)gs_ldq(n);
     return up(ldq * (m + 1)) + 3 * up(ldq) + up((size_t)kGsBlocks * (kChunk + 1)) + up(16) + up(2 * (m + 2) + 2) +
-           up((size_t)(m + 1) * m) + 4 * up(m + 1);
+           up((size_t)(m + 1) * m) + 3 * up(m + 1);
 }
 static GmresWork gmres_work_carve(double *base, long n, int m) {
     auto up = [](size_t v) { return (v + 31) & ~(size_t)31; };
@@ -1895,7 +1882,6 @@ static GmresWork gmres_work_carve(double *base, long n, int m) {
     wk.gd = take(m + 1);
     wk.csd = take(m + 1);
     wk.snd = take(m + 1);
-    wk.yd = take(m + 1);
     return wk;
 }
 
@@ -1911,7 +1897,7 @@ int gmres_device(fvp_csr *W, hipStream_t s, long n, const Op &A, const Op &M, co
     if (p->reorthogonalise < 0 || p->reorthogonalise > 2) { set_error("reorthogonalise must be 0, 1 or 2"); return -1; }
     if (ensure_work(W, m)) return -1;
     GmresWork wk{W->Q.p, W->w.p, W->r.p, W->z.p, W->part.p, W->scal.p, W->hdev.p, W->Hd.p, W->gd.p, W->csd.p,
-                 W->snd.p, W->yd.p, W->hstat.p, &W->hstat.tag, &W->skip, diag};
+                 W->snd.p, W->hstat.p, &W->hstat.tag, &W->skip, diag};
     const int rc = gmres_core(wk, s, n, A, M, b, x, p, st, zero);
     W->skip = nullptr;
     return rc;
@@ -3127,7 +3113,7 @@ extern "C" int fvp_csr_destroy(fvp_csr *A) {
     A->ia.release(); A->ja.release(); A->a.release(); A->lu.release(); A->jac.release(); A->diag.release();
     A->lrows.release(); A->urows.release(); A->flag.release(); A->Q.release(); A->w.release(); A->r.release();
     A->z.release(); A->part.release(); A->scal.release(); A->hdev.release();
-    A->Hd.release(); A->gd.release(); A->csd.release(); A->snd.release(); A->yd.release(); A->Qk.release();
+    A->Hd.release(); A->gd.release(); A->csd.release(); A->snd.release(); A->Qk.release();
     A->hstat.release();
     A->hflag.release();
     A->b_ia.release(); A->b_src.release(); A->b_lu.release(); A->b_lu32.release();

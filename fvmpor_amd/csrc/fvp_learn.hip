@@ -940,7 +940,6 @@ struct fvp_mpnn {
     DevBuf<float> p, m, v, g;
     DevBuf<unsigned short> pb, wt1, wt2, wb;  // BF16 copy, per layer: transposed W1, W2; W1 and W2 (aligned)
     long step = 0;
-    // activations
     // activations: H (L + 1) x (N + 1) x 64, each layer's last row zero (padding of the
     // neighbour sums); A, Z: L x N x 64 (the backward pass puts dZ in Z's place); dA:
     // two of (N + 1) x 64, last rows zero

@@ -13,12 +13,19 @@
 // Kernels:
 //   vg_kernel      per node: van Genuchten Sw, dSw/dpsi, k_r for every zone the
 //                  CV touches, CV-averaged capacity ahh (fvmpor.h:874-945)
-//   tile_lds_kernel  per node tile: gradient, 3 or 6 face fluxes and upwinded
-//                  k_r of every element touching the tile, flux sums in LDS,
-//                  then F = acc / V - psi' ahh, boundary fluxes, Dirichlet rows
-//                  (fvmpor_ODE_impl.cpp:99-115)
-//   elem_kernel    per element, atomic scatter: the averaged-weight pass of
-//                  begin_step (fvmpor_ODE_impl.cpp:118-142), then finalize
+//   owner_lds, owner_imports  per node tile: gradient, 3 or 6 face fluxes and
+//                  upwinded k_r of the tile's elements, once each, from node records
+//                  in LDS, flux sums there, then F = acc / V - psi' ahh, boundary
+//                  fluxes, Dirichlet rows (fvmpor_ODE_impl.cpp:99-115); small problems
+//                  with vg_kernel's pass inside
+//   owner_kernel, owner_finalize  the same gathering from memory, where a tile's
+//                  records do not fit the LDS
+//   tile_lds_kernel  the same from staged windows, every element touching the tile
+//   face_flux_kernel, edge_flux_kernel, mask_kernel  begin_step's upwind weights
+//                  (fvmpor_ODE_impl.cpp:118-142)
+//   fd_nodes, fd_elem_kernel, fd_gather  the element-local FD Jacobian
+//   elem_kernel    per element, atomic scatter: the residual with averaged
+//                  weights, before the first begin_step, then finalize
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
