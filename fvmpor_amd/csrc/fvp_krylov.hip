@@ -78,6 +78,16 @@ struct BjPack {
     }
 };
 
+// Launch of the block factorisation: its threads, the levels in pieces of one slot per
+// lane group, the LDS bytes that staging the values takes and whether they are staged
+struct FacPieces {
+    DevBuf<int> lev, lptr;
+    int most = 0, threads = 0;  // pieces of one block
+    size_t lds = 0;
+    bool staged = false;
+    void release() { lev.release(); lptr.release(); }
+};
+
 struct fvp_csr {
     int device = 0;
     hipStream_t stream = nullptr, own_stream = nullptr;
@@ -114,8 +124,7 @@ struct fvp_csr {
     IluTri otri[2];
     int o_threads = 64, o_fthreads = 512, o_win = 0;  // threads of the solve and of the factorisation
     size_t o_lds = 0;
-    DevBuf<int> f_lev[2], f_lptr[2];        // the factorisation's level pieces for 512 and 1024 threads
-    int f_levmax[2] = {0, 0};
+    FacPieces fp[2];                        // FP64's and FP32's
     // packed solve layouts, FP64's and FP32's (the same one where their windows are);
     // values, which bj_factor writes (the rest stays zero), and per U slot the inverted
     // diagonal
@@ -998,17 +1007,24 @@ __device__ __forceinline__ void lds_barrier() {
 // memory one L entry after another, and a packing pass, took 500 + 25 us.
 // STAGED: the block's values are held in LDS; otherwise in place in memory.
 constexpr int kBjGroup = 16;
-// Threads: 512 or, for rows of up to 16 entries, 1024 (32 or 64 rows of a level at once;
-// longer rows' registers leave room for 512).  Both leave 16 wavefronts a CU, so 1024
-// halve the blocks in flight: taken where the pieces of levels they save are worth it,
-// with 1.2 for a piece's cost against 512's.  Blocks of 1024 rows with an overlap
-// layer, FP32, 138 of them: 110 us with 512 threads, 86 with 1024; 281 blocks of 512 rows
-// without overlap: 54 against 70.
-static int bj_factor_threads(int nc, long blocks, size_t lds, long lds_max, int pieces512, int pieces1024) {
-    if (nc > 1) return 512;
-    const long cus = 256, fit = lds ? std::max(1L, lds_max / (long)lds) : 2;
-    const long r512 = (blocks + cus * std::min(2L, fit) - 1) / (cus * std::min(2L, fit)), r1024 = (blocks + cus - 1) / cus;
-    return 1.2 * (double)r1024 * pieces1024 <= (double)r512 * pieces512 ? 1024 : 512;
+// Threads: 64 to 512 or, for rows of up to 16 entries, 1024 (4 to 64 rows of a level at
+// once; longer rows' registers leave room for 512), the cheapest by this estimate, the
+// more of equal ones.  A round of resident blocks costs its pieces of levels, each a
+// latency or, where that is longer, what its wavefronts issue (a wavefront without a row
+// loads ahead all the same), and the values' way in and out.  The constants fit 386
+// builds (blocks of 64 to 4096 rows, with and without overlap, of meshes, grids, bands
+// and random patterns, each with every thread count) to 8 % of each one's best.  138 blocks
+// of 1024 rows with an overlap layer, FP32: 110 us with 512 threads, 86 with 1024; 977
+// chains of 256 rows, FP64: 210 us with 64, 428 with 512; 129 blocks with levels of 4
+// rows: 437 us with 64, 216 with 512.
+constexpr int kFacThreads[] = {1024, 512, 256, 128, 64};
+static double fac_cost(int th, int nc, size_t vb, long blocks, long nz, size_t lds, long lds_max, int pieces) {
+    if (th == 1024 && nc > 1) return 1e300;
+    const int waves = th / 64, most = nc == 1 ? 16 : nc == 2 && vb == 4 ? 12 : 8;  // wavefronts a CU holds
+    const long cus = 256, fit = std::max(1L, std::min((long)most / waves, lds ? lds_max / (long)lds : 64L));
+    const long rounds = (blocks + cus * fit - 1) / (cus * fit);
+    const double issue = 0.35 * (double)std::min(fit, (blocks + cus - 1) / cus) * waves / 4;
+    return (double)rounds * (pieces * std::max(1., issue) + 0.8 * (double)nz / th);
 }
 constexpr int kAhead = 2;  // offset words of eight L entries loaded a level ahead
 
@@ -1182,7 +1198,7 @@ __device__ __forceinline__ void fac_row_store(const FacRow<T, NC> &w, int gl, T 
 // factor.  vl, vu, vd: the solve's packed L, U and inverted diagonal.  STAGED: values and piece pointers (npmax + 1 ints) in LDS, so that a
 // barrier waits for LDS accesses only and rows are loaded kRing levels ahead.
 template <typename T, int NC, bool STAGED, int TH>
-__global__ void __launch_bounds__(TH) bj_factor(
+__global__ void __launch_bounds__(TH, NC == 1 ? 4 : 2) bj_factor(
     const int *__restrict__ roff, const int *__restrict__ ia, const int *__restrict__ src,
     const double *__restrict__ a, const uint4 *__restrict__ slot, const uint4 *__restrict__ sout,
     const unsigned *__restrict__ piv, const uint2 *__restrict__ off, const int *__restrict__ blev,
@@ -2400,7 +2416,7 @@ static int build_one(fvp_csr *A, const std::vector<int> &diag, const std::vector
     std::vector<int> fp, fp1024;
     level_pieces(A->lptr_h, 512 / kBjGroup, fp);
     level_pieces(A->lptr_h, 1024 / kBjGroup, fp1024);
-    A->o_fthreads = bj_factor_threads(maxrow <= kBjGroup ? 1 : 2, 1, 0, 0, (int)fp.size() - 1, (int)fp1024.size() - 1);
+    A->o_fthreads = maxrow <= kBjGroup && 1.2 * fp1024.size() <= fp.size() ? 1024 : 512;
     if (A->o_fthreads == 1024) fp.swap(fp1024);
     const int head[4] = {0, n, 0, (int)fp.size() - 1};
     fp.insert(fp.begin(), head, head + 4);
@@ -2535,7 +2551,51 @@ static int build_pack(BjPack &P, int W, int nb, const std::vector<int> &roff, co
     return 0;
 }
 
-// Block-local CSR and the per-block level sets of L and U.  Block b owns rows
+static void bj_attrs(int lds_max);
+
+// The factorisation's levels (blev per block into lptr) in pieces, at the cheapest width
+static int factor_pieces(FacPieces &F, int nb, const std::vector<int> &blev, const std::vector<int> &lptr, int maxnz,
+                         int nc, size_t vb, int lds_max) {
+    double best = 1e300;
+    const char *given = getenv("FVP_BJ_FACTOR_THREADS");  // forces the threads: a tuning and test knob
+    F.threads = 0;
+    for (int th : kFacThreads) {
+        if (given && (nc > 1 ? std::min(atoi(given), 512) : atoi(given)) != th) continue;
+        const int width = th / kBjGroup;
+        int most = 0;
+        for (int b = 0; b < nb; ++b) {
+            int n1 = 0;
+            for (int l = blev[b]; l < blev[b + 1]; ++l) n1 += (lptr[l + 1] - lptr[l] + width - 1) / width;
+            most = std::max(most, n1);
+        }
+        // Values staged in LDS wherever a block fits (rows past 32 entries in FP64
+        // spill registers in that form and stay in place).  Whole builds, staged
+        // against in place: 67 / 75 us (276 blocks of 512 rows, FP32), 200 / 307
+        // (1024 with one overlap layer, FP32), 323 / 365 (the same, FP64), 517 / 549
+        // (1000 blocks of 1024 with overlap, FP32); at worst 91 / 83 (276 blocks of
+        // 512, FP64), all with 512 threads.
+        const size_t lds = (size_t)maxnz * vb + 8 * (size_t)((most + 2) / 2);
+        const bool staged = lds <= (size_t)lds_max && !(nc == 4 && vb == 8);
+        const double cost = fac_cost(th, nc, vb, nb, maxnz, staged ? lds : 0, lds_max, most);
+        if (cost >= best) continue;
+        best = cost;
+        F.threads = th;
+        F.most = most;
+        F.lds = lds;
+        F.staged = staged;
+    }
+    if (!F.threads) { set_error("FVP_BJ_FACTOR_THREADS must be 64, 128, 256, 512 or 1024"); return -1; }
+    const int width = F.threads / kBjGroup;
+    std::vector<int> fb(nb + 1, 0), fp(1, 0);
+    for (int b = 0; b < nb; ++b) {
+        for (int l = blev[b]; l < blev[b + 1]; ++l)
+            for (int p = lptr[l]; p < lptr[l + 1]; p += width) fp.push_back(std::min(p + width, lptr[l + 1]));
+        fb[b + 1] = (int)fp.size() - 1;
+    }
+    return F.lev.upload(fb.data(), nb + 1) || F.lptr.upload(fp.data(), fp.size()) ? -1 : 0;
+}
+
+// Block-local CSR and the per-block level sets of L.  Block b owns rows
 // [b bs, (b+1) bs); with overlap > 0 its local rows are the owned rows plus
 // `overlap` layers of their graph neighbours (sorted by global row, so the
 // local ILU(0) follows the global row order), and only the owned rows of its
@@ -2637,19 +2697,6 @@ static int build_bj(fvp_csr *A) {
         for (int f32 = 0; f32 <= A->pack32; ++f32)
             if (build_pack(A->pack[f32], win[f32], nb, roff, bia, bja, bdiag, rows_l)) return -1;
         if (factor_tables(A->fac, nb, roff, bia, bja, bdiag, rows_l, maxrow)) return -1;
-        // the factor's levels in pieces of one slot per lane group
-        for (int w = 0; w < 2; ++w) {
-            const int width = (w ? 1024 : 512) / kBjGroup;
-            std::vector<int> fb(nb + 1, 0), fp(1, 0);
-            A->f_levmax[w] = 0;
-            for (int b = 0; b < nb; ++b) {
-                for (int l = blev_l[b]; l < blev_l[b + 1]; ++l)
-                    for (int p = lptr_l[l]; p < lptr_l[l + 1]; p += width) fp.push_back(std::min(p + width, lptr_l[l + 1]));
-                fb[b + 1] = (int)fp.size() - 1;
-                A->f_levmax[w] = std::max(A->f_levmax[w], fb[b + 1] - fb[b]);
-            }
-            if (A->f_lev[w].upload(fb.data(), nb + 1) || A->f_lptr[w].upload(fp.data(), fp.size())) return -1;
-        }
         A->val_l.release(); A->val_u.release(); A->dinv.release();
         A->val32_l.release(); A->val32_u.release(); A->dinv32.release();
     }
@@ -2659,14 +2706,10 @@ static int build_bj(fvp_csr *A) {
         A->lds_max = 64 * 1024;
     // per-kernel attributes (shared by every matrix): allow the device maximum;
     // each build checks its own block against it
-    for (const void *f : {(const void *)bj_factor<double, 1, true, 512>, (const void *)bj_factor<double, 1, true, 1024>,
-                          (const void *)bj_factor<double, 2, true, 512>, (const void *)bj_factor<double, 4, true, 512>,
-                          (const void *)bj_factor<float, 1, true, 512>, (const void *)bj_factor<float, 1, true, 1024>,
-                          (const void *)bj_factor<float, 2, true, 512>, (const void *)bj_factor<float, 4, true, 512>,
-                          (const void *)bj_solve<double, 4>, (const void *)bj_solve<double, 8>,
-                          (const void *)bj_solve<float, 4>, (const void *)bj_solve<float, 8>,
-                          (const void *)bj_solve<float, 12>})
-        (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, A->lds_max);
+    bj_attrs(A->lds_max);
+    for (int f32 = 0; f32 < 2; ++f32)
+        if (factor_pieces(A->fp[f32], nb, blev_l, lptr_l, maxnz, A->fac.nc, f32 ? sizeof(float) : sizeof(double), A->lds_max))
+            return -1;
     A->nblk = nb;
     A->bj = true;
     return 0;
@@ -2866,18 +2909,41 @@ struct FactorArgs {
     int threads;
 };
 template <typename T, int NC, int TH>
-static void bj_factor_launch_nc(hipStream_t s, const FactorArgs &f, T *lu, T *vl, T *vu, T *vd) {
+static void bj_factor_launch_th(hipStream_t s, const FactorArgs &f, T *lu, T *vl, T *vu, T *vd) {
     const FactorTab &t = *f.tab;
     const auto kernel = f.staged ? bj_factor<T, NC, true, TH> : bj_factor<T, NC, false, TH>;
     kernel<<<f.nblk, TH, f.staged, s>>>(f.roff, f.ia, f.src, f.a, t.slot.p, f.sout, t.piv.p, t.off.p, f.lev, f.lptr, lu,
                                         vl, vu, vd, f.out, f.flag, f.npmax);
 }
+template <typename T, int NC>
+static void bj_factor_launch_nc(hipStream_t s, const FactorArgs &f, T *lu, T *vl, T *vu, T *vd) {
+    if (f.threads == 64) bj_factor_launch_th<T, NC, 64>(s, f, lu, vl, vu, vd);
+    else if (f.threads == 128) bj_factor_launch_th<T, NC, 128>(s, f, lu, vl, vu, vd);
+    else if (f.threads == 256) bj_factor_launch_th<T, NC, 256>(s, f, lu, vl, vu, vd);
+    else if (f.threads == 512 || NC > 1) bj_factor_launch_th<T, NC, 512>(s, f, lu, vl, vu, vd);
+    else bj_factor_launch_th<T, NC, NC == 1 ? 1024 : 512>(s, f, lu, vl, vu, vd);
+}
 template <typename T>
 static void bj_factor_launch(hipStream_t s, const FactorArgs &f, T *lu, T *vl, T *vu, T *vd) {
-    if (f.tab->nc == 1 && f.threads == 1024) bj_factor_launch_nc<T, 1, 1024>(s, f, lu, vl, vu, vd);
-    else if (f.tab->nc == 1) bj_factor_launch_nc<T, 1, 512>(s, f, lu, vl, vu, vd);
-    else if (f.tab->nc == 2) bj_factor_launch_nc<T, 2, 512>(s, f, lu, vl, vu, vd);
-    else bj_factor_launch_nc<T, 4, 512>(s, f, lu, vl, vu, vd);
+    if (f.tab->nc == 1) bj_factor_launch_nc<T, 1>(s, f, lu, vl, vu, vd);
+    else if (f.tab->nc == 2) bj_factor_launch_nc<T, 2>(s, f, lu, vl, vu, vd);
+    else bj_factor_launch_nc<T, 4>(s, f, lu, vl, vu, vd);
+}
+
+template <typename T, int NC>
+static void bj_factor_attrs(int lds_max) {
+    for (const void *f : {(const void *)bj_factor<T, NC, true, 64>, (const void *)bj_factor<T, NC, true, 128>,
+                          (const void *)bj_factor<T, NC, true, 256>, (const void *)bj_factor<T, NC, true, 512>,
+                          (const void *)bj_factor<T, NC, true, NC == 1 ? 1024 : 512>})
+        (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
+}
+static void bj_attrs(int lds_max) {
+    bj_factor_attrs<double, 1>(lds_max); bj_factor_attrs<double, 2>(lds_max); bj_factor_attrs<double, 4>(lds_max);
+    bj_factor_attrs<float, 1>(lds_max); bj_factor_attrs<float, 2>(lds_max); bj_factor_attrs<float, 4>(lds_max);
+    for (const void *f : {(const void *)bj_solve<double, 4>, (const void *)bj_solve<double, 8>,
+                          (const void *)bj_solve<float, 4>, (const void *)bj_solve<float, 8>,
+                          (const void *)bj_solve<float, 12>})
+        (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
 }
 
 static int precon_build_impl(fvp_csr *A, int type) {
@@ -2898,42 +2964,34 @@ static int precon_build_impl(fvp_csr *A, int type) {
         int rc = schur_factor(A);
         if (rc) { A->ptype = -1; return rc; }
     } else if (type == FVP_PRECON_BJILU0 || type == FVP_PRECON_BJILU0_F32) {
+        const bool f32 = type == FVP_PRECON_BJILU0_F32;
         if (!A->bj) {
             int rc = build_bj(A);
             if (rc) { A->ptype = -1; return rc; }
         }
-        const size_t vb = type == FVP_PRECON_BJILU0 ? sizeof(double) : sizeof(float);
-        // Values staged in LDS wherever a block fits (rows past 32 entries in FP64
-        // spill registers in that form and stay in place).  Whole builds, staged
-        // against in place: 67 / 75 us (276 blocks of 512 rows, FP32), 200 / 307
-        // (1024 with one overlap layer, FP32), 323 / 365 (the same, FP64), 517 / 549
-        // (1000 blocks of 1024 with overlap, FP32); at worst 91 / 83 (276 blocks of
-        // 512, FP64), all with 512 threads.  FVP_BJ_FACTOR_MODE 0 / 1 forces in place /
-        // staged where it fits the workgroup: a tuning and test knob.
-        const size_t staged = (size_t)A->b_maxnz * vb + 8 * (size_t)((A->f_levmax[0] + 2) / 2);
-        bool stage = staged <= (size_t)A->lds_max && !(A->fac.nc == 4 && vb == 8);
-        if (const char *e = getenv("FVP_BJ_FACTOR_MODE")) stage = atoi(e) > 0 && staged <= (size_t)A->lds_max;
-        A->factor_mode = stage ? 1 : 0;
-        const int th = bj_factor_threads(A->fac.nc, A->nblk, stage ? staged : 0, A->lds_max, A->f_levmax[0], A->f_levmax[1]);
-        const int w = th == 1024;
-        const BjPack &P = A->pack[vb == 4 ? A->pack32 : 0];
-        const FactorArgs fa{A->nblk, A->b_roff.p, A->b_ia.p, A->b_src.p, A->a.p, &A->fac, A->f_lev[w].p,
-                            A->f_lptr[w].p, A->flag.p,
+        const FacPieces &F = A->fp[f32];
+        const BjPack &P = A->pack[f32 ? A->pack32 : 0];
+        // FVP_BJ_FACTOR_MODE 0 / 1 forces values in place / staged where they fit the
+        // workgroup: a tuning and test knob
+        bool stage = F.staged;
+        if (const char *e = getenv("FVP_BJ_FACTOR_MODE")) stage = atoi(e) > 0 && F.lds <= (size_t)A->lds_max;
+        A->factor_mode = stage;
+        const FactorArgs fa{A->nblk, A->b_roff.p, A->b_ia.p, A->b_src.p, A->a.p, &A->fac, F.lev.p, F.lptr.p, A->flag.p,
                             FacOut{(unsigned)P.win, P.place.p, P.lev_l.p, P.lptr_l.p, P.lev_u.p, P.lptr_u.p},
-                            P.out.p, stage ? staged : 0, A->f_levmax[w], th};
+                            P.out.p, stage ? F.lds : 0, F.most, F.threads};
         const size_t nl = P.row_l.n * P.win, nu = P.row_u.n * P.win, nd = P.row_u.n;
         // the packed arrays' padding stays zero: only the factor's entries are written
         auto ensure = [&](auto &lu, auto &vl, auto &vu, auto &vd) {
             if (!lu.p && lu.alloc(A->b_src.n)) return -1;
-            if (vl.p) return 0;
+            if (vd.p) return 0;  // the last of them
             // ... and a slot without a diagonal keeps d = 1
             const std::vector<std::decay_t<decltype(*vd.p)>> ones(nd, 1);
-            if (vl.alloc(nl) || vu.alloc(nu) || vd.upload(ones.data(), nd)) return -1;
+            if (vl.alloc(nl) || vu.alloc(nu)) return -1;
             FVP_HIP(hipMemsetAsync(vl.p, 0, sizeof(*vl.p) * nl, s));
             FVP_HIP(hipMemsetAsync(vu.p, 0, sizeof(*vu.p) * nu, s));
-            return 0;
+            return vd.upload(ones.data(), nd);
         };
-        if (type == FVP_PRECON_BJILU0) {
+        if (!f32) {
             if (ensure(A->b_lu, A->val_l, A->val_u, A->dinv)) return -1;
             bj_factor_launch<double>(s, fa, A->b_lu.p, A->val_l.p, A->val_u.p, A->dinv.p);
         } else {
@@ -3121,7 +3179,7 @@ extern "C" int fvp_csr_destroy(fvp_csr *A) {
     A->pack[0].release(); A->pack[1].release(); A->val_l.release();
     A->val_u.release(); A->dinv.release(); A->val32_l.release(); A->val32_u.release(); A->dinv32.release();
     A->fac.release(); A->ofac.release(); A->otri[0].release(); A->otri[1].release(); A->o_fptr.release();
-    for (int w = 0; w < 2; ++w) { A->f_lev[w].release(); A->f_lptr[w].release(); }
+    A->fp[0].release(); A->fp[1].release();
     schur_free(A);
     if (A->own_stream) (void)hipStreamDestroy(A->own_stream);
     delete A;
