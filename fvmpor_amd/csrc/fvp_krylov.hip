@@ -63,11 +63,12 @@ struct IluTri {
 };
 
 // Packed layout of the block solve (see bj_solve), per triangle: the levels of at most
-// 64 slots, win entries per slot, their columns (two per word) and the row; out: where
+// 64 slots, kBjWin entries per slot, their columns (two per word) and the row; out: where
 // the factorisation puts a row (see factor_tables), place: the entries of a row of
 // several slots
 struct BjPack {
-    int win = 0, levmax_l = 0, levmax_u = 0;
+    int levmax_l = 0, levmax_u = 0;
+    bool several = false;  // some row has several slots
     fvp::DevBuf<int> lev_l, lptr_l, lev_u, lptr_u;
     fvp::DevBuf<unsigned> col_l, col_u, place;
     fvp::DevBuf<unsigned short> row_l, row_u;
@@ -125,11 +126,9 @@ struct fvp_csr {
     int o_threads = 64, o_fthreads = 512, o_win = 0;  // threads of the solve and of the factorisation
     size_t o_lds = 0;
     FacPieces fp[2];                        // FP64's and FP32's
-    // packed solve layouts, FP64's and FP32's (the same one where their windows are);
-    // values, which bj_factor writes (the rest stays zero), and per U slot the inverted
-    // diagonal
-    BjPack pack[2];
-    int pack32 = 0;
+    // packed solve layout; values, which bj_factor writes (the rest stays zero), and per
+    // U slot the inverted diagonal
+    BjPack pack;
     DevBuf<double> val_l, val_u, dinv;
     DevBuf<float> val32_l, val32_u, dinv32;
     // workspace
@@ -1300,67 +1299,61 @@ __global__ void __launch_bounds__(TH, NC == 1 ? 4 : 2) bj_factor(
 // Solve: one wavefront per block.  Only the block's solution and its level
 // pointers live in LDS (so that every block of the matrix is resident at once
 // and the CU interleaves their dependency chains).  The factor streams from a
-// level-ordered packed copy per triangle, which bj_factor writes: slots of W
+// level-ordered packed copy per triangle, which bj_factor writes: slots of kBjWin
 // entries, zero past the row's length (their column is the row itself), one lane
-// each, up to 64 a level.  A row of more than W entries takes further slots in
+// each, up to 64 a level.  A row of more than kBjWin entries takes further slots in
 // earlier levels, for the entries whose rows are final there: each subtracts its
-// share from v[r] (with d = 1 in U).  T is the factor's arithmetic type (double, or
-// float for the FP32 preconditioner); x and y stay FP64.
+// share from v[r] (with d = 1 in U).  T is the factor's type (double, or float for the
+// FP32 preconditioner), V the solution's and the sums': double, or float for FP32
+// factors whose rows have one slot each (and where double does not fit the LDS); x and y
+// stay FP64.  A row of several slots is rounded several times on its way: with V float
+// that showed (||y - y64|| / ||y64|| of a 194 672-row box in blocks of 1024 with an
+// overlap layer: 1.14e-7, rows whole 1.09e-7, V double 0.93e-7).
 // What bounds it is one wavefront's instruction issue and LDS latency per level, and
-// for large matrices the factor's bytes.  Rows end to end, a lane pair to a row and
-// windows of 12 entries (levels of 32, starts and lengths from the LDS, two selects an
-// entry) needed 71 vector instructions a level and twice the levels where those are
-// wide.  With a tetrahedral box's rows (at most 7 entries a triangle, 10 next to
-// other blocks), one overlap layer, us: 144 000 rows in blocks of 1024, FP64 51 -> 32,
-// FP32 49 -> 32; 614 000 in blocks of 512, FP64 49 -> 42, FP32 46 -> 39; in two
-// dimensions 23 000 in blocks of 1024, 43 -> 25 both.
-// W: in FP64 8, or 4 where nine rows in ten fit that; in FP32 the least of 4, 8 and 12
-// that all rows fit (12 beyond): a row's sum is kept in the order of the form before
-// (entries 0 to 5, then 6 to 11), which FP32 would show.
-template <typename T, int W>
+// for many blocks the factor's bytes.  Slots of 4 entries: a tetrahedral box's rows have
+// 7 a triangle (10 next to other blocks) inside a block, 5 on average in blocks of 256
+// rows, 2.5 in blocks of 64, and the rest of a wider slot is read for nothing.
+// One overlap layer, us, slots of 8 (FP64) and 12 (FP32) -> 4: 524 288 rows in blocks
+// of 64, 179 -> 134 and 166 -> 78; in blocks of 256, 69 -> 47 and 52 -> 38; 194 672 in
+// blocks of 1024, 48 -> 40 and 46 -> 42; the same by rows end to end (no padding, a lane
+// pair to a row, twice the levels): 160 and 114, 54 and 50, 66 and 65.  Longer rows find
+// room in earlier levels: a band of 41, 346 -> 263.  Only where wide levels are full of
+// long rows are 8 the better: 27-point stencil, 27 000 rows in blocks of 1024
+// with overlap, FP64, 52 against 57 (end to end 114).
+constexpr int kBjWin = 4;
+template <typename T>
 struct BjWin {
-    T a[W];
-    unsigned c[W / 2];  // local columns, two per word
+    T a[kBjWin];
+    unsigned c[kBjWin / 2];  // local columns, two per word
     unsigned r;
     T d;                // inverted diagonal (U)
     bool mine;
 };
 
 // slot s of the block's
-template <typename T, int W, bool UPPER>
-__device__ __forceinline__ void bj_win_load(BjWin<T, W> &w, unsigned s, bool mine, const T *__restrict__ val,
+template <typename T, bool UPPER>
+__device__ __forceinline__ void bj_win_load(BjWin<T> &w, unsigned s, bool mine, const T *__restrict__ val,
                                             const unsigned *__restrict__ col, const unsigned short *__restrict__ row,
                                             const T *__restrict__ dinv) {
     if constexpr (sizeof(T) == 4) {
-        const float4 *p = reinterpret_cast<const float4 *>(val + W * s);
-#pragma unroll
-        for (int i = 0; i < W / 4; ++i) {
-            const float4 q = p[i];
-            w.a[4 * i] = q.x; w.a[4 * i + 1] = q.y; w.a[4 * i + 2] = q.z; w.a[4 * i + 3] = q.w;
-        }
+        const float4 q = *reinterpret_cast<const float4 *>(val + kBjWin * s);
+        w.a[0] = q.x; w.a[1] = q.y; w.a[2] = q.z; w.a[3] = q.w;
     } else {
-        const double2 *p = reinterpret_cast<const double2 *>(val + W * s);
-#pragma unroll
-        for (int i = 0; i < W / 2; ++i) {
-            const double2 q = p[i];
-            w.a[2 * i] = q.x; w.a[2 * i + 1] = q.y;
-        }
+        const double2 *p = reinterpret_cast<const double2 *>(val + kBjWin * s);
+        const double2 q0 = p[0], q1 = p[1];
+        w.a[0] = q0.x; w.a[1] = q0.y; w.a[2] = q1.x; w.a[3] = q1.y;
     }
-    const uint2 *pc = reinterpret_cast<const uint2 *>(col + W / 2 * s);
-#pragma unroll
-    for (int i = 0; i < W / 4; ++i) {
-        const uint2 q = pc[i];
-        w.c[2 * i] = q.x; w.c[2 * i + 1] = q.y;
-    }
+    const uint2 q = *reinterpret_cast<const uint2 *>(col + kBjWin / 2 * s);
+    w.c[0] = q.x; w.c[1] = q.y;
     w.r = row[s];
     w.d = UPPER ? dinv[s] : T(0);
     w.mine = mine;
 }
 
 // levels loaded ahead: deep enough to cover a memory round trip with the short
-// per-level arithmetic, as far as the registers go
-template <typename T, int W>
-constexpr int bj_ahead() { return sizeof(T) == 4 ? (W == 12 ? 5 : 8) : W == 4 ? 7 : 4; }
+// per-level arithmetic, as far as the registers of four wavefronts a SIMD go
+template <typename T>
+constexpr int bj_ahead() { return sizeof(T) == 4 ? 8 : 7; }
 
 // One triangle of one block: lane t takes the t-th slot of each level (lp: the
 // levels' slots within the block).  The windows are loads in flight, kA levels
@@ -1371,17 +1364,17 @@ constexpr int bj_ahead() { return sizeof(T) == 4 ? (W == 12 ? 5 : 8) : W == 4 ? 
 // stores s, lanes without a slot to their own spare place vd, so that v[r]'s read
 // stays with the window's (rows of one level do not depend on each other, so it
 // is final here).
-template <typename T, int W, bool UPPER>
-__device__ __forceinline__ void bj_sweep(T *v, T *vd, int nl, const int *lp, const T *__restrict__ val,
+template <typename T, typename V, bool UPPER>
+__device__ __forceinline__ void bj_sweep(V *v, V *vd, int nl, const int *lp, const T *__restrict__ val,
                                          const unsigned *__restrict__ col, const unsigned short *__restrict__ row,
                                          const T *__restrict__ dinv) {
     if (nl <= 0) return;
-    constexpr int kA = bj_ahead<T, W>();
-    auto load = [&](BjWin<T, W> &w, int l, int p0, int p1) {
+    constexpr int kA = bj_ahead<T>();
+    auto load = [&](BjWin<T> &w, int l, int p0, int p1) {
         const int s = p0 + (int)threadIdx.x;
-        bj_win_load<T, W, UPPER>(w, min(s, p1 - 1), l < nl && s < p1, val, col, row, dinv);
+        bj_win_load<T, UPPER>(w, min(s, p1 - 1), l < nl && s < p1, val, col, row, dinv);
     };
-    BjWin<T, W> wr[kA];
+    BjWin<T> wr[kA];
 #pragma unroll
     for (int d = 0; d < kA; ++d) {
         const int lc = min(d, nl - 1);
@@ -1395,16 +1388,16 @@ __device__ __forceinline__ void bj_sweep(T *v, T *vd, int nl, const int *lp, con
         for (int d = 0; d < kA; ++d) {
             const int ln = lb + d + kA, lc = min(ln, nl - 1);
             const int p0 = lp[lc], p1 = lp[lc + 1];
-            const BjWin<T, W> &w = wr[d];
-            constexpr int kFirst = sizeof(T) == 4 ? 6 : W / 2;
-            T q0 = T(0), q1 = T(0);
+            const BjWin<T> &w = wr[d];
+            constexpr int kFirst = sizeof(V) == 4 ? kBjWin : kBjWin / 2;
+            V q0 = V(0), q1 = V(0);
 #pragma unroll
-            for (int u = 0; u < W; ++u) {
-                const T x = v[(u & 1) ? w.c[u / 2] >> 16 : w.c[u / 2] & 0xffffu];
+            for (int u = 0; u < kBjWin; ++u) {
+                const V x = v[(u & 1) ? w.c[u / 2] >> 16 : w.c[u / 2] & 0xffffu];
                 if (u < kFirst) q0 += w.a[u] * x;
                 else q1 += w.a[u] * x;
             }
-            T s = v[w.r] - (q0 + q1);
+            V s = v[w.r] - (q0 + q1);
             if (UPPER) s *= w.d;
             *(w.mine ? v + w.r : vd) = s;
             load(wr[d], ln, p0, p1);
@@ -1415,10 +1408,10 @@ __device__ __forceinline__ void bj_sweep(T *v, T *vd, int nl, const int *lp, con
     }
 }
 
-// LDS bytes of one block's solve: the solution (T x maxrows) and a spare
-// place per lane (T x 64), its L and U level pointers
-__host__ __device__ inline size_t bj_solve_lds(size_t tsize, int maxrows, int levl, int levu) {
-    return ((tsize * (size_t)(maxrows + 64) + 7) & ~(size_t)7) + 4 * (size_t)(levl + levu + 2);
+// LDS bytes of one block's solve: the solution (V x maxrows) and a spare
+// place per lane (V x 64), its L and U level pointers
+__host__ __device__ inline size_t bj_solve_lds(size_t vsize, int maxrows, int levl, int levu) {
+    return ((vsize * (size_t)(maxrows + 64) + 7) & ~(size_t)7) + 4 * (size_t)(levl + levu + 2);
 }
 
 // rowid: global row of each local row (nullptr: block b's rows are the
@@ -1429,7 +1422,7 @@ __host__ __device__ inline size_t bj_solve_lds(size_t tsize, int maxrows, int le
 // one wavefront stages too slowly.)  Per triangle: solve levels blev (per
 // block) into lptr (per level, into the level-ordered slots, at most 64 per
 // level), the slots' values, columns and rows, U's inverted diagonals.
-template <typename T, int W>
+template <typename T, typename V>
 __global__ void __launch_bounds__(64) bj_solve(const int *__restrict__ roff, const int *__restrict__ rowid,
                                                const int *__restrict__ own, const int *__restrict__ blev_l,
                                                const int *__restrict__ lptr_l, const T *__restrict__ val_l,
@@ -1447,13 +1440,13 @@ __global__ void __launch_bounds__(64) bj_solve(const int *__restrict__ roff, con
     const int base = roff[b];
     const int cnt = roff[b + 1] - base;
     char *lds = reinterpret_cast<char *>(smem);
-    T *v = reinterpret_cast<T *>(lds);
+    V *v = reinterpret_cast<V *>(lds);
     // v: the block's rows, then one spare place per lane
-    T *vd = v + maxrows + threadIdx.x;
+    V *vd = v + maxrows + threadIdx.x;
     const int l0 = blev_l[b], nl = blev_l[b + 1] - l0;
     const int u0 = blev_u[b], nu = blev_u[b + 1] - u0;
     const long sl = lptr_l[l0], su = lptr_u[u0];  // the block's first slots
-    int *lpl = reinterpret_cast<int *>(lds + ((sizeof(T) * (size_t)(maxrows + 64) + 7) & ~(size_t)7));
+    int *lpl = reinterpret_cast<int *>(lds + ((sizeof(V) * (size_t)(maxrows + 64) + 7) & ~(size_t)7));
     int *lpu = lpl + nl + 1;
     for (int k = threadIdx.x; k <= nl; k += 64) lpl[k] = lptr_l[l0 + k] - (int)sl;
     for (int k = threadIdx.x; k <= nu; k += 64) lpu[k] = lptr_u[u0 + k] - (int)su;
@@ -1476,13 +1469,13 @@ __global__ void __launch_bounds__(64) bj_solve(const int *__restrict__ roff, con
 #pragma unroll
         for (int k = 0; k < kBjStage; ++k) {
             const int r = r0 + 64 * k;
-            if (r < cnt) v[r] = (T)(xdiv ? xv[k] / dv[k] : xv[k]);
+            if (r < cnt) v[r] = (V)(xdiv ? xv[k] / dv[k] : xv[k]);
         }
     }
     wave_lds_order();
     if (over != 0.) return;
-    bj_sweep<T, W, false>(v, vd, nl, lpl, val_l + W * sl, col_l + W / 2 * sl, row_l + sl, nullptr);
-    bj_sweep<T, W, true>(v, vd, nu, lpu, val_u + W * su, col_u + W / 2 * su, row_u + su, dinv + su);
+    bj_sweep<T, V, false>(v, vd, nl, lpl, val_l + kBjWin * sl, col_l + kBjWin / 2 * sl, row_l + sl, nullptr);
+    bj_sweep<T, V, true>(v, vd, nu, lpu, val_u + kBjWin * su, col_u + kBjWin / 2 * su, row_u + su, dinv + su);
     const int olo = own[2 * b], ohi = own[2 * b + 1];
     double q = 0.;
     for (int r0 = olo + threadIdx.x; r0 < ohi; r0 += 64 * kBjStage) {
@@ -2433,13 +2426,13 @@ static int build_one(fvp_csr *A, const std::vector<int> &diag, const std::vector
     return 0;
 }
 
-// The solve's packed layout with windows of W entries for the blocks roff, bia, bja,
-// bdiag (as in factor_tables), rows_l their rows in the factorisation's order
-static int build_pack(BjPack &P, int W, int nb, const std::vector<int> &roff, const std::vector<int> &bia,
+// The solve's packed layout for the blocks roff, bia, bja, bdiag (as in factor_tables), rows_l their rows in the factorisation's order
+static int build_pack(BjPack &P, int nb, const std::vector<int> &roff, const std::vector<int> &bia,
                       const std::vector<unsigned short> &bja, const std::vector<int> &bdiag,
                       const std::vector<unsigned short> &rows_l) {
     const int total = roff[nb];
-    P.win = W;
+    constexpr int W = kBjWin;
+    P.several = false;
     std::vector<int> lev;
     std::vector<uint4> out(total, make_uint4(0u, 0u, 0u, 0u));  // by row at first, then by slot of L's level order
     std::vector<unsigned> place;
@@ -2517,7 +2510,7 @@ static int build_pack(BjPack &P, int W, int nb, const std::vector<int> &roff, co
                 const int sl = s0 + at[step[q]]++;
                 by[q] = sl;
                 srow[sl] = (unsigned short)m.row;
-                unsigned short c[12];
+                unsigned short c[W];
                 for (int k = 0; k < W; ++k) c[k] = k < m.n ? bja[order[m.first + k]] : (unsigned short)m.row;
                 for (int k = 0; k < W; k += 2) col[(size_t)sl * (W / 2) + k / 2] = c[k] | (unsigned)c[k + 1] << 16;
                 if (m.main) (tri ? out[base + m.row].y : out[base + m.row].x) = (unsigned)(sl - s0);
@@ -2528,6 +2521,7 @@ static int build_pack(BjPack &P, int W, int nb, const std::vector<int> &roff, co
                 const int i = base + m.row, len = bia[i + 1] - bia[i];
                 const bool several = std::max(bdiag[i] - bia[i], bia[i + 1] - bdiag[i] - 1) > W;
                 if (!several) continue;
+                P.several = true;
                 if (!out[i].w) {
                     out[i].w = (unsigned)place.size() + 1;
                     place.resize(place.size() + len, 0);
@@ -2683,23 +2677,11 @@ static int build_bj(fvp_csr *A) {
     if (ident) A->b_rowid.release();
     A->b_lu.release();
     A->b_lu32.release();
-    {
-        // packed solve layout (see bj_solve)
-        long small = 0;
-        int longest = 0;
-        for (int i = 0; i < total; ++i) {
-            const int l = bdiag[i] - bia[i], u = bia[i + 1] - bdiag[i] - 1;
-            small += (l <= 4) + (u <= 4);
-            longest = std::max({longest, l, u});
-        }
-        const int win[2] = {small >= 9 * (2 * (long)total) / 10 ? 4 : 8, longest <= 4 ? 4 : longest <= 8 ? 8 : 12};
-        A->pack32 = win[1] != win[0];
-        for (int f32 = 0; f32 <= A->pack32; ++f32)
-            if (build_pack(A->pack[f32], win[f32], nb, roff, bia, bja, bdiag, rows_l)) return -1;
-        if (factor_tables(A->fac, nb, roff, bia, bja, bdiag, rows_l, maxrow)) return -1;
-        A->val_l.release(); A->val_u.release(); A->dinv.release();
-        A->val32_l.release(); A->val32_u.release(); A->dinv32.release();
-    }
+    if (build_pack(A->pack, nb, roff, bia, bja, bdiag, rows_l) ||
+        factor_tables(A->fac, nb, roff, bia, bja, bdiag, rows_l, maxrow))
+        return -1;
+    A->val_l.release(); A->val_u.release(); A->dinv.release();
+    A->val32_l.release(); A->val32_u.release(); A->dinv32.release();
     A->b_maxnz = maxnz;
     A->b_maxrows = maxrows;
     if (hipDeviceGetAttribute(&A->lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, A->device) != hipSuccess)
@@ -2940,9 +2922,8 @@ static void bj_factor_attrs(int lds_max) {
 static void bj_attrs(int lds_max) {
     bj_factor_attrs<double, 1>(lds_max); bj_factor_attrs<double, 2>(lds_max); bj_factor_attrs<double, 4>(lds_max);
     bj_factor_attrs<float, 1>(lds_max); bj_factor_attrs<float, 2>(lds_max); bj_factor_attrs<float, 4>(lds_max);
-    for (const void *f : {(const void *)bj_solve<double, 4>, (const void *)bj_solve<double, 8>,
-                          (const void *)bj_solve<float, 4>, (const void *)bj_solve<float, 8>,
-                          (const void *)bj_solve<float, 12>})
+    for (const void *f : {(const void *)bj_solve<double, double>, (const void *)bj_solve<float, double>,
+                          (const void *)bj_solve<float, float>})
         (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
 }
 
@@ -2970,16 +2951,16 @@ static int precon_build_impl(fvp_csr *A, int type) {
             if (rc) { A->ptype = -1; return rc; }
         }
         const FacPieces &F = A->fp[f32];
-        const BjPack &P = A->pack[f32 ? A->pack32 : 0];
+        const BjPack &P = A->pack;
         // FVP_BJ_FACTOR_MODE 0 / 1 forces values in place / staged where they fit the
         // workgroup: a tuning and test knob
         bool stage = F.staged;
         if (const char *e = getenv("FVP_BJ_FACTOR_MODE")) stage = atoi(e) > 0 && F.lds <= (size_t)A->lds_max;
         A->factor_mode = stage;
         const FactorArgs fa{A->nblk, A->b_roff.p, A->b_ia.p, A->b_src.p, A->a.p, &A->fac, F.lev.p, F.lptr.p, A->flag.p,
-                            FacOut{(unsigned)P.win, P.place.p, P.lev_l.p, P.lptr_l.p, P.lev_u.p, P.lptr_u.p},
+                            FacOut{(unsigned)kBjWin, P.place.p, P.lev_l.p, P.lptr_l.p, P.lev_u.p, P.lptr_u.p},
                             P.out.p, stage ? F.lds : 0, F.most, F.threads};
-        const size_t nl = P.row_l.n * P.win, nu = P.row_u.n * P.win, nd = P.row_u.n;
+        const size_t nl = P.row_l.n * kBjWin, nu = P.row_u.n * kBjWin, nd = P.row_u.n;
         // the packed arrays' padding stays zero: only the factor's entries are written
         auto ensure = [&](auto &lu, auto &vl, auto &vu, auto &vd) {
             if (!lu.p && lu.alloc(A->b_src.n)) return -1;
@@ -3076,25 +3057,21 @@ static int precon_apply_impl(fvp_csr *A, const double *x, double *y, const doubl
     case FVP_PRECON_BJILU0:
     case FVP_PRECON_BJILU0_F32: {
         const bool f64 = A->ptype == FVP_PRECON_BJILU0;
-        const size_t ts = f64 ? sizeof(double) : sizeof(float);
-        const BjPack &P = A->pack[f64 ? 0 : A->pack32];
-        const size_t lds = bj_solve_lds(ts, A->b_maxrows, P.levmax_l, P.levmax_u);
+        const BjPack &P = A->pack;
+        size_t lds = bj_solve_lds(sizeof(double), A->b_maxrows, P.levmax_l, P.levmax_u);
+        const bool v64 = f64 || (P.several && lds <= (size_t)A->lds_max);
+        if (!v64) lds = bj_solve_lds(sizeof(float), A->b_maxrows, P.levmax_l, P.levmax_u);
         if (lds > (size_t)A->lds_max) {
             set_error("block-Jacobi ILU(0): a block's solution does not fit the LDS");
             return -1;
         }
-#define FVP_BJ_SOLVE(TT, W, VL, VU, DI)                                                                            \
-    bj_solve<TT, W><<<A->nblk, 64, lds, s>>>(A->b_roff.p, A->b_rowid.p, A->b_own.p, P.lev_l.p, P.lptr_l.p, VL,     \
-                                             P.col_l.p, P.row_l.p, P.lev_u.p, P.lptr_u.p, VU, P.col_u.p, P.row_u.p, \
-                                             DI, A->b_maxrows, x, xdiv, y, yn2, A->skip)
-        if (f64) {
-            if (P.win == 8) FVP_BJ_SOLVE(double, 8, A->val_l.p, A->val_u.p, A->dinv.p);
-            else FVP_BJ_SOLVE(double, 4, A->val_l.p, A->val_u.p, A->dinv.p);
-        } else {
-            if (P.win == 12) FVP_BJ_SOLVE(float, 12, A->val32_l.p, A->val32_u.p, A->dinv32.p);
-            else if (P.win == 8) FVP_BJ_SOLVE(float, 8, A->val32_l.p, A->val32_u.p, A->dinv32.p);
-            else FVP_BJ_SOLVE(float, 4, A->val32_l.p, A->val32_u.p, A->dinv32.p);
-        }
+#define FVP_BJ_SOLVE(T, V, VL, VU, DI)                                                                             \
+    bj_solve<T, V><<<A->nblk, 64, lds, s>>>(A->b_roff.p, A->b_rowid.p, A->b_own.p, P.lev_l.p, P.lptr_l.p, VL,      \
+                                            P.col_l.p, P.row_l.p, P.lev_u.p, P.lptr_u.p, VU, P.col_u.p, P.row_u.p, \
+                                            DI, A->b_maxrows, x, xdiv, y, yn2, A->skip)
+        if (f64) FVP_BJ_SOLVE(double, double, A->val_l.p, A->val_u.p, A->dinv.p);
+        else if (v64) FVP_BJ_SOLVE(float, double, A->val32_l.p, A->val32_u.p, A->dinv32.p);
+        else FVP_BJ_SOLVE(float, float, A->val32_l.p, A->val32_u.p, A->dinv32.p);
 #undef FVP_BJ_SOLVE
         break;
     }
@@ -3176,7 +3153,7 @@ extern "C" int fvp_csr_destroy(fvp_csr *A) {
     A->hflag.release();
     A->b_ia.release(); A->b_src.release(); A->b_lu.release(); A->b_lu32.release();
     A->b_roff.release(); A->b_rowid.release(); A->b_own.release(); A->b_zn2.release();
-    A->pack[0].release(); A->pack[1].release(); A->val_l.release();
+    A->pack.release(); A->val_l.release();
     A->val_u.release(); A->dinv.release(); A->val32_l.release(); A->val32_u.release(); A->dinv32.release();
     A->fac.release(); A->ofac.release(); A->otri[0].release(); A->otri[1].release(); A->o_fptr.release();
     A->fp[0].release(); A->fp[1].release();
