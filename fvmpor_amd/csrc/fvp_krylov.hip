@@ -92,7 +92,7 @@ struct FacPieces {
 struct fvp_csr {
     int device = 0;
     hipStream_t stream = nullptr, own_stream = nullptr;
-    int n = 0, nnz = 0;
+    int n = 0, nnz = 0, longest = 0;    // longest: entries of the longest row
     std::vector<int> ia_h, ja_h;
     DevBuf<int> ia, ja;
     DevBuf<double> a;
@@ -167,20 +167,24 @@ namespace fvp {
 constexpr int kThreads = 256;
 
 // ---- kernels ------------------------------------------------------------------
-// y = alpha A x + beta y.  A workgroup's kGemvRows rows are one contiguous range of
+// y = alpha A x + beta y.  A workgroup's R rows are one contiguous range of
 // entries: its threads load them entry by entry (whole lines, four values of x in flight
-// each) into the LDS, a chunk of 16 a row at a time, and four lanes to a row sum them
+// each) into the LDS, a chunk of 1024 at a time, and 256 / R lanes to a row sum them
 // from there.  What bounds it is the latency of row pointer -> column -> x, then its
 // bytes (4.5 TB/s at 524 288 rows of 14.6).  Against eight lanes to a row straight from
-// memory: 191 771 rows of 14.6 11.3 -> 9.3 us, 524 288 of 14.6 26.9 -> 21.0, 600 000 of
-// 7 18.2 -> 17.0, 4 141 of 6.9 4.8 -> 4.0.  Rows per workgroup 32 / 64 / 128: 10.9 / 9.3 /
-// 9.1 us, 24.4 / 21.0 / 21.5, 24.1 / 17.0 / 17.0, 4.5 / 4.0 / 4.5.
-constexpr int kGemvRows = 64;
+// memory: 191 771 rows of 14.6 11.3 -> 9.3 us, 524 288 of 14.6 26.9 -> 21.0, 4 141 of 6.9
+// 4.8 -> 4.0.  R, so that a workgroup's rows fill a chunk or two: 128 for rows of up to 9
+// entries on average (64 / 128: 200 000 rows of 2 6.2 / 4.8 us, 10^6 of 3 23.9 / 14.0,
+// 800 000 of 5 20.2 / 13.0, 400 000 of 9 12.1 / 12.5, 200 000 random of 11 13.1 / 14.5),
+// not where single rows are long (one of 100 000: 1051 / 2054, lanes to a row straight
+// from memory 1736); 16 for more than 40 (16 / 64: 4 000 rows of 61 4.8 / 6.6, 60 000 of 61
+// 10.0 / 11.2, 60 000 of 45 8.3 / 7.6, 120 000 of 41 14.3 / 13.6, 3 000 of 480 17.6 / 184).
+template <int R>
 __global__ void __launch_bounds__(256) csr_gemv_kernel(int n, const int *__restrict__ ia, const int *__restrict__ ja,
                                                        const double *__restrict__ a, double alpha,
                                                        const double *__restrict__ x, double beta,
                                                        double *__restrict__ y, const double *skip) {
-    constexpr int R = kGemvRows, L = 256 / R, U = R / 16, CH = 256 * U;
+    constexpr int L = 256 / R, U = 4, CH = 256 * U;
     __shared__ double qa[CH], qx[CH];
     const double over = skip_word(skip);
     const int r0 = blockIdx.x * R, row = r0 + threadIdx.x / L, lane = threadIdx.x % L;
@@ -2239,9 +2243,16 @@ using namespace fvp;
 
 namespace fvp {
 
+template <int R>
+static void csr_gemv_launch(fvp_csr *A, double alpha, const double *x, double beta, double *y) {
+    csr_gemv_kernel<R><<<nblk(A->n, R), 256, 0, A->stream>>>(A->n, A->ia.p, A->ja.p, A->a.p, alpha, x, beta, y, A->skip);
+}
 static int csr_gemv_impl(fvp_csr *A, double alpha, const double *x, double beta, double *y) {
-    csr_gemv_kernel<<<nblk(A->n, kGemvRows), 256, 0, A->stream>>>(A->n, A->ia.p, A->ja.p, A->a.p, alpha, x, beta, y,
-                                                                 A->skip);
+    // rows per workgroup: see csr_gemv_kernel
+    const long n = A->n, nnz = A->nnz;
+    if (nnz <= 9 * n && A->longest <= 256) csr_gemv_launch<128>(A, alpha, x, beta, y);
+    else if (nnz <= 40 * n) csr_gemv_launch<64>(A, alpha, x, beta, y);
+    else csr_gemv_launch<16>(A, alpha, x, beta, y);
     FVP_HIP(hipGetLastError());
     return 0;
 }
@@ -3112,8 +3123,10 @@ static int precon_apply_impl(fvp_csr *A, const double *x, double *y, const doubl
 int csr_create_impl(int device, int n, const int *ia, const int *ja, fvp_csr **out) {
     if (!out || !ia || !ja || n <= 0) { set_error("invalid CSR arguments"); return -1; }
     *out = nullptr;
+    int longest = 0;
     for (int i = 0; i < n; ++i) {
         if (ia[i + 1] < ia[i]) { set_error("row pointers must be non-decreasing"); return -1; }
+        longest = std::max(longest, ia[i + 1] - ia[i]);
         for (int k = ia[i]; k < ia[i + 1]; ++k) {
             if (ja[k] < 0 || ja[k] >= n) { set_error("column index out of range"); return -1; }
             if (k > ia[i] && ja[k] <= ja[k - 1]) { set_error("column indices must be sorted and unique"); return -1; }
@@ -3124,6 +3137,7 @@ int csr_create_impl(int device, int n, const int *ia, const int *ja, fvp_csr **o
     A->device = device;
     A->n = n;
     A->nnz = ia[n];
+    A->longest = longest;
     A->ia_h.assign(ia, ia + n + 1);
     A->ja_h.assign(ja, ja + A->nnz);
     if (hipStreamCreateWithFlags(&A->own_stream, hipStreamNonBlocking) != hipSuccess) {
