@@ -2474,8 +2474,13 @@ static int build_pack(BjPack &P, int nb, const std::vector<int> &roff, const std
                 const int f = (int)order.size();
                 for (int k = 0; k < n; ++k) order.push_back(k0 + k);
                 int l = 0;
-                if (n > W)
-                    std::stable_sort(order.begin() + f, order.end(), [&](int x, int y) { return lev[bja[x]] < lev[bja[y]]; });
+                if (n > W)  // few entries: by insertion
+                    for (int k = 1; k < n; ++k) {
+                        const int e = order[f + k], le = lev[bja[e]];
+                        int j = k;
+                        for (; j > 0 && lev[bja[order[f + j - 1]]] > le; --j) order[f + j] = order[f + j - 1];
+                        order[f + j] = e;
+                    }
                 for (int k = 0; k < n; ++k) l = std::max(l, lev[bja[order[f + k]]] + 1);
                 for (int j = 1, e = n - W; e > 0; ++j, e -= W) l = std::max(l, lev[bja[order[f + e - 1]]] + 1 + j);
                 lev[r] = l;
@@ -2558,21 +2563,28 @@ static int build_pack(BjPack &P, int nb, const std::vector<int> &roff, const std
 
 static void bj_attrs(int lds_max);
 
+// The most pieces of one block, by kFacThreads
+static std::array<int, 5> most_pieces(int nb, const std::vector<int> &blev, const std::vector<int> &lptr) {
+    std::array<int, 5> most{};
+    for (int b = 0; b < nb; ++b) {
+        std::array<int, 5> m{};
+        for (int l = blev[b]; l < blev[b + 1]; ++l)
+            for (int w = 0; w < 5; ++w) m[w] += (lptr[l + 1] - lptr[l] + (64 >> w) - 1) >> (6 - w);
+        for (int w = 0; w < 5; ++w) most[w] = std::max(most[w], m[w]);
+    }
+    return most;
+}
+
 // The factorisation's levels (blev per block into lptr) in pieces, at the cheapest width
-static int factor_pieces(FacPieces &F, int nb, const std::vector<int> &blev, const std::vector<int> &lptr, int maxnz,
-                         int nc, size_t vb, int lds_max) {
+static int factor_pieces(FacPieces &F, int nb, const std::vector<int> &blev, const std::vector<int> &lptr,
+                         const std::array<int, 5> &pieces, int maxnz, int nc, size_t vb, int lds_max) {
+    static_assert(sizeof(kFacThreads) == 5 * sizeof(int) && kFacThreads[0] / kBjGroup == 64 && kFacThreads[4] / kBjGroup == 4);
     double best = 1e300;
     const char *given = getenv("FVP_BJ_FACTOR_THREADS");  // forces the threads: a tuning and test knob
     F.threads = 0;
-    for (int th : kFacThreads) {
+    for (int w = 0; w < 5; ++w) {
+        const int th = kFacThreads[w], most = pieces[w];
         if (given && (nc > 1 ? std::min(atoi(given), 512) : atoi(given)) != th) continue;
-        const int width = th / kBjGroup;
-        int most = 0;
-        for (int b = 0; b < nb; ++b) {
-            int n1 = 0;
-            for (int l = blev[b]; l < blev[b + 1]; ++l) n1 += (lptr[l + 1] - lptr[l] + width - 1) / width;
-            most = std::max(most, n1);
-        }
         // Values staged in LDS wherever a block fits (rows past 32 entries in FP64
         // spill registers in that form and stay in place).  Whole builds, staged
         // against in place: 67 / 75 us (276 blocks of 512 rows, FP32), 200 / 307
@@ -2700,8 +2712,10 @@ static int build_bj(fvp_csr *A) {
     // per-kernel attributes (shared by every matrix): allow the device maximum;
     // each build checks its own block against it
     bj_attrs(A->lds_max);
+    const std::array<int, 5> pieces = most_pieces(nb, blev_l, lptr_l);
     for (int f32 = 0; f32 < 2; ++f32)
-        if (factor_pieces(A->fp[f32], nb, blev_l, lptr_l, maxnz, A->fac.nc, f32 ? sizeof(float) : sizeof(double), A->lds_max))
+        if (factor_pieces(A->fp[f32], nb, blev_l, lptr_l, pieces, maxnz, A->fac.nc, f32 ? sizeof(float) : sizeof(double),
+                          A->lds_max))
             return -1;
     A->nblk = nb;
     A->bj = true;
