@@ -25,6 +25,7 @@
 #include <complex>
 #include <cstring>
 #include <functional>
+#include <memory>
 #include <mutex>
 #include <numeric>
 #include <set>
@@ -63,12 +64,11 @@ struct IluTri {
 };
 
 // Packed layout of the block solve (see bj_solve), per triangle: the levels of at most
-// 64 slots, kBjWin entries per slot, their columns (two per word) and the row; out: where
+// 64 lanes, win entries per lane, their columns (two per word) and the row; out: where
 // the factorisation puts a row (see factor_tables), place: the entries of a row of
 // several slots
 struct BjPack {
-    int levmax_l = 0, levmax_u = 0;
-    bool several = false;  // some row has several slots
+    int win = 0, levmax_l = 0, levmax_u = 0;  // win 0: not made
     fvp::DevBuf<int> lev_l, lptr_l, lev_u, lptr_u;
     fvp::DevBuf<unsigned> col_l, col_u, place;
     fvp::DevBuf<unsigned short> row_l, row_u;
@@ -87,6 +87,13 @@ struct FacPieces {
     size_t lds = 0;
     bool staged = false;
     void release() { lev.release(); lptr.release(); }
+};
+
+// The blocks as the host lays them out (see build_bj), kept until both precisions have
+// their layout of the solve
+struct BjTables {
+    std::vector<int> roff, bia, bdiag;
+    std::vector<unsigned short> bja, rows;
 };
 
 struct fvp_csr {
@@ -126,9 +133,13 @@ struct fvp_csr {
     int o_threads = 64, o_fthreads = 512, o_win = 0;  // threads of the solve and of the factorisation
     size_t o_lds = 0;
     FacPieces fp[2];                        // FP64's and FP32's
-    // packed solve layout; values, which bj_factor writes (the rest stays zero), and per
-    // U slot the inverted diagonal
-    BjPack pack;
+    // packed solve layouts, FP64's (also FP32's where no row is longer than its lanes)
+    // and FP32's, made at the first build that wants them; values, which bj_factor writes
+    // (the rest stays zero), and per U lane the inverted diagonal
+    std::unique_ptr<BjTables> tables;
+    BjPack pack[2];
+    int b_longest = 0;                      // entries of the longest row of a triangle
+    const BjPack &pack_of(bool f32) const { return pack[f32 && b_longest > 4]; }
     DevBuf<double> val_l, val_u, dinv;
     DevBuf<float> val32_l, val32_u, dinv32;
     // workspace
@@ -1047,7 +1058,7 @@ __device__ __forceinline__ double row_bcast(double x) {
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// The layout of the solve's packed copies: win values per slot; place: where
+// The layout of the solve's packed copies: win values per lane; place: where
 // the entries of a row of several slots go (out.w > 0), from out.w - 1 on; all within
 // the block, whose first slots are ptr[lev[b]] of the solve's levels (null: 0)
 struct FacOut {
@@ -1303,55 +1314,57 @@ __global__ void __launch_bounds__(TH, NC == 1 ? 4 : 2) bj_factor(
 // Solve: one wavefront per block.  Only the block's solution and its level
 // pointers live in LDS (so that every block of the matrix is resident at once
 // and the CU interleaves their dependency chains).  The factor streams from a
-// level-ordered packed copy per triangle, which bj_factor writes: slots of kBjWin
-// entries, zero past the row's length (their column is the row itself), one lane
-// each, up to 64 a level.  A row of more than kBjWin entries takes further slots in
-// earlier levels, for the entries whose rows are final there: each subtracts its
-// share from v[r] (with d = 1 in U).  T is the factor's type (double, or float for the
-// FP32 preconditioner), V the solution's and the sums': double, or float for FP32
-// factors whose rows have one slot each (and where double does not fit the LDS); x and y
-// stay FP64.  A row of several slots is rounded several times on its way: with V float
-// that showed (||y - y64|| / ||y64|| of a 194 672-row box in blocks of 1024 with an
-// overlap layer: 1.14e-7, rows whole 1.09e-7, V double 0.93e-7).
+// level-ordered packed copy per triangle, which bj_factor writes: slots of one lane or,
+// with PAIR, of up to two, W entries to a lane (zero past the row's length, with the row
+// itself as the column), up to 64 lanes a level.  A pair's second lane (its row: its own
+// spare place) passes its sum to the first.  A row longer than a slot takes further slots
+// in earlier levels, for the entries whose rows are final there: each subtracts its share
+// from v[r] (with d = 1 in U).  T is the factor's arithmetic type (double, or float for the
+// FP32 preconditioner); x and y stay FP64.
+// W = 4 and one lane, in FP32 where every row fits it; else 6 in pairs: a row's sum is that
+// of entries 0 to 5 and of 6 to 11, whatever lanes they lie in, since FP32 shows a row
+// rounded once more (194 672-row box in blocks of 1024, one overlap layer, against FP64:
+// 1.09e-7; with slots of 4 1.14e-7).
 // What bounds it is one wavefront's instruction issue and LDS latency per level, and
-// for many blocks the factor's bytes.  Slots of 4 entries: a tetrahedral box's rows have
-// 7 a triangle (10 next to other blocks) inside a block, 5 on average in blocks of 256
-// rows, 2.5 in blocks of 64, and the rest of a wider slot is read for nothing.
-// One overlap layer, us, slots of 8 (FP64) and 12 (FP32) -> 4: 524 288 rows in blocks
-// of 64, 179 -> 134 and 166 -> 78; in blocks of 256, 69 -> 47 and 52 -> 38; 194 672 in
-// blocks of 1024, 48 -> 40 and 46 -> 42; the same by rows end to end (no padding, a lane
-// pair to a row, twice the levels): 160 and 114, 54 and 50, 66 and 65.  Longer rows find
-// room in earlier levels: a band of 41, 346 -> 263.  Only where wide levels are full of
-// long rows are 8 the better: 27-point stencil, 27 000 rows in blocks of 1024
-// with overlap, FP64, 52 against 57 (end to end 114).
-constexpr int kBjWin = 4;
-template <typename T>
+// for many blocks the factor's bytes.  A tetrahedral box's rows have 7 entries a
+// triangle (10 next to other blocks) inside a block, 5 on average in blocks of 256 rows,
+// 2.5 in blocks of 64; lanes of 8 entries (12 in FP32) read zeros for the rest.
+// One overlap layer, us, FP64 / FP32, now, with lanes of 8 and 12, and with rows end to end
+// (no padding, a lane pair to a row, twice the levels): 524 288 rows in blocks of 64
+// 135 / 116, 179 / 166, 160 / 114; in blocks of 256 48 / 43, 69 / 51, 54 / 50; 194 672 in
+// blocks of 1024 40 / 39, 48 / 46, 66 / 65; a band of 61, 9 000 rows, no overlap,
+// 262 / 314, 345 / 405, 3565 / 3564.  Only where wide levels are full of long rows are lanes
+// of 8 the better in FP64: 27-point stencil, 27 000 rows in blocks of 1024, 58, 52, 114.
+template <typename T, int W>
 struct BjWin {
-    T a[kBjWin];
-    unsigned c[kBjWin / 2];  // local columns, two per word
+    T a[W];
+    unsigned c[W / 2];  // local columns, two per word
     unsigned r;
     T d;                // inverted diagonal (U)
     bool mine;
 };
 
-// slot s of the block's
-template <typename T, bool UPPER>
-__device__ __forceinline__ void bj_win_load(BjWin<T> &w, unsigned s, bool mine, const T *__restrict__ val,
+// lane s of the block's
+template <typename T, int W, bool UPPER>
+__device__ __forceinline__ void bj_win_load(BjWin<T, W> &w, unsigned s, bool mine, const T *__restrict__ val,
                                             const unsigned *__restrict__ col, const unsigned short *__restrict__ row,
                                             const T *__restrict__ dinv) {
-    if constexpr (sizeof(T) == 4) {
-        const float4 q = *reinterpret_cast<const float4 *>(val + kBjWin * s);
-        w.a[0] = q.x; w.a[1] = q.y; w.a[2] = q.z; w.a[3] = q.w;
-    } else {
-        const double2 *p = reinterpret_cast<const double2 *>(val + kBjWin * s);
-        const double2 q0 = p[0], q1 = p[1];
-        w.a[0] = q0.x; w.a[1] = q0.y; w.a[2] = q1.x; w.a[3] = q1.y;
+    using T2 = typename std::conditional<sizeof(T) == 4, float2, double2>::type;
+    const T2 *p = reinterpret_cast<const T2 *>(val + W * s);
+#pragma unroll
+    for (int i = 0; i < W / 2; ++i) {
+        const T2 q = p[i];
+        w.a[2 * i] = q.x; w.a[2 * i + 1] = q.y;
+        w.c[i] = col[W / 2 * s + i];
     }
-    const uint2 q = *reinterpret_cast<const uint2 *>(col + kBjWin / 2 * s);
-    w.c[0] = q.x; w.c[1] = q.y;
     w.r = row[s];
     w.d = UPPER ? dinv[s] : T(0);
     w.mine = mine;
+}
+
+// the other lane's of a pair
+__device__ __forceinline__ float swap_pair(float x) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xb1, 0xf, 0xf, true));
 }
 
 // levels loaded ahead: deep enough to cover a memory round trip with the short
@@ -1359,26 +1372,26 @@ __device__ __forceinline__ void bj_win_load(BjWin<T> &w, unsigned s, bool mine, 
 template <typename T>
 constexpr int bj_ahead() { return sizeof(T) == 4 ? 8 : 7; }
 
-// One triangle of one block: lane t takes the t-th slot of each level (lp: the
-// levels' slots within the block).  The windows are loads in flight, kA levels
-// ahead, one per lane and level, each consumed by the same unrolled stage that
+// One triangle of one block: lane t takes the t-th lane of each level (lp: the
+// levels' lanes within the block; spare: the first spare place).  The windows are
+// loads in flight, kA levels ahead, one per lane and level, each consumed by the same unrolled stage that
 // issued it kA stages earlier (no loop-carried register holds a pending load, so
 // the compiler's wait counts keep all kA levels in flight).  Every pass runs all
 // kA levels (those past the last have no lane with work).  Every lane forms and
 // stores s, lanes without a slot to their own spare place vd, so that v[r]'s read
 // stays with the window's (rows of one level do not depend on each other, so it
 // is final here).
-template <typename T, typename V, bool UPPER>
-__device__ __forceinline__ void bj_sweep(V *v, V *vd, int nl, const int *lp, const T *__restrict__ val,
+template <typename T, int W, bool PAIR, bool UPPER>
+__device__ __forceinline__ void bj_sweep(T *v, T *vd, unsigned spare, int nl, const int *lp, const T *__restrict__ val,
                                          const unsigned *__restrict__ col, const unsigned short *__restrict__ row,
                                          const T *__restrict__ dinv) {
     if (nl <= 0) return;
     constexpr int kA = bj_ahead<T>();
-    auto load = [&](BjWin<T> &w, int l, int p0, int p1) {
+    auto load = [&](BjWin<T, W> &w, int l, int p0, int p1) {
         const int s = p0 + (int)threadIdx.x;
-        bj_win_load<T, UPPER>(w, min(s, p1 - 1), l < nl && s < p1, val, col, row, dinv);
+        bj_win_load<T, W, UPPER>(w, min(s, p1 - 1), l < nl && s < p1, val, col, row, dinv);
     };
-    BjWin<T> wr[kA];
+    BjWin<T, W> wr[kA];
 #pragma unroll
     for (int d = 0; d < kA; ++d) {
         const int lc = min(d, nl - 1);
@@ -1392,16 +1405,17 @@ __device__ __forceinline__ void bj_sweep(V *v, V *vd, int nl, const int *lp, con
         for (int d = 0; d < kA; ++d) {
             const int ln = lb + d + kA, lc = min(ln, nl - 1);
             const int p0 = lp[lc], p1 = lp[lc + 1];
-            const BjWin<T> &w = wr[d];
-            constexpr int kFirst = sizeof(V) == 4 ? kBjWin : kBjWin / 2;
-            V q0 = V(0), q1 = V(0);
+            const BjWin<T, W> &w = wr[d];
+            T q0 = T(0), q1 = T(0);
 #pragma unroll
-            for (int u = 0; u < kBjWin; ++u) {
-                const V x = v[(u & 1) ? w.c[u / 2] >> 16 : w.c[u / 2] & 0xffffu];
-                if (u < kFirst) q0 += w.a[u] * x;
+            for (int u = 0; u < W; ++u) {
+                const T x = v[(u & 1) ? w.c[u / 2] >> 16 : w.c[u / 2] & 0xffffu];
+                if (sizeof(T) == 4 || u < W / 2) q0 += w.a[u] * x;
                 else q1 += w.a[u] * x;
             }
-            V s = v[w.r] - (q0 + q1);
+            const T vr = v[w.r];
+            if constexpr (PAIR) q1 = swap_pair(w.r >= spare ? q0 : T(0));
+            T s = vr - (q0 + q1);
             if (UPPER) s *= w.d;
             *(w.mine ? v + w.r : vd) = s;
             load(wr[d], ln, p0, p1);
@@ -1412,10 +1426,10 @@ __device__ __forceinline__ void bj_sweep(V *v, V *vd, int nl, const int *lp, con
     }
 }
 
-// LDS bytes of one block's solve: the solution (V x maxrows) and a spare
-// place per lane (V x 64), its L and U level pointers
-__host__ __device__ inline size_t bj_solve_lds(size_t vsize, int maxrows, int levl, int levu) {
-    return ((vsize * (size_t)(maxrows + 64) + 7) & ~(size_t)7) + 4 * (size_t)(levl + levu + 2);
+// LDS bytes of one block's solve: the solution (T x maxrows) and a spare
+// place per lane (T x 64), its L and U level pointers
+__host__ __device__ inline size_t bj_solve_lds(size_t tsize, int maxrows, int levl, int levu) {
+    return ((tsize * (size_t)(maxrows + 64) + 7) & ~(size_t)7) + 4 * (size_t)(levl + levu + 2);
 }
 
 // rowid: global row of each local row (nullptr: block b's rows are the
@@ -1426,7 +1440,7 @@ __host__ __device__ inline size_t bj_solve_lds(size_t vsize, int maxrows, int le
 // one wavefront stages too slowly.)  Per triangle: solve levels blev (per
 // block) into lptr (per level, into the level-ordered slots, at most 64 per
 // level), the slots' values, columns and rows, U's inverted diagonals.
-template <typename T, typename V>
+template <typename T, int W, bool PAIR>
 __global__ void __launch_bounds__(64) bj_solve(const int *__restrict__ roff, const int *__restrict__ rowid,
                                                const int *__restrict__ own, const int *__restrict__ blev_l,
                                                const int *__restrict__ lptr_l, const T *__restrict__ val_l,
@@ -1444,13 +1458,13 @@ __global__ void __launch_bounds__(64) bj_solve(const int *__restrict__ roff, con
     const int base = roff[b];
     const int cnt = roff[b + 1] - base;
     char *lds = reinterpret_cast<char *>(smem);
-    V *v = reinterpret_cast<V *>(lds);
+    T *v = reinterpret_cast<T *>(lds);
     // v: the block's rows, then one spare place per lane
-    V *vd = v + maxrows + threadIdx.x;
+    T *vd = v + maxrows + threadIdx.x;
     const int l0 = blev_l[b], nl = blev_l[b + 1] - l0;
     const int u0 = blev_u[b], nu = blev_u[b + 1] - u0;
     const long sl = lptr_l[l0], su = lptr_u[u0];  // the block's first slots
-    int *lpl = reinterpret_cast<int *>(lds + ((sizeof(V) * (size_t)(maxrows + 64) + 7) & ~(size_t)7));
+    int *lpl = reinterpret_cast<int *>(lds + ((sizeof(T) * (size_t)(maxrows + 64) + 7) & ~(size_t)7));
     int *lpu = lpl + nl + 1;
     for (int k = threadIdx.x; k <= nl; k += 64) lpl[k] = lptr_l[l0 + k] - (int)sl;
     for (int k = threadIdx.x; k <= nu; k += 64) lpu[k] = lptr_u[u0 + k] - (int)su;
@@ -1473,13 +1487,13 @@ __global__ void __launch_bounds__(64) bj_solve(const int *__restrict__ roff, con
 #pragma unroll
         for (int k = 0; k < kBjStage; ++k) {
             const int r = r0 + 64 * k;
-            if (r < cnt) v[r] = (V)(xdiv ? xv[k] / dv[k] : xv[k]);
+            if (r < cnt) v[r] = (T)(xdiv ? xv[k] / dv[k] : xv[k]);
         }
     }
     wave_lds_order();
     if (over != 0.) return;
-    bj_sweep<T, V, false>(v, vd, nl, lpl, val_l + kBjWin * sl, col_l + kBjWin / 2 * sl, row_l + sl, nullptr);
-    bj_sweep<T, V, true>(v, vd, nu, lpu, val_u + kBjWin * su, col_u + kBjWin / 2 * su, row_u + su, dinv + su);
+    bj_sweep<T, W, PAIR, false>(v, vd, maxrows, nl, lpl, val_l + W * sl, col_l + W / 2 * sl, row_l + sl, nullptr);
+    bj_sweep<T, W, PAIR, true>(v, vd, maxrows, nu, lpu, val_u + W * su, col_u + W / 2 * su, row_u + su, dinv + su);
     const int olo = own[2 * b], ohi = own[2 * b + 1];
     double q = 0.;
     for (int r0 = olo + threadIdx.x; r0 < ohi; r0 += 64 * kBjStage) {
@@ -2437,13 +2451,11 @@ static int build_one(fvp_csr *A, const std::vector<int> &diag, const std::vector
     return 0;
 }
 
-// The solve's packed layout for the blocks roff, bia, bja, bdiag (as in factor_tables), rows_l their rows in the factorisation's order
-static int build_pack(BjPack &P, int nb, const std::vector<int> &roff, const std::vector<int> &bia,
-                      const std::vector<unsigned short> &bja, const std::vector<int> &bdiag,
-                      const std::vector<unsigned short> &rows_l) {
+// The solve's packed layout with W entries to a lane, S to a slot; maxrows: of any block
+static int build_pack(BjPack &P, int W, int S, int nb, int maxrows, const BjTables &t) {
+    const std::vector<int> &roff = t.roff, &bia = t.bia, &bdiag = t.bdiag;
+    const std::vector<unsigned short> &bja = t.bja, &rows_l = t.rows;
     const int total = roff[nb];
-    constexpr int W = kBjWin;
-    P.several = false;
     std::vector<int> lev;
     std::vector<uint4> out(total, make_uint4(0u, 0u, 0u, 0u));  // by row at first, then by slot of L's level order
     std::vector<unsigned> place;
@@ -2452,7 +2464,7 @@ static int build_pack(BjPack &P, int nb, const std::vector<int> &roff, const std
         int first;      // in `order`
         bool main;
     };
-    std::vector<int> order, at, count, step;
+    std::vector<int> order, at, count, step, by, single, pair;
     std::vector<Slot> slots;
     for (int tri = 0; tri < 2; ++tri) {
         std::vector<unsigned> col;
@@ -2466,7 +2478,7 @@ static int build_pack(BjPack &P, int nb, const std::vector<int> &roff, const std
             order.clear();
             slots.clear();
             step.clear();
-            // rows in dependency order: the row's entries by level, the last W in its own
+            // rows in dependency order: the row's entries by level, the last S in its own
             // slot; a row of further slots waits until each can precede the next
             for (int q = 0; q < cnt; ++q) {
                 const int r = tri ? cnt - 1 - q : q, i = base + r;
@@ -2474,7 +2486,7 @@ static int build_pack(BjPack &P, int nb, const std::vector<int> &roff, const std
                 const int f = (int)order.size();
                 for (int k = 0; k < n; ++k) order.push_back(k0 + k);
                 int l = 0;
-                if (n > W)  // few entries: by insertion
+                if (n > S)  // few entries: by insertion
                     for (int k = 1; k < n; ++k) {
                         const int e = order[f + k], le = lev[bja[e]];
                         int j = k;
@@ -2482,35 +2494,35 @@ static int build_pack(BjPack &P, int nb, const std::vector<int> &roff, const std
                         order[f + j] = e;
                     }
                 for (int k = 0; k < n; ++k) l = std::max(l, lev[bja[order[f + k]]] + 1);
-                for (int j = 1, e = n - W; e > 0; ++j, e -= W) l = std::max(l, lev[bja[order[f + e - 1]]] + 1 + j);
+                for (int j = 1, e = n - S; e > 0; ++j, e -= S) l = std::max(l, lev[bja[order[f + e - 1]]] + 1 + j);
                 lev[r] = l;
-                slots.push_back({r, std::min(n, W), f + std::max(0, n - W), true});
+                slots.push_back({r, std::min(n, S), f + std::max(0, n - S), true});
                 step.push_back(l);
             }
             int nl = 0;
             for (int s : step) nl = std::max(nl, s + 1);
             count.assign(nl + 1, 0);
-            for (int s : step) ++count[s];
+            for (int q = 0; q < cnt; ++q) count[step[q]] += slots[q].n > W ? 2 : 1;
             for (int q = 0; q < cnt; ++q) {  // the further slots, where there is room
                 const Slot m = slots[q];
                 const int r = m.row, i = base + r, n = tri ? bia[i + 1] - bdiag[i] - 1 : bdiag[i] - bia[i];
                 int hi = step[q];
-                for (int e = n - W; e > 0; e -= W) {
-                    const int f0 = m.first - (n - W) + std::max(0, e - W), ne = std::min(e, W);
+                for (int e = n - S; e > 0; e -= S) {
+                    const int f0 = m.first - (n - S) + std::max(0, e - S), ne = std::min(e, S), lanes = ne > W ? 2 : 1;
                     // not before its rows are final, nor so early that the slots before it are
                     int lo = lev[bja[order[f0 + ne - 1]]] + 1;
-                    for (int k = e - W, j = 1; k > 0; k -= W, ++j)
-                        lo = std::max(lo, lev[bja[order[m.first - (n - W) + k - 1]]] + 1 + j);
-                    int best = hi - 1;  // the latest level with a free lane in its last piece
+                    for (int k = e - S, j = 1; k > 0; k -= S, ++j)
+                        lo = std::max(lo, lev[bja[order[m.first - (n - S) + k - 1]]] + 1 + j);
+                    int best = hi - 1;  // the latest level with free lanes in its last piece
                     for (int s = hi - 1; s >= lo; --s)
-                        if (count[s] % 64) { best = s; break; }
+                        if (count[s] % 64 && count[s] % 64 + lanes <= 64) { best = s; break; }
                     hi = best;
                     slots.push_back({r, ne, f0, false});
                     step.push_back(hi);
-                    ++count[hi];
+                    count[hi] += lanes;
                 }
             }
-            // level by level, pieces of at most 64
+            // level by level, pieces of at most 64 lanes, slots of two lanes first
             at.assign(nl + 1, 0);
             for (int l = 0; l < nl; ++l) at[l + 1] = at[l] + count[l];
             const int s0 = (int)srow.size();
@@ -2518,26 +2530,33 @@ static int build_pack(BjPack &P, int nb, const std::vector<int> &roff, const std
                 for (int p = at[l]; p < at[l + 1]; p += 64) sp.push_back(s0 + std::min(p + 64, at[l + 1]));
             sb[b + 1] = (int)sp.size() - 1;
             levmax = std::max(levmax, sb[b + 1] - sb[b]);
-            srow.resize(s0 + slots.size());
+            srow.resize(s0 + at[nl]);
             col.resize((size_t)srow.size() * (W / 2));
-            std::vector<int> by(slots.size());
+            by.assign(slots.size(), 0);
+            single.assign(at.begin(), at.end());
+            for (size_t q = 0; q < slots.size(); ++q)
+                if (slots[q].n > W) single[step[q]] += 2;
+            pair = at;
             for (size_t q = 0; q < slots.size(); ++q) {
                 const Slot &m = slots[q];
-                const int sl = s0 + at[step[q]]++;
+                const bool two = m.n > W;
+                const int in = two ? pair[step[q]] : single[step[q]], sl = s0 + in;
+                (two ? pair : single)[step[q]] += two ? 2 : 1;
                 by[q] = sl;
                 srow[sl] = (unsigned short)m.row;
-                unsigned short c[W];
-                for (int k = 0; k < W; ++k) c[k] = k < m.n ? bja[order[m.first + k]] : (unsigned short)m.row;
-                for (int k = 0; k < W; k += 2) col[(size_t)sl * (W / 2) + k / 2] = c[k] | (unsigned)c[k + 1] << 16;
+                if (two) srow[sl + 1] = (unsigned short)(maxrows + (in + 1 - at[step[q]]) % 64);
+                for (int k = 0; k < (two ? S : W); k += 2) {
+                    auto c = [&](int k) { return (unsigned)(k < m.n ? bja[order[m.first + k]] : m.row); };
+                    col[(size_t)sl * (W / 2) + k / 2] = c(k) | c(k + 1) << 16;
+                }
                 if (m.main) (tri ? out[base + m.row].y : out[base + m.row].x) = (unsigned)(sl - s0);
             }
             // rows of several slots in either triangle: each entry's place
             for (size_t q = 0; q < slots.size(); ++q) {
                 const Slot &m = slots[q];
                 const int i = base + m.row, len = bia[i + 1] - bia[i];
-                const bool several = std::max(bdiag[i] - bia[i], bia[i + 1] - bdiag[i] - 1) > W;
+                const bool several = std::max(bdiag[i] - bia[i], bia[i + 1] - bdiag[i] - 1) > S;
                 if (!several) continue;
-                P.several = true;
                 if (!out[i].w) {
                     out[i].w = (unsigned)place.size() + 1;
                     place.resize(place.size() + len, 0);
@@ -2558,6 +2577,7 @@ static int build_pack(BjPack &P, int nb, const std::vector<int> &roff, const std
             for (int sl = roff[b]; sl < roff[b + 1]; ++sl) by[sl] = out[roff[b] + rows_l[sl]];
         if (P.out.upload(by.data(), by.size()) || P.place.upload(place.data(), place.size())) return -1;
     }
+    P.win = W;
     return 0;
 }
 
@@ -2621,8 +2641,13 @@ static int build_bj(fvp_csr *A) {
     const int n = A->n, BS = A->bs;
     const bool given = !A->bstart.empty();
     const int nb = given ? (int)A->bstart.size() - 1 : (n + BS - 1) / BS;
-    std::vector<int> roff(nb + 1, 0), rowid, own(2 * (size_t)nb), bia(1, 0), bsrc, bdiag;
-    std::vector<unsigned short> bja;
+    A->tables.reset();
+    auto tables = std::make_unique<BjTables>();
+    std::vector<int> &roff = tables->roff, &bia = tables->bia, &bdiag = tables->bdiag;
+    std::vector<unsigned short> &bja = tables->bja, &rows_l = tables->rows;
+    roff.assign(nb + 1, 0);
+    bia.assign(1, 0);
+    std::vector<int> rowid, own(2 * (size_t)nb), bsrc;
     std::vector<int> stamp(n, -1), loc(n, 0), ext, frontier, next;
     for (int b = 0; b < nb; ++b) {
         const int lo = given ? A->bstart[b] : b * BS, hi = given ? A->bstart[b + 1] : std::min(n, lo + BS);
@@ -2664,14 +2689,17 @@ static int build_bj(fvp_csr *A) {
     }
     const int total = roff[nb];
     std::vector<int> blev_l(nb + 1, 0), lptr_l(1, 0);
-    std::vector<unsigned short> rows_l(total);
+    rows_l.resize(total);
     std::vector<int> lev;
-    int maxnz = 0, maxrow = 0, maxrows = 0;
+    int maxnz = 0, maxrow = 0, maxrows = 0, longest = 0;
     for (int b = 0; b < nb; ++b) {
         const int base = roff[b], cnt = roff[b + 1] - base;
         maxrows = std::max(maxrows, cnt);
         maxnz = std::max(maxnz, bia[base + cnt] - bia[base]);
-        for (int r = 0; r < cnt; ++r) maxrow = std::max(maxrow, bia[base + r + 1] - bia[base + r]);
+        for (int i = base; i < base + cnt; ++i) {
+            maxrow = std::max(maxrow, bia[i + 1] - bia[i]);
+            longest = std::max({longest, bdiag[i] - bia[i], bia[i + 1] - bdiag[i] - 1});
+        }
         // the factorisation's levels
         lev.assign(cnt, 0);
         int nl = 0;
@@ -2698,13 +2726,11 @@ static int build_bj(fvp_csr *A) {
         A->b_own.upload(own.data(), own.size()) || (!ident && A->b_rowid.upload(rowid.data(), total)))
         return -1;
     if (ident) A->b_rowid.release();
-    A->b_lu.release();
-    A->b_lu32.release();
-    if (build_pack(A->pack, nb, roff, bia, bja, bdiag, rows_l) ||
-        factor_tables(A->fac, nb, roff, bia, bja, bdiag, rows_l, maxrow))
-        return -1;
-    A->val_l.release(); A->val_u.release(); A->dinv.release();
-    A->val32_l.release(); A->val32_u.release(); A->dinv32.release();
+    if (factor_tables(A->fac, nb, roff, bia, bja, bdiag, rows_l, maxrow)) return -1;
+    A->b_lu.release(); A->val_l.release(); A->val_u.release(); A->dinv.release();
+    A->b_lu32.release(); A->val32_l.release(); A->val32_u.release(); A->dinv32.release();
+    A->pack[0].win = A->pack[1].win = 0;
+    A->b_longest = longest;
     A->b_maxnz = maxnz;
     A->b_maxrows = maxrows;
     if (hipDeviceGetAttribute(&A->lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, A->device) != hipSuccess)
@@ -2717,8 +2743,18 @@ static int build_bj(fvp_csr *A) {
         if (factor_pieces(A->fp[f32], nb, blev_l, lptr_l, pieces, maxnz, A->fac.nc, f32 ? sizeof(float) : sizeof(double),
                           A->lds_max))
             return -1;
+    A->tables = std::move(tables);
     A->nblk = nb;
     A->bj = true;
+    return 0;
+}
+
+// A precision's layout of the solve
+static int bj_layout(fvp_csr *A, bool f32) {
+    const int w = f32 && A->b_longest > 4;
+    if (A->pack[w].win) return 0;
+    if (build_pack(A->pack[w], w ? 6 : 4, w ? 12 : 4, A->nblk, A->b_maxrows, *A->tables)) return -1;
+    if (A->b_longest <= 4 || A->pack[!w].win) A->tables.reset();
     return 0;
 }
 
@@ -2947,8 +2983,8 @@ static void bj_factor_attrs(int lds_max) {
 static void bj_attrs(int lds_max) {
     bj_factor_attrs<double, 1>(lds_max); bj_factor_attrs<double, 2>(lds_max); bj_factor_attrs<double, 4>(lds_max);
     bj_factor_attrs<float, 1>(lds_max); bj_factor_attrs<float, 2>(lds_max); bj_factor_attrs<float, 4>(lds_max);
-    for (const void *f : {(const void *)bj_solve<double, double>, (const void *)bj_solve<float, double>,
-                          (const void *)bj_solve<float, float>})
+    for (const void *f : {(const void *)bj_solve<double, 4, false>, (const void *)bj_solve<float, 4, false>,
+                          (const void *)bj_solve<float, 6, true>})
         (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
 }
 
@@ -2971,21 +3007,20 @@ static int precon_build_impl(fvp_csr *A, int type) {
         if (rc) { A->ptype = -1; return rc; }
     } else if (type == FVP_PRECON_BJILU0 || type == FVP_PRECON_BJILU0_F32) {
         const bool f32 = type == FVP_PRECON_BJILU0_F32;
-        if (!A->bj) {
-            int rc = build_bj(A);
-            if (rc) { A->ptype = -1; return rc; }
-        }
+        int rc = A->bj ? 0 : build_bj(A);
+        if (!rc) rc = bj_layout(A, f32);
+        if (rc) { A->ptype = -1; return rc; }
         const FacPieces &F = A->fp[f32];
-        const BjPack &P = A->pack;
+        const BjPack &P = A->pack_of(f32);
         // FVP_BJ_FACTOR_MODE 0 / 1 forces values in place / staged where they fit the
         // workgroup: a tuning and test knob
         bool stage = F.staged;
         if (const char *e = getenv("FVP_BJ_FACTOR_MODE")) stage = atoi(e) > 0 && F.lds <= (size_t)A->lds_max;
         A->factor_mode = stage;
         const FactorArgs fa{A->nblk, A->b_roff.p, A->b_ia.p, A->b_src.p, A->a.p, &A->fac, F.lev.p, F.lptr.p, A->flag.p,
-                            FacOut{(unsigned)kBjWin, P.place.p, P.lev_l.p, P.lptr_l.p, P.lev_u.p, P.lptr_u.p},
+                            FacOut{(unsigned)P.win, P.place.p, P.lev_l.p, P.lptr_l.p, P.lev_u.p, P.lptr_u.p},
                             P.out.p, stage ? F.lds : 0, F.most, F.threads};
-        const size_t nl = P.row_l.n * kBjWin, nu = P.row_u.n * kBjWin, nd = P.row_u.n;
+        const size_t nl = P.row_l.n * P.win, nu = P.row_u.n * P.win, nd = P.row_u.n;
         // the packed arrays' padding stays zero: only the factor's entries are written
         auto ensure = [&](auto &lu, auto &vl, auto &vu, auto &vd) {
             if (!lu.p && lu.alloc(A->b_src.n)) return -1;
@@ -3082,21 +3117,19 @@ static int precon_apply_impl(fvp_csr *A, const double *x, double *y, const doubl
     case FVP_PRECON_BJILU0:
     case FVP_PRECON_BJILU0_F32: {
         const bool f64 = A->ptype == FVP_PRECON_BJILU0;
-        const BjPack &P = A->pack;
-        size_t lds = bj_solve_lds(sizeof(double), A->b_maxrows, P.levmax_l, P.levmax_u);
-        const bool v64 = f64 || (P.several && lds <= (size_t)A->lds_max);
-        if (!v64) lds = bj_solve_lds(sizeof(float), A->b_maxrows, P.levmax_l, P.levmax_u);
+        const BjPack &P = A->pack_of(!f64);
+        const size_t lds = bj_solve_lds(f64 ? sizeof(double) : sizeof(float), A->b_maxrows, P.levmax_l, P.levmax_u);
         if (lds > (size_t)A->lds_max) {
             set_error("block-Jacobi ILU(0): a block's solution does not fit the LDS");
             return -1;
         }
-#define FVP_BJ_SOLVE(T, V, VL, VU, DI)                                                                             \
-    bj_solve<T, V><<<A->nblk, 64, lds, s>>>(A->b_roff.p, A->b_rowid.p, A->b_own.p, P.lev_l.p, P.lptr_l.p, VL,      \
+#define FVP_BJ_SOLVE(T, W, PAIR, VL, VU, DI)                                                                       \
+    bj_solve<T, W, PAIR><<<A->nblk, 64, lds, s>>>(A->b_roff.p, A->b_rowid.p, A->b_own.p, P.lev_l.p, P.lptr_l.p, VL,      \
                                             P.col_l.p, P.row_l.p, P.lev_u.p, P.lptr_u.p, VU, P.col_u.p, P.row_u.p, \
                                             DI, A->b_maxrows, x, xdiv, y, yn2, A->skip)
-        if (f64) FVP_BJ_SOLVE(double, double, A->val_l.p, A->val_u.p, A->dinv.p);
-        else if (v64) FVP_BJ_SOLVE(float, double, A->val32_l.p, A->val32_u.p, A->dinv32.p);
-        else FVP_BJ_SOLVE(float, float, A->val32_l.p, A->val32_u.p, A->dinv32.p);
+        if (f64) FVP_BJ_SOLVE(double, 4, false, A->val_l.p, A->val_u.p, A->dinv.p);
+        else if (P.win == 6) FVP_BJ_SOLVE(float, 6, true, A->val32_l.p, A->val32_u.p, A->dinv32.p);
+        else FVP_BJ_SOLVE(float, 4, false, A->val32_l.p, A->val32_u.p, A->dinv32.p);
 #undef FVP_BJ_SOLVE
         break;
     }
@@ -3181,7 +3214,7 @@ extern "C" int fvp_csr_destroy(fvp_csr *A) {
     A->hflag.release();
     A->b_ia.release(); A->b_src.release(); A->b_lu.release(); A->b_lu32.release();
     A->b_roff.release(); A->b_rowid.release(); A->b_own.release(); A->b_zn2.release();
-    A->pack.release(); A->val_l.release();
+    A->pack[0].release(); A->pack[1].release(); A->val_l.release();
     A->val_u.release(); A->dinv.release(); A->val32_l.release(); A->val32_u.release(); A->dinv32.release();
     A->fac.release(); A->ofac.release(); A->otri[0].release(); A->otri[1].release(); A->o_fptr.release();
     A->fp[0].release(); A->fp[1].release();

@@ -1,8 +1,7 @@
-"""The block solve with FP32 factors.  Where a block has rows of more than four entries a
-triangle, which the solve takes in several slots, the solution and the sums are FP64: y is
-the FP64 solution with the FP32 factors, to rounding (1e-12).  Where rows have one slot
-each, or where a block's solution fits the LDS in FP32 only, they are FP32: at most ten
-roundings of 2^-24 a row, growth by the dominant diagonal below 2, five rows deep (1e-5)."""
+"""The block solve with FP32 factors, rows of one lane (up to four or six entries a
+triangle), of two, and of several slots, and blocks of 20480 rows, against the FP64 solution
+with the same factors: at most ten roundings of 2^-24 a row, growth by the dominant diagonal
+below 2, five rows deep (1e-5)."""
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -49,23 +48,20 @@ def _solve(ia, ja, lu, rows, x):
 
 
 @pytest.mark.parametrize("rows", [64, 512])
-@pytest.mark.parametrize("which", ["band of 4", "band of 5", "row of 8 L entries", "row of 9 L entries",
+@pytest.mark.parametrize("which", ["band of 4", "band of 5", "band of 6", "band of 7", "row of 8 L entries",
+                                   "row of 9 L entries",
                                    "row of 17 L entries", "rows of 63 entries", "a chain and rows of 20 entries",
                                    "box"])
 def test_solution_with_the_fp32_factors(which, rows):
     ia, ja, a = _csr(_band(300, int(which[-1])) if which.startswith("band") else SHAPES[which], 5)
     A, x, y = _fp32(ia, ja, a, rows)
     ref = _solve(ia, ja, A.precon_values(len(ja)), rows, x)
-    row = np.repeat(np.arange(len(ia) - 1), np.diff(ia))
-    keep = row // rows == ja // rows
-    several = max(np.bincount(row[keep & (ja < row)]).max(), np.bincount(row[keep & (ja > row)]).max()) > 4
-    tol = 1e-12 if several else 1e-5
-    np.testing.assert_allclose(y, ref, rtol=0, atol=tol * np.abs(ref).max())
+    np.testing.assert_allclose(y, ref, rtol=0, atol=1e-5 * np.abs(ref).max())
 
 
-def test_a_block_whose_solution_fits_in_fp32_only():
+def test_a_block_of_20480_rows():
     # block 0: 4096 rows and, one layer out, four neighbours of each; and a row of 5
-    # entries a triangle.  20480 rows of 8 bytes are past 160 KB of LDS.
+    # entries a triangle
     m = 4096
     hub = np.repeat(np.arange(m), 4)
     P = sp.coo_matrix((np.ones(4 * m + 5), (np.r_[hub, np.full(5, 9)], np.r_[m + np.arange(4 * m), np.arange(5)])),
