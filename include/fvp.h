@@ -316,11 +316,12 @@ int fvp_integrator_get_stats(const fvp_integrator *I, fvp_integrator_stats *st);
 /* ---------------------------------------------------------------------------
  * Launch shape of the residual.  Nodes are processed in tiles of tile_nodes
  * consecutive ids (a power of two in [64, 4096]; default 256, 128 below 65 536
- * nodes, 512 where a tile's node window does not fit the LDS), one workgroup
+ * nodes, 512 where some tile's window of records does not fit), one workgroup
  * per tile; xcd_map = 1 deals consecutive tiles to one XCD (shared L2 for
  * their halos).  Variants: FVP_RESIDUAL_OWNER evaluates each element once, in
- * the tile of its lowest node, from node records staged in LDS (gathered from
- * memory where the tile's window does not fit), with LDS sums and export slots
+ * the tile of its lowest node, from node records staged in LDS (for the whole
+ * mesh gathered from memory if a node touches more than four zones or any tile's
+ * records take more than 78 KB), with LDS sums and export slots
  * for nodes of other tiles, which a node pass adds while it finalises (default;
  * no global atomics); FVP_RESIDUAL_WINDOW
  * stages every tile's node window in LDS and evaluates each element once per
