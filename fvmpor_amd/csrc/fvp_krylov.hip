@@ -49,7 +49,8 @@ struct FactorTab {
     DevBuf<uint4> slot, out;
     DevBuf<unsigned> piv;
     DevBuf<uint2> off;
-    int nc = 1;  // longest row in entries, in units of 16
+    int nc = 1;  // registers of the longest row (16 entries each): 1, 2 or 4
+    bool mostly_long = false;  // more than one row in eight needs four
     void release() { slot.release(); out.release(); piv.release(); off.release(); }
 };
 
@@ -1078,6 +1079,40 @@ struct FacRow {
     unsigned off[2 * kAhead][NC];  // distances, four L entries a word, 0: none
 };
 
+// The registers (1, 2 or 4) that the rows of a wavefront need, uniform: rows of up to 16
+// entries take one, also where others of the matrix have more.  100 000 tridiagonal rows
+// in blocks of 1024 with overlap, FP64 / FP32, us: 737 / 715; with one row of 24 entries
+// 804 / 802 (1096 / 1053 with two registers for every row), of 40 900 / 860 (1654 / 1431).
+template <int NC>
+__device__ __forceinline__ int fac_regs(int len) {
+    if (NC == 1 || !__any(len > kBjGroup)) return 1;
+    return NC == 2 || !__any(len > 2 * kBjGroup) ? 2 : NC;
+}
+
+template <int C0, int C1, typename T, int NC>
+__device__ __forceinline__ void fac_load_part(FacRow<T, NC> &w, uint4 out, int gl, const uint2 *__restrict__ off,
+                                              const FacOut &fo, const T *val) {
+    const int nch = (w.len + kBjGroup - 1) / kBjGroup;
+#pragma unroll
+    for (int c = C0; c < C1; ++c) {
+        const int e = gl + kBjGroup * c;
+        w.at[c] = e < w.d ? out.x * fo.win + e : e > w.d ? out.y * fo.win + (e - w.d - 1) : out.y;
+        if (out.w && e < w.len && e != w.d) w.at[c] = fo.place[out.w - 1 + e];
+    }
+#pragma unroll
+    for (int c = C0; c < C1; ++c) w.a[c] = gl + kBjGroup * c < w.len ? val[w.s0 + gl + kBjGroup * c] : T(0);
+#pragma unroll
+    for (int b = 0; b < kAhead; ++b)
+#pragma unroll
+        for (int c = C0; c < C1; ++c) {
+            const uint2 o = 8 * b < w.d && c < nch ? off[(size_t)(w.tab + b * nch + c) * kBjGroup + gl]
+                                                   : make_uint2(0u, 0u);
+            w.off[2 * b][c] = o.x;
+            w.off[2 * b + 1][c] = o.y;
+        }
+}
+
+// Registers that no row of the wavefront needs (see fac_regs) are left as they are.
 template <typename T, int NC>
 __device__ __forceinline__ void fac_row_load(FacRow<T, NC> &w, uint4 m, uint4 out, int gl,
                                              const unsigned *__restrict__ piv, const uint2 *__restrict__ off,
@@ -1087,94 +1122,80 @@ __device__ __forceinline__ void fac_row_load(FacRow<T, NC> &w, uint4 m, uint4 ou
     w.d = (int)((m.y >> 8) & 0xffu);
     w.tab = m.z;
     w.l0 = m.w;
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-        const int e = gl + kBjGroup * c;
-        w.at[c] = e < w.d ? out.x * fo.win + e : e > w.d ? out.y * fo.win + (e - w.d - 1) : out.y;
-        if (out.w && e < w.len && e != w.d) w.at[c] = fo.place[out.w - 1 + e];
-    }
-    const int nch = (w.len + kBjGroup - 1) / kBjGroup;
-#pragma unroll
-    for (int c = 0; c < NC; ++c) w.a[c] = gl + kBjGroup * c < w.len ? val[w.s0 + gl + kBjGroup * c] : T(0);
+    const int regs = fac_regs<NC>(w.len);
+    fac_load_part<0, 1>(w, out, gl, off, fo, val);
     w.piv = gl < w.d ? piv[w.l0 + gl] : 0u;
-#pragma unroll
-    for (int b = 0; b < kAhead; ++b)
-#pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            const uint2 o = 8 * b < w.d && c < nch ? off[(size_t)(w.tab + b * nch + c) * kBjGroup + gl]
-                                                   : make_uint2(0u, 0u);
-            w.off[2 * b][c] = o.x;
-            w.off[2 * b + 1][c] = o.y;
-        }
+    if constexpr (NC > 1)
+        if (regs > 1) fac_load_part<1, 2>(w, out, gl, off, fo, val);
+    if constexpr (NC > 2)
+        if (regs > 2) fac_load_part<2, NC>(w, out, gl, off, fo, val);
 }
 
 // L entries 4 B .. 4 B + 3 of a row: their u_kj (an entry without one loads the pivot, unused)
-template <int B, typename T, int NC>
-__device__ __forceinline__ void fac_load_u(const FacRow<T, NC> &w, bool wide, const T *val, T (&u)[4][NC]) {
+template <int B, int M, typename T, int NC>
+__device__ __forceinline__ void fac_load_u(const FacRow<T, NC> &w, const T *val, T (&u)[4][M]) {
     constexpr int K0 = 4 * B;
     const unsigned p[4] = {row_bcast<K0>(w.piv), row_bcast<K0 + 1>(w.piv), row_bcast<K0 + 2>(w.piv),
                            row_bcast<K0 + 3>(w.piv)};
 #pragma unroll
     for (int k = 0; k < 4; ++k)
 #pragma unroll
-        for (int c = 0; c < NC; ++c)
-            if (c == 0 || wide) u[k][c] = val[p[k] + ((w.off[B][c] >> (8 * k)) & 0xffu)];
+        for (int c = 0; c < M; ++c) u[k][c] = val[p[k] + ((w.off[B][c] >> (8 * k)) & 0xffu)];
 }
 
 // L entry K: l_ik = a_ik u_kk^-1 (lane K's product, final since only earlier L
 // entries update entry K), then the row's entries that row k has too
-template <int K, typename T, int NC>
-__device__ __forceinline__ void fac_step(FacRow<T, NC> &w, bool wide, T pv, const T (&u)[4][NC]) {
+template <int K, int M, typename T, int NC>
+__device__ __forceinline__ void fac_step(FacRow<T, NC> &w, T pv, const T (&u)[4][M]) {
     const T lik = row_bcast<K>(w.a[0] * pv);
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-        if (c > 0 && !wide) break;
+    for (int c = 0; c < M; ++c) {
         const T t = w.a[c] - lik * u[K & 3][c];
         w.a[c] = (w.off[K / 4][c] & (0xffu << (8 * (K & 3)))) ? t : w.a[c];
     }
 }
 
-template <int B, typename T, int NC>
-__device__ __forceinline__ void fac_chain(FacRow<T, NC> &w, bool wide, T pv, const T (&u)[4][NC]) {
-    fac_step<4 * B>(w, wide, pv, u);
-    fac_step<4 * B + 1>(w, wide, pv, u);
-    fac_step<4 * B + 2>(w, wide, pv, u);
-    fac_step<4 * B + 3>(w, wide, pv, u);
+template <int B, int M, typename T, int NC>
+__device__ __forceinline__ void fac_chain(FacRow<T, NC> &w, T pv, const T (&u)[4][M]) {
+    fac_step<4 * B>(w, pv, u);
+    fac_step<4 * B + 1>(w, pv, u);
+    fac_step<4 * B + 2>(w, pv, u);
+    fac_step<4 * B + 3>(w, pv, u);
 }
 
-// One row, once every row that it uses is final: the u_kj of its first sixteen L
-// entries in one round of loads, then their chain; more L entries one at a time.
-template <typename T, int NC>
-__device__ __forceinline__ void fac_row(FacRow<T, NC> &w, int gl, const unsigned *__restrict__ piv,
-                                        const uint2 *__restrict__ off, const T *val) {
+// One row of up to M registers, once every row that it uses is final: the u_kj of its
+// first sixteen L entries in one round of loads, then their chain; more L entries one at
+// a time.
+template <int M, typename T, int NC>
+__device__ __forceinline__ void fac_row_m(FacRow<T, NC> &w, int gl, const unsigned *__restrict__ piv,
+                                          const uint2 *__restrict__ off, const T *val) {
     // uniform: batches, and entries past the sixteenth, that no row of the wavefront has
     const bool b1 = __any(w.d > 4), b2 = __any(w.d > 8), b3 = __any(w.d > 12);
-    const bool wide = NC > 1 && __any(w.len > kBjGroup);
     const T pv = val[w.piv];
-    T u0[4][NC], u1[4][NC], u2[4][NC], u3[4][NC];
-    fac_load_u<0>(w, wide, val, u0);
-    if (b1) fac_load_u<1>(w, wide, val, u1);
-    if (b2) fac_load_u<2>(w, wide, val, u2);
-    if (b3) fac_load_u<3>(w, wide, val, u3);
-    fac_chain<0>(w, wide, pv, u0);
-    if (b1) fac_chain<1>(w, wide, pv, u1);
-    if (b2) fac_chain<2>(w, wide, pv, u2);
-    if (b3) fac_chain<3>(w, wide, pv, u3);
+    T u0[4][M], u1[4][M], u2[4][M], u3[4][M];
+    fac_load_u<0>(w, val, u0);
+    if (b1) fac_load_u<1>(w, val, u1);
+    if (b2) fac_load_u<2>(w, val, u2);
+    if (b3) fac_load_u<3>(w, val, u3);
+    fac_chain<0>(w, pv, u0);
+    if (b1) fac_chain<1>(w, pv, u1);
+    if (b2) fac_chain<2>(w, pv, u2);
+    if (b3) fac_chain<3>(w, pv, u3);
     if (gl < w.d) w.a[0] *= pv;
-    if (NC > 1 && __any(w.d > 8 * kAhead)) {
+    if (M > 1 && __any(w.d > 8 * kAhead)) {
         const int nch = (w.len + kBjGroup - 1) / kBjGroup;
         for (int k = 8 * kAhead; __any(k < w.d); ++k) {
             const bool in = k < w.d;
             T ak = T(0);
 #pragma unroll
-            for (int c = 0; c < NC; ++c) {
+            for (int c = 0; c < M; ++c) {
                 const T q = __shfl(w.a[c], k & (kBjGroup - 1), kBjGroup);
                 if (c == k / kBjGroup) ak = q;
             }
             const unsigned pk = in ? piv[w.l0 + k] : 0u;
             const T lik = in ? ak * val[pk] : T(0);
 #pragma unroll
-            for (int c = 0; c < NC; ++c) {
+            for (int c = 0; c < M; ++c) {
                 const uint2 o2 = in && c < nch ? off[(size_t)(w.tab + (k >> 3) * nch + c) * kBjGroup + gl]
                                                : make_uint2(0u, 0u);
                 const unsigned o = ((k & 4 ? o2.y : o2.x) >> (8 * (k & 3))) & 0xffu;
@@ -1187,12 +1208,12 @@ __device__ __forceinline__ void fac_row(FacRow<T, NC> &w, int gl, const unsigned
 
 // The factored row to val and to the solve's packed copies, its pivot inverted
 // (a zero pivot sets the flag).
-template <typename T, int NC>
+template <int M, typename T, int NC>
 __device__ __forceinline__ void fac_row_store(const FacRow<T, NC> &w, int gl, T *val, T *__restrict__ vl,
                                               T *__restrict__ vu, T *__restrict__ vd,
                                               int *__restrict__ flag) {
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
+    for (int c = 0; c < M; ++c) {
         const int e = gl + kBjGroup * c;
         T v = w.a[c];
         if (e == w.d) {
@@ -1206,11 +1227,34 @@ __device__ __forceinline__ void fac_row_store(const FacRow<T, NC> &w, int gl, T 
     }
 }
 
+// a wavefront's rows (have: those it has), factored and stored
+template <typename T, int NC>
+__device__ __forceinline__ void fac_row(FacRow<T, NC> &w, bool have, int gl, const unsigned *__restrict__ piv,
+                                        const uint2 *__restrict__ off, T *val, T *__restrict__ vl,
+                                        T *__restrict__ vu, T *__restrict__ vd, int *__restrict__ flag) {
+    const int regs = fac_regs<NC>(w.len);
+    if (regs == 1) {
+        fac_row_m<1>(w, gl, piv, off, val);
+        if (have) fac_row_store<1>(w, gl, val, vl, vu, vd, flag);
+    }
+    if constexpr (NC > 1)
+        if (regs == 2) {
+            fac_row_m<2>(w, gl, piv, off, val);
+            if (have) fac_row_store<2>(w, gl, val, vl, vu, vd, flag);
+        }
+    if constexpr (NC > 2)
+        if (regs == NC) {
+            fac_row_m<NC>(w, gl, piv, off, val);
+            if (have) fac_row_store<NC>(w, gl, val, vl, vu, vd, flag);
+        }
+}
+
 // One workgroup per block b: values ia[roff[b]] ... ia[roff[b + 1]] of lu, the
 // slots of its level pieces (at most TH / kBjGroup each)
 // lptr[blev[b]] ... lptr[blev[b + 1]].  src null: lu already holds the values to
-// factor.  vl, vu, vd: the solve's packed L, U and inverted diagonal.  STAGED: values and piece pointers (npmax + 1 ints) in LDS, so that a
-// barrier waits for LDS accesses only and rows are loaded kRing levels ahead.
+// factor.  vl, vu, vd: the solve's packed L, U and inverted diagonal.  STAGED: values
+// and piece pointers (npmax + 1 ints) in LDS, so that a barrier waits for LDS accesses
+// only and rows are loaded kRing levels ahead.
 template <typename T, int NC, bool STAGED, int TH>
 __global__ void __launch_bounds__(TH, NC == 1 ? 4 : 2) bj_factor(
     const int *__restrict__ roff, const int *__restrict__ ia, const int *__restrict__ src,
@@ -1272,10 +1316,7 @@ __global__ void __launch_bounds__(TH, NC == 1 ? 4 : 2) bj_factor(
         for (int lb = 0; lb < nl; lb += kRing) {
 #pragma unroll
             for (int q = 0; q < kRing; ++q) {
-                if (__any(have[q])) {
-                    fac_row(w[q], gl, piv, off, val);
-                    if (have[q]) fac_row_store(w[q], gl, val, vl, vu, vd, flag);
-                }
+                if (__any(have[q])) fac_row(w[q], have[q], gl, piv, off, val, vl, vu, vd, flag);
                 fac_row_load(w[q], m[q], o[q], gl, piv, off, fo, val);
                 have[q] = have1[q];
                 const int sl = slot_of(lb + q + 2 * kRing, have1[q]);
@@ -1296,10 +1337,7 @@ __global__ void __launch_bounds__(TH, NC == 1 ? 4 : 2) bj_factor(
             fac_row_load(nx, m1, o1, gl, piv, off, fo, val);
             const int sl = slot_of(l + 2, have2);
             const uint4 m2 = slot[sl], o2 = sout[sl];
-            if (__any(have)) {
-                fac_row(w, gl, piv, off, val);
-                if (have) fac_row_store(w, gl, val, vl, vu, vd, flag);
-            }
+            if (__any(have)) fac_row(w, have, gl, piv, off, val, vl, vu, vd, flag);
             __threadfence_block();
             __syncthreads();
             w = nx;
@@ -2358,6 +2396,9 @@ static int factor_tables(FactorTab &F, int nb, const std::vector<int> &roff, con
     if (piv.empty()) piv.push_back(0u);
     if (off.empty()) off.resize(8 * kBjGroup, (unsigned char)0);
     F.nc = maxrow <= kBjGroup ? 1 : maxrow <= 2 * kBjGroup ? 2 : 4;
+    long longs = 0;
+    for (int i = 0; i < total; ++i) longs += bia[i + 1] - bia[i] > 2 * kBjGroup;
+    F.mostly_long = 8 * longs > total;
     return F.slot.upload(slot.data(), slot.size()) || F.piv.upload(piv.data(), piv.size()) ||
            F.off.upload(reinterpret_cast<const uint2 *>(off.data()), off.size() / 8);
 }
@@ -2597,22 +2638,24 @@ static std::array<int, 5> most_pieces(int nb, const std::vector<int> &blev, cons
 
 // The factorisation's levels (blev per block into lptr) in pieces, at the cheapest width
 static int factor_pieces(FacPieces &F, int nb, const std::vector<int> &blev, const std::vector<int> &lptr,
-                         const std::array<int, 5> &pieces, int maxnz, int nc, size_t vb, int lds_max) {
+                         const std::array<int, 5> &pieces, int maxnz, const FactorTab &tab, size_t vb, int lds_max) {
     static_assert(sizeof(kFacThreads) == 5 * sizeof(int) && kFacThreads[0] / kBjGroup == 64 && kFacThreads[4] / kBjGroup == 4);
+    const int nc = tab.nc;
     double best = 1e300;
     const char *given = getenv("FVP_BJ_FACTOR_THREADS");  // forces the threads: a tuning and test knob
     F.threads = 0;
     for (int w = 0; w < 5; ++w) {
         const int th = kFacThreads[w], most = pieces[w];
         if (given && (nc > 1 ? std::min(atoi(given), 512) : atoi(given)) != th) continue;
-        // Values staged in LDS wherever a block fits (rows past 32 entries in FP64
-        // spill registers in that form and stay in place).  Whole builds, staged
-        // against in place: 67 / 75 us (276 blocks of 512 rows, FP32), 200 / 307
+        // Values staged in LDS wherever a block fits, but not where many FP64 rows have
+        // more than 32 entries: four registers a row spill in that form.  Whole builds,
+        // staged against in place: 67 / 75 us (276 blocks of 512 rows, FP32), 200 / 307
         // (1024 with one overlap layer, FP32), 323 / 365 (the same, FP64), 517 / 549
         // (1000 blocks of 1024 with overlap, FP32); at worst 91 / 83 (276 blocks of
-        // 512, FP64), all with 512 threads.
+        // 512, FP64), all with 512 threads; FP64, one row of 41 among tridiagonal ones,
+        // blocks of 1024 with overlap, 900 / 1142; all of 41, blocks of 64, 436 / 353.
         const size_t lds = (size_t)maxnz * vb + 8 * (size_t)((most + 2) / 2);
-        const bool staged = lds <= (size_t)lds_max && !(nc == 4 && vb == 8);
+        const bool staged = lds <= (size_t)lds_max && !(vb == 8 && tab.mostly_long);
         const double cost = fac_cost(th, nc, vb, nb, maxnz, staged ? lds : 0, lds_max, most);
         if (cost >= best) continue;
         best = cost;
@@ -2740,7 +2783,7 @@ static int build_bj(fvp_csr *A) {
     bj_attrs(A->lds_max);
     const std::array<int, 5> pieces = most_pieces(nb, blev_l, lptr_l);
     for (int f32 = 0; f32 < 2; ++f32)
-        if (factor_pieces(A->fp[f32], nb, blev_l, lptr_l, pieces, maxnz, A->fac.nc, f32 ? sizeof(float) : sizeof(double),
+        if (factor_pieces(A->fp[f32], nb, blev_l, lptr_l, pieces, maxnz, A->fac, f32 ? sizeof(float) : sizeof(double),
                           A->lds_max))
             return -1;
     A->tables = std::move(tables);
